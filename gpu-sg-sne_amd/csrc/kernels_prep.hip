@@ -26,176 +26,276 @@ namespace sgt {
 namespace {
 
 // ---- exact kNN -----------------------------------------------------------
-// Work-group tile: 64 queries x 32 references; 256 threads each own a 4x2
-// micro-tile of (query, reference) distances accumulated over the dimensions
-// in order with fma(diff, diff, acc).  Candidates below a query's current
-// worst key (distance, index) are queued in LDS and merged by one thread per
-// query into a max-heap of k entries kept in global memory.  Queries are the
-// slots [0, nq): slot s is point qlist[s] (point s without a list); heaps are
-// indexed by slot.
-constexpr int kKnnQ = 64;
-constexpr int kKnnR = 32;
+// Two kernels over a slab of query slots [0, nq) (slot s is point qlist[s],
+// point s without a list): the FP64 distances of every (slot, point) pair,
+// then per slot the k smallest (distance, index) keys.
+//
+// Distances: a 256-thread work-group owns a tile of 16 RQ queries x 16 RR
+// references, each thread an RQ x RR micro-tile whose sums run over the
+// dimensions in order, acc = fma(diff, diff, acc) (zero-padded dimensions add
+// an exact 0), with 16 dimensions of the tile staged in LDS and the next 16 in
+// flight.  Bound by FP64 vector issue, two operations per pair and dimension.
+// The squared difference does not depend on which point is subtracted from
+// which, so when the slab holds every point in order the tiles below the
+// diagonal are not computed: tile (a, b) also writes (b, a).
 constexpr int kKnnDC = 16;  // dimensions staged per round
 constexpr int kKnnThreads = 256;
+constexpr int kKnnMaxK = 2048;
 
-__device__ __forceinline__ bool key_less(double da, int ia, double db, int ib) {
-  return da < db || (da == db && ia < ib);
+template <int RQ, int RR>
+__global__ __launch_bounds__(kKnnThreads) void knn_dist_kernel(const double *__restrict__ X, int n, int dim,
+                                                               const int *__restrict__ qlist, int s0, int nq,
+                                                               int mirror, double *__restrict__ dist) {
+  constexpr int TQ = 16 * RQ, TR = 16 * RR;
+  constexpr int LQ = TQ * kKnnDC / kKnnThreads, LR = TR * kKnnDC / kKnnThreads;
+  static_assert(RQ % 2 == 0 && RR % 2 == 0 && LQ >= 1 && LR >= 1, "micro-tiles of pairs");
+  if (mirror && (int)blockIdx.x < (int)blockIdx.y) return;  // square tiles: the mirrored one writes it
+  __shared__ double2 qs2[kKnnDC][TQ / 2 + 1], rs2[kKnnDC][TR / 2 + 1];
+  double *qs = reinterpret_cast<double *>(qs2), *rs = reinterpret_cast<double *>(rs2);
+  constexpr int SQ = TQ + 2, SR = TR + 2;  // doubles per staged dimension
+  const int q0 = blockIdx.y * TQ, r0 = blockIdx.x * TR;
+  const int tid = threadIdx.x;
+  const int tq = tid >> 4, tr = tid & 15;  // queries 2 tq + 32 a, references 2 tr + 32 b (and the next)
+  // this thread's share of a staged round: dimension tid % 16 of rows tid / 16 + 16 u
+  const int ll = tid & 15;
+  const double *qp[LQ], *rp[LR];
+#pragma unroll
+  for (int u = 0; u < LQ; ++u) {
+    const int sl = q0 + (tid >> 4) + 16 * u;
+    const int q = sl < nq ? (qlist ? qlist[s0 + sl] : s0 + sl) : -1;
+    qp[u] = q >= 0 ? X + (size_t)q * dim : nullptr;
+  }
+#pragma unroll
+  for (int u = 0; u < LR; ++u) {
+    const int r = r0 + (tid >> 4) + 16 * u;
+    rp[u] = r < n ? X + (size_t)r * dim : nullptr;
+  }
+  double qb[LQ], rb[LR];
+  auto load = [&](int l0) {
+    const int l = l0 + ll;
+#pragma unroll
+    for (int u = 0; u < LQ; ++u) qb[u] = (qp[u] && l < dim) ? qp[u][l] : 0.0;
+#pragma unroll
+    for (int u = 0; u < LR; ++u) rb[u] = (rp[u] && l < dim) ? rp[u][l] : 0.0;
+  };
+  double acc[RQ][RR];
+#pragma unroll
+  for (int a = 0; a < RQ; ++a)
+#pragma unroll
+    for (int b = 0; b < RR; ++b) acc[a][b] = 0.0;
+  load(0);
+  for (int l0 = 0; l0 < dim; l0 += kKnnDC) {
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < LQ; ++u) qs[ll * SQ + (tid >> 4) + 16 * u] = qb[u];
+#pragma unroll
+    for (int u = 0; u < LR; ++u) rs[ll * SR + (tid >> 4) + 16 * u] = rb[u];
+    __syncthreads();
+    if (l0 + kKnnDC < dim) load(l0 + kKnnDC);
+#pragma unroll 2
+    for (int d = 0; d < kKnnDC; ++d) {
+      double qv[RQ], rv[RR];
+#pragma unroll
+      for (int a = 0; a < RQ; a += 2) {
+        const double2 v = qs2[d][tq + 8 * a];
+        qv[a] = v.x;
+        qv[a + 1] = v.y;
+      }
+#pragma unroll
+      for (int b = 0; b < RR; b += 2) {
+        const double2 v = rs2[d][tr + 8 * b];
+        rv[b] = v.x;
+        rv[b + 1] = v.y;
+      }
+#pragma unroll
+      for (int a = 0; a < RQ; ++a)
+#pragma unroll
+        for (int b = 0; b < RR; ++b) {
+          const double df = qv[a] - rv[b];
+          acc[a][b] = fma(df, df, acc[a][b]);
+        }
+    }
+  }
+#pragma unroll
+  for (int a = 0; a < RQ; ++a) {
+    const int sl = q0 + 2 * tq + 16 * (a & ~1) + (a & 1);
+#pragma unroll
+    for (int b = 0; b < RR; ++b) {
+      const int r = r0 + 2 * tr + 16 * (b & ~1) + (b & 1);
+      if (sl < nq && r < n) {
+        dist[(size_t)sl * n + r] = acc[a][b];
+        if (mirror) dist[(size_t)r * n + sl] = acc[a][b];
+      }
+    }
+  }
 }
 
-__global__ __launch_bounds__(kKnnThreads) void knn_kernel(const double *__restrict__ X, int n,
-                                                          int dim, int k, double *__restrict__ hd,
-                                                          int *__restrict__ hi, const int *__restrict__ qlist,
-                                                          int nq) {
-  __shared__ double qs[kKnnDC][kKnnQ + 1];
-  __shared__ double rs[kKnnDC][kKnnR + 1];
-  __shared__ double qd[kKnnQ][kKnnR];
-  __shared__ int qi[kKnnQ][kKnnR];
-  __shared__ int qcnt[kKnnQ];
-  __shared__ double thr_d[kKnnQ];
-  __shared__ int thr_i[kKnnQ];
-  __shared__ int qid[kKnnQ];  // point of each slot (-1: none)
-
-  const int q0 = blockIdx.x * kKnnQ;
-  const int tid = threadIdx.x;
-  const int tq = tid >> 4;   // 0..15 -> queries tq*4 .. tq*4+3
-  const int tr = tid & 15;   // 0..15 -> references tr + 16*c
-  if (tid < kKnnQ) {
-    qcnt[tid] = 0;
-    thr_d[tid] = INFINITY;
-    thr_i[tid] = INT_MAX;
-    const int slot = q0 + tid;
-    qid[tid] = slot < nq ? (qlist ? qlist[slot] : slot) : -1;
-    if (slot < nq)
-      for (int e = 0; e < k; ++e) {
-        hd[(size_t)slot * k + e] = INFINITY;
-        hi[(size_t)slot * k + e] = INT_MAX;
+// Ascending bitonic sort of P2 (a power of two) (key, index) pairs in LDS by
+// the key, then the index; every thread of the work-group calls it.
+__device__ void sort_keys(unsigned long long *key, int *id, int P2) {
+  for (int size = 2; size <= P2; size <<= 1)
+    for (int stride = size >> 1; stride > 0; stride >>= 1) {
+      __syncthreads();
+      for (int t = threadIdx.x; t < P2 / 2; t += blockDim.x) {
+        const int i = 2 * stride * (t / stride) + (t & (stride - 1)), j = i + stride;
+        const bool up = (i & size) == 0;
+        const unsigned long long a = key[i], b = key[j];
+        const int ia = id[i], ib = id[j];
+        const bool a_after_b = b < a || (b == a && ib < ia);
+        if (a_after_b == up) {
+          key[i] = b;
+          key[j] = a;
+          id[i] = ib;
+          id[j] = ia;
+        }
       }
+    }
+  __syncthreads();
+}
+
+// The k smallest (distance, index) keys of each slot's row of distances, in
+// ascending order after the point itself; one work-group per slot.  Distances
+// are non-negative, so their bits order as they do; NaN is no neighbour, and a
+// row left short ends in (infinity, INT_MAX).  The row is narrowed by
+// histograms of 2048 equal ranges of the key between the bounds of the k-th
+// smallest, until at most CAP keys lie at or below the upper bound; those are
+// sorted.  When the keys tied at the k-th smallest are too many for that, the
+// ones of lowest index are taken in index order.  A row costs three passes
+// over it (bounds, one histogram, collection) unless its keys crowd.
+constexpr int kSelBins = 2048;
+
+template <int CAP>
+__global__ __launch_bounds__(kKnnThreads) void knn_select_kernel(const double *__restrict__ dist, int n, int k,
+                                                                 const int *__restrict__ qlist, int s0,
+                                                                 int32_t *__restrict__ I, double *__restrict__ D) {
+  __shared__ unsigned long long key[CAP];
+  __shared__ int id[CAP];
+  __shared__ int hist[kSelBins];
+  __shared__ unsigned long long wlo[kKnnThreads / 64], whi[kKnnThreads / 64];
+  __shared__ int wcnt[kKnnThreads / 64];
+  __shared__ int total, pick_bin, pick_below;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int q = qlist ? qlist[s0 + blockIdx.x] : s0 + (int)blockIdx.x;
+  const unsigned long long *row = reinterpret_cast<const unsigned long long *>(dist) + (size_t)blockIdx.x * n;
+  constexpr unsigned long long kInf = 0x7FF0000000000000ull;
+  // bounds and count of the row's keys
+  unsigned long long lo = ~0ull, hi = 0;
+  int cnt = 0;
+  for (int r = tid; r < n; r += kKnnThreads) {
+    const unsigned long long u = row[r];
+    if (u <= kInf && r != q) {
+      lo = u < lo ? u : lo;
+      hi = u > hi ? u : hi;
+      ++cnt;
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const unsigned long long a = __shfl_xor(lo, o, 64), b = __shfl_xor(hi, o, 64);
+    lo = a < lo ? a : lo;
+    hi = b > hi ? b : hi;
+    cnt += __shfl_xor(cnt, o, 64);
+  }
+  if (lane == 0) {
+    wlo[w] = lo;
+    whi[w] = hi;
+    wcnt[w] = cnt;
+  }
+  if (tid == 0) total = 0;
+  __syncthreads();
+  cnt = 0;
+#pragma unroll
+  for (int v = 0; v < kKnnThreads / 64; ++v) {
+    lo = wlo[v] < lo ? wlo[v] : lo;
+    hi = whi[v] > hi ? whi[v] : hi;
+    cnt += wcnt[v];
+  }
+  // narrow [lo, hi] around the k-th smallest key; `below` keys lie under lo
+  int below = 0, ties = 0;  // ties > 0: that many keys equal to hi, lowest indices first
+  if (cnt > CAP)
+    for (;;) {
+      const unsigned long long range = hi - lo;
+      const int bits = 64 - __clzll((long long)(range | 1ull));
+      const int shift = bits > 11 ? bits - 11 : 0;
+      for (int b = tid; b < kSelBins; b += kKnnThreads) hist[b] = 0;
+      __syncthreads();
+      for (int r = tid; r < n; r += kKnnThreads) {
+        const unsigned long long u = row[r];
+        if (u >= lo && u <= hi && u <= kInf && r != q) atomicAdd(&hist[(int)((u - lo) >> shift)], 1);
+      }
+      __syncthreads();
+      if (w == 0) {  // the first bin whose running total reaches k: 32 bins per lane
+        int sum = 0;
+        for (int b = 0; b < kSelBins / 64; ++b) sum += hist[lane * (kSelBins / 64) + b];
+        int pre = sum;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+          const int v = __shfl_up(pre, o, 64);
+          if (lane >= o) pre += v;
+        }
+        const int before = below + pre - sum;
+        const unsigned long long reach = __ballot(before + sum >= k);
+        if (lane == __ffsll((long long)reach) - 1) {
+          int run = before, b = lane * (kSelBins / 64);
+          while (run + hist[b] < k) run += hist[b++];
+          pick_bin = b;
+          pick_below = run;
+        }
+      }
+      __syncthreads();
+      const int b = pick_bin, upto = pick_below + hist[b];
+      below = pick_below;
+      lo += (unsigned long long)b << shift;
+      hi = lo + ((1ull << shift) - 1);
+      __syncthreads();  // pick_bin and hist are rewritten by the next round
+      if (upto <= CAP) break;
+      if (shift == 0) {
+        ties = k - below;
+        break;
+      }
+    }
+  // collect: every key at or below hi, or those under hi and the first ties
+  for (int r = tid; r < n; r += kKnnThreads) {
+    const unsigned long long u = row[r];
+    if (u <= kInf && r != q && (ties ? u < hi : (u <= hi))) {
+      const int pos = atomicAdd(&total, 1);
+      key[pos] = u;
+      id[pos] = r;
+    }
   }
   __syncthreads();
-
-  for (int r0 = 0; r0 < n; r0 += kKnnR) {
-    double acc[4][2];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 2; ++b) acc[a][b] = 0.0;
-    for (int l0 = 0; l0 < dim; l0 += kKnnDC) {
-      for (int idx = tid; idx < kKnnDC * kKnnQ; idx += kKnnThreads) {
-        const int qq = idx / kKnnDC, ll = idx % kKnnDC;
-        const int q = qid[qq], l = l0 + ll;
-        qs[ll][qq] = (q >= 0 && l < dim) ? X[(size_t)q * dim + l] : 0.0;
-        if (qq < kKnnR) {
-          const int r = r0 + qq;
-          rs[ll][qq] = (r < n && l < dim) ? X[(size_t)r * dim + l] : 0.0;
-        }
+  if (ties && w == 0) {
+    int have = total;
+    for (int r = 0; r < n && have < k; r += 64) {
+      const bool eq = r + lane < n && r + lane != q && row[r + lane] == hi;
+      const unsigned long long m = __ballot(eq);
+      const int pos = have + __popcll(m & ((1ull << lane) - 1ull));
+      if (eq && pos < k) {
+        key[pos] = hi;
+        id[pos] = r + lane;
       }
-      __syncthreads();
-      const int lc = min(kKnnDC, dim - l0);
-      for (int ll = 0; ll < lc; ++ll) {
-        double qv[4], rv[2];
-#pragma unroll
-        for (int a = 0; a < 4; ++a) qv[a] = qs[ll][tq * 4 + a];
-#pragma unroll
-        for (int b = 0; b < 2; ++b) rv[b] = rs[ll][tr + 16 * b];
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-#pragma unroll
-          for (int b = 0; b < 2; ++b) {
-            const double df = qv[a] - rv[b];
-            acc[a][b] = fma(df, df, acc[a][b]);
-          }
-      }
-      __syncthreads();
+      have += __popcll(m);
     }
-    // queue candidates
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      const int ql = tq * 4 + a;
-      const int q = qid[ql];
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        const int r = r0 + tr + 16 * b;
-        if (q >= 0 && r < n && r != q && key_less(acc[a][b], r, thr_d[ql], thr_i[ql])) {
-          const int pos = atomicAdd(&qcnt[ql], 1);
-          qd[ql][pos] = acc[a][b];
-          qi[ql][pos] = r;
-        }
-      }
-    }
-    __syncthreads();
-    // merge queued candidates into the heaps (one thread per query)
-    if (tid < kKnnQ) {
-      const int slot = q0 + tid;
-      const int cnt = qcnt[tid];
-      if (slot < nq && cnt > 0) {
-        double *H = hd + (size_t)slot * k;
-        int *HI = hi + (size_t)slot * k;
-        double rd = H[0];
-        int ri = HI[0];
-        for (int c = 0; c < cnt; ++c) {
-          const double cd = qd[tid][c];
-          const int ci = qi[tid][c];
-          if (!key_less(cd, ci, rd, ri)) continue;
-          int pos = 0;
-          for (;;) {
-            const int l = 2 * pos + 1, rr = l + 1;
-            int m = -1;
-            double md = cd;
-            int mi = ci;
-            if (l < k && key_less(md, mi, H[l], HI[l])) { m = l; md = H[l]; mi = HI[l]; }
-            if (rr < k && key_less(md, mi, H[rr], HI[rr])) { m = rr; md = H[rr]; mi = HI[rr]; }
-            if (m < 0) break;
-            H[pos] = md;
-            HI[pos] = mi;
-            pos = m;
-          }
-          H[pos] = cd;
-          HI[pos] = ci;
-          rd = H[0];
-          ri = HI[0];
-        }
-        thr_d[tid] = rd;
-        thr_i[tid] = ri;
-      }
-      qcnt[tid] = 0;
-    }
-    __syncthreads();
+    if (lane == 0) total = have < k ? have : k;
   }
-}
-
-// Heap -> ascending rows with the point itself first (slots as knn_kernel).
-__global__ void knn_finalize_kernel(int nq, int k, double *__restrict__ hd, int *__restrict__ hi,
-                                    const int *__restrict__ qlist, int32_t *__restrict__ I,
-                                    double *__restrict__ D) {
-  const int slot = blockIdx.x * blockDim.x + threadIdx.x;
-  if (slot >= nq) return;
-  const int q = qlist ? qlist[slot] : slot;
-  double *H = hd + (size_t)slot * k;
-  int *HI = hi + (size_t)slot * k;
+  __syncthreads();
+  const int m = total;
+  int P2 = 2;
+  while (P2 < m) P2 <<= 1;
+  for (int t = m + tid; t < P2; t += kKnnThreads) {
+    key[t] = ~0ull;
+    id[t] = INT_MAX;
+  }
+  sort_keys(key, id, P2);
   int32_t *Iq = I + (size_t)q * (k + 1);
   double *Dq = D + (size_t)q * (k + 1);
-  Iq[0] = q;
-  Dq[0] = 0.0;
-  for (int e = k - 1; e >= 0; --e) {
-    Iq[1 + e] = HI[0];
-    Dq[1 + e] = H[0];
-    const double cd = H[e];
-    const int ci = HI[e];
-    int pos = 0;
-    for (;;) {
-      const int l = 2 * pos + 1, rr = l + 1;
-      int m = -1;
-      double md = cd;
-      int mi = ci;
-      if (l < e && key_less(md, mi, H[l], HI[l])) { m = l; md = H[l]; mi = HI[l]; }
-      if (rr < e && key_less(md, mi, H[rr], HI[rr])) { m = rr; md = H[rr]; mi = HI[rr]; }
-      if (m < 0) break;
-      H[pos] = md;
-      HI[pos] = mi;
-      pos = m;
-    }
-    H[pos] = cd;
-    HI[pos] = ci;
+  if (tid == 0) {
+    Iq[0] = q;
+    Dq[0] = 0.0;
+  }
+  for (int t = tid; t < k; t += kKnnThreads) {
+    Iq[1 + t] = t < m ? id[t] : INT_MAX;
+    Dq[1 + t] = t < m ? __longlong_as_double((long long)key[t]) : (double)INFINITY;
   }
 }
 
@@ -1324,19 +1424,40 @@ __global__ void to_double_kernel(const float *__restrict__ in, double *__restric
 
 namespace {
 
-// Exact kNN of the query slots [0, nq) (points qlist[slot], or all points).
+// Exact kNN of the query slots [0, nq) (points qlist[slot], or all points),
+// in slabs of slots whose distances to every point take at most about 512 MB.
+// All points of a matrix that fits one slab (n <= 8192): mirrored tiles of 128
+// x 128.  Lists of up to 256 slots (rows the certificate left) take tiles of
+// 32 x 64, which spread a few rows over the device: 128 x 128 tiles would
+// leave n / 128 work-groups.  Measured: 6007 points of 784 dimensions 1.40 ms
+// for the distances (20 G pair-dimensions/s of the 39 G/s FP64 issue allows)
+// and 0.17 ms for the selection (one work-group per 64 queries with serial
+// heaps: 37.1 ms); the 82 uncertified rows of a 20,011-point 50-D job 0.08 ms
+// (11.5 ms).
+constexpr size_t kKnnSlabBytes = (size_t)1 << 29;
+
 int knn_exact_rows(hipStream_t s, const double *X, int n, int dim, int k, const int *qlist, int nq, int32_t *I,
                    double *D) {
-  double *hd = nullptr;
-  int *hi = nullptr;
-  SGT_HIP(hipMallocAsync((void **)&hd, sizeof(double) * (size_t)nq * k, s));
-  SGT_HIP(hipMallocAsync((void **)&hi, sizeof(int) * (size_t)nq * k, s));
-  knn_kernel<<<div_up(nq, kKnnQ), kKnnThreads, 0, s>>>(X, n, dim, k, hd, hi, qlist, nq);
-  SGT_LAUNCH_CHECK();
-  knn_finalize_kernel<<<div_up(nq, 256), 256, 0, s>>>(nq, k, hd, hi, qlist, I, D);
-  SGT_LAUNCH_CHECK();
-  SGT_HIP(hipFreeAsync(hd, s));
-  SGT_HIP(hipFreeAsync(hi, s));
+  const int slab = (int)std::min<int64_t>(nq, std::max<int64_t>(128, (int64_t)(kKnnSlabBytes / 8 / n) / 128 * 128));
+  const int mirror = !qlist && nq == n && slab == n;
+  const bool few = qlist && nq <= 256;
+  double *dist = nullptr;
+  SGT_HIP(hipMallocAsync((void **)&dist, sizeof(double) * (size_t)slab * n, s));
+  for (int s0 = 0; s0 < nq; s0 += slab) {
+    const int m = std::min(slab, nq - s0);
+    if (few)
+      knn_dist_kernel<2, 4><<<dim3(div_up(n, 64), div_up(m, 32)), kKnnThreads, 0, s>>>(X, n, dim, qlist, s0, m, 0, dist);
+    else
+      knn_dist_kernel<8, 8><<<dim3(div_up(n, 128), div_up(m, 128)), kKnnThreads, 0, s>>>(X, n, dim, qlist, s0, m,
+                                                                                        mirror, dist);
+    SGT_LAUNCH_CHECK();
+    if (k <= 256)
+      knn_select_kernel<512><<<m, kKnnThreads, 0, s>>>(dist, n, k, qlist, s0, I, D);
+    else
+      knn_select_kernel<2 * kKnnMaxK><<<m, kKnnThreads, 0, s>>>(dist, n, k, qlist, s0, I, D);
+    SGT_LAUNCH_CHECK();
+  }
+  SGT_HIP(hipFreeAsync(dist, s));
   return SGTSNE_OK;
 }
 
@@ -1346,7 +1467,7 @@ int knn_begin(hipStream_t s, const double *X, int n, int dim, int k, int32_t *I,
               int *count_host, KnnPending *pend) {
   *pend = KnnPending{};
   SGT_CHECK(n > k && k >= 1 && dim >= 1, SGTSNE_ERR_ARG, "kNN needs n > k >= 1 (n=%d k=%d)", n, k);
-  SGT_CHECK(k <= kKnnR * 64, SGTSNE_ERR_ARG, "k too large");
+  SGT_CHECK(k <= kKnnMaxK, SGTSNE_ERR_ARG, "k too large");
   const bool filter_ok = k + kFiltSlack <= kRerank && dim <= kFiltMaxDp && n >= kFiltQ;
   if (method == SGTSNE_KNN_EXACT_FP64 || (method == SGTSNE_KNN_AUTO && !filter_ok))
     return knn_exact_rows(s, X, n, dim, k, nullptr, n, I, D);  // nothing left for knn_end

@@ -1,0 +1,57 @@
+"""kNN kernels at the edges of their tiles: rows bit for bit against the FP64 oracle."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def sg():
+    import sgtsne_amd
+
+    return sgtsne_amd
+
+
+@pytest.fixture(scope="module")
+def O():
+    from oracle import oracle
+
+    return oracle
+
+
+def _points(n, dim, seed):
+    rng = np.random.default_rng(seed)
+    centres = rng.normal(0, 4, size=(6, dim))
+    return (centres[rng.integers(0, 6, n)] + rng.standard_normal((n, dim))).astype(np.float32)
+
+
+# one point beyond / at / under the 128 x 128 tiles, dimensions around the 16
+# staged at a time, k around the two selection widths
+@pytest.mark.parametrize("n,dim,k", [(2, 1, 1), (127, 16, 126), (128, 17, 40), (129, 1, 3), (257, 15, 256), (300, 130, 257),
+                                     (700, 784, 90), (2100, 5, 2048), (1000, 33, 600)])
+def test_knn_exact_tiles(sg, O, n, dim, k):
+    X = _points(n, dim, n + dim)
+    I, D, fb = sg.knn(X, k, sg.KNN_EXACT_FP64)
+    Io, Do = O.knn_exact(X, k)
+    assert fb == -1 and np.array_equal(I, Io) and np.array_equal(D, Do)
+
+
+@pytest.mark.parametrize("n,distinct,k", [(3000, 2, 90), (3000, 1, 300), (5000, 7, 20)])
+def test_knn_exact_wide_ties(sg, O, n, distinct, k):
+    # far more keys tie at the k-th smallest than the selection sorts
+    X = np.repeat((np.arange(n) % distinct).astype(np.float32)[:, None], 3, axis=1)
+    I, D, _ = sg.knn(X, k, sg.KNN_EXACT_FP64)
+    Io, Do = O.knn_exact(X, k)
+    assert np.array_equal(I, Io) and np.array_equal(D, Do)
+
+
+def test_knn_exact_infinite_points(sg):
+    # a pair with one infinite point is infinitely far (taken by index after
+    # every finite one), a pair of them has no distance (NaN) and is no neighbour
+    X = _points(200, 4, 8)
+    X[[3, 50, 199], 1] = np.inf
+    I, D, _ = sg.knn(X, 198, sg.KNN_EXACT_FP64)
+    far = [3, 50, 199]
+    assert I[0, -2:].tolist() == [3, 50] and np.isinf(D[0, -2:]).all() and np.isfinite(D[0, :-2]).all()
+    near = [i for i in range(200) if i not in far]
+    assert I[3, 1:198].tolist() == near and np.isinf(D[3, 1:]).all() and I[3, 198] == np.iinfo(np.int32).max
