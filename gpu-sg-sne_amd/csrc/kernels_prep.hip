@@ -526,7 +526,10 @@ __global__ void knn_cell_offsets_kernel(const int *__restrict__ cnt, int P, int 
 }
 
 // The reference stream in cell order: slot of sorted position i, its point
-// id (padding slots keep -1 and zero rows) and the id -> slot map.
+// id (padding slots keep -1 and zero values) and the id -> slot map.  Each 16
+// slots are stored as the filter's matrix instructions take them: step st
+// (dimensions 4 st .. 4 st + 3) of slot j, dimension 4 st + g, belongs to lane
+// 16 g + j, and a lane's steps come in pairs, 64 lanes side by side.
 __global__ void knn_ref_scatter_kernel(const float *__restrict__ Xc, int n, int dp,
                                        const int32_t *__restrict__ order, const int32_t *__restrict__ cell,
                                        const int *__restrict__ start, const int *__restrict__ slot0,
@@ -538,8 +541,14 @@ __global__ void knn_ref_scatter_kernel(const float *__restrict__ Xc, int n, int 
   rid[sl] = id;
   rinv[id] = sl;
   const float4 *src = reinterpret_cast<const float4 *>(Xc + (size_t)id * dp);
-  float4 *dst = reinterpret_cast<float4 *>(Xr + (size_t)sl * dp);
-  for (int c4 = 0; c4 < dp / 4; ++c4) dst[c4] = src[c4];
+  float2 *dst = reinterpret_cast<float2 *>(Xr + (size_t)(sl >> 4) * dp * 16) + (sl & 15);
+  for (int h = 0; h < dp / 8; ++h) {
+    const float4 a = src[2 * h], b = src[2 * h + 1];
+    dst[64 * h] = make_float2(a.x, b.x);
+    dst[64 * h + 16] = make_float2(a.y, b.y);
+    dst[64 * h + 32] = make_float2(a.z, b.z);
+    dst[64 * h + 48] = make_float2(a.w, b.w);
+  }
 }
 
 // Bounding sphere of each reference tile (one wave per tile), in the
@@ -728,56 +737,123 @@ __global__ __launch_bounds__(256) void knn_filter_kernel(const float *__restrict
   }
 }
 
-// The same filter with the candidate heaps in LDS (lists of up to kF2MaxKp):
-// 32 queries per work-group (two waves).  A tile's approximate distances go
-// to LDS; each query's candidates of the tile form a 64-bit mask built from
-// wave ballots (16 bits per 16-lane group), and the merge walks the mask in
-// reference order and sifts into the LDS heap.
+// The same filter with the candidate lists in LDS (lists of up to kF2MaxKp).
+// A work-group of four waves owns NQ = 16 QB queries of one frame.  The
+// references come in tiles of 64, 16 to a wave, stored in the order the matrix
+// instructions take them (knn_ref_scatter_kernel), so a wave reads its B
+// operands straight from memory, coalesced, the next tile's in flight, and
+// nothing is staged or transposed in LDS.
 //
-// The references come as tiles of a cell order (see knn_cell_kernel), each
-// tile with a bounding sphere.  A block starts at the tiles around its own
-// queries' (its lists fill with near candidates), then visits the others,
-// 128 at a time, skipping every tile that cannot hold a candidate: with D
-// the distance between the block's and the tile's spheres, every query a and
-// reference b of them have a true distance of at least D, and the filter
-// value of the pair is within 2^-12 S^2 of its squared distance (S = block
-// radius + centre distance + tile radius + R + |c_b - mu|: more than eight
-// times the certificate's error bounds for the rounding of the centred
-// points and the FP32 dot products), so a tile with D^2 - 2^-12 S^2 above
-// every query's current worst key holds no candidate.  Skipped tiles thus
-// leave the lists as a full scan would: the k + kFiltSlack smallest keys.
-constexpr int kF2Q = 32;
+// A query's list is a buffer of CAP (distance, slot) entries in no order and a
+// threshold: a lane appends its pair when the distance is under the threshold
+// (ballots give the places).  Once a list holds more than kTrig entries one
+// wave cuts it back to the kp smallest (a few spare): the threshold is found by
+// bisecting the bits of the distances with ballot counts, and becomes the
+// list's new threshold.  An entry dropped or turned away has kp entries at or
+// below it, so the list always holds kp smallest values, and the ties dropped
+// at the kp-th have that very value: what the certificate needs.  The waves
+// meet once a round (a tile, or two with QB = 1).  An insertion thus costs a
+// few instructions of one wave and a cut about 300 per ~100 insertions; the
+// binary heaps this replaces took one lane log2(kp) dependent LDS round trips
+// per insertion while both waves of the work-group waited.  20,011 points of 50
+// dimensions: 4.09 -> 0.57 ms; a job of 500-8000 points: 1.58 -> 0.12 ms on
+// average; the whole kNN of 1.3M points 2.76 -> 1.15 s.
+//
+// The tiles follow a cell order (see knn_cell_kernel), each with a bounding
+// sphere.  A block starts at the tiles around its own queries' (its lists fill
+// with near candidates), then visits the others in groups, skipping every tile
+// that cannot hold a candidate: with D the distance between the block's and
+// the tile's spheres, every query a and reference b of them have a true
+// distance of at least D, and the filter value of the pair is within 2^-12 S^2
+// of its squared distance (S = block radius + centre distance + tile radius +
+// R + |c_b - mu|: more than eight times the certificate's error bounds for the
+// rounding of the centred points and the FP32 dot products), so a tile with
+// D^2 - 2^-12 S^2 above every query's current threshold holds no candidate.
+// Skipped tiles thus leave the lists as a full scan would: the k + kFiltSlack
+// smallest values.
+constexpr int kF2Q = 32;  // queries of a frame
 constexpr int kF2MaxKp = 128;
 constexpr int kFiltHomeBack = 16;  // tiles visited before a block's own
+constexpr int kTrig = 192;         // entries beyond which a list is cut
+constexpr int kCutSpare = 12;      // entries a cut may leave beyond kp
+static_assert(kF2MaxKp + kCutSpare < kTrig, "a cut list is below the trigger");
 
-// A reference tile shifted into a query block's frame: rt holds
-// fl32(x~ - delta) transposed, and rnp[t] the partial squared norm of the
-// row this thread stored (rows t % 64: two threads cover every row, so a
-// row's norm is rnp[j] + rnp[j + 64]).
-template <int NST>
-__device__ __forceinline__ void tile_store_shift(float *rt, float *rnp, const float4 (&buf)[kFiltR * NST / 128],
-                                                 const float4 (&dl)[kFiltR * NST / 128]) {
-  float ss = 0.0f;
-#pragma unroll
-  for (int u = 0; u < kFiltR * NST / 128; ++u) {
-    const int t = threadIdx.x + u * 128;
-    const int j = t % kFiltR, c4 = t / kFiltR;
-    const float4 v = make_float4(buf[u].x - dl[u].x, buf[u].y - dl[u].y, buf[u].z - dl[u].z, buf[u].w - dl[u].w);
-    float *col = rt + 4 * c4 * kFiltRS + j;
-    col[0] = v.x;
-    col[kFiltRS] = v.y;
-    col[2 * kFiltRS] = v.z;
-    col[3 * kFiltRS] = v.w;
-    ss = fmaf(v.x, v.x, ss);
-    ss = fmaf(v.y, v.y, ss);
-    ss = fmaf(v.z, v.z, ss);
-    ss = fmaf(v.w, v.w, ss);
-  }
-  rnp[threadIdx.x] = ss;
+// Unsigned integers ordered as the floats (none of them NaN), and back.
+__device__ __forceinline__ uint32_t float_order(float f) {
+  const uint32_t u = __float_as_uint(f);
+  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+__device__ __forceinline__ float order_float(uint32_t u) {
+  return __uint_as_float((u & 0x80000000u) ? (u & 0x7FFFFFFFu) : ~u);
 }
 
-// The reference stream of the LDS-heap filter: tiles of kFiltR slots in
-// cell order (Xr rows, -1 ids for padding), their spheres, and the query
+// Cuts a list of c >= kp entries to its smallest: at least kp, at most kp +
+// spare; returns the new count and, in *thr, a value at or below which at
+// least kp of them lie.  One wave; the list's entries must be written.
+template <int CAP>
+__device__ __forceinline__ int cut_list(float *key, int *id, int c, int kp, int spare, int lane, float *thr) {
+  constexpr int E = CAP / 64;
+  uint32_t u[E];
+  int x[E];
+  uint32_t lo = 0xFFFFFFFFu, hi = 0;
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    const int e = lane + 64 * i;
+    u[i] = e < c ? float_order(key[e]) : 0xFFFFFFFFu;  // above every value (not a float's image)
+    x[i] = e < c ? id[e] : -1;
+    if (e < c) {
+      lo = min(lo, u[i]);
+      hi = max(hi, u[i]);
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    lo = min(lo, (uint32_t)__shfl_xor((int)lo, o, 64));
+    hi = max(hi, (uint32_t)__shfl_xor((int)hi, o, 64));
+  }
+  int upto = c;  // entries at or below hi
+  while (lo < hi) {
+    const uint32_t mid = lo + ((hi - lo) >> 1);
+    int m = 0;
+#pragma unroll
+    for (int i = 0; i < E; ++i) m += __popcll(__ballot(u[i] <= mid));
+    if (m >= kp) {
+      hi = mid;
+      upto = m;
+      if (m <= kp + spare) break;
+    } else {
+      lo = mid + 1;
+    }
+  }
+  int tie_room = CAP;  // entries equal to hi that are kept (all, unless they are too many)
+  if (upto > kp + spare) {
+    int under = 0;
+#pragma unroll
+    for (int i = 0; i < E; ++i) under += __popcll(__ballot(u[i] < hi));
+    tie_room = kp - under;
+  }
+  const unsigned long long below = (1ull << lane) - 1ull;
+  int pos0 = 0, tie0 = 0;
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    const unsigned long long tm = __ballot(u[i] == hi);
+    const bool tie = u[i] == hi && tie0 + __popcll(tm & below) < tie_room;
+    tie0 += __popcll(tm);
+    const bool keep = u[i] < hi || tie;
+    const unsigned long long km = __ballot(keep);
+    if (keep) {
+      const int p = pos0 + __popcll(km & below);
+      key[p] = order_float(u[i]);
+      id[p] = x[i];
+    }
+    pos0 += __popcll(km);
+  }
+  *thr = order_float(hi);
+  return pos0;
+}
+
+// The reference stream of the LDS-list filter: tiles of kFiltR slots in
+// cell order (Xr, -1 ids for padding), their spheres, and the query
 // blocks' spheres (centre cb, radius from the queries' norms qa, |c_b - mu|
 // in dn; R the largest |x - mu|).
 struct RefTiles {
@@ -792,197 +868,233 @@ struct RefTiles {
   const int *slot0;     // cell -> its first slot (a tile boundary)
 };
 
-template <int NST>
-__global__ __launch_bounds__(128) void knn_filter_lds_kernel(const RefTiles rf, const float *__restrict__ Xq,
-                                                             const float *__restrict__ qn32,
-                                                             const int32_t *__restrict__ qorder,
-                                                             const float *__restrict__ delta, int n, int kp,
-                                                             float *__restrict__ hd, int *__restrict__ hi) {
-  static_assert((kFiltR * NST) % 128 == 0, "a tile must split evenly over the work-group");
-  extern __shared__ float dyn[];  // heap keys [kF2Q][kp] | heap indices [kF2Q][kp]
-  float *hk = dyn;
-  int *hx = reinterpret_cast<int *>(hk + (size_t)kF2Q * kp);
-  __shared__ float rt[4 * NST * kFiltRS];
-  __shared__ float dist[kF2Q][kFiltR];
-  __shared__ unsigned long long mask[kF2Q];
-  __shared__ float rnp[128];
-  __shared__ float qn[kF2Q];
-  __shared__ int qid[kF2Q];
-  __shared__ unsigned long long skipm[2];
-  __shared__ float sthr;
-  __shared__ double srho;
-
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, g = lane >> 4;
-  const int q0 = blockIdx.x * kF2Q;  // first slot of this query block
+template <int NST, int QB>
+__global__ __launch_bounds__(256) void knn_filter_list_kernel(const RefTiles rf, const float *__restrict__ Xq,
+                                                              const float *__restrict__ qn32,
+                                                              const int32_t *__restrict__ qorder,
+                                                              const float *__restrict__ delta, int n, int kp,
+                                                              float *__restrict__ hd, int *__restrict__ hi) {
+  constexpr int NQ = 16 * QB;
+  constexpr int TPR = QB == 1 ? 2 : 1;       // tiles between the meetings of the waves
+  constexpr int CAP = kTrig + 64 * TPR;      // no list overflows in a round
+  static_assert(NST % 2 == 0 && kF2Q % NQ == 0, "steps come in pairs, work-groups lie in one frame");
+  __shared__ float lkey[NQ][CAP];
+  __shared__ int lid[NQ][CAP];
+  __shared__ int lcnt[NQ];
+  __shared__ float lthr[NQ];  // -infinity for a slot without a query: nothing enters
+  __shared__ int lqid[NQ];
+  __shared__ int need[3];     // round r uses need[r % 3]
+  __shared__ unsigned long long skipm[4];
+  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, g = lane >> 4, j = lane & 15;
+  const int q0 = blockIdx.x * NQ, frame = q0 / kF2Q;
   const int ntiles = rf.ntiles;
-  float areg[NST];
-  {
-    const int sa = q0 + 16 * w + (lane & 15);
+  float areg[QB][NST], dl[NST];
 #pragma unroll
-    for (int st = 0; st < NST; ++st) areg[st] = sa < n ? Xq[(size_t)sa * 4 * NST + 4 * st + (lane >> 4)] : 0.0f;
-  }
-  // this thread's float4 columns of the block's shift
-  float4 dl[kFiltR * NST / 128];
-  {
-    const float4 *D4 = reinterpret_cast<const float4 *>(delta) + (size_t)blockIdx.x * NST;
+  for (int b = 0; b < QB; ++b) {
+    const int sa = q0 + 16 * b + j;
 #pragma unroll
-    for (int u = 0; u < kFiltR * NST / 128; ++u) dl[u] = D4[(threadIdx.x + u * 128) / kFiltR];
+    for (int st = 0; st < NST; ++st) areg[b][st] = sa < n ? Xq[(size_t)sa * 4 * NST + 4 * st + g] : 0.0f;
   }
-  for (int t = tid; t < kF2Q * kp; t += 128) {
-    hk[t] = INFINITY;
-    hx[t] = INT_MAX;
+#pragma unroll
+  for (int st = 0; st < NST; ++st) dl[st] = delta[(size_t)frame * 4 * NST + 4 * st + g];
+  if (tid < NQ) {
+    const bool in = q0 + tid < n;
+    lcnt[tid] = 0;
+    lqid[tid] = in ? qorder[q0 + tid] : -1;
+    lthr[tid] = in ? INFINITY : -INFINITY;
   }
-  if (tid < kF2Q) {
-    qn[tid] = q0 + tid < n ? qn32[q0 + tid] : 0.0f;
-    qid[tid] = q0 + tid < n ? qorder[q0 + tid] : -1;
-  }
-  if (w == 0) {  // the block's radius: its queries' largest |x - c_b| (|a| rounded up)
-    const int q = lane < kF2Q && q0 + lane < n ? qorder[q0 + lane] : -1;
-    const double r = wave_max(q >= 0 ? rf.qa[q] * (1.0 + 0x1p-20) : 0.0);
-    if (lane == 0) srho = r;
-  }
+  if (tid < 3) need[tid] = 0;
+  // the block's radius: its queries' largest |x - c_b| (|a| rounded up)
+  const double rho =
+      wave_max(lane < NQ && q0 + lane < n ? rf.qa[qorder[q0 + lane]] * (1.0 + 0x1p-20) : 0.0);
+  __syncthreads();
+  // this lane's queries: rows 4 g + v of each block of 16
+  float qv[QB][4], th[QB][4];
+  int qq[QB][4];
+#pragma unroll
+  for (int b = 0; b < QB; ++b)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int ql = 16 * b + 4 * g + v;
+      qv[b][v] = q0 + ql < n ? qn32[q0 + ql] : 0.0f;
+      qq[b][v] = lqid[ql];
+      th[b][v] = lthr[ql];
+    }
   // the first tile visited: kFiltHomeBack tiles before the block's own, but
   // not before its cell's first tile, so the lists fill from the block's
   // own cell and its threshold prunes the other cells' tiles early
   const int home = rf.rinv[qorder[q0]] / kFiltR;
   const int start = max(home - kFiltHomeBack, rf.slot0[rf.cell[qorder[q0]]] / kFiltR);
   const double R = __longlong_as_double((long long)*rf.rmax);
-  const double dnb = rf.dn[blockIdx.x];
-  const double *cbb = rf.cb + (size_t)blockIdx.x * rf.dim;
+  const double dnb = rf.dn[frame];
+  const double *cbb = rf.cb + (size_t)frame * rf.dim;
   auto visit = [&](int sq) { return (start + sq) % ntiles; };  // the sq-th tile visited
-  float4 buf[kFiltR * NST / 128];
-  float rnv;
-  for (int g0 = 0; g0 < ntiles; g0 += 128) {
-    __syncthreads();  // the previous tile's merge is done
-    if (w == 0) {  // the worst key over the block's queries (infinite until every list is full)
-      const float th = lane < kF2Q && qid[lane] >= 0 ? hk[lane * kp] : -INFINITY;
-      const float m = (float)wave_max((double)th);
-      if (lane == 0) sthr = m;
+  const float2 *Xr2 = reinterpret_cast<const float2 *>(rf.Xr);
+  float2 nb[NST / 2];
+  int nid = -1;
+  auto load = [&](int tile) {  // this wave's 16 references of a tile
+    const size_t t16 = (size_t)tile * 4 + w;
+    const float2 *src = Xr2 + t16 * (NST / 2) * 64 + lane;
+#pragma unroll
+    for (int u = 0; u < NST / 2; ++u) nb[u] = src[u * 64];
+    nid = rf.rid[t16 * 16 + j];
+  };
+  auto cut = [&](int ql, int spare) {
+    float t;
+    const int c = cut_list<CAP>(lkey[ql], lid[ql], lcnt[ql], kp, spare, lane, &t);
+    if (lane == 0) {
+      lcnt[ql] = c;
+      lthr[ql] = t;
     }
+  };
+  auto refresh = [&]() {
+#pragma unroll
+    for (int b = 0; b < QB; ++b)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) th[b][v] = lthr[16 * b + 4 * g + v];
+  };
+  int round = 0;
+  // groups of tiles: the first ones small, so that the thresholds prune soon
+  for (int g0 = 0, gsz = 32; g0 < ntiles; g0 += gsz, gsz = min(256, g0 >= 64 ? 256 : 2 * gsz)) {
+    // tighten every list that has kp entries, then the tiles of the group
+    // that some query's threshold reaches
+    for (int ql = w; ql < NQ; ql += 4)
+      if (lcnt[ql] > kp) cut(ql, kCutSpare);
     __syncthreads();
+    refresh();
+    const float thr = (float)wave_max(lane < NQ ? (double)lthr[lane] : -INFINITY);
     bool skip = true;
-    if (g0 + tid < ntiles) {
+    if (tid < gsz && g0 + tid < ntiles) {
       const int t = visit(g0 + tid);
       const double rt_ = rf.trad[t];
-      const double thr = (double)sthr;
-      if (rt_ < 0.0) {
-        skip = true;  // padding only
-      } else if (!(thr < INFINITY)) {
+      if (rt_ >= 0.0) {  // not padding only
         skip = false;
-      } else {
-        const double *tc = rf.tcen + (size_t)t * rf.dim;
-        double d2 = 0.0;
-        for (int l = 0; l < rf.dim; ++l) {
-          const double v = cbb[l] - tc[l];
-          d2 = fma(v, v, d2);
+        if (thr < INFINITY) {
+          const double *tc = rf.tcen + (size_t)t * rf.dim;
+          double d2 = 0.0;
+          for (int l = 0; l < rf.dim; ++l) {
+            const double v = cbb[l] - tc[l];
+            d2 = fma(v, v, d2);
+          }
+          const double dcm = sqrt(d2);
+          const double dlb = dcm - rho - rt_;
+          const double S = rho + dcm + rt_ + R + dnb;
+          skip = dlb > 0.0 && dlb * dlb - 0x1p-12 * S * S > (double)thr;
         }
-        const double dcm = sqrt(d2), rho = srho;
-        const double dlb = dcm - rho - rt_;
-        const double S = rho + dcm + rt_ + R + dnb;
-        skip = dlb > 0.0 && dlb * dlb - 0x1p-12 * S * S > thr;
       }
     }
     const unsigned long long sb = __ballot(skip);
     if (lane == 0) skipm[w] = sb;
     __syncthreads();
-    const unsigned long long todo[2] = {~skipm[0], ~skipm[1]};
-    auto next_tile = [&](int i) {  // the next visited index of this group after i, or -1
-      const int k = i + 1;
-      if (k >= 128) return -1;
-      if (k < 64) {
-        const unsigned long long m = todo[0] & (~0ull << k);
-        if (m) return __builtin_ctzll(m);
+    unsigned long long t0 = ~skipm[0], t1 = ~skipm[1], t2 = ~skipm[2], t3 = ~skipm[3];
+    auto next_tile = [&]() {  // takes the next tile of the group, -1: none left
+      int i = -1;
+      if (t0) {
+        i = __builtin_ctzll(t0);
+        t0 &= t0 - 1;
+      } else if (t1) {
+        i = 64 + __builtin_ctzll(t1);
+        t1 &= t1 - 1;
+      } else if (t2) {
+        i = 128 + __builtin_ctzll(t2);
+        t2 &= t2 - 1;
+      } else if (t3) {
+        i = 192 + __builtin_ctzll(t3);
+        t3 &= t3 - 1;
       }
-      const unsigned long long m = todo[1] & (k <= 64 ? ~0ull : ~0ull << (k - 64));
-      return m ? 64 + __builtin_ctzll(m) : -1;
+      return i < 0 ? -1 : visit(g0 + i);
     };
-    int i = next_tile(-1);
-    if (i >= 0) tile_load<128, NST>(rf.Xr, rf.Xr, ntiles * kFiltR, visit(g0 + i) * kFiltR, buf, rnv);
-    while (i >= 0) {
-      const int r0 = visit(g0 + i) * kFiltR;
-      const int inext = next_tile(i);
-      __syncthreads();  // the previous tile's merge is done
-      tile_store_shift<NST>(rt, rnp, buf, dl);
-      __syncthreads();
-      if (inext >= 0) tile_load<128, NST>(rf.Xr, rf.Xr, ntiles * kFiltR, visit(g0 + inext) * kFiltR, buf, rnv);
-      int rr[4];  // ids of this lane's reference columns 16 t + lane % 16 (in flight over the dot products)
+    int tile = next_tile();
+    if (tile >= 0) load(tile);
+    while (tile >= 0) {
+#pragma unroll 1
+      for (int u = 0; u < TPR && tile >= 0; ++u) {
+        float bv[NST];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) rr[t] = rf.rid[r0 + 16 * t + (lane & 15)];
-      fv4 acc[4];
-      tile_dots<NST>(areg, rt, lane, acc);
-      // this lane's four query rows 16 w + 4 g + v: norms and current worst keys
-      float qv[4], thd[4];
-      int thi[4], qq[4];
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int ql = 16 * w + 4 * g + v;
-        qv[v] = qn[ql];
-        thd[v] = hk[ql * kp];
-        thi[v] = hx[ql * kp];
-        qq[v] = qid[ql];
-      }
-      unsigned long long mq[4] = {0ull, 0ull, 0ull, 0ull};
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int jl = 16 * t + (lane & 15);
-        const float rv = rnp[jl] + rnp[jl + 64];
-        const int r = rr[t];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int ql = 16 * w + 4 * g + v;
-          const float dd = (qv[v] + rv) - 2.0f * acc[t][v];
-          dist[ql][jl] = dd;
-          const bool cand = qq[v] >= 0 && r >= 0 && r != qq[v] && key_lessf(dd, r, thd[v], thi[v]);
-          const unsigned long long b = __ballot(cand);
-          mq[v] |= ((b >> (16 * g)) & 0xFFFFull) << (16 * t);
+        for (int h = 0; h < NST / 2; ++h) {
+          bv[2 * h] = nb[h].x;
+          bv[2 * h + 1] = nb[h].y;
         }
-      }
-      if ((lane & 15) == 0)
+        const int rid = nid;
+        tile = next_tile();
+        if (tile >= 0) load(tile);
+        // into the block's frame, with the squared norms of the references
+        float rn = 0.0f;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) mask[16 * w + 4 * g + v] = mq[v];
-      __syncthreads();
-      if (tid < kF2Q) {
-        float *H = hk + tid * kp;
-        int *HI = hx + tid * kp;
-        unsigned long long m = mask[tid];
-        while (m) {
-          const int j = __ffsll((long long)m) - 1;
-          m &= m - 1;
-          const float cd = dist[tid][j];
-          const int ci = rf.rid[r0 + j];
-          if (!key_lessf(cd, ci, H[0], HI[0])) continue;
-          int pos = 0;
-          for (;;) {
-            const int l = 2 * pos + 1, rr2 = l + 1;
-            int mm = -1;
-            float md = cd;
-            int mi = ci;
-            if (l < kp && key_lessf(md, mi, H[l], HI[l])) { mm = l; md = H[l]; mi = HI[l]; }
-            if (rr2 < kp && key_lessf(md, mi, H[rr2], HI[rr2])) { mm = rr2; md = H[rr2]; mi = HI[rr2]; }
-            if (mm < 0) break;
-            H[pos] = md;
-            HI[pos] = mi;
-            pos = mm;
+        for (int st = 0; st < NST; ++st) {
+          bv[st] -= dl[st];
+          rn = fmaf(bv[st], bv[st], rn);
+        }
+        rn += __shfl_xor(rn, 16, 64);
+        rn += __shfl_xor(rn, 32, 64);
+        fv4 acc[QB];
+#pragma unroll
+        for (int b = 0; b < QB; ++b) acc[b] = fv4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int st = 0; st < NST; ++st)
+#pragma unroll
+          for (int b = 0; b < QB; ++b)
+            acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(areg[b][st], bv[st], acc[b], 0, 0, 0);
+        float dd[QB][4];
+        bool any = false;
+#pragma unroll
+        for (int b = 0; b < QB; ++b)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            dd[b][v] = (qv[b][v] + rn) - 2.0f * acc[b][v];
+            any |= dd[b][v] < th[b][v];
           }
-          H[pos] = cd;
-          HI[pos] = ci;
+        if (__ballot(any)) {
+#pragma unroll
+          for (int b = 0; b < QB; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+              const bool in = dd[b][v] < th[b][v] && rid >= 0 && rid != qq[b][v];
+              const unsigned gm = (unsigned)(__ballot(in) >> (16 * g)) & 0xFFFFu;  // this query's 16 references
+              const int c = __popc(gm), ql = 16 * b + 4 * g + v;
+              int base = 0;
+              if (j == 0 && c) {
+                base = atomicAdd(&lcnt[ql], c);
+                if (base + c > kTrig) need[round % 3] = 1;
+              }
+              base = __shfl(base, 16 * g, 64);
+              if (in) {
+                const int p = base + __popc(gm & ((1u << j) - 1u));
+                lkey[ql][p] = dd[b][v];
+                lid[ql][p] = rid;
+              }
+            }
         }
       }
-      i = inext;
+      __syncthreads();
+      // every wave reads need[round % 3] before the next meeting; it is
+      // cleared after that one, and used again after the one that follows
+      const bool full = need[round % 3] != 0;
+      if (tid == 0) need[(round + 2) % 3] = 0;
+      ++round;
+      if (full) {
+        for (int ql = w; ql < NQ; ql += 4)
+          if (lcnt[ql] > kTrig - 32) cut(ql, kCutSpare);
+        __syncthreads();
+        refresh();
+      }
     }
   }
   __syncthreads();
-  for (int t = tid; t < kF2Q * kp; t += 128) {
-    const int ql = t / kp, q = qid[ql];
-    if (q >= 0) {
-      hd[(size_t)q * kp + (t - ql * kp)] = hk[t];
-      hi[(size_t)q * kp + (t - ql * kp)] = hx[t];
+  for (int ql = w; ql < NQ; ql += 4) {
+    const int q = lqid[ql];
+    if (q < 0) continue;  // wave-uniform
+    if (lcnt[ql] > kp) cut(ql, 0);
+    const int c = lcnt[ql];
+    for (int e = lane; e < kp; e += 64) {  // a list left short (NaN distances) is not certified
+      hd[(size_t)q * kp + e] = e < c ? lkey[ql][e] : INFINITY;
+      hi[(size_t)q * kp + e] = e < c ? lid[ql][e] : INT_MAX;
     }
   }
 }
 
 // Step counts (dimensions / 4, rounded up) the filters are built for.
-// The block-centred arrays of the LDS-heap filter (kp <= kF2MaxKp).
+// The block-centred arrays of the LDS-list filter (kp <= kF2MaxKp).
 struct BlockCentred {
   const float *Xq;         // queries in slot order, centred at their block's mean
   const float *qn32;       // their squared norms
@@ -991,13 +1103,23 @@ struct BlockCentred {
   RefTiles rf;             // the references in cell order, with tile spheres
 };
 
+// Points from which a work-group takes 32 queries instead of 16.  32 halve the
+// reads of the references but leave half as many waves per CU (66 KB of lists
+// against 41) and half as many work-groups: whole kNN calls at 50 dimensions
+// with 16 / 32: 2.24 / 2.46 ms at 10,000 points, 4.23 / 4.58 at 20,000, 82.4 /
+// 84.2 at 200,000, 1272 / 1148 at 1.3M.
+constexpr int kFiltWide = 1 << 19;
+
 template <int NST>
 int launch_filter(hipStream_t s, const float *Xc, const float *n32, int n, int kp, const BlockCentred &bc,
                   float *hd, int *hi) {
   if (kp <= kF2MaxKp) {
-    const size_t lds = (sizeof(float) + sizeof(int)) * (size_t)kF2Q * kp;
-    knn_filter_lds_kernel<NST><<<div_up(n, kF2Q), 128, lds, s>>>(bc.rf, bc.Xq, bc.qn32, bc.qorder, bc.delta, n, kp,
-                                                                 hd, hi);
+    if (n < kFiltWide)
+      knn_filter_list_kernel<NST, 1><<<div_up(n, 16), 256, 0, s>>>(bc.rf, bc.Xq, bc.qn32, bc.qorder, bc.delta, n, kp,
+                                                                   hd, hi);
+    else
+      knn_filter_list_kernel<NST, 2><<<div_up(n, 32), 256, 0, s>>>(bc.rf, bc.Xq, bc.qn32, bc.qorder, bc.delta, n, kp,
+                                                                   hd, hi);
   } else {
     if constexpr ((kFiltR * NST) % 256 == 0) {
       knn_filter_kernel<NST><<<div_up(n, kFiltQ), 256, 0, s>>>(Xc, n32, n, kp, hd, hi);
@@ -1010,10 +1132,9 @@ int launch_filter(hipStream_t s, const float *Xc, const float *n32, int n, int k
 }
 
 // float4 steps of the filter's padded dimension.  14 (dims 49-56: the usual
-// 50-D PCA input) only with the LDS-heap kernel, whose 128-thread tile load
-// splits 64 x 14 float4 evenly: its LDS then fits three work-groups per CU,
-// where 16 steps fit two.  The zero padding adds exact zeros, so the FP32
-// distances, the candidates and the rows are the same either way.
+// 50-D PCA input) only with the LDS-list kernel, which takes any even number
+// of steps.  The zero padding adds exact zeros, so the FP32 distances, the
+// candidates and the rows are the same either way.
 int filter_steps(int dim, int kp) {
   const int nst = (dim + 3) / 4;
   if (nst > 12 && nst <= 14 && kp <= kF2MaxKp) return 14;

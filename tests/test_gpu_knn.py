@@ -55,3 +55,39 @@ def test_knn_exact_infinite_points(sg):
     assert I[0, -2:].tolist() == [3, 50] and np.isinf(D[0, -2:]).all() and np.isfinite(D[0, :-2]).all()
     near = [i for i in range(200) if i not in far]
     assert I[3, 1:198].tolist() == near and np.isinf(D[3, 1:]).all() and I[3, 198] == np.iinfo(np.int32).max
+
+
+# query blocks and reference tiles one point short / full / one over, every
+# step count of the filter's template, lists at their largest (k + 16 = 128)
+@pytest.mark.parametrize("n,dim,k", [(64, 3, 40), (65, 16, 30), (129, 17, 112), (193, 31, 90), (1000, 48, 112), (1025, 49, 16),
+                                     (2048, 64, 90), (3001, 96, 45), (2500, 100, 1)])
+def test_knn_filtered_lists(sg, O, n, dim, k):
+    X = _points(n, dim, 3 * n + dim)
+    I, D, fb = sg.knn(X, k, sg.KNN_FILTERED)
+    Io, Do = O.knn_exact(X, k)
+    assert fb >= 0 and np.array_equal(I, Io) and np.array_equal(D, Do)
+
+
+@pytest.mark.parametrize("step", [1.0, -1.0])
+def test_knn_filtered_every_reference_enters(sg, O, step):
+    # points on a line, ever farther from (or nearer to) the first ones: in one
+    # direction every reference beats the list's threshold as it is visited
+    n = 4000
+    X = np.zeros((n, 4), np.float32)
+    X[:, 0] = step * np.arange(n, dtype=np.float32) ** 1.5
+    I, D, fb = sg.knn(X, 90, sg.KNN_FILTERED)
+    Io, Do = O.knn_exact(X, 90)
+    assert np.array_equal(I, Io) and np.array_equal(D, Do)
+
+
+def test_knn_filtered_wide_blocks(sg):
+    # the 32-query work-groups of very large jobs, on rows sampled from one
+    X = _points(530_000, 8, 4)
+    I, D, fb = sg.knn(X, 20, sg.KNN_FILTERED)
+    rows = np.arange(0, X.shape[0], 1877)
+    Xd = X.astype(np.float64)
+    for q in rows:
+        d2 = ((Xd - Xd[q]) ** 2).sum(1)
+        d2[q] = np.inf
+        near = np.sort(np.partition(d2, 19)[:20])
+        assert I[q, 0] == q and np.allclose(D[q, 1:], near, rtol=1e-12) and np.allclose(d2[I[q, 1:]], near, rtol=1e-12)
