@@ -6,9 +6,9 @@
 // iteration 250, alpha -> 1 after iteration early_iter, mean-centring every
 // iteration (HYB semantics), h-driven grid size (HY/qq.cpp:159-166).
 //
-// Per iteration there is one device->host transfer of the (min, max) of Y,
-// needed to size the grid; the attractive SpMV is issued before the host
-// waits for it, so the GPU stays busy across the round trip.
+// Per iteration the centring kernel writes the (min, max) of Y, needed to size
+// the grid, into pinned memory the host polls; the attractive SpMV is issued
+// before the host waits for it, so the GPU stays busy across the round trip.
 #include "common.hpp"
 #include "kernels.hpp"
 #include "grid_device.hpp"
@@ -60,11 +60,6 @@ static int optimal_ell_width(int n, const std::vector<int32_t> &rowptr) {
   return maxlen;
 }
 
-struct PhaseEvents {
-  hipEvent_t e[6];  // attr start, attr end, s2g end, conv end, g2s end, update end
-  bool valid = false;
-};
-
 }  // namespace sgt
 
 using namespace sgt;
@@ -114,8 +109,8 @@ struct sgtsne_ctx {
   // reductions
   RedWork rw{};
   DevScalars *sc = nullptr;       // device
-  DevScalars *sc_host = nullptr;  // pinned
-  hipEvent_t ev_scal = nullptr;
+  HostScalars *hs = nullptr;      // pinned: what the device publishes to the host
+  unsigned long long seq = 0;     // sequence number of the last publication queued
 
   // grid workspace
   size_t grid_cap = 0, w_cap = 0, k_cap = 0;
@@ -126,7 +121,8 @@ struct sgtsne_ctx {
 
   // timing
   bool timing = true;
-  PhaseEvents pe[2];
+  bool stamped = false;  // the last publication carries an iteration's phase times
+  double ms_per_tick = 1e-5;  // of the device clock
   double acc_ms[7] = {0, 0, 0, 0, 0, 0, 0};
   double *time_info = nullptr;  // optional per-iteration output (sgtsne_run)
   int time_info_base = 0;
@@ -260,7 +256,7 @@ int check_params(const sgtsne_params *p) {
 double default_h(int d) { return d == 1 ? 0.5 : d == 2 ? 0.7 : 1.2; }
 
 // Host side of one iteration's grid mapping (HY/qq.cpp:159-166, HY/nuconv.cpp:28-47).
-int make_grid(sgtsne_ctx *c, const DevScalars &s, GridParams &g) {
+int make_grid(sgtsne_ctx *c, const HostScalars &s, GridParams &g) {
   const int d = c->d;
   double maxy = 0.0;
   for (int a = 0; a < d; a++) {
@@ -352,37 +348,51 @@ int attractive(sgtsne_ctx *c) {
   }
 }
 
-// Repulsive term for the current (centred) Y: S2G -> convolution -> G2S.
-int repulsive(sgtsne_ctx *c, const GridParams &g, PhaseEvents *pe) {
+// Repulsive term for the current (centred) Y: S2G -> convolution -> G2S; *nz
+// receives the number of partials of Z.
+int repulsive(sgtsne_ctx *c, const GridParams &g, bool stamp, int *nz) {
   const int zdirect = c->p.zeta_mode == SGTSNE_ZETA_DIRECT;
+  DevScalars *st = stamp ? c->sc : nullptr;
   SGT_TRY(ensure_grid(c, g));
   int64_t need = 0;
-  SGT_TRY(launch_s2g(c->stream, g, c->n, c->Y, c->V, c->s2g_part, c->s2g_cap, &need, c->p.spread));
-  if (pe) SGT_HIP(hipEventRecord(pe->e[2], c->stream));
+  SGT_TRY(launch_s2g(c->stream, g, c->n, c->Y, c->V, c->s2g_part, c->s2g_cap, &need, c->p.spread, st));
   SGT_TRY(launch_conv(c->stream, g, zdirect, c->V, c->Phi, c->cb));
-  if (pe) SGT_HIP(hipEventRecord(pe->e[3], c->stream));
-  SGT_TRY(launch_g2s_force(c->stream, g, c->n, c->Y, c->Phi, c->Frep, zdirect, c->rw, c->sc));
-  if (pe) SGT_HIP(hipEventRecord(pe->e[4], c->stream));
+  SGT_TRY(launch_g2s_force(c->stream, g, c->n, c->Y, c->Phi, c->Frep, zdirect, c->rw, nz, st));
   c->last_grid = g;
   return SGTSNE_OK;
 }
 
-int center_and_fetch(sgtsne_ctx *c, int apply_mean, PhaseEvents *pe = nullptr) {
-  SGT_TRY(launch_center_minmax(c->stream, c->d, c->n, c->Y, apply_mean, c->rw, c->sc));
-  if (pe) {
-    SGT_HIP(hipEventRecord(pe->e[5], c->stream));
-    pe->valid = true;
-  }
-  SGT_HIP(hipMemcpyAsync(c->sc_host, c->sc, sizeof(DevScalars), hipMemcpyDeviceToHost, c->stream));
-  SGT_HIP(hipEventRecord(c->ev_scal, c->stream));
-  return SGTSNE_OK;
+// Centres Y by the mean in c->sc (when asked) and queues the publication of
+// its bounds.
+int center_and_publish(sgtsne_ctx *c, int apply_mean) {
+  c->stamped = false;
+  return launch_center_minmax(c->stream, c->d, c->n, c->Y, apply_mean, c->rw, c->sc, c->hs, ++c->seq);
 }
 
-void harvest_timing(sgtsne_ctx *c, PhaseEvents &pe, int it) {
-  if (!pe.valid) return;
-  float t[5] = {0, 0, 0, 0, 0};
-  for (int k = 0; k < 5; k++) (void)hipEventElapsedTime(&t[k], pe.e[k], pe.e[k + 1]);
-  // t: attr, s2g(+fill), conv, g2s, update(+centre)
+// Waits for the last queued publication.  The device writes the sequence
+// number after everything else; a stream that has drained (or failed) without
+// it ends the wait.
+int wait_published(sgtsne_ctx *c) {
+  for (unsigned spin = 1;; ++spin) {
+    if (__atomic_load_n(&c->hs->seq, __ATOMIC_ACQUIRE) == c->seq) return SGTSNE_OK;
+    if (spin % 1024 == 0) {
+      const hipError_t e = hipStreamQuery(c->stream);
+      if (e == hipErrorNotReady) continue;
+      SGT_HIP(e);
+      SGT_CHECK(__atomic_load_n(&c->hs->seq, __ATOMIC_ACQUIRE) == c->seq, SGTSNE_ERR_STATE,
+                "the device did not publish its scalars (iteration %d)", c->iter);
+      return SGTSNE_OK;
+    }
+    __builtin_ia32_pause();
+  }
+}
+
+// Adds the phase times of iteration `it`, published with its centring.
+void harvest_timing(sgtsne_ctx *c, int it) {
+  if (!c->stamped) return;
+  c->stamped = false;
+  double t[5];  // attr (and any wait for the host), s2g, conv, g2s, update(+centre)
+  for (int k = 0; k < 5; k++) t[k] = (double)(c->hs->stamp[k + 1] - c->hs->stamp[k]) * c->ms_per_tick;
   c->acc_ms[0] += t[0];
   c->acc_ms[1] += t[1];
   c->acc_ms[2] += t[2];
@@ -400,7 +410,6 @@ void harvest_timing(sgtsne_ctx *c, PhaseEvents &pe, int it) {
     ti[5] = t[1] + t[2] + t[3];
     ti[6] = 0.0;
   }
-  pe.valid = false;
 }
 
 // Iterations at which a re-order of the points along a Morton curve of the
@@ -410,6 +419,10 @@ void harvest_timing(sgtsne_ctx *c, PhaseEvents &pe, int it) {
 // (large N converges slowly) the breadth-first order of P is better.  So the
 // new order is kept only when the attractive kernel measures faster on it.
 constexpr int kSpatialReorderIters[] = {50, 150, 300, 600};
+// A smaller job's Y (at most 64 KB) stays in cache in any order: the gathers
+// of 1800 points took 4.5 us in either, so the comparison kept one of them by
+// chance, at 1.0-1.5 ms of host work per attempt.
+constexpr int kSpatialReorderMin = 4096;
 
 int tune_attractive(sgtsne_ctx *c);
 int build_localised(sgtsne_ctx *c);
@@ -457,8 +470,8 @@ int time_attractive(sgtsne_ctx *c, int32_t *rp, int32_t *col, float *val, float 
 
 int spatial_reorder(sgtsne_ctx *c) {
   const int n = c->n, d = c->d, ds = c->ds;
-  SGT_HIP(hipEventSynchronize(c->ev_scal));
-  const DevScalars sh = *c->sc_host;
+  SGT_TRY(wait_published(c));
+  const HostScalars sh = *c->hs;
   double lo[3] = {0, 0, 0}, extent = 0.0;
   for (int a = 0; a < d; a++) {
     lo[a] = sh.minv[a];
@@ -552,25 +565,29 @@ int spatial_reorder(sgtsne_ctx *c) {
 
 int iterate(sgtsne_ctx *c) {
   const int it = c->iter;
-  if (c->p.reorder >= 2 && (c->p.format == SGTSNE_FORMAT_CSR_SEG || c->p.format == SGTSNE_FORMAT_CSR))
+  if (c->p.reorder >= 2 && c->n >= kSpatialReorderMin &&
+      (c->p.format == SGTSNE_FORMAT_CSR_SEG || c->p.format == SGTSNE_FORMAT_CSR))
     for (int r : kSpatialReorderIters)
-      if (it == r) SGT_TRY(spatial_reorder(c));
+      if (it == r) {
+        SGT_TRY(wait_published(c));
+        harvest_timing(c, it - 1);
+        SGT_TRY(spatial_reorder(c));
+        if (c->timing) SGT_TRY(launch_stamp(c->stream, c->sc, STAMP_END));  // not part of the iteration
+      }
   const double alpha = it <= c->p.early_iter ? c->p.alpha : 1.0;
   const double momentum = it <= 250 ? 0.5 : 0.8;
   const double eta = 200.0;
-  PhaseEvents *pe = c->timing ? &c->pe[it & 1] : nullptr;
-  if (pe) SGT_HIP(hipEventRecord(pe->e[0], c->stream));
   SGT_TRY(attractive(c));
-  if (pe) SGT_HIP(hipEventRecord(pe->e[1], c->stream));
-  // wait for the (min, max) of this iteration's Y (issued by the previous centring)
-  SGT_HIP(hipEventSynchronize(c->ev_scal));
-  if (c->timing) harvest_timing(c, c->pe[(it + 1) & 1], it - 1);
-  const DevScalars s = *c->sc_host;
+  // wait for the (min, max) of this iteration's Y (published by the previous centring)
+  SGT_TRY(wait_published(c));
+  harvest_timing(c, it - 1);
   GridParams g{};
-  SGT_TRY(make_grid(c, s, g));
-  SGT_TRY(repulsive(c, g, pe));
+  SGT_TRY(make_grid(c, *c->hs, g));
+  int nz = 0;
+  SGT_TRY(repulsive(c, g, c->timing, &nz));
   if (c->p.compute_error > 0 && it % 10 == 0) {
     // relative L2 error of the interpolated repulsion (CU/gradient_descend.cu:206-215)
+    SGT_TRY(launch_finalize_z(c->stream, nz, c->n, c->rw, c->sc));
     SGT_HIP(hipStreamSynchronize(c->stream));
     const size_t nb = (size_t)c->n * c->ds;
     std::vector<float> fi(nb), fe(nb);
@@ -579,7 +596,10 @@ int iterate(sgtsne_ctx *c) {
     SGT_HIP(hipMemcpy(&sh, c->sc, sizeof(DevScalars), hipMemcpyDeviceToHost));
     float *tmp = nullptr;
     SGT_TRY(alloc_dev((void **)&tmp, nb * sizeof(float)));
-    int st = launch_rep_exact(c->stream, c->d, c->n, c->Y, tmp, c->rw, c->sc);
+    RedWork rx = c->rw;  // past the partials of Z, which the update still reads
+    rx.part += (size_t)8 * 4096;
+    rx.max_blocks -= 4096;
+    int st = launch_rep_exact(c->stream, c->d, c->n, c->Y, tmp, rx, c->sc);
     if (st == SGTSNE_OK) {
       (void)hipStreamSynchronize(c->stream);
       (void)hipMemcpy(fe.data(), tmp, nb * sizeof(float), hipMemcpyDeviceToHost);
@@ -597,9 +617,9 @@ int iterate(sgtsne_ctx *c) {
     free_dev(tmp);
     SGT_TRY(st);
   }
-  SGT_TRY(launch_update(c->stream, c->d, c->n, c->Y, c->uY, c->gains, c->Fattr, c->Frep,
-                        (float)alpha, (float)momentum, (float)eta, c->rw, c->sc));
-  SGT_TRY(center_and_fetch(c, 1, pe));
+  SGT_TRY(launch_update_center(c->stream, c->d, c->n, c->Y, c->uY, c->gains, c->Fattr, c->Frep, (float)alpha,
+                               (float)momentum, (float)eta, nz, c->rw, c->sc, c->hs, ++c->seq, c->timing));
+  c->stamped = c->timing;
   c->iter++;
   return SGTSNE_OK;
 }
@@ -1026,7 +1046,7 @@ int sgtsne_ctx_create(sgtsne_ctx **out, const sgtsne_params *params) {
     set_error("hipStreamCreate failed");
     return fail(SGTSNE_ERR_HIP);
   }
-  c->rw.max_blocks = 65536;
+  c->rw.max_blocks = 65536 + 4096;
   if ((st = alloc_dev((void **)&c->rw.part, sizeof(double) * 8 * c->rw.max_blocks))) return fail(st);
   if ((st = alloc_dev((void **)&c->rw.ticket, sizeof(unsigned) * 4))) return fail(st);
   if ((st = alloc_dev((void **)&c->sc, sizeof(DevScalars)))) return fail(st);
@@ -1035,21 +1055,14 @@ int sgtsne_ctx_create(sgtsne_ctx **out, const sgtsne_params *params) {
     set_error("hipMemset failed");
     return fail(SGTSNE_ERR_HIP);
   }
-  if (hipHostMalloc((void **)&c->sc_host, sizeof(DevScalars), hipHostMallocDefault) != hipSuccess) {
+  if (hipHostMalloc((void **)&c->hs, sizeof(HostScalars), hipHostMallocCoherent) != hipSuccess) {
     set_error("hipHostMalloc failed");
     return fail(SGTSNE_ERR_NOMEM);
   }
-  std::memset(c->sc_host, 0, sizeof(DevScalars));
-  if (hipEventCreateWithFlags(&c->ev_scal, hipEventDisableTiming) != hipSuccess) {
-    set_error("hipEventCreate failed");
-    return fail(SGTSNE_ERR_HIP);
-  }
-  for (auto &pe : c->pe)
-    for (auto &ev : pe.e)
-      if (hipEventCreate(&ev) != hipSuccess) {
-        set_error("hipEventCreate failed");
-        return fail(SGTSNE_ERR_HIP);
-      }
+  std::memset(c->hs, 0, sizeof(HostScalars));
+  int khz = 0;
+  if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, c->device) == hipSuccess && khz > 0)
+    c->ms_per_tick = 1.0 / (double)khz;
   if ((st = alloc_dev((void **)&c->cb.tw, sizeof(float2) * twiddle_count()))) return fail(st);
   if ((st = init_twiddles(c->stream, c->cb.tw))) return fail(st);
   *out = c;
@@ -1076,11 +1089,7 @@ int sgtsne_ctx_destroy(sgtsne_ctx *c) {
   free_dev(c->cb.Kt2);
   free_dev(c->cb.Kh);
   free_dev(c->cb.tw);
-  if (c->sc_host) (void)hipHostFree(c->sc_host);
-  if (c->ev_scal) (void)hipEventDestroy(c->ev_scal);
-  for (auto &pe : c->pe)
-    for (auto &ev : pe.e)
-      if (ev) (void)hipEventDestroy(ev);
+  if (c->hs) (void)hipHostFree(c->hs);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
   return SGTSNE_OK;
@@ -1214,7 +1223,7 @@ int sgtsne_ctx_set_Y(sgtsne_ctx *c, const float *y, int layout, int reset_state)
     SGT_TRY(launch_fill(c->stream, c->gains, (int64_t)nb, 1.0f));
     c->iter = 0;
   }
-  SGT_TRY(center_and_fetch(c, 1));
+  SGT_TRY(center_and_publish(c, 1));
   SGT_HIP(hipStreamSynchronize(c->stream));
   c->have_Y = true;
   return SGTSNE_OK;
@@ -1234,11 +1243,13 @@ int sgtsne_ctx_step(sgtsne_ctx *c, int iters) {
   SGT_CHECK(c != nullptr && iters >= 0, SGTSNE_ERR_ARG, "bad arguments");
   SGT_CHECK(c->have_P && c->have_Y, SGTSNE_ERR_STATE, "upload P and set Y before stepping");
   for (auto &v : c->acc_ms) v = 0.0;
-  for (auto &pe : c->pe) pe.valid = false;
+  c->stamped = false;
   int st = SGTSNE_OK;
+  if (c->timing && iters > 0) st = launch_stamp(c->stream, c->sc, STAMP_END);
   for (int k = 0; k < iters && st == SGTSNE_OK; k++) st = iterate(c);
   SGT_HIP(hipStreamSynchronize(c->stream));
-  if (c->timing && c->iter > 0) harvest_timing(c, c->pe[(c->iter - 1) & 1], c->iter - 1);
+  if (st == SGTSNE_OK) harvest_timing(c, c->iter - 1);
+  c->stamped = false;
   return st;
 }
 
@@ -1246,12 +1257,14 @@ int sgtsne_ctx_terms(sgtsne_ctx *c, float *Fattr, float *Frep, double *Z, int *n
   SGT_CHECK(c != nullptr, SGTSNE_ERR_ARG, "ctx is NULL");
   SGT_CHECK(c->have_P && c->have_Y, SGTSNE_ERR_STATE, "upload P and set Y first");
   SGT_HIP(hipStreamSynchronize(c->stream));
-  SGT_TRY(center_and_fetch(c, 0));
-  SGT_HIP(hipEventSynchronize(c->ev_scal));
+  SGT_TRY(center_and_publish(c, 0));
   SGT_TRY(attractive(c));
+  SGT_TRY(wait_published(c));
   GridParams g{};
-  SGT_TRY(make_grid(c, *c->sc_host, g));
-  SGT_TRY(repulsive(c, g, nullptr));
+  SGT_TRY(make_grid(c, *c->hs, g));
+  int nz = 0;
+  SGT_TRY(repulsive(c, g, false, &nz));
+  SGT_TRY(launch_finalize_z(c->stream, nz, c->n, c->rw, c->sc));
   SGT_HIP(hipStreamSynchronize(c->stream));
   DevScalars s{};
   SGT_HIP(hipMemcpy(&s, c->sc, sizeof(DevScalars), hipMemcpyDeviceToHost));

@@ -17,6 +17,21 @@ struct DevScalars {
   double kl;        // KL divergence (tsneCost)
   double zexact;    // exact-repulsion Z (validation)
   double pad;
+  // device clock (wall_clock64) at the starts of an iteration's spread,
+  // convolution, gather and update, written by those phases' own kernels, and
+  // at the end of the last centring: phases are timed without event packets
+  // between the kernels (six timed events cost 19-25 us per iteration)
+  unsigned long long stamp[5];
+};
+enum StampAt { STAMP_S2G = 0, STAMP_CONV = 1, STAMP_G2S = 2, STAMP_UPDATE = 3, STAMP_END = 4 };
+
+// The part of it the host reads every iteration, in pinned memory, written by
+// the centring itself: `seq` last, so the host polls one word instead of
+// queuing a copy and waiting for an event.
+struct HostScalars {
+  double minv[4], maxv[4];
+  unsigned long long stamp[6];  // iteration start, the five above
+  unsigned long long seq;
 };
 
 // Partial-reduction workspace: one slot per block plus a ticket counter.
@@ -74,20 +89,29 @@ int launch_kl(hipStream_t s, int d, int n, const int32_t *rowptr, const int32_t 
 // ---- repulsion (kernels_grid.hip) ----
 int launch_fill(hipStream_t s, float *p, int64_t count, float v);
 int launch_stream_copy(hipStream_t s, const float4 *in, float4 *out, int64_t count);
+// Y -= sc->mean (when asked), then min / max of Y into sc and hs.
 int launch_center_minmax(hipStream_t s, int d, int n, float *Y, int apply_mean, RedWork rw,
-                         DevScalars *sc);
+                         DevScalars *sc, HostScalars *hs, unsigned long long seq);
 // S2G into V [d+1][ng^d] (V is overwritten).  scratch: float workspace for the
 // per-block private grids of the LDS path; *needed receives the floats it
 // wants (when larger than scratch_floats the global-atomic path runs).
+// sc (may be NULL): the phase stamps STAMP_S2G and STAMP_CONV are written to it.
 int launch_s2g(hipStream_t s, const GridParams &g, int n, const float *Y, float *V, float *scratch,
-               int64_t scratch_floats, int64_t *needed, int mode = 0);
+               int64_t scratch_floats, int64_t *needed, int mode = 0, DevScalars *stamp = nullptr);
 int64_t s2g_scratch_need(const GridParams &g, int n, int mode = 0);
+// Frep and the partials of Z; *nz receives how many there are: launch_update
+// adds them up itself, launch_finalize_z puts their sum into sc->Z for others.
 int launch_g2s_force(hipStream_t s, const GridParams &g, int n, const float *Y, const float *Phi,
-                     float *Frep, int zdirect, RedWork rw, DevScalars *sc);
+                     float *Frep, int zdirect, RedWork rw, int *nz, DevScalars *stamp = nullptr);
+int launch_finalize_z(hipStream_t s, int nz, int n, RedWork rw, DevScalars *sc);
 int launch_finalize_kl(hipStream_t s, int nblocks, RedWork rw, DevScalars *sc);
-int launch_update(hipStream_t s, int d, int n, float *Y, float *uY, float *gains,
-                  const float *Fattr, const float *Frep, float alpha, float momentum, float eta,
-                  RedWork rw, DevScalars *sc);
+// The update of Y from the forces and the nz partials of Z, then the centring
+// of the new Y with its min / max into sc and hs (two kernels).
+int launch_update_center(hipStream_t s, int d, int n, float *Y, float *uY, float *gains, const float *Fattr,
+                         const float *Frep, float alpha, float momentum, float eta, int nz, RedWork rw,
+                         DevScalars *sc, HostScalars *hs, unsigned long long seq, bool stamp);
+// Device clock now, into sc->stamp[at].
+int launch_stamp(hipStream_t s, DevScalars *sc, int at);
 int launch_rep_exact(hipStream_t s, int d, int n, const float *Y, float *Frep, RedWork rw,
                      DevScalars *sc);
 

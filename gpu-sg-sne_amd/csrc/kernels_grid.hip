@@ -10,9 +10,16 @@
 //   forces and Z      HY/qq.cpp:75-106 / CU/Frep.cu:43-80
 //   update            CU/gradient_descend.cu:12-44, HY/gradient_descendHYB.cpp:29-78
 //
-// Reductions: every block writes its partials to rw.part[block * 8 + k]; a
-// one-block finalize kernel combines them in a fixed order (deterministic),
-// so no kernel needs a device-wide fence.
+// Reductions: every block writes its partials to rw.part[block * 8 + k], and
+// they are combined in a fixed order (deterministic), so no kernel needs a
+// device-wide fence: in the iteration by every block of the kernel that uses
+// the result (the update adds up Z, the centring the mean and the bounding box:
+// at most 2048 partials of 16 bytes and 256 of 64, read from L2), elsewhere by
+// a one-block finalize kernel.  An iteration of a small job is a chain of
+// kernels of 3-9 us each, so a launch saved is worth more than those reads:
+// without the three finalize kernels, the copy of the scalars to the host and
+// six timed events an iteration of 2011 points takes 69 us instead of 94, one of
+// 60,000 points late in a run 174 instead of 200.
 #include "common.hpp"
 #include "kernels.hpp"
 #include "grid_device.hpp"
@@ -25,7 +32,22 @@ namespace {
 
 constexpr int kBlock = 256;
 
-enum FinMode { FIN_MINMAX = 0, FIN_ZNEU = 1, FIN_MEAN = 2, FIN_ZEXACT = 3, FIN_KL = 4 };
+enum FinMode { FIN_MINMAX = 0, FIN_ZNEU = 1, FIN_ZEXACT = 2, FIN_KL = 3 };
+
+// Device clock into stamp[at], by one thread of the launch (NULL: no timing).
+__device__ __forceinline__ void stamp_now(DevScalars *sc, int at) {
+  if (sc && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) sc->stamp[at] = wall_clock64();
+}
+__global__ void stamp_kernel(DevScalars *sc, int at) { stamp_now(sc, at); }
+
+// The scalars the host waits for; the sequence number is released last.
+__device__ void publish(HostScalars *hs, const DevScalars *sc, unsigned long long seq) {
+  for (int a = 0; a < 4; ++a) {
+    hs->minv[a] = sc->minv[a];
+    hs->maxv[a] = sc->maxv[a];
+  }
+  __hip_atomic_store(&hs->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // ---- plain streaming copy (bandwidth / counter calibration) ----------------------
 __global__ __launch_bounds__(kBlock) void stream_copy_kernel(const float4 *__restrict__ in, float4 *__restrict__ out,
@@ -115,7 +137,8 @@ constexpr int kS2GUnroll = 4;    // points per lane whose loads are issued toget
 
 template <int D>
 __global__ __launch_bounds__(kS2GBlock) void s2g_lds_kernel(GridParams g, int n, const float *__restrict__ Y,
-                                                            float *__restrict__ part, int chunk, int copies) {
+                                                            float *__restrict__ part, int chunk, int copies, DevScalars *stamp) {
+  stamp_now(stamp, STAMP_S2G);
   extern __shared__ float sgrid[];
   constexpr int M = D + 1;
   constexpr int PPW = NodeLanes<D>::PPW;
@@ -213,7 +236,8 @@ __device__ __forceinline__ float lagrange_node(int r, float dl) {
 
 template <int NT>
 __global__ __launch_bounds__(kMfmaBlock) void s2g_mfma_kernel(GridParams g, int n, const float *__restrict__ Y,
-                                                              float *__restrict__ part, int chunk) {
+                                                              float *__restrict__ part, int chunk, DevScalars *stamp) {
+  stamp_now(stamp, STAMP_S2G);
   constexpr int T = 16 * NT;  // side of the tiled grid (>= ng)
   __shared__ float red[4][3][T * T];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -311,7 +335,8 @@ __global__ __launch_bounds__(kMfmaBlock) void s2g_mfma_kernel(GridParams g, int 
 constexpr int kMfma3Chunk = 2048;  // points per work-group (a multiple of the work-group size)
 
 __global__ __launch_bounds__(kMfmaBlock) void s2g_mfma3_kernel(GridParams g, int n, const float *__restrict__ Y,
-                                                               float *__restrict__ part, int chunk) {
+                                                               float *__restrict__ part, int chunk, DevScalars *stamp) {
+  stamp_now(stamp, STAMP_S2G);
   __shared__ float grid[4 * 16 * 16 * 16];  // [channel][z][y][x], side ng
   __shared__ uint32_t key[kMfma3Chunk];
   __shared__ int zcnt[kMfma3Chunk / kMfmaBlock][4][16];
@@ -480,7 +505,8 @@ __global__ __launch_bounds__(kMfmaBlock) void s2g_mfma3_kernel(GridParams g, int
 template <int D>
 __global__ __launch_bounds__(kBlock) void s2g_atomic_kernel(GridParams g, int n,
                                                             const float *__restrict__ Y,
-                                                            float *__restrict__ V) {
+                                                            float *__restrict__ V, DevScalars *stamp) {
+  stamp_now(stamp, STAMP_S2G);
   constexpr int PPW = NodeLanes<D>::PPW;
   constexpr int NODES = NodeLanes<D>::NODES;
   const int G = grid_cells<D>(g.ng);
@@ -506,7 +532,7 @@ __global__ __launch_bounds__(kBlock) void s2g_atomic_kernel(GridParams g, int n,
 // Sum of the per-block private grids (deterministic): 64 cells per block,
 // 16 partial groups per cell summed in a fixed order, then combined in LDS.
 __global__ __launch_bounds__(1024) void grid_reduce_kernel(const float *__restrict__ part, int nparts,
-                                                           int cells, float *__restrict__ V) {
+                                                           int cells, float *__restrict__ V, DevScalars *stamp) {
   __shared__ float red[16][64];
   const int c = blockIdx.x * 64 + (threadIdx.x & 63);
   const int gidx = threadIdx.x >> 6;
@@ -527,6 +553,7 @@ __global__ __launch_bounds__(1024) void grid_reduce_kernel(const float *__restri
     for (int k = 0; k < 16; ++k) t += red[k][threadIdx.x];
     V[c] = t;
   }
+  stamp_now(stamp, STAMP_CONV);  // the spread ends here
 }
 
 // ---- G2S + forces + Z ------------------------------------------------------------
@@ -541,7 +568,8 @@ template <int D, bool ZDIRECT>
 __global__ __launch_bounds__(kBlock) void g2s_force_kernel(GridParams g, int n,
                                                            const float *__restrict__ Y,
                                                            const float *__restrict__ Phi,
-                                                           float *__restrict__ Frep, double *part) {
+                                                           float *__restrict__ Frep, double *part, DevScalars *stamp) {
+  stamp_now(stamp, STAMP_G2S);
   __shared__ double lds[8];
   const int ng = g.ng;
   const int G = grid_cells<D>(ng);
@@ -599,7 +627,8 @@ inline bool g2s_lds_fits(int d, int ng) { return (d == 2 && ng <= 64) || (d == 3
 template <int D, bool ZDIRECT>
 __global__ __launch_bounds__(kG2sLdsBlock) void g2s_lds_kernel(GridParams g, int n, const float *__restrict__ Y,
                                                                const float *__restrict__ Phi,
-                                                               float *__restrict__ Frep, double *part) {
+                                                               float *__restrict__ Frep, double *part, DevScalars *stamp) {
+  stamp_now(stamp, STAMP_G2S);
   constexpr int C = ZDIRECT ? D + 2 : D + 1;
   static_assert(C >= 3 && C <= 5, "2-D or 3-D only");
   __shared__ float4 q4[kG2sLdsCells];
@@ -678,19 +707,94 @@ __global__ __launch_bounds__(kG2sLdsBlock) void g2s_lds_kernel(GridParams g, int
 // dy = alpha Fattr - Frep / Z; gains, uy, y exactly as CU/gradient_descend.cu:29-44;
 // per-block sums of the new Y feed the mean of the next centring.
 
+// Sum of nz Neumaier partials (part[8 b], part[8 b + 1]) by threads 0..255 of
+// the block, in the finalize kernel's order; every thread receives it.
+__device__ Neu block_neu(const double *__restrict__ part, int nz, double (*red)[kBlock]) {
+  const int t = threadIdx.x;
+  if (t < kBlock) {
+    Neu z{0.0, 0.0};
+    for (int b = t; b < nz; b += kBlock) neu_merge(z, Neu{part[(size_t)b * 8], part[(size_t)b * 8 + 1]});
+    red[0][t] = z.s;
+    red[1][t] = z.c;
+  }
+  __syncthreads();
+  for (int s = kBlock / 2; s > 0; s >>= 1) {
+    if (t < s) {
+      Neu x{red[0][t], red[1][t]};
+      neu_merge(x, Neu{red[0][t + s], red[1][t + s]});
+      red[0][t] = x.s;
+      red[1][t] = x.c;
+    }
+    __syncthreads();
+  }
+  return Neu{red[0][0], red[1][0]};
+}
+
+// One block's part of the new Y: the sum per dimension, the count of
+// non-finite coordinates and the bounds.
+struct BoxPart {
+  double sum[3], bad;
+  float mn[3], mx[3];
+  double pad;
+};
+static_assert(sizeof(BoxPart) == 64, "one partial slot");
+constexpr int kMaxBoxParts = 256;  // every wave of the centring reads them all
+
 template <int D>
-__global__ __launch_bounds__(kBlock) void update_kernel(int n, float *__restrict__ Y,
+__device__ __forceinline__ void wave_box(BoxPart &v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+      v.sum[a] += __shfl_xor(v.sum[a], o, 64);
+      v.mn[a] = fminf(v.mn[a], __shfl_xor(v.mn[a], o, 64));
+      v.mx[a] = fmaxf(v.mx[a], __shfl_xor(v.mx[a], o, 64));
+    }
+    v.bad += __shfl_xor(v.bad, o, 64);
+  }
+}
+
+template <int D>
+__device__ __forceinline__ void empty_box(BoxPart &v) {
+  v = BoxPart{};
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    v.mn[a] = INFINITY;
+    v.mx[a] = -INFINITY;
+  }
+}
+
+template <int D>
+__device__ __forceinline__ void merge_box(BoxPart &v, const BoxPart &w) {
+#pragma unroll
+  for (int a = 0; a < D; ++a) {
+    v.sum[a] += w.sum[a];
+    v.mn[a] = fminf(v.mn[a], w.mn[a]);
+    v.mx[a] = fmaxf(v.mx[a], w.mx[a]);
+  }
+  v.bad += w.bad;
+}
+
+constexpr int kUpdBlock = 1024;  // largest work-group of the update and the centring
+
+template <int D>
+__global__ __launch_bounds__(kUpdBlock) void update_kernel(int n, float *__restrict__ Y,
                                                         float *__restrict__ uY,
                                                         float *__restrict__ gains,
                                                         const float *__restrict__ Fattr,
                                                         const float *__restrict__ Frep,
                                                         float alpha, float momentum, float eta,
-                                                        const DevScalars *sc, double *part) {
-  __shared__ double lds[D * 4];
-  const float zinv = (float)(1.0 / sc->Z);
-  double s[D];
-#pragma unroll
-  for (int a = 0; a < D; ++a) s[a] = 0.0;
+                                                        const double *__restrict__ zpart, int nz, DevScalars *sc,
+                                                        BoxPart *__restrict__ box, int stamp) {
+  stamp_now(stamp ? sc : nullptr, STAMP_UPDATE);
+  __shared__ double red[2][kBlock];
+  __shared__ BoxPart wbox[kUpdBlock / 64];
+  const Neu zs = block_neu(zpart, nz, red);
+  const double Z = (zs.s + zs.c) - (double)n;
+  if (blockIdx.x == 0 && threadIdx.x == 0) sc->Z = Z;
+  const float zinv = (float)(1.0 / Z);
+  BoxPart v;
+  empty_box<D>(v);
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     float y[D], u[D], gn[D], fa[D], fr[D];
     load_pt<D>(Y, i, y);
@@ -706,23 +810,71 @@ __global__ __launch_bounds__(kBlock) void update_kernel(int n, float *__restrict
       gn[a] = gg;
       u[a] = momentum * u[a] - eta * gg * dy;
       y[a] = y[a] + u[a];
-      s[a] += (double)y[a];
+      v.sum[a] += (double)y[a];
+      v.mn[a] = fminf(v.mn[a], y[a]);
+      v.mx[a] = fmaxf(v.mx[a], y[a]);
+      v.bad += isfinite(y[a]) ? 0.0 : 1.0;
     }
     store_pt<D>(Y, i, y);
     store_pt<D>(uY, i, u);
     store_pt<D>(gains, i, gn);
   }
+  wave_box<D>(v);
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-  for (int a = 0; a < D; ++a) s[a] = wave_sum(s[a]);
-  if (lane == 0)
-#pragma unroll
-    for (int a = 0; a < D; ++a) lds[a * 4 + wid] = s[a];
+  if (lane == 0) wbox[wid] = v;
   __syncthreads();
-  if (threadIdx.x == 0)
+  if (threadIdx.x == 0) {
+    for (int k = 1; k < (int)(blockDim.x >> 6); ++k) merge_box<D>(v, wbox[k]);
+    box[blockIdx.x] = v;
+  }
+}
+
+// The centring of the updated Y (HY/gradient_descendHYB.cpp:64-76): every
+// block adds up the update's partials in the same fixed order, subtracts the
+// mean from its points, and block 0 publishes the centred bounds (rounding is
+// monotone, so fl(min y - m) is the minimum of the centred points).
+template <int D>
+__global__ __launch_bounds__(kUpdBlock) void center_kernel(int n, float *__restrict__ Y,
+                                                           const BoxPart *__restrict__ box, int nbox, DevScalars *sc,
+                                                           HostScalars *hs, unsigned long long seq, int stamp) {
+  // every wave adds all the partials itself, as a binary tree over 256 places:
+  // no work-group memory or barrier, and the same bits in every wave
+  const int lane = threadIdx.x & 63;
+  BoxPart v, w;
+  empty_box<D>(v);
+  empty_box<D>(w);
+  if (lane < nbox) v = box[lane];
+  if (lane + 128 < nbox) merge_box<D>(v, box[lane + 128]);
+  if (lane + 64 < nbox) w = box[lane + 64];
+  if (lane + 192 < nbox) merge_box<D>(w, box[lane + 192]);
+  merge_box<D>(v, w);
+  wave_box<D>(v);
+  float m[D];
 #pragma unroll
-    for (int a = 0; a < D; ++a)
-      part[(size_t)blockIdx.x * 8 + a] = lds[a * 4] + lds[a * 4 + 1] + lds[a * 4 + 2] + lds[a * 4 + 3];
+  for (int a = 0; a < D; ++a) m[a] = (float)(v.sum[a] / (double)n);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    for (int a = 0; a < D; ++a) {
+      sc->sum[a] = v.sum[a];
+      sc->mean[a] = 0.0;
+      sc->minv[a] = v.bad > 0.0 ? NAN : (double)(v.mn[a] - m[a]);  // a non-finite coordinate poisons the extent
+      sc->maxv[a] = (double)(v.mx[a] - m[a]);
+    }
+    if (stamp) {
+      const unsigned long long t = wall_clock64();
+      hs->stamp[0] = sc->stamp[STAMP_END];  // this iteration began where the last one ended
+      for (int k = 0; k < 4; ++k) hs->stamp[1 + k] = sc->stamp[k];
+      hs->stamp[5] = t;
+      sc->stamp[STAMP_END] = t;
+    }
+    publish(hs, sc, seq);
+  }
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    float y[D];
+    load_pt<D>(Y, i, y);
+#pragma unroll
+    for (int a = 0; a < D; ++a) y[a] -= m[a];
+    store_pt<D>(Y, i, y);
+  }
 }
 
 // ---- exact O(N^2) repulsion (validation, CU/compute_error.cu:8-53) -------------
@@ -782,7 +934,7 @@ __global__ __launch_bounds__(kBlock) void rep_exact_kernel(int n, const float *_
 // ---- one-block finalisation of the block partials (fixed order) ---------------
 __global__ __launch_bounds__(kBlock) void finalize_kernel(int mode, int nblocks, int d, int n,
                                                           int apply_mean, const double *__restrict__ part,
-                                                          DevScalars *sc) {
+                                                          DevScalars *sc, HostScalars *hs, unsigned long long seq) {
   __shared__ double red[8][kBlock];
   __shared__ double redc[kBlock];
   const int t = threadIdx.x;
@@ -835,13 +987,9 @@ __global__ __launch_bounds__(kBlock) void finalize_kernel(int mode, int nblocks,
         sc->maxv[a] = red[4 + a][0];
         if (apply_mean) sc->mean[a] = 0.0;
       }
+      publish(hs, sc, seq);
     } else if (mode == FIN_ZNEU) {
       sc->Z = (red[0][0] + red[1][0]) - (double)n;
-    } else if (mode == FIN_MEAN) {
-      for (int a = 0; a < d; ++a) {
-        sc->sum[a] = red[a][0];
-        sc->mean[a] = red[a][0] / (double)n;
-      }
     } else if (mode == FIN_ZEXACT) {
       sc->zexact = red[0][0];
     } else if (mode == FIN_KL) {
@@ -855,8 +1003,9 @@ int grid_blocks(int n, int max_blocks) {
   return b < max_blocks ? b : max_blocks;
 }
 
-int finalize(hipStream_t s, int mode, int nblocks, int d, int n, int apply_mean, RedWork rw, DevScalars *sc) {
-  finalize_kernel<<<1, kBlock, 0, s>>>(mode, nblocks, d, n, apply_mean, rw.part, sc);
+int finalize(hipStream_t s, int mode, int nblocks, int d, int n, int apply_mean, RedWork rw, DevScalars *sc,
+             HostScalars *hs = nullptr, unsigned long long seq = 0) {
+  finalize_kernel<<<1, kBlock, 0, s>>>(mode, nblocks, d, n, apply_mean, rw.part, sc, hs, seq);
   SGT_LAUNCH_CHECK();
   return SGTSNE_OK;
 }
@@ -870,7 +1019,8 @@ template <int D>
 __global__ __launch_bounds__(s2g_threads<D>()) void s2g_fix_kernel(GridParams g, float fsf, int n,
                                                                    const float *__restrict__ Y,
                                                                    unsigned long long *__restrict__ Vf, int unit,
-                                                                   int lds_slots) {
+                                                                   int lds_slots, DevScalars *stamp) {
+  stamp_now(stamp, STAMP_S2G);
   extern __shared__ unsigned long long win[];
   __shared__ int sbox[6];
   const int nunits = (n + unit - 1) / unit;
@@ -879,12 +1029,14 @@ __global__ __launch_bounds__(s2g_threads<D>()) void s2g_fix_kernel(GridParams g,
 }
 
 // V = Vf * 2^-e in FP32 (the FP64 product rounded once), Vf cleared.
-__global__ void fix_to_float_kernel(long long *__restrict__ Vf, float *__restrict__ V, int64_t count, double inv) {
+__global__ void fix_to_float_kernel(long long *__restrict__ Vf, float *__restrict__ V, int64_t count, double inv,
+                                    DevScalars *stamp) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += stride) {
     V[i] = (float)((double)Vf[i] * inv);
     Vf[i] = 0;
   }
+  stamp_now(stamp, STAMP_CONV);
 }
 
 }  // namespace
@@ -904,8 +1056,14 @@ int launch_fill(hipStream_t s, float *p, int64_t count, float v) {
   return SGTSNE_OK;
 }
 
+int launch_stamp(hipStream_t s, DevScalars *sc, int at) {
+  stamp_kernel<<<1, 1, 0, s>>>(sc, at);
+  SGT_LAUNCH_CHECK();
+  return SGTSNE_OK;
+}
+
 int launch_center_minmax(hipStream_t s, int d, int n, float *Y, int apply_mean, RedWork rw,
-                         DevScalars *sc) {
+                         DevScalars *sc, HostScalars *hs, unsigned long long seq) {
   const int blocks = grid_blocks(n, std::min(rw.max_blocks, 1024));
   switch (d) {
     case 1: center_minmax_kernel<1><<<blocks, kBlock, 0, s>>>(Y, n, apply_mean, rw.part, sc); break;
@@ -914,7 +1072,7 @@ int launch_center_minmax(hipStream_t s, int d, int n, float *Y, int apply_mean, 
     default: SGT_CHECK(false, SGTSNE_ERR_ARG, "d must be 1..3");
   }
   SGT_LAUNCH_CHECK();
-  return finalize(s, FIN_MINMAX, blocks, d, n, apply_mean, rw, sc);
+  return finalize(s, FIN_MINMAX, blocks, d, n, apply_mean, rw, sc, hs, seq);
 }
 
 // LDS grid copies for the spread: one per point slot of a wave when they fit.
@@ -935,7 +1093,7 @@ int64_t s2g_scratch_need(const GridParams &g, int n, int mode) {
 }
 
 int launch_s2g(hipStream_t s, const GridParams &g, int n, const float *Y, float *V, float *scratch,
-               int64_t scratch_floats, int64_t *needed, int mode) {
+               int64_t scratch_floats, int64_t *needed, int mode, DevScalars *stamp) {
   const bool query = n < 0;  // size query only
   if (query) n = -n;
   if (n > 0 && g.d == 2 && g.ng <= 32 && mode != SGTSNE_SPREAD_ATOMIC) {
@@ -947,11 +1105,11 @@ int launch_s2g(hipStream_t s, const GridParams &g, int n, const float *Y, float 
     if (query) return SGTSNE_OK;
     SGT_CHECK((int64_t)blocks * cells <= scratch_floats, SGTSNE_ERR_STATE, "spread scratch too small");
     if (g.ng <= 16)
-      s2g_mfma_kernel<1><<<blocks, kMfmaBlock, 0, s>>>(g, n, Y, scratch, chunk);
+      s2g_mfma_kernel<1><<<blocks, kMfmaBlock, 0, s>>>(g, n, Y, scratch, chunk, stamp);
     else
-      s2g_mfma_kernel<2><<<blocks, kMfmaBlock, 0, s>>>(g, n, Y, scratch, chunk);
+      s2g_mfma_kernel<2><<<blocks, kMfmaBlock, 0, s>>>(g, n, Y, scratch, chunk, stamp);
     SGT_LAUNCH_CHECK();
-    grid_reduce_kernel<<<div_up(cells, 64), 1024, 0, s>>>(scratch, blocks, (int)cells, V);
+    grid_reduce_kernel<<<div_up(cells, 64), 1024, 0, s>>>(scratch, blocks, (int)cells, V, stamp);
     SGT_LAUNCH_CHECK();
     return SGTSNE_OK;
   }
@@ -961,9 +1119,9 @@ int launch_s2g(hipStream_t s, const GridParams &g, int n, const float *Y, float 
     if (needed) *needed = (int64_t)blocks * cells;
     if (query) return SGTSNE_OK;
     SGT_CHECK((int64_t)blocks * cells <= scratch_floats, SGTSNE_ERR_STATE, "spread scratch too small");
-    s2g_mfma3_kernel<<<blocks, kMfmaBlock, 0, s>>>(g, n, Y, scratch, kMfma3Chunk);
+    s2g_mfma3_kernel<<<blocks, kMfmaBlock, 0, s>>>(g, n, Y, scratch, kMfma3Chunk, stamp);
     SGT_LAUNCH_CHECK();
-    grid_reduce_kernel<<<div_up(cells, 64), 1024, 0, s>>>(scratch, blocks, (int)cells, V);
+    grid_reduce_kernel<<<div_up(cells, 64), 1024, 0, s>>>(scratch, blocks, (int)cells, V, stamp);
     SGT_LAUNCH_CHECK();
     return SGTSNE_OK;
   }
@@ -987,12 +1145,12 @@ int launch_s2g(hipStream_t s, const GridParams &g, int n, const float *Y, float 
     const int lds_b = 64512;  // two work-groups per CU
     const int blocks = (int)std::min<int64_t>(div_up(n, unit), 2048);
     if (g.d == 2)
-      s2g_fix_kernel<2><<<blocks, s2g_threads<2>(), lds_b, s>>>(g, std::ldexp(1.0f, e), n, Y, Vf, unit, lds_b / 8);
+      s2g_fix_kernel<2><<<blocks, s2g_threads<2>(), lds_b, s>>>(g, std::ldexp(1.0f, e), n, Y, Vf, unit, lds_b / 8, stamp);
     else
-      s2g_fix_kernel<3><<<blocks, s2g_threads<3>(), lds_b, s>>>(g, std::ldexp(1.0f, e), n, Y, Vf, unit, lds_b / 8);
+      s2g_fix_kernel<3><<<blocks, s2g_threads<3>(), lds_b, s>>>(g, std::ldexp(1.0f, e), n, Y, Vf, unit, lds_b / 8, stamp);
     SGT_LAUNCH_CHECK();
     fix_to_float_kernel<<<(int)std::min<int64_t>(div_up(cells, 256), 4096), 256, 0, s>>>(
-        reinterpret_cast<long long *>(Vf), V, cells, std::ldexp(1.0, -e));
+        reinterpret_cast<long long *>(Vf), V, cells, std::ldexp(1.0, -e), stamp);
     SGT_LAUNCH_CHECK();
     return SGTSNE_OK;
   }
@@ -1009,48 +1167,51 @@ int launch_s2g(hipStream_t s, const GridParams &g, int n, const float *Y, float 
   if (query) return SGTSNE_OK;
   if (blocks > 0 && (int64_t)blocks * cells <= scratch_floats) {
     switch (g.d) {
-      case 1: s2g_lds_kernel<1><<<blocks, kS2GBlock, lds, s>>>(g, n, Y, scratch, chunk, copies); break;
-      case 2: s2g_lds_kernel<2><<<blocks, kS2GBlock, lds, s>>>(g, n, Y, scratch, chunk, copies); break;
-      case 3: s2g_lds_kernel<3><<<blocks, kS2GBlock, lds, s>>>(g, n, Y, scratch, chunk, copies); break;
+      case 1: s2g_lds_kernel<1><<<blocks, kS2GBlock, lds, s>>>(g, n, Y, scratch, chunk, copies, stamp); break;
+      case 2: s2g_lds_kernel<2><<<blocks, kS2GBlock, lds, s>>>(g, n, Y, scratch, chunk, copies, stamp); break;
+      case 3: s2g_lds_kernel<3><<<blocks, kS2GBlock, lds, s>>>(g, n, Y, scratch, chunk, copies, stamp); break;
       default: SGT_CHECK(false, SGTSNE_ERR_ARG, "d must be 1..3");
     }
     SGT_LAUNCH_CHECK();
-    grid_reduce_kernel<<<div_up(cells, 64), 1024, 0, s>>>(scratch, blocks, (int)cells, V);
+    grid_reduce_kernel<<<div_up(cells, 64), 1024, 0, s>>>(scratch, blocks, (int)cells, V, stamp);
   } else {
     SGT_TRY(launch_fill(s, V, cells, 0.0f));
     const int ppb = (kBlock / 64) * (g.d == 1 ? 16 : g.d == 2 ? 4 : 1);  // points per block per step
     const int ab = (int)std::min<int64_t>(div_up(n > 0 ? n : 1, ppb), 65536);
     switch (g.d) {
-      case 1: s2g_atomic_kernel<1><<<ab, kBlock, 0, s>>>(g, n, Y, V); break;
-      case 2: s2g_atomic_kernel<2><<<ab, kBlock, 0, s>>>(g, n, Y, V); break;
-      case 3: s2g_atomic_kernel<3><<<ab, kBlock, 0, s>>>(g, n, Y, V); break;
+      case 1: s2g_atomic_kernel<1><<<ab, kBlock, 0, s>>>(g, n, Y, V, stamp); break;
+      case 2: s2g_atomic_kernel<2><<<ab, kBlock, 0, s>>>(g, n, Y, V, stamp); break;
+      case 3: s2g_atomic_kernel<3><<<ab, kBlock, 0, s>>>(g, n, Y, V, stamp); break;
       default: SGT_CHECK(false, SGTSNE_ERR_ARG, "d must be 1..3");
     }
+    SGT_LAUNCH_CHECK();
+    if (stamp) SGT_TRY(launch_stamp(s, stamp, STAMP_CONV));
   }
   SGT_LAUNCH_CHECK();
   return SGTSNE_OK;
 }
 
 int launch_g2s_force(hipStream_t s, const GridParams &g, int n, const float *Y, const float *Phi,
-                     float *Frep, int zdirect, RedWork rw, DevScalars *sc) {
+                     float *Frep, int zdirect, RedWork rw, int *nz, DevScalars *stamp) {
   if (g2s_lds_fits(g.d, g.ng)) {
     // one 16-wave work-group per CU (the grid copy takes half of its LDS)
     const int lb = std::max(1, std::min({rw.max_blocks, 256, div_up(n > 0 ? n : 1, kG2sLdsBlock)}));
     if (g.d == 2) {
-      if (zdirect) g2s_lds_kernel<2, true><<<lb, kG2sLdsBlock, 0, s>>>(g, n, Y, Phi, Frep, rw.part);
-      else g2s_lds_kernel<2, false><<<lb, kG2sLdsBlock, 0, s>>>(g, n, Y, Phi, Frep, rw.part);
+      if (zdirect) g2s_lds_kernel<2, true><<<lb, kG2sLdsBlock, 0, s>>>(g, n, Y, Phi, Frep, rw.part, stamp);
+      else g2s_lds_kernel<2, false><<<lb, kG2sLdsBlock, 0, s>>>(g, n, Y, Phi, Frep, rw.part, stamp);
     } else {
-      if (zdirect) g2s_lds_kernel<3, true><<<lb, kG2sLdsBlock, 0, s>>>(g, n, Y, Phi, Frep, rw.part);
-      else g2s_lds_kernel<3, false><<<lb, kG2sLdsBlock, 0, s>>>(g, n, Y, Phi, Frep, rw.part);
+      if (zdirect) g2s_lds_kernel<3, true><<<lb, kG2sLdsBlock, 0, s>>>(g, n, Y, Phi, Frep, rw.part, stamp);
+      else g2s_lds_kernel<3, false><<<lb, kG2sLdsBlock, 0, s>>>(g, n, Y, Phi, Frep, rw.part, stamp);
     }
     SGT_LAUNCH_CHECK();
-    return finalize(s, FIN_ZNEU, lb, g.d, n, 0, rw, sc);
+    *nz = lb;
+    return SGTSNE_OK;
   }
   const int blocks = grid_blocks(n, std::min(rw.max_blocks, 2048));
 #define G2S_CASE(DD)                                                                               \
   case DD:                                                                                         \
-    if (zdirect) g2s_force_kernel<DD, true><<<blocks, kBlock, 0, s>>>(g, n, Y, Phi, Frep, rw.part); \
-    else g2s_force_kernel<DD, false><<<blocks, kBlock, 0, s>>>(g, n, Y, Phi, Frep, rw.part);        \
+    if (zdirect) g2s_force_kernel<DD, true><<<blocks, kBlock, 0, s>>>(g, n, Y, Phi, Frep, rw.part, stamp); \
+    else g2s_force_kernel<DD, false><<<blocks, kBlock, 0, s>>>(g, n, Y, Phi, Frep, rw.part, stamp);        \
     break;
   switch (g.d) {
     G2S_CASE(1)
@@ -1060,25 +1221,44 @@ int launch_g2s_force(hipStream_t s, const GridParams &g, int n, const float *Y, 
   }
 #undef G2S_CASE
   SGT_LAUNCH_CHECK();
-  return finalize(s, FIN_ZNEU, blocks, g.d, n, 0, rw, sc);
+  *nz = blocks;
+  return SGTSNE_OK;
+}
+
+int launch_finalize_z(hipStream_t s, int nz, int n, RedWork rw, DevScalars *sc) {
+  return finalize(s, FIN_ZNEU, nz, 1, n, 0, rw, sc);
 }
 
 int launch_finalize_kl(hipStream_t s, int nblocks, RedWork rw, DevScalars *sc) {
   return finalize(s, FIN_KL, nblocks, 1, 0, 0, rw, sc);
 }
 
-int launch_update(hipStream_t s, int d, int n, float *Y, float *uY, float *gains,
-                  const float *Fattr, const float *Frep, float alpha, float momentum, float eta,
-                  RedWork rw, DevScalars *sc) {
-  const int blocks = grid_blocks(n, std::min(rw.max_blocks, 2048));
+// Work-groups of 256 while one per point fits kMaxBoxParts of them, else of
+// 1024, so that the few partials still leave four waves per SIMD in flight.
+int launch_update_center(hipStream_t s, int d, int n, float *Y, float *uY, float *gains, const float *Fattr,
+                         const float *Frep, float alpha, float momentum, float eta, int nz, RedWork rw,
+                         DevScalars *sc, HostScalars *hs, unsigned long long seq, bool stamp) {
+  const int tpb = n <= kMaxBoxParts * kBlock ? kBlock : kUpdBlock;
+  const int blocks = std::min(div_up(n > 0 ? n : 1, tpb), kMaxBoxParts);
+  // the Z partials take the front of the workspace (at most 2048 slots)
+  SGT_CHECK(nz >= 1 && nz <= 2048 && rw.max_blocks >= 2048 + kMaxBoxParts, SGTSNE_ERR_STATE, "%d partials of Z", nz);
+  BoxPart *box = reinterpret_cast<BoxPart *>(rw.part + (size_t)8 * 2048);
+#define UPD_CASE(DD)                                                                                            \
+  case DD:                                                                                                      \
+    update_kernel<DD><<<blocks, tpb, 0, s>>>(n, Y, uY, gains, Fattr, Frep, alpha, momentum, eta, rw.part, nz, sc, box, \
+                                             stamp);                                                            \
+    SGT_LAUNCH_CHECK();                                                                                         \
+    center_kernel<DD><<<blocks, tpb, 0, s>>>(n, Y, box, blocks, sc, hs, seq, stamp);                            \
+    break;
   switch (d) {
-    case 1: update_kernel<1><<<blocks, kBlock, 0, s>>>(n, Y, uY, gains, Fattr, Frep, alpha, momentum, eta, sc, rw.part); break;
-    case 2: update_kernel<2><<<blocks, kBlock, 0, s>>>(n, Y, uY, gains, Fattr, Frep, alpha, momentum, eta, sc, rw.part); break;
-    case 3: update_kernel<3><<<blocks, kBlock, 0, s>>>(n, Y, uY, gains, Fattr, Frep, alpha, momentum, eta, sc, rw.part); break;
+    UPD_CASE(1)
+    UPD_CASE(2)
+    UPD_CASE(3)
     default: SGT_CHECK(false, SGTSNE_ERR_ARG, "d must be 1..3");
   }
+#undef UPD_CASE
   SGT_LAUNCH_CHECK();
-  return finalize(s, FIN_MEAN, blocks, d, n, 0, rw, sc);
+  return SGTSNE_OK;
 }
 
 int launch_rep_exact(hipStream_t s, int d, int n, const float *Y, float *Frep, RedWork rw,

@@ -94,7 +94,7 @@ typedef struct sgtsne_params {
                          Cuthill-McKee order of P at upload; 2 also tries a
                          Morton order of Y at iterations 50, 150, 300, 600
                          and keeps it when the attractive kernel measures
-                         faster (CSR formats)                            (2)   */
+                         faster (CSR formats, from 4096 points on)       (2)   */
   int spread;         /* SGTSNE_SPREAD_*: how points are spread onto the grid
                          (AUTO: the matrix-core form for 2-D grids of side
                          <= 32 and 3-D grids of side <= 16, else
@@ -224,7 +224,8 @@ int sgtsne_ctx_kl(sgtsne_ctx *ctx, double alpha, double *kl);
 int sgtsne_ctx_repulsive_exact(sgtsne_ctx *ctx, float *Frep, double *Z, int layout);
 
 /* Per-phase device time of the last sgtsne_ctx_step call, ms summed over
- * its iterations: [0] attractive, [1] S2G (incl. binning), [2] G2G (FFT
+ * its iterations, from the device clock at the start of each phase's first
+ * kernel: [0] attractive (with any wait for the host to size the grid), [1] S2G (incl. binning), [2] G2G (FFT
  * convolution), [3] G2S + forces, [4] update, [5] total, [6] iterations. */
 int sgtsne_ctx_timing(sgtsne_ctx *ctx, double *out7);
 
@@ -252,7 +253,7 @@ int sgtsne_ctx_set_attractive(sgtsne_ctx *ctx, int group, int unroll, int rows_p
  * declined because the attractive kernel measured slower on them. */
 int sgtsne_ctx_reorders(sgtsne_ctx *ctx, int *applied, int *declined);
 
-/* Enables (default) or disables the per-phase event timing of ctx_step. */
+/* Enables (default) or disables the per-phase timing of ctx_step. */
 int sgtsne_ctx_set_timing(sgtsne_ctx *ctx, int on);
 
 /* Relative L2 errors recorded by params.compute_error > 0 (one every 10
