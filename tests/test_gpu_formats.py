@@ -1,0 +1,60 @@
+"""COO and hybrid attractive kernels at the edges of their runs, against the FP64 oracle."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-5  # FP32 sums of up to 3000 terms: below 3000 * 2^-24 / sqrt(3000) of their size
+
+
+@pytest.fixture(scope="module")
+def sg():
+    import sgtsne_amd
+
+    return sgtsne_amd
+
+
+@pytest.fixture(scope="module")
+def O():
+    from oracle import oracle
+
+    return oracle
+
+
+def _matrix(kind, n, rng):
+    """Symmetric patterns whose rows end inside lanes, fill them, and span waves."""
+    if kind == "single":  # rows of one entry: every entry ends a run
+        i = np.arange(n)
+        rows, cols = i, i ^ 1
+    elif kind == "hub":  # one row of n - 1 entries (many waves), the others of one
+        rows = np.concatenate([np.zeros(n - 1, int), np.arange(1, n)])
+        cols = np.concatenate([np.arange(1, n), np.zeros(n - 1, int)])
+    else:  # ragged rows, some of them empty
+        dense = rng.random((n, n)) < np.minimum(0.9, rng.pareto(1.0, n) * 0.02)[:, None]
+        dense[::7] = False
+        dense[:, ::7] = False
+        dense |= dense.T
+        np.fill_diagonal(dense, False)
+        rows, cols = np.nonzero(dense)
+    order = np.lexsort((cols, rows))
+    rows, cols = rows[order], cols[order]
+    rp = np.zeros(n + 1, np.int64)
+    np.add.at(rp, rows + 1, 1)
+    val = np.full(rows.size, 1.0 / rows.size)
+    return np.cumsum(rp), cols.astype(np.int32), val
+
+
+@pytest.mark.parametrize("fmt,width", [("COO", 0), ("HYBRID", 0), ("HYBRID", 1), ("HYBRID", 33)])
+@pytest.mark.parametrize("kind,n,d", [("single", 514, 2), ("hub", 3000, 1), ("ragged", 257, 3), ("ragged", 640, 2)])
+def test_attractive_runs(sg, O, fmt, width, kind, n, d):
+    rng = np.random.default_rng(n + d)
+    rp, col, val = _matrix(kind, n, rng)
+    Y = (rng.standard_normal((n, d)) * 3).astype(np.float32)
+    prm = sg.tsneparams(d=d, format=getattr(sg, "FORMAT_" + fmt), ell_width=width, reorder=0)
+    with sg.Context(prm) as ctx:
+        ctx.upload_P(sg.CSR(n, rp, col, val), symmetrize=False)
+        ctx.set_Y(Y)
+        Fa = ctx.terms()[0]
+        Yc = ctx.get_Y().astype(np.float64)
+    ref = O.attractive(O.CSR(n, rp.astype(np.int64), col, val.astype(np.float32).astype(np.float64)), Yc)
+    assert np.linalg.norm(Fa - ref) <= TOL * np.linalg.norm(ref)
