@@ -136,6 +136,8 @@ struct sgtsne_ctx {
   int reorders = 0;
   int reorders_declined = 0;  // Morton orders measured slower than the current one
   std::vector<int32_t> perm, iperm;
+  int32_t *perm_d = nullptr;  // perm on the device (when permuted)
+  float *io = nullptr;        // a point array in the caller's order, on its way in or out
 };
 
 namespace {
@@ -362,13 +364,6 @@ int repulsive(sgtsne_ctx *c, const GridParams &g, bool stamp, int *nz) {
   return SGTSNE_OK;
 }
 
-// Centres Y by the mean in c->sc (when asked) and queues the publication of
-// its bounds.
-int center_and_publish(sgtsne_ctx *c, int apply_mean) {
-  c->stamped = false;
-  return launch_center_minmax(c->stream, c->d, c->n, c->Y, apply_mean, c->rw, c->sc, c->hs, ++c->seq);
-}
-
 // Waits for the last queued publication.  The device writes the sequence
 // number after everything else; a stream that has drained (or failed) without
 // it ends the wait.
@@ -544,6 +539,9 @@ int spatial_reorder(sgtsne_ctx *c) {
   c->perm.swap(np);
   c->iperm.assign(n, 0);
   for (int r = 0; r < n; r++) c->iperm[c->perm[r]] = r;
+  if (!c->perm_d) SGT_TRY(alloc_dev((void **)&c->perm_d, sizeof(int32_t) * (size_t)n));
+  SGT_HIP(hipMemcpyAsync(c->perm_d, c->perm.data(), sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice, c->stream));
+  SGT_HIP(hipStreamSynchronize(c->stream));
   c->permuted = true;
   c->reorders++;
   // the column-localised blocks follow the order
@@ -624,27 +622,12 @@ int iterate(sgtsne_ctx *c) {
   return SGTSNE_OK;
 }
 
-// caller order <-> device order (perm empty: identity)
-void pack_y(const float *y, int layout, int n, int d, int ds, const std::vector<int32_t> &perm,
-            std::vector<float> &out) {
-  out.assign((size_t)n * ds, 0.0f);
-  for (int r = 0; r < n; r++) {
-    const int i = perm.empty() ? r : perm[r];
-    for (int a = 0; a < d; a++)
-      out[(size_t)r * ds + a] = layout == SGTSNE_LAYOUT_AOS ? y[(size_t)i * d + a] : y[(size_t)a * n + i];
-  }
-}
-
-void unpack_y(const std::vector<float> &in, int layout, int n, int d, int ds, const std::vector<int32_t> &perm,
-              float *y, double scale = 1.0) {
-  for (int r = 0; r < n; r++) {
-    const int i = perm.empty() ? r : perm[r];
-    for (int a = 0; a < d; a++) {
-      float v = (float)(in[(size_t)r * ds + a] * scale);
-      if (layout == SGTSNE_LAYOUT_AOS) y[(size_t)i * d + a] = v;
-      else y[(size_t)a * n + i] = v;
-    }
-  }
+// A point array of the device (its order) into the caller's order and layout.
+int fetch_points(sgtsne_ctx *c, const float *in, int layout, double scale, float *out) {
+  SGT_TRY(launch_get_points(c->stream, c->d, c->n, in, layout, c->permuted ? c->perm_d : nullptr, scale, c->io));
+  SGT_HIP(hipMemcpyAsync(out, c->io, sizeof(float) * (size_t)c->n * c->d, hipMemcpyDeviceToHost, c->stream));
+  SGT_HIP(hipStreamSynchronize(c->stream));
+  return SGTSNE_OK;
 }
 
 // Breadth-first order of the graph of P (Cuthill-McKee without the degree
@@ -789,7 +772,8 @@ int apply_locality_order(sgtsne_ctx *c) {
   SGT_HIP(hipMemcpyAsync(diperm, c->iperm.data(), sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice, c->stream));
   int st = launch_permute_csr(c->stream, n, c->nnz, dperm, diperm, c->rowptr, c->col, c->val, rp2, col2, val2);
   (void)hipStreamSynchronize(c->stream);
-  free_dev(dperm);
+  free_dev(c->perm_d);
+  c->perm_d = dperm;  // kept: the points' way in and out
   free_dev(diperm);
   free_dev(c->rowptr);
   free_dev(c->col);
@@ -810,6 +794,9 @@ int alloc_points(sgtsne_ctx *c) {
   free_dev(c->gains);
   free_dev(c->Fattr);
   free_dev(c->Frep);
+  free_dev(c->io);
+  c->points_n = 0;
+  SGT_TRY(alloc_dev((void **)&c->io, sizeof(float) * (size_t)c->n * c->d));
   SGT_TRY(alloc_dev((void **)&c->Y, nb * sizeof(float)));
   SGT_TRY(alloc_dev((void **)&c->uY, nb * sizeof(float)));
   SGT_TRY(alloc_dev((void **)&c->gains, nb * sizeof(float)));
@@ -1078,6 +1065,8 @@ int sgtsne_ctx_destroy(sgtsne_ctx *c) {
   free_dev(c->gains);
   free_dev(c->Fattr);
   free_dev(c->Frep);
+  free_dev(c->io);
+  free_dev(c->perm_d);
   free_dev(c->rw.part);
   free_dev(c->rw.ticket);
   free_dev(c->sc);
@@ -1119,6 +1108,7 @@ int sgtsne_ctx_upload_P(sgtsne_ctx *c, int n, int64_t nnz, const int32_t *rowptr
   c->permuted = false;
   c->perm.clear();
   c->iperm.clear();
+  free_dev(c->perm_d);
   int32_t *rp = nullptr, *cc = nullptr;
   float *vv = nullptr;
   SGT_TRY(alloc_dev((void **)&rp, sizeof(int32_t) * ((size_t)n + 1)));
@@ -1201,29 +1191,13 @@ int sgtsne_ctx_set_Y(sgtsne_ctx *c, const float *y, int layout, int reset_state)
   SGT_CHECK(layout == SGTSNE_LAYOUT_SOA || layout == SGTSNE_LAYOUT_AOS, SGTSNE_ERR_ARG, "bad layout");
   int n = c->n;
   SGT_CHECK(n > 0, SGTSNE_ERR_STATE, "upload P before Y (n unknown)");
-  const size_t nb = (size_t)n * c->ds;
   SGT_TRY(alloc_points(c));
   if (!c->have_Y) reset_state = 1;
-  std::vector<float> h;
-  pack_y(y, layout, n, c->d, c->ds, c->perm, h);
-  double mean[4] = {0, 0, 0, 0};
-  for (int a = 0; a < c->d; a++) {
-    double s = 0;
-    for (int i = 0; i < n; i++) s += h[(size_t)i * c->ds + a];
-    mean[a] = s / n;
-  }
-  SGT_HIP(hipMemcpyAsync(c->Y, h.data(), nb * sizeof(float), hipMemcpyHostToDevice, c->stream));
-  SGT_HIP(hipStreamSynchronize(c->stream));
-  DevScalars s{};
-  SGT_HIP(hipMemcpy(&s, c->sc, sizeof(DevScalars), hipMemcpyDeviceToHost));
-  for (int a = 0; a < 4; a++) s.mean[a] = mean[a];
-  SGT_HIP(hipMemcpy(c->sc, &s, sizeof(DevScalars), hipMemcpyHostToDevice));
-  if (reset_state) {
-    SGT_TRY(launch_fill(c->stream, c->uY, (int64_t)nb, 0.0f));
-    SGT_TRY(launch_fill(c->stream, c->gains, (int64_t)nb, 1.0f));
-    c->iter = 0;
-  }
-  SGT_TRY(center_and_publish(c, 1));
+  SGT_HIP(hipMemcpyAsync(c->io, y, sizeof(float) * (size_t)n * c->d, hipMemcpyHostToDevice, c->stream));
+  if (reset_state) c->iter = 0;
+  c->stamped = false;
+  SGT_TRY(launch_set_points(c->stream, c->d, n, c->io, layout, c->permuted ? c->perm_d : nullptr, c->Y, reset_state,
+                            c->uY, c->gains, c->rw, c->sc, c->hs, ++c->seq));
   SGT_HIP(hipStreamSynchronize(c->stream));
   c->have_Y = true;
   return SGTSNE_OK;
@@ -1232,11 +1206,7 @@ int sgtsne_ctx_set_Y(sgtsne_ctx *c, const float *y, int layout, int reset_state)
 int sgtsne_ctx_get_Y(sgtsne_ctx *c, float *y, int layout) {
   SGT_CHECK(c != nullptr && y != nullptr, SGTSNE_ERR_ARG, "bad arguments");
   SGT_CHECK(c->have_Y, SGTSNE_ERR_STATE, "Y not set");
-  std::vector<float> h((size_t)c->n * c->ds);
-  SGT_HIP(hipStreamSynchronize(c->stream));
-  SGT_HIP(hipMemcpy(h.data(), c->Y, h.size() * sizeof(float), hipMemcpyDeviceToHost));
-  unpack_y(h, layout, c->n, c->d, c->ds, c->perm, y);
-  return SGTSNE_OK;
+  return fetch_points(c, c->Y, layout, 1.0, y);
 }
 
 int sgtsne_ctx_step(sgtsne_ctx *c, int iters) {
@@ -1256,28 +1226,18 @@ int sgtsne_ctx_step(sgtsne_ctx *c, int iters) {
 int sgtsne_ctx_terms(sgtsne_ctx *c, float *Fattr, float *Frep, double *Z, int *ng, int layout) {
   SGT_CHECK(c != nullptr, SGTSNE_ERR_ARG, "ctx is NULL");
   SGT_CHECK(c->have_P && c->have_Y, SGTSNE_ERR_STATE, "upload P and set Y first");
-  SGT_HIP(hipStreamSynchronize(c->stream));
-  SGT_TRY(center_and_publish(c, 0));
   SGT_TRY(attractive(c));
-  SGT_TRY(wait_published(c));
+  SGT_TRY(wait_published(c));  // the bounds of the current Y
   GridParams g{};
   SGT_TRY(make_grid(c, *c->hs, g));
   int nz = 0;
   SGT_TRY(repulsive(c, g, false, &nz));
   SGT_TRY(launch_finalize_z(c->stream, nz, c->n, c->rw, c->sc));
-  SGT_HIP(hipStreamSynchronize(c->stream));
   DevScalars s{};
-  SGT_HIP(hipMemcpy(&s, c->sc, sizeof(DevScalars), hipMemcpyDeviceToHost));
-  const size_t nb = (size_t)c->n * c->ds;
-  std::vector<float> h(nb);
-  if (Fattr) {
-    SGT_HIP(hipMemcpy(h.data(), c->Fattr, nb * sizeof(float), hipMemcpyDeviceToHost));
-    unpack_y(h, layout, c->n, c->d, c->ds, c->perm, Fattr);
-  }
-  if (Frep) {
-    SGT_HIP(hipMemcpy(h.data(), c->Frep, nb * sizeof(float), hipMemcpyDeviceToHost));
-    unpack_y(h, layout, c->n, c->d, c->ds, c->perm, Frep, 1.0 / s.Z);
-  }
+  SGT_HIP(hipMemcpyAsync(&s, c->sc, sizeof(DevScalars), hipMemcpyDeviceToHost, c->stream));
+  SGT_HIP(hipStreamSynchronize(c->stream));
+  if (Fattr) SGT_TRY(fetch_points(c, c->Fattr, layout, 1.0, Fattr));
+  if (Frep) SGT_TRY(fetch_points(c, c->Frep, layout, 1.0 / s.Z, Frep));
   if (Z) *Z = s.Z;
   if (ng) *ng = g.ng;
   return SGTSNE_OK;
@@ -1300,20 +1260,17 @@ int sgtsne_ctx_repulsive_exact(sgtsne_ctx *c, float *Frep, double *Z, int layout
   SGT_CHECK(c != nullptr, SGTSNE_ERR_ARG, "ctx is NULL");
   SGT_CHECK(c->have_Y, SGTSNE_ERR_STATE, "Y not set");
   SGT_HIP(hipStreamSynchronize(c->stream));
-  const size_t nb = (size_t)c->n * c->ds;
   float *tmp = nullptr;
-  SGT_TRY(alloc_dev((void **)&tmp, nb * sizeof(float)));
+  SGT_TRY(alloc_dev((void **)&tmp, sizeof(float) * (size_t)c->n * c->ds));
   int st = launch_rep_exact(c->stream, c->d, c->n, c->Y, tmp, c->rw, c->sc);
-  std::vector<float> h(nb);
   DevScalars s{};
   if (st == SGTSNE_OK) {
     (void)hipStreamSynchronize(c->stream);
-    (void)hipMemcpy(h.data(), tmp, nb * sizeof(float), hipMemcpyDeviceToHost);
     (void)hipMemcpy(&s, c->sc, sizeof(DevScalars), hipMemcpyDeviceToHost);
+    if (Frep) st = fetch_points(c, tmp, layout, 1.0 / s.zexact, Frep);
   }
   free_dev(tmp);
   SGT_TRY(st);
-  if (Frep) unpack_y(h, layout, c->n, c->d, c->ds, c->perm, Frep, 1.0 / s.zexact);
   if (Z) *Z = s.zexact;
   return SGTSNE_OK;
 }

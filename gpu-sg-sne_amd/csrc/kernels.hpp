@@ -9,10 +9,8 @@ namespace sgt {
 
 // Scalars the iteration keeps on the device (reductions and Z).
 struct DevScalars {
-  double sum[4];    // sum of Y per dimension (after the update)
   double minv[4];   // min of the centred Y per dimension
   double maxv[4];   // max of the centred Y per dimension
-  double mean[4];   // mean subtracted by the centring kernel
   double Z;         // normalisation term (sum z_i - N)
   double kl;        // KL divergence (tsneCost)
   double zexact;    // exact-repulsion Z (validation)
@@ -89,9 +87,14 @@ int launch_kl(hipStream_t s, int d, int n, const int32_t *rowptr, const int32_t 
 // ---- repulsion (kernels_grid.hip) ----
 int launch_fill(hipStream_t s, float *p, int64_t count, float v);
 int launch_stream_copy(hipStream_t s, const float4 *in, float4 *out, int64_t count);
-// Y -= sc->mean (when asked), then min / max of Y into sc and hs.
-int launch_center_minmax(hipStream_t s, int d, int n, float *Y, int apply_mean, RedWork rw,
-                         DevScalars *sc, HostScalars *hs, unsigned long long seq);
+// Caller's points (raw [n][d] or [d][n], perm: row -> caller's index, NULL: the
+// same) into Y, centred, with min / max into sc and hs; reset: uY = 0, gains = 1.
+int launch_set_points(hipStream_t s, int d, int n, const float *raw, int layout, const int32_t *perm, float *Y,
+                      int reset, float *uY, float *gains, RedWork rw, DevScalars *sc, HostScalars *hs,
+                      unsigned long long seq);
+// The reverse for Y or a force, each coordinate times scale (in FP64).
+int launch_get_points(hipStream_t s, int d, int n, const float *in, int layout, const int32_t *perm, double scale,
+                      float *raw);
 // S2G into V [d+1][ng^d] (V is overwritten).  scratch: float workspace for the
 // per-block private grids of the LDS path; *needed receives the floats it
 // wants (when larger than scratch_floats the global-atomic path runs).

@@ -32,7 +32,7 @@ namespace {
 
 constexpr int kBlock = 256;
 
-enum FinMode { FIN_MINMAX = 0, FIN_ZNEU = 1, FIN_ZEXACT = 2, FIN_KL = 3 };
+enum FinMode { FIN_ZNEU, FIN_ZEXACT, FIN_KL };
 
 // Device clock into stamp[at], by one thread of the launch (NULL: no timing).
 __device__ __forceinline__ void stamp_now(DevScalars *sc, int at) {
@@ -62,66 +62,6 @@ __global__ void fill_kernel(float *__restrict__ p, int64_t count, float v) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (; i < count; i += stride) p[i] = v;
-}
-
-// ---- centring + min/max ------------------------------------------------------
-// Y -= mean (the mean of the last update, HY/gradient_descendHYB.cpp:64-76),
-// then per-block min/max of the centred Y (HY/qq.cpp:147-163) and a count of
-// non-finite coordinates.
-template <int D>
-__global__ __launch_bounds__(kBlock) void center_minmax_kernel(float *__restrict__ Y, int n,
-                                                               int apply_mean, double *part,
-                                                               const DevScalars *sc) {
-  __shared__ double lds[(2 * D + 1) * 4];
-  float m[D];
-#pragma unroll
-  for (int a = 0; a < D; ++a) m[a] = apply_mean ? (float)sc->mean[a] : 0.0f;
-  float mn[D], mx[D];
-  float bad = 0.0f;
-#pragma unroll
-  for (int a = 0; a < D; ++a) { mn[a] = INFINITY; mx[a] = -INFINITY; }
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    float y[D];
-    load_pt<D>(Y, i, y);
-    if (apply_mean) {
-#pragma unroll
-      for (int a = 0; a < D; ++a) y[a] -= m[a];
-      store_pt<D>(Y, i, y);
-    }
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-      mn[a] = fminf(mn[a], y[a]);
-      mx[a] = fmaxf(mx[a], y[a]);
-      bad += isfinite(y[a]) ? 0.0f : 1.0f;
-    }
-  }
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  double vmin[D], vmax[D];
-#pragma unroll
-  for (int a = 0; a < D; ++a) {
-    vmin[a] = wave_min((double)mn[a]);
-    vmax[a] = wave_max((double)mx[a]);
-  }
-  const double vbad = wave_sum((double)bad);
-  if (lane == 0) {
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-      lds[a * 4 + wid] = vmin[a];
-      lds[(D + a) * 4 + wid] = vmax[a];
-    }
-    lds[2 * D * 4 + wid] = vbad;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double *pb = part + (size_t)blockIdx.x * 8;
-#pragma unroll
-    for (int a = 0; a < D; ++a) {
-      pb[a] = fmin(fmin(lds[a * 4], lds[a * 4 + 1]), fmin(lds[a * 4 + 2], lds[a * 4 + 3]));
-      pb[4 + a] = fmax(fmax(lds[(D + a) * 4], lds[(D + a) * 4 + 1]),
-                       fmax(lds[(D + a) * 4 + 2], lds[(D + a) * 4 + 3]));
-    }
-    pb[3] = lds[2 * D * 4] + lds[2 * D * 4 + 1] + lds[2 * D * 4 + 2] + lds[2 * D * 4 + 3];
-  }
 }
 
 // ---- S2G, LDS-privatised whole grid -------------------------------------------
@@ -778,6 +718,31 @@ __device__ __forceinline__ void merge_box(BoxPart &v, const BoxPart &w) {
 constexpr int kUpdBlock = 1024;  // largest work-group of the update and the centring
 
 template <int D>
+__device__ __forceinline__ void add_box(BoxPart &v, const float (&y)[D]) {
+#pragma unroll
+  for (int a = 0; a < D; ++a) {
+    v.sum[a] += (double)y[a];
+    v.mn[a] = fminf(v.mn[a], y[a]);
+    v.mx[a] = fmaxf(v.mx[a], y[a]);
+    v.bad += isfinite(y[a]) ? 0.0 : 1.0;
+  }
+}
+
+// The block's partial from its threads' (every thread calls it).
+template <int D>
+__device__ __forceinline__ void block_box(BoxPart &v, BoxPart *__restrict__ box) {
+  __shared__ BoxPart wbox[kUpdBlock / 64];
+  wave_box<D>(v);
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  if (lane == 0) wbox[wid] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int k = 1; k < (int)(blockDim.x >> 6); ++k) merge_box<D>(v, wbox[k]);
+    box[blockIdx.x] = v;
+  }
+}
+
+template <int D>
 __global__ __launch_bounds__(kUpdBlock) void update_kernel(int n, float *__restrict__ Y,
                                                         float *__restrict__ uY,
                                                         float *__restrict__ gains,
@@ -788,7 +753,6 @@ __global__ __launch_bounds__(kUpdBlock) void update_kernel(int n, float *__restr
                                                         BoxPart *__restrict__ box, int stamp) {
   stamp_now(stamp ? sc : nullptr, STAMP_UPDATE);
   __shared__ double red[2][kBlock];
-  __shared__ BoxPart wbox[kUpdBlock / 64];
   const Neu zs = block_neu(zpart, nz, red);
   const double Z = (zs.s + zs.c) - (double)n;
   if (blockIdx.x == 0 && threadIdx.x == 0) sc->Z = Z;
@@ -810,22 +774,56 @@ __global__ __launch_bounds__(kUpdBlock) void update_kernel(int n, float *__restr
       gn[a] = gg;
       u[a] = momentum * u[a] - eta * gg * dy;
       y[a] = y[a] + u[a];
-      v.sum[a] += (double)y[a];
-      v.mn[a] = fminf(v.mn[a], y[a]);
-      v.mx[a] = fmaxf(v.mx[a], y[a]);
-      v.bad += isfinite(y[a]) ? 0.0 : 1.0;
     }
+    add_box<D>(v, y);
     store_pt<D>(Y, i, y);
     store_pt<D>(uY, i, u);
     store_pt<D>(gains, i, gn);
   }
-  wave_box<D>(v);
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  if (lane == 0) wbox[wid] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int k = 1; k < (int)(blockDim.x >> 6); ++k) merge_box<D>(v, wbox[k]);
-    box[blockIdx.x] = v;
+  block_box<D>(v, box);
+}
+
+// Caller's points into the device's order and layout, with the partials the
+// centring needs; the fresh optimiser state along with them.
+template <int D>
+__global__ __launch_bounds__(kUpdBlock) void set_points_kernel(int n, const float *__restrict__ raw, int aos,
+                                                               const int32_t *__restrict__ perm,
+                                                               float *__restrict__ Y, int reset,
+                                                               float *__restrict__ uY, float *__restrict__ gains,
+                                                               BoxPart *__restrict__ box) {
+  BoxPart v;
+  empty_box<D>(v);
+  for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < n; r += gridDim.x * blockDim.x) {
+    const int64_t i = perm ? perm[r] : r;
+    float y[D];
+#pragma unroll
+    for (int a = 0; a < D; ++a) y[a] = aos ? raw[i * D + a] : raw[(int64_t)a * n + i];
+    store_pt<D>(Y, r, y);
+    add_box<D>(v, y);
+    if (reset) {
+      float z[D], o[D];
+#pragma unroll
+      for (int a = 0; a < D; ++a) {
+        z[a] = 0.0f;
+        o[a] = 1.0f;
+      }
+      store_pt<D>(uY, r, z);
+      store_pt<D>(gains, r, o);
+    }
+  }
+  block_box<D>(v, box);
+}
+
+template <int D>
+__global__ __launch_bounds__(kBlock) void get_points_kernel(int n, const float *__restrict__ in, int aos,
+                                                            const int32_t *__restrict__ perm, double scale,
+                                                            float *__restrict__ raw) {
+  for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < n; r += gridDim.x * blockDim.x) {
+    const int64_t i = perm ? perm[r] : r;
+    float y[D];
+    load_pt<D>(in, r, y);
+#pragma unroll
+    for (int a = 0; a < D; ++a) raw[aos ? i * D + a : (int64_t)a * n + i] = (float)((double)y[a] * scale);
   }
 }
 
@@ -854,8 +852,6 @@ __global__ __launch_bounds__(kUpdBlock) void center_kernel(int n, float *__restr
   for (int a = 0; a < D; ++a) m[a] = (float)(v.sum[a] / (double)n);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     for (int a = 0; a < D; ++a) {
-      sc->sum[a] = v.sum[a];
-      sc->mean[a] = 0.0;
       sc->minv[a] = v.bad > 0.0 ? NAN : (double)(v.mn[a] - m[a]);  // a non-finite coordinate poisons the extent
       sc->maxv[a] = (double)(v.mx[a] - m[a]);
     }
@@ -932,70 +928,24 @@ __global__ __launch_bounds__(kBlock) void rep_exact_kernel(int n, const float *_
 }
 
 // ---- one-block finalisation of the block partials (fixed order) ---------------
-__global__ __launch_bounds__(kBlock) void finalize_kernel(int mode, int nblocks, int d, int n,
-                                                          int apply_mean, const double *__restrict__ part,
-                                                          DevScalars *sc, HostScalars *hs, unsigned long long seq) {
-  __shared__ double red[8][kBlock];
-  __shared__ double redc[kBlock];
-  const int t = threadIdx.x;
-  double acc[8];
-  Neu zn{0.0, 0.0};
-  for (int k = 0; k < 8; ++k) acc[k] = (mode == FIN_MINMAX) ? (k < 4 ? INFINITY : -INFINITY) : 0.0;
-  if (mode == FIN_MINMAX) acc[3] = 0.0;
-  for (int b = t; b < nblocks; b += kBlock) {
-    const double *pb = part + (size_t)b * 8;
-    if (mode == FIN_MINMAX) {
-      for (int a = 0; a < d; ++a) {
-        acc[a] = fmin(acc[a], pb[a]);
-        acc[4 + a] = fmax(acc[4 + a], pb[4 + a]);
-      }
-      acc[3] += pb[3];
-    } else if (mode == FIN_ZNEU) {
-      neu_merge(zn, Neu{pb[0], pb[1]});
-    } else {
-      for (int a = 0; a < 4; ++a) acc[a] += pb[a];
-    }
+__global__ __launch_bounds__(kBlock) void finalize_kernel(int mode, int nblocks, int n,
+                                                          const double *__restrict__ part, DevScalars *sc) {
+  __shared__ double red[2][kBlock];
+  if (mode == FIN_ZNEU) {
+    const Neu z = block_neu(part, nblocks, red);
+    if (threadIdx.x == 0) sc->Z = (z.s + z.c) - (double)n;
+    return;
   }
-  if (mode == FIN_ZNEU) { acc[0] = zn.s; acc[1] = zn.c; }
-  for (int k = 0; k < 8; ++k) red[k][t] = acc[k];
+  const int t = threadIdx.x;
+  double acc = 0.0;
+  for (int b = t; b < nblocks; b += kBlock) acc += part[(size_t)b * 8];
+  red[0][t] = acc;
   __syncthreads();
   for (int s = kBlock / 2; s > 0; s >>= 1) {
-    if (t < s) {
-      if (mode == FIN_MINMAX) {
-        for (int a = 0; a < 3; ++a) {
-          red[a][t] = fmin(red[a][t], red[a][t + s]);
-          red[4 + a][t] = fmax(red[4 + a][t], red[4 + a][t + s]);
-        }
-        red[3][t] += red[3][t + s];
-      } else if (mode == FIN_ZNEU) {
-        Neu x{red[0][t], red[1][t]};
-        neu_merge(x, Neu{red[0][t + s], red[1][t + s]});
-        red[0][t] = x.s;
-        red[1][t] = x.c;
-      } else {
-        for (int a = 0; a < 4; ++a) red[a][t] += red[a][t + s];
-      }
-    }
+    if (t < s) red[0][t] += red[0][t + s];
     __syncthreads();
   }
-  (void)redc;
-  if (t == 0) {
-    if (mode == FIN_MINMAX) {
-      const bool bad = red[3][0] > 0.0;
-      for (int a = 0; a < d; ++a) {
-        sc->minv[a] = bad ? NAN : red[a][0];  // a non-finite coordinate poisons the extent
-        sc->maxv[a] = red[4 + a][0];
-        if (apply_mean) sc->mean[a] = 0.0;
-      }
-      publish(hs, sc, seq);
-    } else if (mode == FIN_ZNEU) {
-      sc->Z = (red[0][0] + red[1][0]) - (double)n;
-    } else if (mode == FIN_ZEXACT) {
-      sc->zexact = red[0][0];
-    } else if (mode == FIN_KL) {
-      sc->kl = red[0][0];
-    }
-  }
+  if (t == 0) (mode == FIN_ZEXACT ? sc->zexact : sc->kl) = red[0][0];
 }
 
 int grid_blocks(int n, int max_blocks) {
@@ -1003,9 +953,8 @@ int grid_blocks(int n, int max_blocks) {
   return b < max_blocks ? b : max_blocks;
 }
 
-int finalize(hipStream_t s, int mode, int nblocks, int d, int n, int apply_mean, RedWork rw, DevScalars *sc,
-             HostScalars *hs = nullptr, unsigned long long seq = 0) {
-  finalize_kernel<<<1, kBlock, 0, s>>>(mode, nblocks, d, n, apply_mean, rw.part, sc, hs, seq);
+int finalize(hipStream_t s, int mode, int nblocks, int n, RedWork rw, DevScalars *sc) {
+  finalize_kernel<<<1, kBlock, 0, s>>>(mode, nblocks, n, rw.part, sc);
   SGT_LAUNCH_CHECK();
   return SGTSNE_OK;
 }
@@ -1060,19 +1009,6 @@ int launch_stamp(hipStream_t s, DevScalars *sc, int at) {
   stamp_kernel<<<1, 1, 0, s>>>(sc, at);
   SGT_LAUNCH_CHECK();
   return SGTSNE_OK;
-}
-
-int launch_center_minmax(hipStream_t s, int d, int n, float *Y, int apply_mean, RedWork rw,
-                         DevScalars *sc, HostScalars *hs, unsigned long long seq) {
-  const int blocks = grid_blocks(n, std::min(rw.max_blocks, 1024));
-  switch (d) {
-    case 1: center_minmax_kernel<1><<<blocks, kBlock, 0, s>>>(Y, n, apply_mean, rw.part, sc); break;
-    case 2: center_minmax_kernel<2><<<blocks, kBlock, 0, s>>>(Y, n, apply_mean, rw.part, sc); break;
-    case 3: center_minmax_kernel<3><<<blocks, kBlock, 0, s>>>(Y, n, apply_mean, rw.part, sc); break;
-    default: SGT_CHECK(false, SGTSNE_ERR_ARG, "d must be 1..3");
-  }
-  SGT_LAUNCH_CHECK();
-  return finalize(s, FIN_MINMAX, blocks, d, n, apply_mean, rw, sc, hs, seq);
 }
 
 // LDS grid copies for the spread: one per point slot of a wave when they fit.
@@ -1226,23 +1162,61 @@ int launch_g2s_force(hipStream_t s, const GridParams &g, int n, const float *Y, 
 }
 
 int launch_finalize_z(hipStream_t s, int nz, int n, RedWork rw, DevScalars *sc) {
-  return finalize(s, FIN_ZNEU, nz, 1, n, 0, rw, sc);
+  return finalize(s, FIN_ZNEU, nz, n, rw, sc);
 }
 
 int launch_finalize_kl(hipStream_t s, int nblocks, RedWork rw, DevScalars *sc) {
-  return finalize(s, FIN_KL, nblocks, 1, 0, 0, rw, sc);
+  return finalize(s, FIN_KL, nblocks, 0, rw, sc);
 }
 
 // Work-groups of 256 while one per point fits kMaxBoxParts of them, else of
 // 1024, so that the few partials still leave four waves per SIMD in flight.
+int upd_threads(int n) { return n <= kMaxBoxParts * kBlock ? kBlock : kUpdBlock; }
+int upd_blocks(int n) { return std::min(div_up(n > 0 ? n : 1, upd_threads(n)), kMaxBoxParts); }
+// the Z partials take the front of the workspace (at most 2048 slots)
+BoxPart *box_parts(const RedWork &rw) { return reinterpret_cast<BoxPart *>(rw.part + (size_t)8 * 2048); }
+
+int launch_set_points(hipStream_t s, int d, int n, const float *raw, int layout, const int32_t *perm, float *Y,
+                      int reset, float *uY, float *gains, RedWork rw, DevScalars *sc, HostScalars *hs,
+                      unsigned long long seq) {
+  const int tpb = upd_threads(n), blocks = upd_blocks(n), aos = layout == SGTSNE_LAYOUT_AOS;
+  BoxPart *box = box_parts(rw);
+#define SET_CASE(DD)                                                                                  \
+  case DD:                                                                                            \
+    set_points_kernel<DD><<<blocks, tpb, 0, s>>>(n, raw, aos, perm, Y, reset, uY, gains, box);        \
+    SGT_LAUNCH_CHECK();                                                                               \
+    center_kernel<DD><<<blocks, tpb, 0, s>>>(n, Y, box, blocks, sc, hs, seq, 0);                      \
+    break;
+  switch (d) {
+    SET_CASE(1)
+    SET_CASE(2)
+    SET_CASE(3)
+    default: SGT_CHECK(false, SGTSNE_ERR_ARG, "d must be 1..3");
+  }
+#undef SET_CASE
+  SGT_LAUNCH_CHECK();
+  return SGTSNE_OK;
+}
+
+int launch_get_points(hipStream_t s, int d, int n, const float *in, int layout, const int32_t *perm, double scale,
+                      float *raw) {
+  const int blocks = std::min(div_up(n > 0 ? n : 1, kBlock), 4096), aos = layout == SGTSNE_LAYOUT_AOS;
+  switch (d) {
+    case 1: get_points_kernel<1><<<blocks, kBlock, 0, s>>>(n, in, aos, perm, scale, raw); break;
+    case 2: get_points_kernel<2><<<blocks, kBlock, 0, s>>>(n, in, aos, perm, scale, raw); break;
+    case 3: get_points_kernel<3><<<blocks, kBlock, 0, s>>>(n, in, aos, perm, scale, raw); break;
+    default: SGT_CHECK(false, SGTSNE_ERR_ARG, "d must be 1..3");
+  }
+  SGT_LAUNCH_CHECK();
+  return SGTSNE_OK;
+}
+
 int launch_update_center(hipStream_t s, int d, int n, float *Y, float *uY, float *gains, const float *Fattr,
                          const float *Frep, float alpha, float momentum, float eta, int nz, RedWork rw,
                          DevScalars *sc, HostScalars *hs, unsigned long long seq, bool stamp) {
-  const int tpb = n <= kMaxBoxParts * kBlock ? kBlock : kUpdBlock;
-  const int blocks = std::min(div_up(n > 0 ? n : 1, tpb), kMaxBoxParts);
-  // the Z partials take the front of the workspace (at most 2048 slots)
+  const int tpb = upd_threads(n), blocks = upd_blocks(n);
   SGT_CHECK(nz >= 1 && nz <= 2048 && rw.max_blocks >= 2048 + kMaxBoxParts, SGTSNE_ERR_STATE, "%d partials of Z", nz);
-  BoxPart *box = reinterpret_cast<BoxPart *>(rw.part + (size_t)8 * 2048);
+  BoxPart *box = box_parts(rw);
 #define UPD_CASE(DD)                                                                                            \
   case DD:                                                                                                      \
     update_kernel<DD><<<blocks, tpb, 0, s>>>(n, Y, uY, gains, Fattr, Frep, alpha, momentum, eta, rw.part, nz, sc, box, \
@@ -1272,7 +1246,7 @@ int launch_rep_exact(hipStream_t s, int d, int n, const float *Y, float *Frep, R
     default: SGT_CHECK(false, SGTSNE_ERR_ARG, "d must be 1..3");
   }
   SGT_LAUNCH_CHECK();
-  return finalize(s, FIN_ZEXACT, blocks, d, n, 0, rw, sc);
+  return finalize(s, FIN_ZEXACT, blocks, n, rw, sc);
 }
 
 }  // namespace sgt
