@@ -90,6 +90,14 @@ enum OutKind { OUT_W = 0, OUT_PHIPAIR = 1, OUT_KT = 2, OUT_PHIQ = 3 };
 enum MidKind { MID_FWD = 0, MID_INV = 1, MID_CONV = 2 };
 
 // The pass shapes of one convolution (template arguments of the pass kernel).
+// A single job's multiply pass transforms the kernel along its own axis too
+// (kfused): its lines' kernel columns, half-transformed along the other axes, go
+// through the same stages before the data, one launch less on a chain that
+// launches bound (the convolution of 60,000 points late in a run 70 -> 56 us
+// with it and the passes launched in pairs).  The batched engine's passes are
+// bound by their work, and a column serves up to 4 mirrored lines: there the
+// kernel's last axis stays a pass of its own (a batch of 3-D jobs of 2000-20,000
+// points 2 % slower with the fused form).
 enum PassKind {
   PK_KGEN = 0,     // kernel values -> half spectrum along the first axis
   PK_KT_T = 1,     // half spectrum along a strided axis
@@ -118,9 +126,10 @@ struct PassArgs {
   int in_c[4][2], out_c[4][2], kcplx[4];  // per-pair channels (-1: none) and spectrum kind
   int npairs;     // channel pairs of the convolution
   int pairloop;   // a 3-D multiply pass: each work-group runs every pair of its lines
+  int kfused;     // a multiply pass: Kh is still to be transformed along the pass axis
   const void *in;
   void *out;
-  const float2 *Kh;
+  const float2 *Kh;  // MID_CONV: kernel spectrum (1-D), or half-transformed kernel
   const float2 *tw;  // twiddle table of length L
 };
 
@@ -445,8 +454,8 @@ __device__ inline void pass_body(const PassArgs &a, int blk, int p, float2 *lds)
     const bool loop = MID == MID_CONV && a.pairloop;
     const int pa = loop ? 0 : p, pb = loop ? a.npairs : p + 1;
     float2 kreg[MID == MID_CONV ? kLineElems : 1];
-    if (MID == MID_CONV && act) {
-      // kernel spectrum at (mirror(e), mirror(outer), mirror(inner)):
+    if (MID == MID_CONV) {
+      // the line's kernel column at (mirror(e), mirror(outer), mirror(inner)):
       // index mirror(e) * ks + kb
       int ks = 1, kb = 0;
       if (a.kdim == 2) {
@@ -456,11 +465,21 @@ __device__ inline void pass_body(const PassArgs &a, int blk, int p, float2 *lds)
         ks = a.H * a.H;
         kb = mirror(outer, L) * a.H + mirror(inner, L);
       }
+      const float2 *col = a.Kh + kb;
+      if (a.kfused) {  // transformed first; the spectrum is even as well
+        float2 *dl = b0 + l * Lp;
+        if (act)
+          for (int e = g; e < L; e += G) dl[e] = lv ? col[mirror(e, L) * ks] : make_float2(0.f, 0.f);
+        __syncthreads();
+        col = stockham(b0, b1, a, nl, false, twl) + l * Lp;
+        ks = 1;
+      }
 #pragma unroll
       for (int k = 0; k < kLineElems; ++k) {
         const int e = g + k * G;
-        kreg[k] = lv && e < L ? a.Kh[mirror(e, L) * ks + kb] : make_float2(0.f, 0.f);
+        kreg[k] = lv && e < L ? col[mirror(e, L) * ks] : make_float2(0.f, 0.f);
       }
+      if (a.kfused) __syncthreads();  // the buffers are the data's next
     }
     for (int pp = pa; pp < pb; ++pp) {
       if (act) {
@@ -623,19 +642,22 @@ __device__ inline void pass_body(const PassArgs &a, int blk, int p, float2 *lds)
 // Work-groups of one pass (per channel pair).
 __host__ __device__ inline int pass_blocks(const PassArgs &a) { return (a.nlines + a.nl - 1) / a.nl; }
 
-// Pass shapes of a d-dimensional convolution, in launch order.
-__host__ __device__ inline int pass_kinds(int d, int *kinds) {
+// Pass shapes of a d-dimensional convolution, in launch order (fused: the
+// kernel's last axis in the multiply pass).
+__host__ __device__ inline int pass_kinds(int d, bool fused, int *kinds) {
+  int n = 0;
+  kinds[n++] = PK_KGEN;
   if (d == 1) {
-    kinds[0] = PK_KGEN; kinds[1] = PK_V_PHI;
-    return 2;
+    kinds[n++] = PK_V_PHI;
+    return n;
   }
-  if (d == 2) {
-    kinds[0] = PK_KGEN; kinds[1] = PK_KT_T; kinds[2] = PK_V_W; kinds[3] = PK_W_W_CONV; kinds[4] = PK_W_PHI;
-    return 5;
-  }
-  kinds[0] = PK_KGEN; kinds[1] = PK_KT_T; kinds[2] = PK_KT_T; kinds[3] = PK_V_W; kinds[4] = PK_W_W_FWD;
-  kinds[5] = PK_W_W_CONV; kinds[6] = PK_W_W_INV; kinds[7] = PK_W_PHI;
-  return 8;
+  for (int i = fused ? 2 : 1; i < d; ++i) kinds[n++] = PK_KT_T;
+  kinds[n++] = PK_V_W;
+  if (d == 3) kinds[n++] = PK_W_W_FWD;
+  kinds[n++] = PK_W_W_CONV;
+  if (d == 3) kinds[n++] = PK_W_W_INV;
+  kinds[n++] = PK_W_PHI;
+  return n;
 }
 
 // Channel plan of one convolution.  zdirect: pair 0 = (V0, -) with the
@@ -702,13 +724,10 @@ __host__ __device__ inline void base_args(PassArgs &a, const GridParams &g, cons
   }
 }
 
-// Passes of a d-dimensional convolution.
-__host__ __device__ inline int conv_npasses(int d) { return d == 1 ? 2 : d == 2 ? 5 : 8; }
-
 // Arguments of pass i (in the order of pass_kinds) of one convolution,
 // written in place, lines unpadded; returns the channel pairs the pass runs over.
-__host__ __device__ inline int conv_pass_shape(const GridParams &g, bool zdirect, const ConvPtrs &b, int i,
-                                               PassArgs &a) {
+__host__ __device__ inline int conv_pass_shape(const GridParams &g, bool zdirect, bool fused, const ConvPtrs &b,
+                                               int i, PassArgs &a) {
   const int d = g.d, ng = g.ng, L = g.L, H = L / 2 + 1;
   const Plan pl = make_plan(d, zdirect);
   const int64_t G = d == 1 ? ng : d == 2 ? (int64_t)ng * ng : (int64_t)ng * ng * ng;
@@ -728,6 +747,9 @@ __host__ __device__ inline int conv_pass_shape(const GridParams &g, bool zdirect
     return pl.pairs;
   }
 
+  // the passes numbered as without fusing: the fused form skips the kernel's
+  // last transform
+  if (fused && i >= d - 1) ++i;
   if (d == 2) {
     const int64_t wp = (int64_t)ng * L;
     switch (i) {
@@ -749,6 +771,8 @@ __host__ __device__ inline int conv_pass_shape(const GridParams &g, bool zdirect
         a.in = b.W; a.i_is = 1; a.i_es = L; a.n_in = ng; a.pair_in = wp;
         a.out = b.W; a.o_is = 1; a.o_es = L; a.n_out = ng; a.pair_out = wp;
         a.kdim = 2;
+        a.kfused = fused;
+        if (fused) a.Kh = b.Kt1;
         return pl.pairs;
       default:  // rows: inverse -> Phi
         a.nlines = ng; a.ninner = ng;
@@ -790,6 +814,8 @@ __host__ __device__ inline int conv_pass_shape(const GridParams &g, bool zdirect
       a.in = b.W; a.i_os = L; a.i_is = 1; a.i_es = L2; a.n_in = ng; a.pair_in = wp;
       a.out = b.W; a.o_os = L; a.o_is = 1; a.o_es = L2; a.n_out = ng; a.pair_out = wp;
       a.kdim = 3;
+      a.kfused = fused;
+      if (fused) a.Kh = b.Kt2;
       return pl.pairs;
     case 6:  // y inverse (y < ng kept)
       a.nlines = ng * L; a.ninner = L;
@@ -812,22 +838,22 @@ __host__ __device__ inline bool pass_strided(int kind) {
 
 // Arguments of pass i (in the order of pass_kinds) of one convolution,
 // written in place; returns the channel pairs the pass runs over.
-__host__ __device__ inline int conv_pass(const GridParams &g, bool zdirect, const ConvPtrs &b, int i, PassArgs &a) {
-  const int pairs = conv_pass_shape(g, zdirect, b, i, a);
+__host__ __device__ inline int conv_pass(const GridParams &g, bool zdirect, bool fused, const ConvPtrs &b, int i,
+                                         PassArgs &a) {
+  const int pairs = conv_pass_shape(g, zdirect, fused, b, i, a);
   int kinds[kMaxPasses];
-  pass_kinds(g.d, kinds);
+  pass_kinds(g.d, fused, kinds);
   set_lines(a, pass_strided(kinds[i]));
   a.npairs = make_plan(g.d, zdirect).pairs;
   a.pairloop = kinds[i] == PK_W_W_CONV && g.d == 3;
   return a.pairloop ? 1 : pairs;  // its work-groups run every pair
 }
 
-// Arguments of every pass of one convolution (in the order of pass_kinds),
-// and the channel pairs each pass runs over.  Returns the pass count.
-__host__ __device__ inline int conv_setup(const GridParams &g, bool zdirect, const ConvPtrs &b, PassArgs *out,
-                                          int *pairs_out) {
-  const int np = conv_npasses(g.d);
-  for (int i = 0; i < np; ++i) pairs_out[i] = conv_pass(g, zdirect, b, i, out[i]);
+// Arguments of every pass of one job's convolution (in the order of pass_kinds,
+// fused), and the channel pairs each pass runs over.  Returns the pass count.
+inline int conv_setup(const GridParams &g, bool zdirect, const ConvPtrs &b, PassArgs *out, int *pairs_out, int *kinds) {
+  const int np = pass_kinds(g.d, true, kinds);
+  for (int i = 0; i < np; ++i) pairs_out[i] = conv_pass(g, zdirect, true, b, i, out[i]);
   return np;
 }
 

@@ -395,13 +395,12 @@ __global__ __launch_bounds__(256) void bplan_kernel(int d, BatchJob *__restrict_
     J->fix_scale = ldexp(1.0, e);
     J->fix_inv = fix_inv;
   }
-  const int np = conv_npasses(d);
+  int kinds[kMaxPasses];
+  const int np = pass_kinds(d, false, kinds);
   if (lane < np) {
-    int kinds[kMaxPasses];
-    pass_kinds(d, kinds);
     ConvPtrs ptr{J->vfix, J->phi, J->W, J->Kt1, J->Kt2, J->Kh, tw};
     PassArgs &a = args[(size_t)j * npasses + lane];
-    conv_pass(g, J->zdirect != 0, ptr, lane, a);
+    conv_pass(g, J->zdirect != 0, false, ptr, lane, a);
     if (pass_reads_grid(kinds[lane])) a.fix_inv = fix_inv;
   }
 }
@@ -544,7 +543,7 @@ size_t batch_pass_args_bytes() { return sizeof(PassArgs); }
 
 int batch_npasses(int d) {
   int kinds[kMaxPasses];
-  return pass_kinds(d, kinds);
+  return pass_kinds(d, false, kinds);
 }
 
 int launch_bs2g(hipStream_t s, int d, const BatchJob *jobs, const BatchItem *items, int nitems, const float *Y,
@@ -563,7 +562,7 @@ int launch_bconv(hipStream_t s, int d, int zdirect, const void *args_v, const in
   if (njobs <= 0) return SGTSNE_OK;
   const PassArgs *args = static_cast<const PassArgs *>(args_v);
   int kinds[kMaxPasses];
-  const int np = pass_kinds(d, kinds);
+  const int np = pass_kinds(d, false, kinds);
   const int pairs = make_plan(d, zdirect != 0).pairs;
   for (int p = 0; p < np; ++p) {
     const int pr = (kinds[p] == PK_KGEN || kinds[p] == PK_KT_T || (kinds[p] == PK_W_W_CONV && d == 3)) ? 1 : pairs;

@@ -7,6 +7,7 @@
 #include "fft_device.hpp"
 #include "../../include/sgtsne.h"
 
+#include <algorithm>
 #include <cmath>
 
 namespace sgt {
@@ -19,6 +20,29 @@ template <int IN, int OUT, int MID, bool EC>
 __global__ __launch_bounds__(kFftThreads) void fft_pass_kernel(PassArgs a) {
   extern __shared__ float2 lds[];
   pass_body<IN, OUT, MID, EC>(a, blockIdx.x, blockIdx.y, lds);
+}
+
+// Two independent passes in one launch: work-groups [0, blocks_k) take a pass
+// of the kernel's, the others (blocks_d per channel pair) one of the data's.
+template <int KI, int KO, bool KE, int IN, int OUT, bool EC>
+__global__ __launch_bounds__(kFftThreads) void fft_two_kernel(PassArgs k, int blocks_k, PassArgs a, int blocks_d) {
+  extern __shared__ float2 lds[];
+  int b = blockIdx.x;
+  if (b < blocks_k) {
+    pass_body<KI, KO, MID_FWD, KE>(k, b, 0, lds);
+  } else {
+    b -= blocks_k;
+    pass_body<IN, OUT, MID_FWD, EC>(a, b % blocks_d, b / blocks_d, lds);
+  }
+}
+
+template <int KI, int KO, bool KE, int IN, int OUT, bool EC>
+int run_two(hipStream_t s, const PassArgs &k, const PassArgs &a, int pairs) {
+  const int bk = pass_blocks(k), bd = pass_blocks(a);
+  const size_t lds = std::max(pass_lds_bytes(k.nl, k.L, k.Lp), pass_lds_bytes(a.nl, a.L, a.Lp));
+  fft_two_kernel<KI, KO, KE, IN, OUT, EC><<<bk + bd * pairs, kFftThreads, lds, s>>>(k, bk, a, bd);
+  SGT_LAUNCH_CHECK();
+  return SGTSNE_OK;
 }
 
 // Fills every twiddle table: entry t of the table of length L is
@@ -52,12 +76,9 @@ int run_pass(hipStream_t s, const PassArgs &a, int pairs) {
 int run_kind(hipStream_t s, int kind, const PassArgs &a, int pairs) {
   switch (kind) {
     case PK_KGEN: return run_pass<IN_KGEN, OUT_KT, MID_FWD, true>(s, a, pairs);
-    case PK_KT_T: return run_pass<IN_KT, OUT_KT, MID_FWD, false>(s, a, pairs);
-    case PK_V_W: return run_pass<IN_VPAIR, OUT_W, MID_FWD, true>(s, a, pairs);
     case PK_W_W_CONV: return run_pass<IN_W, OUT_W, MID_CONV, false>(s, a, pairs);
     case PK_W_PHI: return run_pass<IN_W, OUT_PHIPAIR, MID_INV, true>(s, a, pairs);
     case PK_V_PHI: return run_pass<IN_VPAIR, OUT_PHIPAIR, MID_CONV, true>(s, a, pairs);
-    case PK_W_W_FWD: return run_pass<IN_W, OUT_W, MID_FWD, false>(s, a, pairs);
     case PK_W_W_INV: return run_pass<IN_W, OUT_W, MID_INV, false>(s, a, pairs);
     default: SGT_CHECK(false, SGTSNE_ERR_ARG, "bad FFT pass kind");
   }
@@ -93,9 +114,18 @@ int launch_conv(hipStream_t s, const GridParams &g, int zdirect, const float *V,
   ConvPtrs ptr{V, Phi, b.W, b.Kt1, b.Kt2, b.Kh, b.tw};
   PassArgs args[kMaxPasses];
   int pairs[kMaxPasses], kinds[kMaxPasses];
-  const int np = conv_setup(g, zdirect != 0, ptr, args, pairs);
-  pass_kinds(g.d, kinds);
-  for (int i = 0; i < np; ++i) SGT_TRY(run_kind(s, kinds[i], args[i], pairs[i]));
+  const int np = conv_setup(g, zdirect != 0, ptr, args, pairs, kinds);
+  // the kernel's passes ride along with the data's they do not depend on
+  int i = 0;
+  if (g.d == 2) {
+    SGT_TRY((run_two<IN_KGEN, OUT_KT, true, IN_VPAIR, OUT_W, true>(s, args[0], args[1], pairs[1])));
+    i = 2;
+  } else if (g.d == 3) {
+    SGT_TRY((run_two<IN_KGEN, OUT_KT, true, IN_VPAIR, OUT_W, true>(s, args[0], args[2], pairs[2])));
+    SGT_TRY((run_two<IN_KT, OUT_KT, false, IN_W, OUT_W, false>(s, args[1], args[3], pairs[3])));
+    i = 4;
+  }
+  for (; i < np; ++i) SGT_TRY(run_kind(s, kinds[i], args[i], pairs[i]));
   return SGTSNE_OK;
 }
 
