@@ -118,6 +118,13 @@ struct sgtsne_ctx {
   float *s2g_part = nullptr;  // per-block private grids of the spread
   int64_t s2g_cap = 0;        // floats
   ConvBuffers cb{};
+  // order of the points along the tiles of a large grid (spread and gather):
+  // renewed every kSpreadOrderIters evaluations, since it only sets how fast
+  // they run, and whenever Y or its device order is replaced
+  int32_t *sord = nullptr;
+  int2 *sord_key = nullptr;
+  int *sord_cnt = nullptr;
+  int sord_left = 0;
 
   // timing
   bool timing = true;
@@ -142,6 +149,8 @@ struct sgtsne_ctx {
 
 namespace {
 
+constexpr int kSpreadOrderIters = 16;
+
 int alloc_dev(void **p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes > 0 ? bytes : 1);
   if (e != hipSuccess) {
@@ -155,6 +164,12 @@ template <class T>
 void free_dev(T *&p) {
   if (p) (void)hipFree((void *)p);
   p = nullptr;
+}
+
+void free_spread_order(sgtsne_ctx *c) {
+  free_dev(c->sord);
+  free_dev(c->sord_key);
+  free_dev(c->sord_cnt);
 }
 
 void free_loc(sgtsne_ctx *c) {
@@ -280,7 +295,7 @@ int make_grid(sgtsne_ctx *c, const HostScalars &s, GridParams &g) {
 }
 
 int ensure_grid(sgtsne_ctx *c, const GridParams &g) {
-  const int m = c->d + 2;  // charges 0..d, plus the direct-Z channel of Phi
+  const int m = std::max(4, c->d + 2);  // charges 0..d; Phi: four channels of a node together, then the fifth
   const size_t G = c->d == 1 ? (size_t)g.ng : c->d == 2 ? (size_t)g.ng * g.ng : (size_t)g.ng * g.ng * g.ng;
   const size_t gb = G * m * sizeof(float);
   size_t wb = 0, kb = 0;
@@ -357,9 +372,23 @@ int repulsive(sgtsne_ctx *c, const GridParams &g, bool stamp, int *nz) {
   DevScalars *st = stamp ? c->sc : nullptr;
   SGT_TRY(ensure_grid(c, g));
   int64_t need = 0;
-  SGT_TRY(launch_s2g(c->stream, g, c->n, c->Y, c->V, c->s2g_part, c->s2g_cap, &need, c->p.spread, st));
-  SGT_TRY(launch_conv(c->stream, g, zdirect, c->V, c->Phi, c->cb));
-  SGT_TRY(launch_g2s_force(c->stream, g, c->n, c->Y, c->Phi, c->Frep, zdirect, c->rw, nz, st));
+  const int32_t *ord = nullptr;
+  if (s2g_takes_order(g, c->p.spread)) {
+    if (!c->sord) {
+      SGT_TRY(alloc_dev((void **)&c->sord_key, sizeof(int2) * (size_t)c->n));
+      SGT_TRY(alloc_dev((void **)&c->sord_cnt, sizeof(int) * kSpreadBins));
+      SGT_TRY(alloc_dev((void **)&c->sord, sizeof(int32_t) * (size_t)c->n));
+      c->sord_left = 0;
+    }
+    if (c->sord_left-- <= 0) {
+      SGT_TRY(launch_spread_order(c->stream, g, c->n, c->Y, c->sord_key, c->sord_cnt, c->sord));
+      c->sord_left = kSpreadOrderIters - 1;
+    }
+    ord = c->sord;
+  }
+  SGT_TRY(launch_s2g(c->stream, g, c->n, c->Y, c->V, c->s2g_part, c->s2g_cap, &need, c->p.spread, st, ord));
+  SGT_TRY(launch_conv(c->stream, g, zdirect, c->V, c->Phi, c->cb, true));
+  SGT_TRY(launch_g2s_force(c->stream, g, c->n, c->Y, c->Phi, c->Frep, zdirect, c->rw, nz, st, ord));
   c->last_grid = g;
   return SGTSNE_OK;
 }
@@ -500,6 +529,7 @@ int spatial_reorder(sgtsne_ctx *c) {
     return SGTSNE_OK;
   }
   if (!st) std::swap(c->Y, tmp);
+  c->sord_left = 0;
   float **state[2] = {&c->uY, &c->gains};
   for (int k = 0; k < 2 && !st; k++) {
     st = launch_gather_points(c->stream, n, ds, order, *state[k], tmp);
@@ -795,6 +825,7 @@ int alloc_points(sgtsne_ctx *c) {
   free_dev(c->Fattr);
   free_dev(c->Frep);
   free_dev(c->io);
+  free_spread_order(c);
   c->points_n = 0;
   SGT_TRY(alloc_dev((void **)&c->io, sizeof(float) * (size_t)c->n * c->d));
   SGT_TRY(alloc_dev((void **)&c->Y, nb * sizeof(float)));
@@ -1066,6 +1097,7 @@ int sgtsne_ctx_destroy(sgtsne_ctx *c) {
   free_dev(c->Fattr);
   free_dev(c->Frep);
   free_dev(c->io);
+  free_spread_order(c);
   free_dev(c->perm_d);
   free_dev(c->rw.part);
   free_dev(c->rw.ticket);
@@ -1196,6 +1228,7 @@ int sgtsne_ctx_set_Y(sgtsne_ctx *c, const float *y, int layout, int reset_state)
   SGT_HIP(hipMemcpyAsync(c->io, y, sizeof(float) * (size_t)n * c->d, hipMemcpyHostToDevice, c->stream));
   if (reset_state) c->iter = 0;
   c->stamped = false;
+  c->sord_left = 0;
   SGT_TRY(launch_set_points(c->stream, c->d, n, c->io, layout, c->permuted ? c->perm_d : nullptr, c->Y, reset_state,
                             c->uY, c->gains, c->rw, c->sc, c->hs, ++c->seq));
   SGT_HIP(hipStreamSynchronize(c->stream));

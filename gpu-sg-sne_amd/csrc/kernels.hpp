@@ -100,12 +100,21 @@ int launch_get_points(hipStream_t s, int d, int n, const float *in, int layout, 
 // wants (when larger than scratch_floats the global-atomic path runs).
 // sc (may be NULL): the phase stamps STAMP_S2G and STAMP_CONV are written to it.
 int launch_s2g(hipStream_t s, const GridParams &g, int n, const float *Y, float *V, float *scratch,
-               int64_t scratch_floats, int64_t *needed, int mode = 0, DevScalars *stamp = nullptr);
+               int64_t scratch_floats, int64_t *needed, int mode = 0, DevScalars *stamp = nullptr,
+               const int32_t *ord = nullptr);
+// Order of the points along the tiles of grid g, for the spread (through ord
+// above) and gather of grids no LDS copy holds: key is scratch of n int2, cnt
+// of kSpreadBins ints.  Any order gives the same bits; this one gives runs of
+// points small windows of the grid.
+constexpr int kSpreadBins = 32768;
+bool s2g_takes_order(const GridParams &g, int mode);
+int launch_spread_order(hipStream_t s, const GridParams &g, int n, const float *Y, int2 *key, int *cnt, int32_t *ord);
 int64_t s2g_scratch_need(const GridParams &g, int n, int mode = 0);
 // Frep and the partials of Z; *nz receives how many there are: launch_update
 // adds them up itself, launch_finalize_z puts their sum into sc->Z for others.
 int launch_g2s_force(hipStream_t s, const GridParams &g, int n, const float *Y, const float *Phi,
-                     float *Frep, int zdirect, RedWork rw, int *nz, DevScalars *stamp = nullptr);
+                     float *Frep, int zdirect, RedWork rw, int *nz, DevScalars *stamp = nullptr,
+                     const int32_t *ord = nullptr);
 int launch_finalize_z(hipStream_t s, int nz, int n, RedWork rw, DevScalars *sc);
 int launch_finalize_kl(hipStream_t s, int nblocks, RedWork rw, DevScalars *sc);
 // The update of Y from the forces and the nz partials of Z, then the centring
@@ -127,9 +136,11 @@ struct ConvBuffers {
   float2 *tw;     // twiddle tables of every supported length (twiddle_count())
 };
 int conv_workspace_bytes(int d, int ng, int L, size_t *w_bytes, size_t *k_bytes);
-// V [d+1][ng^d] -> Phi [d+1 (+1 with zdirect: K1 * V0 in channel d+1)][ng^d]
+// V [d+1][ng^d] -> Phi [d+1 (+1 with zdirect: K1 * V0 in channel d+1)][ng^d];
+// node_major: channels 0-3 of a node as one float4, then channel 4 as a plane
+// (what the gather reads; max(4, d + 2) ng^d floats)
 int launch_conv(hipStream_t s, const GridParams &g, int zdirect, const float *V, float *Phi,
-                const ConvBuffers &b);
+                const ConvBuffers &b, bool node_major = false);
 // twiddle tables of every supported FFT length (twiddle_count() float2)
 size_t twiddle_count();
 int init_twiddles(hipStream_t s, float2 *tw);

@@ -64,7 +64,7 @@ __global__ __launch_bounds__(s2g_threads<D>()) void bs2g_kernel(const BatchJob *
       if (itm.begin >= itm.end) continue;
     }
     spread_fix_unit<D>(J->g, (float)J->fix_scale, reinterpret_cast<unsigned long long *>(J->vfix), itm.begin,
-                       itm.end, Y, win, lds_slots, sbox);
+                       itm.end, Y, nullptr, win, lds_slots, sbox);
   }
 }
 

@@ -73,12 +73,16 @@ int run_pass(hipStream_t s, const PassArgs &a, int pairs) {
   return SGTSNE_OK;
 }
 
-int run_kind(hipStream_t s, int kind, const PassArgs &a, int pairs) {
+int run_kind(hipStream_t s, int kind, const PassArgs &a, int pairs, bool node_major) {
   switch (kind) {
     case PK_KGEN: return run_pass<IN_KGEN, OUT_KT, MID_FWD, true>(s, a, pairs);
     case PK_W_W_CONV: return run_pass<IN_W, OUT_W, MID_CONV, false>(s, a, pairs);
-    case PK_W_PHI: return run_pass<IN_W, OUT_PHIPAIR, MID_INV, true>(s, a, pairs);
-    case PK_V_PHI: return run_pass<IN_VPAIR, OUT_PHIPAIR, MID_CONV, true>(s, a, pairs);
+    case PK_W_PHI:
+      return node_major ? run_pass<IN_W, OUT_PHIQ, MID_INV, true>(s, a, pairs)
+                        : run_pass<IN_W, OUT_PHIPAIR, MID_INV, true>(s, a, pairs);
+    case PK_V_PHI:
+      return node_major ? run_pass<IN_VPAIR, OUT_PHIQ, MID_CONV, true>(s, a, pairs)
+                        : run_pass<IN_VPAIR, OUT_PHIPAIR, MID_CONV, true>(s, a, pairs);
     case PK_W_W_INV: return run_pass<IN_W, OUT_W, MID_INV, false>(s, a, pairs);
     default: SGT_CHECK(false, SGTSNE_ERR_ARG, "bad FFT pass kind");
   }
@@ -108,7 +112,7 @@ int conv_workspace_bytes(int d, int ng, int L, size_t *w_bytes, size_t *k_bytes)
 }
 
 int launch_conv(hipStream_t s, const GridParams &g, int zdirect, const float *V, float *Phi,
-                const ConvBuffers &b) {
+                const ConvBuffers &b, bool node_major) {
   SGT_CHECK(g.L <= kMaxL && g.L >= 2 * g.ng - 1 && fft_smooth(g.L), SGTSNE_ERR_ARG,
             "FFT length %d invalid for ng %d", g.L, g.ng);
   ConvPtrs ptr{V, Phi, b.W, b.Kt1, b.Kt2, b.Kh, b.tw};
@@ -125,7 +129,7 @@ int launch_conv(hipStream_t s, const GridParams &g, int zdirect, const float *V,
     SGT_TRY((run_two<IN_KT, OUT_KT, false, IN_W, OUT_W, false>(s, args[1], args[3], pairs[3])));
     i = 4;
   }
-  for (; i < np; ++i) SGT_TRY(run_kind(s, kinds[i], args[i], pairs[i]));
+  for (; i < np; ++i) SGT_TRY(run_kind(s, kinds[i], args[i], pairs[i], node_major));
   return SGTSNE_OK;
 }
 

@@ -497,7 +497,9 @@ __global__ __launch_bounds__(1024) void grid_reduce_kernel(const float *__restri
 }
 
 // ---- G2S + forces + Z ------------------------------------------------------------
-// Phi_c(y_i) by the same stencil; Frep_i (unnormalised) = ~y_i Phi0 - Phi_{1..d}.
+// Phi (node-major, see launch_conv) at y_i by the same stencil, the points along
+// the tiles of the grid (ord), so that neighbouring lanes read the same nodes:
+// 200,003 points late in a 3-D run 68 -> 21 us with both; Frep_i (unnormalised) = ~y_i Phi0 - Phi_{1..d}.
 // Z per point, compensated sum over points, FP64:
 //   ZDIRECT: z_i = psi_i, the gathered convolution of the unit charges with
 //            1/(1 + r^2) (channel D+1), so Z = sum_i psi_i - N;
@@ -508,14 +510,18 @@ template <int D, bool ZDIRECT>
 __global__ __launch_bounds__(kBlock) void g2s_force_kernel(GridParams g, int n,
                                                            const float *__restrict__ Y,
                                                            const float *__restrict__ Phi,
-                                                           float *__restrict__ Frep, double *part, DevScalars *stamp) {
+                                                           float *__restrict__ Frep, double *part, DevScalars *stamp,
+                                                           const int32_t *__restrict__ ord) {
   stamp_now(stamp, STAMP_G2S);
   __shared__ double lds[8];
   const int ng = g.ng;
   const int G = grid_cells<D>(ng);
   constexpr int C = ZDIRECT ? D + 2 : D + 1;
+  const float4 *__restrict__ Phi4 = reinterpret_cast<const float4 *>(Phi);
+  const float *__restrict__ Phi1 = Phi + 4 * (int64_t)G;
   Neu z{0.0, 0.0};
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+    const int i = ord ? ord[k] : k;
     float y[D];
     load_pt<D>(Y, i, y);
     int f[D];
@@ -525,8 +531,12 @@ __global__ __launch_bounds__(kBlock) void g2s_force_kernel(GridParams g, int n,
 #pragma unroll
     for (int c = 0; c < C; ++c) ph[c] = 0.0f;
     for_stencil<D>(ng, f, w, [&](int idx, float ww) {
-#pragma unroll
-      for (int c = 0; c < C; ++c) ph[c] = __builtin_fmaf(Phi[c * G + idx], ww, ph[c]);
+      const float4 q = Phi4[idx];
+      ph[0] = __builtin_fmaf(q.x, ww, ph[0]);
+      ph[1] = __builtin_fmaf(q.y, ww, ph[1]);
+      if constexpr (C > 2) ph[2] = __builtin_fmaf(q.z, ww, ph[2]);
+      if constexpr (C > 3) ph[3] = __builtin_fmaf(q.w, ww, ph[3]);
+      if constexpr (C > 4) ph[4] = __builtin_fmaf(Phi1[idx], ww, ph[4]);
     });
     float fr[D];
     double ysq = 0.0, ydot = 0.0;
@@ -577,13 +587,8 @@ __global__ __launch_bounds__(kG2sLdsBlock) void g2s_lds_kernel(GridParams g, int
   const int ng = g.ng;
   const int G = grid_cells<D>(ng);
   for (int e = threadIdx.x; e < G; e += blockDim.x) {
-    float4 v;
-    v.x = Phi[e];
-    v.y = Phi[G + e];
-    v.z = Phi[2 * G + e];
-    v.w = C > 3 ? Phi[3 * G + e] : 0.0f;
-    q4[e] = v;
-    if constexpr (C == 5) q5[e] = Phi[4 * G + e];
+    q4[e] = reinterpret_cast<const float4 *>(Phi)[e];
+    if constexpr (C == 5) q5[e] = Phi[4 * (int64_t)G + e];
   }
   __syncthreads();
   Neu z{0.0, 0.0};
@@ -960,21 +965,25 @@ int finalize(hipStream_t s, int mode, int nblocks, int n, RedWork rw, DevScalars
 }
 
 // Large grids (those no LDS copy or matrix-core tile holds): the points in
-// runs of `unit` consecutive ones (the engine's locality order), each run's
-// stencil window accumulated in LDS as 64-bit fixed point and added to the
+// runs of `unit` along the tiles of the grid (ord, see spread_bin_kernel), each
+// run's stencil window accumulated in LDS as 64-bit fixed point and added to the
 // fixed-point grid Vf (spread_fix.hpp), so the grid is exact and the same
-// whatever the order of the atomics.
+// whatever the order of the points and the atomics.  Bound by the global atomics
+// of the windows' cells: in the device order of P a run's window often did not
+// fit LDS and every node of every point went to memory.  200,003 points late in
+// a run: 3-D 238 -> 69 us, 2-D spread 180 -> 40 us with the order (23 us, renewed
+// every 16 evaluations).
 template <int D>
 __global__ __launch_bounds__(s2g_threads<D>()) void s2g_fix_kernel(GridParams g, float fsf, int n,
                                                                    const float *__restrict__ Y,
                                                                    unsigned long long *__restrict__ Vf, int unit,
-                                                                   int lds_slots, DevScalars *stamp) {
+                                                                   int lds_slots, const int32_t *__restrict__ ord, DevScalars *stamp) {
   stamp_now(stamp, STAMP_S2G);
   extern __shared__ unsigned long long win[];
   __shared__ int sbox[6];
   const int nunits = (n + unit - 1) / unit;
   for (int u = blockIdx.x; u < nunits; u += gridDim.x)
-    spread_fix_unit<D>(g, fsf, Vf, u * unit, min(n, (u + 1) * unit), Y, win, lds_slots, sbox);
+    spread_fix_unit<D>(g, fsf, Vf, u * unit, min(n, (u + 1) * unit), Y, ord, win, lds_slots, sbox);
 }
 
 // V = Vf * 2^-e in FP32 (the FP64 product rounded once), Vf cleared.
@@ -1022,6 +1031,113 @@ int s2g_lds_fits(int d, int ng, size_t *lds_bytes, int *copies) {
   return *lds_bytes <= 65536;
 }
 
+// Grids that go through the fixed-point windows (and the gather from memory).
+bool s2g_takes_order(const GridParams &g, int mode) {
+  size_t lds = 0;
+  int copies = 1;
+  return g.d >= 2 && mode != SGTSNE_SPREAD_ATOMIC && !(g.d == 3 && g.ng <= 16) &&
+         !s2g_lds_fits(g.d, g.ng, &lds, &copies);
+}
+
+// Tiles of 2^tb cells per axis (at most 32 per axis in 3-D, 128 in 2-D) in
+// Morton order: the bin of each point and its place among the bin's points.  A
+// work-group counts its 4096 points in LDS first, so a crowded bin takes one
+// global atomic per work-group: with one per point, 200,003 points late in a 3-D
+// run (1900 in a crowded tile) took 414 us on the serial additions to a bin, now
+// 9.
+constexpr int kBinPoints = 4;  // per thread
+
+template <int D>
+__global__ __launch_bounds__(1024) void spread_bin_kernel(GridParams g, int n, const float *__restrict__ Y, int tb,
+                                                          int2 *__restrict__ key, int *__restrict__ cnt) {
+  constexpr int B = D == 3 ? 5 : 7, BINS = 1 << (D * B);
+  static_assert(BINS <= kSpreadBins, "bins");
+  extern __shared__ int bcnt[];
+  for (int b = threadIdx.x; b < BINS; b += 1024) bcnt[b] = 0;
+  __syncthreads();
+  int bin[kBinPoints], rank[kBinPoints];
+#pragma unroll
+  for (int u = 0; u < kBinPoints; ++u) {
+    const int i = (blockIdx.x * kBinPoints + u) * 1024 + threadIdx.x;
+    bin[u] = -1;
+    if (i < n) {
+      float y[D];
+      load_pt<D>(Y, i, y);
+      int f[D];
+      float w[D][4];
+      stencil<D>(g, y, f, w);
+      int k = 0;
+#pragma unroll
+      for (int b = 0; b < B; ++b)
+#pragma unroll
+        for (int a = 0; a < D; ++a) k |= ((f[a] >> (tb + b)) & 1) << (D * b + a);
+      bin[u] = k;
+      rank[u] = atomicAdd(&bcnt[k], 1);
+    }
+  }
+  __syncthreads();
+  for (int b = threadIdx.x; b < BINS; b += 1024) {
+    const int c = bcnt[b];
+    if (c) bcnt[b] = atomicAdd(&cnt[b], c);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kBinPoints; ++u)
+    if (bin[u] >= 0) key[(blockIdx.x * kBinPoints + u) * 1024 + threadIdx.x] = make_int2(bin[u], bcnt[bin[u]] + rank[u]);
+}
+
+// Counts -> first place of each bin (one work-group).
+__global__ __launch_bounds__(1024) void spread_scan_kernel(int *__restrict__ cnt) {
+  __shared__ int wsum[16];
+  constexpr int PER = kSpreadBins / 1024;
+  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+  int v[PER], sum = 0;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    v[k] = cnt[t * PER + k];
+    sum += v[k];
+  }
+  int inc = sum;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int u = __shfl_up(inc, o, 64);
+    if (lane >= o) inc += u;
+  }
+  if (lane == 63) wsum[wid] = inc;
+  __syncthreads();
+  int run = inc - sum;
+  for (int k = 0; k < wid; ++k) run += wsum[k];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    cnt[t * PER + k] = run;
+    run += v[k];
+  }
+}
+
+__global__ void spread_place_kernel(int n, const int2 *__restrict__ key, const int *__restrict__ start,
+                                    int32_t *__restrict__ ord) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int2 k = key[i];
+  ord[start[k.x] + k.y] = i;
+}
+
+int launch_spread_order(hipStream_t s, const GridParams &g, int n, const float *Y, int2 *key, int *cnt, int32_t *ord) {
+  if (n <= 0) return SGTSNE_OK;
+  int tb = 2;
+  while ((g.ng >> tb) >= (g.d == 3 ? 32 : 128)) ++tb;
+  SGT_TRY(launch_fill(s, reinterpret_cast<float *>(cnt), kSpreadBins, 0.0f));
+  const int blocks = div_up(n, kBlock), bblocks = div_up(n, 1024 * kBinPoints);
+  if (g.d == 2) spread_bin_kernel<2><<<bblocks, 1024, sizeof(int) << 14, s>>>(g, n, Y, tb, key, cnt);
+  else spread_bin_kernel<3><<<bblocks, 1024, sizeof(int) << 15, s>>>(g, n, Y, tb, key, cnt);
+  SGT_LAUNCH_CHECK();
+  spread_scan_kernel<<<1, 1024, 0, s>>>(cnt);
+  SGT_LAUNCH_CHECK();
+  spread_place_kernel<<<blocks, kBlock, 0, s>>>(n, key, cnt, ord);
+  SGT_LAUNCH_CHECK();
+  return SGTSNE_OK;
+}
+
 int64_t s2g_scratch_need(const GridParams &g, int n, int mode) {
   int64_t need = 0;
   (void)launch_s2g(nullptr, g, -n, nullptr, nullptr, nullptr, 0, &need, mode);
@@ -1029,7 +1145,7 @@ int64_t s2g_scratch_need(const GridParams &g, int n, int mode) {
 }
 
 int launch_s2g(hipStream_t s, const GridParams &g, int n, const float *Y, float *V, float *scratch,
-               int64_t scratch_floats, int64_t *needed, int mode, DevScalars *stamp) {
+               int64_t scratch_floats, int64_t *needed, int mode, DevScalars *stamp, const int32_t *ord) {
   const bool query = n < 0;  // size query only
   if (query) n = -n;
   if (n > 0 && g.d == 2 && g.ng <= 32 && mode != SGTSNE_SPREAD_ATOMIC) {
@@ -1064,7 +1180,7 @@ int launch_s2g(hipStream_t s, const GridParams &g, int n, const float *Y, float 
   size_t lds = 0;
   int copies = 1;
   const int64_t cells = (int64_t)(g.d == 1 ? g.ng : g.d == 2 ? g.ng * g.ng : g.ng * g.ng * g.ng) * (g.d + 1);
-  if (n > 0 && g.d >= 2 && mode != SGTSNE_SPREAD_ATOMIC && !s2g_lds_fits(g.d, g.ng, &lds, &copies)) {
+  if (n > 0 && s2g_takes_order(g, mode)) {
     // fixed point in the scratch (2 floats per 64-bit cell): cleared, spread,
     // converted into V and cleared again
     if (needed) *needed = 2 * cells;
@@ -1081,9 +1197,9 @@ int launch_s2g(hipStream_t s, const GridParams &g, int n, const float *Y, float 
     const int lds_b = 64512;  // two work-groups per CU
     const int blocks = (int)std::min<int64_t>(div_up(n, unit), 2048);
     if (g.d == 2)
-      s2g_fix_kernel<2><<<blocks, s2g_threads<2>(), lds_b, s>>>(g, std::ldexp(1.0f, e), n, Y, Vf, unit, lds_b / 8, stamp);
+      s2g_fix_kernel<2><<<blocks, s2g_threads<2>(), lds_b, s>>>(g, std::ldexp(1.0f, e), n, Y, Vf, unit, lds_b / 8, ord, stamp);
     else
-      s2g_fix_kernel<3><<<blocks, s2g_threads<3>(), lds_b, s>>>(g, std::ldexp(1.0f, e), n, Y, Vf, unit, lds_b / 8, stamp);
+      s2g_fix_kernel<3><<<blocks, s2g_threads<3>(), lds_b, s>>>(g, std::ldexp(1.0f, e), n, Y, Vf, unit, lds_b / 8, ord, stamp);
     SGT_LAUNCH_CHECK();
     fix_to_float_kernel<<<(int)std::min<int64_t>(div_up(cells, 256), 4096), 256, 0, s>>>(
         reinterpret_cast<long long *>(Vf), V, cells, std::ldexp(1.0, -e), stamp);
@@ -1128,7 +1244,7 @@ int launch_s2g(hipStream_t s, const GridParams &g, int n, const float *Y, float 
 }
 
 int launch_g2s_force(hipStream_t s, const GridParams &g, int n, const float *Y, const float *Phi,
-                     float *Frep, int zdirect, RedWork rw, int *nz, DevScalars *stamp) {
+                     float *Frep, int zdirect, RedWork rw, int *nz, DevScalars *stamp, const int32_t *ord) {
   if (g2s_lds_fits(g.d, g.ng)) {
     // one 16-wave work-group per CU (the grid copy takes half of its LDS)
     const int lb = std::max(1, std::min({rw.max_blocks, 256, div_up(n > 0 ? n : 1, kG2sLdsBlock)}));
@@ -1146,8 +1262,8 @@ int launch_g2s_force(hipStream_t s, const GridParams &g, int n, const float *Y, 
   const int blocks = grid_blocks(n, std::min(rw.max_blocks, 2048));
 #define G2S_CASE(DD)                                                                               \
   case DD:                                                                                         \
-    if (zdirect) g2s_force_kernel<DD, true><<<blocks, kBlock, 0, s>>>(g, n, Y, Phi, Frep, rw.part, stamp); \
-    else g2s_force_kernel<DD, false><<<blocks, kBlock, 0, s>>>(g, n, Y, Phi, Frep, rw.part, stamp);        \
+    if (zdirect) g2s_force_kernel<DD, true><<<blocks, kBlock, 0, s>>>(g, n, Y, Phi, Frep, rw.part, stamp, ord); \
+    else g2s_force_kernel<DD, false><<<blocks, kBlock, 0, s>>>(g, n, Y, Phi, Frep, rw.part, stamp, ord);        \
     break;
   switch (g.d) {
     G2S_CASE(1)

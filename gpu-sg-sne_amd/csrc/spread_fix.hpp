@@ -45,12 +45,14 @@ __device__ __forceinline__ int wave_max_i(int v) {
   return v;
 }
 
-// Spreads points [begin, end) (3-D: at most kFixUnit3 of them) onto the
-// fixed-point grid V of g with scale fsf = 2^e.  Every thread of the
-// work-group calls it; win holds lds_slots 64-bit cells, sbox 6 ints.
+// Spreads points [begin, end) (3-D: at most kFixUnit3 of them) of the order ord
+// (NULL: as stored) onto the fixed-point grid V of g with scale fsf = 2^e.
+// Every thread of the work-group calls it; win holds lds_slots 64-bit cells,
+// sbox 6 ints.
 template <int D>
 __device__ __forceinline__ void spread_fix_unit(const GridParams &g, float fsf, unsigned long long *V, int begin,
-                                                int end, const float *__restrict__ Y, unsigned long long *win,
+                                                int end, const float *__restrict__ Y,
+                                                const int32_t *__restrict__ ord, unsigned long long *win,
                                                 int lds_slots, int *sbox) {
   constexpr int M = D + 1;
   constexpr int NODES = NodeLanes<D>::NODES;
@@ -77,7 +79,7 @@ __device__ __forceinline__ void spread_fix_unit(const GridParams &g, float fsf, 
   float y3[D];
 #pragma unroll
   for (int a = 0; a < D; ++a) y3[a] = 0.0f;
-  if (D == 3 && node < cnt) load_pt<D>(Y, r0 + node, y3);
+  if (D == 3 && node < cnt) load_pt<D>(Y, ord ? ord[r0 + node] : r0 + node, y3);
   if (threadIdx.x < 3) {
     sbox[threadIdx.x] = INT_MAX;
     sbox[3 + threadIdx.x] = INT_MIN;
@@ -99,7 +101,7 @@ __device__ __forceinline__ void spread_fix_unit(const GridParams &g, float fsf, 
     } else {
       for (int i = begin + threadIdx.x; i < end; i += blockDim.x) {
         float y[D];
-        load_pt<D>(Y, i, y);
+        load_pt<D>(Y, ord ? ord[i] : i, y);
         widen(y);
       }
     }
@@ -139,7 +141,7 @@ __device__ __forceinline__ void spread_fix_unit(const GridParams &g, float fsf, 
       for (int b = 0; b < per_slot; b += NODES) {
         float yv[D];
         if (b + node < cnt) {
-          load_pt<D>(Y, r0 + b + node, yv);
+          load_pt<D>(Y, ord ? ord[r0 + b + node] : r0 + b + node, yv);
         } else {
 #pragma unroll
           for (int a = 0; a < D; ++a) yv[a] = 0.0f;

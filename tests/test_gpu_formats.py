@@ -58,3 +58,31 @@ def test_attractive_runs(sg, O, fmt, width, kind, n, d):
         Yc = ctx.get_Y().astype(np.float64)
     ref = O.attractive(O.CSR(n, rp.astype(np.int64), col, val.astype(np.float32).astype(np.float64)), Yc)
     assert np.linalg.norm(Fa - ref) <= TOL * np.linalg.norm(ref)
+
+
+# grids that go through the tile order and the fixed-point windows: points that
+# end a batch of 4096, one crowded tile, every point on the box's faces
+@pytest.mark.parametrize("d,n,kind", [(2, 4096, "wide"), (2, 4097, "crowd"), (2, 9000, "faces"), (3, 4095, "wide"),
+                                      (3, 8193, "crowd"), (3, 5000, "faces")])
+def test_large_grid_order(sg, O, d, n, kind):
+    rng = np.random.default_rng(7 * n + d)
+    R = 40.0 if d == 2 else 20.0
+    Y = rng.uniform(-R, R, (n, d))
+    if kind == "crowd":
+        Y[n // 10:] = 0.3 * rng.standard_normal((n - n // 10, d)) + 5.0
+    elif kind == "faces":
+        Y[np.arange(n), rng.integers(0, d, n)] = R * rng.choice([-1, 1], n)
+    Y = Y.astype(np.float32)
+    i = np.arange(n)
+    P = sg.CSR(n, np.arange(n + 1), i[::-1], np.full(n, 1.0 / n))
+    with sg.Context(sg.tsneparams(d=d, reorder=0)) as ctx:
+        ctx.upload_P(P, symmetrize=True)
+        ctx.set_Y(Y)
+        _, Fr, Z, ng = ctx.terms()
+        Yc = ctx.get_Y().astype(np.float64)
+        again = ctx.terms()
+    assert ng > (73 if d == 2 else 16)
+    Fo, Zo, ngo = O.repulsive_interp(Yc.copy(), 0.7 if d == 2 else 1.2, O.ZETA_DIRECT)
+    # FP32 grids and transforms against FP64: the single-precision bar of the other term tests
+    assert ng == ngo and abs(Z - Zo) <= 1e-4 * Zo and np.linalg.norm(Fr - Fo) <= 1e-4 * np.linalg.norm(Fo)
+    assert np.array_equal(Fr, again[1]) and Z == again[2]
