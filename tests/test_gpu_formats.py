@@ -86,3 +86,28 @@ def test_large_grid_order(sg, O, d, n, kind):
     # FP32 grids and transforms against FP64: the single-precision bar of the other term tests
     assert ng == ngo and abs(Z - Zo) <= 1e-4 * Zo and np.linalg.norm(Fr - Fo) <= 1e-4 * np.linalg.norm(Fo)
     assert np.array_equal(Fr, again[1]) and Z == again[2]
+
+
+# the small grids: work-groups of one short, full and one long round of points,
+# fixed sides below 16, both Z modes
+@pytest.mark.parametrize("zeta", ["DIRECT", "ALGEBRAIC"])
+@pytest.mark.parametrize("d,n,ng_fixed", [(2, 255, 0), (2, 3000, 25), (2, 700, 6), (3, 255, 0), (3, 257, 0), (3, 32769, 0), (3, 900, 9)])
+def test_small_grids(sg, O, d, n, ng_fixed, zeta):
+    rng = np.random.default_rng(n + d)
+    Y = (1.5 * rng.standard_normal((n, d))).astype(np.float32)
+    i = np.arange(n)
+    P = sg.CSR(n, np.arange(n + 1), i[::-1], np.full(n, 1.0 / n))
+    prm = sg.tsneparams(d=d, reorder=0, zeta_mode=getattr(sg, "ZETA_" + zeta))
+    if ng_fixed:
+        prm.grid_mode, prm.ng = sg.GRID_FIXED, ng_fixed
+    with sg.Context(prm) as ctx:
+        ctx.upload_P(P, symmetrize=True)
+        ctx.set_Y(Y)
+        _, Fr, Z, ng = ctx.terms()
+        Yc = ctx.get_Y().astype(np.float64)
+    Fo, Zo, ngo = O.repulsive_interp(Yc.copy(), 0.7 if d == 2 else 1.2, getattr(O, "ZETA_" + zeta), ng_fixed)
+    # FP32 against FP64, the single-precision bar of the other term tests; the
+    # algebraic Z cancels N |y|^2-sized terms of FP32 potentials: ten times it
+    tz = 1e-4 if zeta == "DIRECT" else 1e-3
+    assert ng == ngo and abs(Z - Zo) <= tz * abs(Zo)
+    assert np.linalg.norm(Fr * Z - Fo * Zo) <= 1e-4 * np.linalg.norm(Fo * Zo)
