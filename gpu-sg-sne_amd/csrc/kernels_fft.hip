@@ -88,6 +88,137 @@ int run_kind(hipStream_t s, int kind, const PassArgs &a, int pairs, bool node_ma
   }
 }
 
+// ---- small grids: the convolution as a sum ---------------------------------------
+// On the grids of a run's first iterations (2-D side <= 32, 3-D side <= 16) the
+// transforms are a chain of three (3-D: five) launches whose work is a few
+// thousand operations per line; the sum over all pairs of nodes is 262,144
+// multiply-adds on a 16 x 16 grid and 84 million on a 16-cube, one launch
+// spread over the device.  FP32 sums in a fixed order: at most 32 terms per
+// thread, then the threads' partials in a fixed order.  16 x 16 grid: 25.5 us of
+// transforms -> 4.4; 16-cube: 58 -> 16.  Potentials come node-major; channel 3 (2-D) or 4 (3-D) is the charge with K1.
+constexpr int kDirect2 = 32, kDirect3 = 16;  // largest sides
+
+// One work-group per grid row y; thread (x, j) adds the nodes of row y' = j.
+template <int XP>
+__global__ __launch_bounds__(XP *XP) void conv_direct2_kernel(int ng, float hsq, const float *__restrict__ V,
+                                                             float4 *__restrict__ Phi) {
+  __shared__ float4 vs[XP][XP];    // charges of (x', y')
+  __shared__ float2 ks[XP][XP];    // K2, K1 at (|x - x'|, |y - y'|)
+  __shared__ float4 red[XP][XP];
+  const int x = threadIdx.x % XP, j = threadIdx.x / XP, y = blockIdx.x, G = ng * ng;
+  const bool in = x < ng && j < ng;
+  const int e = j * ng + x;
+  vs[j][x] = in ? make_float4(V[e], V[G + e], V[2 * G + e], 0.0f) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const float dy = (float)(y - j), r2 = (float)x * (float)x + dy * dy;
+  const float k1 = 1.0f / (1.0f + hsq * r2);
+  ks[j][x] = make_float2(k1 * k1, k1);
+  __syncthreads();
+  float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll 8
+  for (int xp = 0; xp < ng; ++xp) {
+    const float4 v = vs[j][xp];
+    const float2 k = ks[j][abs(x - xp)];
+    acc.x = fmaf(k.x, v.x, acc.x);
+    acc.y = fmaf(k.x, v.y, acc.y);
+    acc.z = fmaf(k.x, v.z, acc.z);
+    acc.w = fmaf(k.y, v.x, acc.w);
+  }
+  red[j][x] = acc;
+  __syncthreads();
+  // rows y' added in order, eight of them per thread, then the eighths
+  if (j < XP / 8) {
+    float4 s = red[8 * j][x];
+#pragma unroll
+    for (int k = 1; k < 8; ++k) {
+      const float4 t = red[8 * j + k][x];
+      s.x += t.x;
+      s.y += t.y;
+      s.z += t.z;
+      s.w += t.w;
+    }
+    red[8 * j][x] = s;
+  }
+  __syncthreads();
+  if (j == 0 && x < ng) {
+    float4 s = red[0][x];
+#pragma unroll
+    for (int k = 1; k < XP / 8; ++k) {
+      const float4 t = red[8 * k][x];
+      s.x += t.x;
+      s.y += t.y;
+      s.z += t.z;
+      s.w += t.w;
+    }
+    Phi[y * ng + x] = s;
+  }
+}
+
+// One work-group per row (y, z); thread (y', z') adds the 16 nodes of its row
+// to the 16 outputs in registers, and the threads' sums are added across each
+// wave and then over the four waves.
+__global__ __launch_bounds__(256) void conv_direct3_kernel(int ng, float hsq, const float *__restrict__ V,
+                                                           float *__restrict__ Phi) {
+  constexpr int S = kDirect3, C = 5;
+  __shared__ float red[4][S * C];
+  const int yp = threadIdx.x % S, zp = threadIdx.x / S;
+  const int y = blockIdx.x % ng, z = blockIdx.x / ng, G = ng * ng * ng;
+  const bool in = yp < ng && zp < ng;
+  float k1[S];
+  const float dy = (float)(y - yp), dz = (float)(z - zp), r0 = dy * dy + dz * dz;
+#pragma unroll
+  for (int d = 0; d < S; ++d) k1[d] = 1.0f / (1.0f + hsq * ((float)(d * d) + r0));
+  float acc[S][C];
+#pragma unroll
+  for (int x = 0; x < S; ++x)
+#pragma unroll
+    for (int c = 0; c < C; ++c) acc[x][c] = 0.0f;
+  const float *row = V + (zp * ng + yp) * ng;
+#pragma unroll
+  for (int xp = 0; xp < S; ++xp) {
+    float v[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) v[c] = in && xp < ng ? row[c * G + xp] : 0.0f;
+#pragma unroll
+    for (int x = 0; x < S; ++x) {
+      const float k = k1[x > xp ? x - xp : xp - x], kk = k * k;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[x][c] = fmaf(kk, v[c], acc[x][c]);
+      acc[x][4] = fmaf(k, v[0], acc[x][4]);
+    }
+  }
+  // across the wave: halves exchanged until 16 groups of four lanes hold 5 sums
+  // each (85 shuffles; 80 butterflies would be 480), then added over the four
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  float a[S * C];
+#pragma unroll
+  for (int x = 0; x < S; ++x)
+#pragma unroll
+    for (int c = 0; c < C; ++c) a[x * C + c] = acc[x][c];
+#pragma unroll
+  for (int half = S * C / 2, o = 32; o >= 4; half /= 2, o /= 2) {
+    const bool up = lane & o;
+#pragma unroll
+    for (int i = 0; i < half; ++i) {
+      const float keep = up ? a[i + half] : a[i], send = up ? a[i] : a[i + half];
+      a[i] = keep + __shfl_xor(send, o, 64);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < C; ++i) {
+    a[i] += __shfl_xor(a[i], 2, 64);
+    a[i] += __shfl_xor(a[i], 1, 64);
+    if ((lane & 3) == 0) red[w][(lane >> 2) * C + i] = a[i];
+  }
+  __syncthreads();
+  for (int o = threadIdx.x; o < S * C; o += blockDim.x) {
+    const int x = o / C, c = o - x * C;
+    if (x >= ng) continue;
+    const float s = (red[0][o] + red[1][o]) + (red[2][o] + red[3][o]);
+    const int e = (z * ng + y) * ng + x;
+    Phi[c < 4 ? 4 * e + c : 4 * G + e] = s;
+  }
+}
+
 }  // namespace
 
 size_t twiddle_count() { return (size_t)fft_table_size(); }
@@ -115,6 +246,19 @@ int launch_conv(hipStream_t s, const GridParams &g, int zdirect, const float *V,
                 const ConvBuffers &b, bool node_major) {
   SGT_CHECK(g.L <= kMaxL && g.L >= 2 * g.ng - 1 && fft_smooth(g.L), SGTSNE_ERR_ARG,
             "FFT length %d invalid for ng %d", g.L, g.ng);
+  const float hsq = (float)(g.hgrid * g.hgrid);
+  if (node_major && g.d == 2 && g.ng <= kDirect2) {
+    float4 *Phi4 = reinterpret_cast<float4 *>(Phi);
+    if (g.ng <= 16) conv_direct2_kernel<16><<<g.ng, 256, 0, s>>>(g.ng, hsq, V, Phi4);
+    else conv_direct2_kernel<32><<<g.ng, 1024, 0, s>>>(g.ng, hsq, V, Phi4);
+    SGT_LAUNCH_CHECK();
+    return SGTSNE_OK;
+  }
+  if (node_major && g.d == 3 && g.ng <= kDirect3) {
+    conv_direct3_kernel<<<g.ng * g.ng, 256, 0, s>>>(g.ng, hsq, V, Phi);
+    SGT_LAUNCH_CHECK();
+    return SGTSNE_OK;
+  }
   ConvPtrs ptr{V, Phi, b.W, b.Kt1, b.Kt2, b.Kh, b.tw};
   PassArgs args[kMaxPasses];
   int pairs[kMaxPasses], kinds[kMaxPasses];
