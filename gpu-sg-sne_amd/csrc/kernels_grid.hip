@@ -576,7 +576,13 @@ __global__ __launch_bounds__(kBlock) void g2s_force_kernel(GridParams g, int n,
 constexpr int kG2sLdsCells = 4096;
 constexpr int kG2sLdsBlock = 1024;
 
-inline bool g2s_lds_fits(int d, int ng) { return (d == 2 && ng <= 64) || (d == 3 && ng <= 16); }
+// Below about 200,000 points the copies of the grid into LDS (and, in 3-D, a
+// work-group per CU of 80 KB) cost more than reading the nodes from cache:
+// 10,000 points 5.9 (LDS) / 3.8 us, 3-D 20,000 20.5 / 8.4, 200,003 2-D 6.5 / 6.5
+// and 3-D 21.3 / 23.1, 400,000 8.4 / 9.3.
+inline bool g2s_lds_fits(int d, int ng, int n) {
+  return n >= 200000 && ((d == 2 && ng <= 64) || (d == 3 && ng <= 16));
+}
 
 template <int D, bool ZDIRECT>
 __global__ __launch_bounds__(kG2sLdsBlock) void g2s_lds_kernel(GridParams g, int n, const float *__restrict__ Y,
@@ -1249,7 +1255,7 @@ int launch_s2g(hipStream_t s, const GridParams &g, int n, const float *Y, float 
 
 int launch_g2s_force(hipStream_t s, const GridParams &g, int n, const float *Y, const float *Phi,
                      float *Frep, int zdirect, RedWork rw, int *nz, DevScalars *stamp, const int32_t *ord) {
-  if (g2s_lds_fits(g.d, g.ng)) {
+  if (g2s_lds_fits(g.d, g.ng, n)) {
     // one 16-wave work-group per CU (the grid copy takes half of its LDS)
     const int lb = std::max(1, std::min({rw.max_blocks, 256, div_up(n > 0 ? n : 1, kG2sLdsBlock)}));
     if (g.d == 2) {
