@@ -206,19 +206,6 @@ int ws_reserve(sgtsne_batch *b, size_t bytes) {
   return SGTSNE_OK;
 }
 
-// Consecutive 256-byte-aligned pieces of one buffer; with a null base it
-// only adds up the size the same pieces need.
-struct Carve {
-  char *base;
-  size_t off = 0;
-  template <class T>
-  T *take(size_t count) {
-    T *p = base ? reinterpret_cast<T *>(base + off) : nullptr;
-    off += (sizeof(T) * std::max<size_t>(count, 1) + 255) & ~(size_t)255;
-    return p;
-  }
-};
-
 double bdefault_h(int d) { return d == 1 ? 0.5 : d == 2 ? 0.7 : 1.2; }
 
 // Largest grid side a job may reach: the embedding extent grows with N, so

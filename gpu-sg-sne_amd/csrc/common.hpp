@@ -44,6 +44,19 @@ constexpr int kWave = 64;  // CDNA wavefront width
 
 inline int div_up(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 
+// Consecutive 256-byte-aligned pieces of one buffer; with a null base it
+// only adds up the size the same pieces need.
+struct Carve {
+  char *base;
+  size_t off = 0;
+  template <class T>
+  T *take(size_t count) {
+    T *p = base ? reinterpret_cast<T *>(base + off) : nullptr;
+    off += (sizeof(T) * (count > 0 ? count : 1) + 255) & ~(size_t)255;
+    return p;
+  }
+};
+
 // Per-point storage stride: Y, uY, gains, Fattr, Frep are AoS with d=1 -> 1,
 // d=2 -> 2 (float2), d=3 -> 4 (float4, the 4th lane is padding) so that one
 // point is one aligned vector load.

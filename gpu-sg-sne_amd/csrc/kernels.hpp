@@ -188,10 +188,10 @@ int gpu_symmetrize(hipStream_t s, int n, int64_t nnz, const int32_t *rowptr_d,
 struct SymPending {
   bool open = false;
   int n = 0;
-  int64_t m2 = 0;
-  unsigned long long *k0 = nullptr, *k1 = nullptr;
-  double *v0 = nullptr, *v1 = nullptr, *total = nullptr;
-  int *nruns = nullptr;
+  void *ws = nullptr;  // the one block the pointers below lie in
+  const int32_t *off = nullptr, *ucnt = nullptr, *rp = nullptr;
+  const int32_t *mcol = nullptr;
+  const double *mval = nullptr, *total = nullptr;
   const int *runs_host = nullptr;
 };
 int sym_begin(hipStream_t s, int n, int64_t nnz, const int32_t *rowptr_d, const int32_t *col_d,
