@@ -79,8 +79,9 @@ struct FrontEnd {
   int n = 0, dim = 0, k = 0, max_iter = 0, ng_cap = 0;
   double u = 0.0;
   const float *y_in = nullptr;  // the caller's, read at admission
+  void *ws = nullptr;  // the block of X, the kNN rows and P
   float *Xf = nullptr, *vv = nullptr, *svv = nullptr;
-  double *Xd = nullptr, *Dd = nullptr;
+  double *Dd = nullptr;
   int32_t *Id = nullptr, *rp = nullptr, *cc = nullptr, *srp = nullptr, *scc = nullptr;
   int64_t m = 0;
   KnnPending knn;
@@ -167,7 +168,7 @@ struct sgtsne_batch {
   // memory released on the iteration stream, returned to the pool once the
   // queued work that used it has passed its event
   struct Deferred {
-    void *p[3];
+    void *p;
     hipEvent_t ev;
   };
   std::vector<Deferred> deferred;
@@ -301,13 +302,13 @@ void release_graph(sgtsne_batch *b) {
   b->graph_valid = false;
 }
 
-// Queues the release of up to three blocks once the iteration stream has
+// Queues the release of a block once the iteration stream has
 // passed this point (see release_deferred).
-int defer_free(sgtsne_batch *b, void *p0, void *p1 = nullptr, void *p2 = nullptr) {
+int defer_free(sgtsne_batch *b, void *p) {
   hipEvent_t ev = nullptr;
   SGT_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
   SGT_HIP(hipEventRecord(ev, b->stream));
-  b->deferred.push_back(sgtsne_batch::Deferred{{p0, p1, p2}, ev});
+  b->deferred.push_back(sgtsne_batch::Deferred{p, ev});
   return SGTSNE_OK;
 }
 
@@ -316,8 +317,7 @@ int defer_free(sgtsne_batch *b, void *p0, void *p1 = nullptr, void *p2 = nullptr
 void release_deferred(sgtsne_batch *b, bool all = false) {
   for (auto it = b->deferred.begin(); it != b->deferred.end();) {
     if (all || hipEventQuery(it->ev) == hipSuccess) {
-      for (void *q : it->p)
-        if (q) (void)hipFreeAsync(q, b->copy);  // idle stream: the block is free at once
+      if (it->p) (void)hipFreeAsync(it->p, b->copy);  // idle stream: the block is free at once
       (void)hipEventDestroy(it->ev);
       it = b->deferred.erase(it);
     } else {
@@ -915,7 +915,7 @@ void fe_release(sgtsne_batch *b, FrontEnd &f) {
   const hipStream_t s = b->prep;
   knn_release(s, &f.knn);
   sym_release(s, &f.sym);
-  void *bufs[] = {f.Xf, f.Xd, f.Dd, f.Id, f.rp, f.cc, f.vv, f.srp, f.scc, f.svv};
+  void *bufs[] = {f.ws, f.srp};
   for (void *q : bufs)
     if (q) (void)hipFreeAsync(q, s);
   fe_clear(f);
@@ -936,12 +936,8 @@ int fe_advance(sgtsne_batch *b, FrontEnd &f, int *job) {
   } else if (f.stage == 2) {  // merged count known: P_sym's CSR
     st = sym_end(s, &f.sym, &f.srp, &f.scc, &f.svv, &f.m, true);
     // released in stream order, after the kernels just queued that read them
-    void *tmp[] = {f.Xf, f.Xd, f.Dd, f.Id, f.rp, f.cc, f.vv};
-    for (void *q : tmp)
-      if (q) (void)hipFreeAsync(q, s);
-    f.Xf = f.vv = nullptr;
-    f.Xd = f.Dd = nullptr;
-    f.Id = f.rp = f.cc = nullptr;
+    if (f.ws) (void)hipFreeAsync(f.ws, s);
+    f.ws = nullptr;
   } else {  // P_sym built: admission
     std::lock_guard<std::mutex> lock(b->mu);
     release_deferred(b);
@@ -951,7 +947,7 @@ int fe_advance(sgtsne_batch *b, FrontEnd &f, int *job) {
       return st;
     }
     // the admitted P is read by copies queued on the iteration stream
-    st = defer_free(b, f.srp, f.scc, f.svv);
+    st = defer_free(b, f.srp);
     fe_clear(f);
     return st ? st : 1;
   }
@@ -1080,9 +1076,14 @@ int sgtsne_batch_add(sgtsne_batch *b, int n, int64_t nnz, const int32_t *rowptr,
   float *vv = nullptr;
   // temporaries come from the stream-ordered pool: no release here waits for
   // the iterations queued on the other stream
-  SGT_HIP(hipMallocAsync((void **)&rp, sizeof(int32_t) * ((size_t)n + 1), s));
-  SGT_HIP(hipMallocAsync((void **)&cc, sizeof(int32_t) * (size_t)std::max<int64_t>(nnz, 1), s));
-  SGT_HIP(hipMallocAsync((void **)&vv, sizeof(float) * (size_t)std::max<int64_t>(nnz, 1), s));
+  void *ws = nullptr;
+  for (int pass = 0; pass < 2; ++pass) {
+    Carve c{static_cast<char *>(ws)};
+    rp = c.take<int32_t>((size_t)n + 1);
+    cc = c.take<int32_t>(nnz);
+    vv = c.take<float>(nnz);
+    if (pass == 0) SGT_HIP(hipMallocAsync(&ws, c.off, s));
+  }
   int st = SGTSNE_OK;
   if (hipMemcpyAsync(rp, rowptr, sizeof(int32_t) * ((size_t)n + 1), hipMemcpyHostToDevice, s) != hipSuccess ||
       (nnz > 0 && (hipMemcpyAsync(cc, col, sizeof(int32_t) * nnz, hipMemcpyHostToDevice, s) != hipSuccess ||
@@ -1104,18 +1105,16 @@ int sgtsne_batch_add(sgtsne_batch *b, int n, int64_t nnz, const int32_t *rowptr,
   std::lock_guard<std::mutex> lock(b->mu);
   release_deferred(b);
   if (!st) st = admit(b, n, m, srp, scc, svv, y_in, max_iter, ng_cap, job);
-  if (srp != rp) {
-    (void)hipFreeAsync(rp, s);
-    (void)hipFreeAsync(cc, s);
-    (void)hipFreeAsync(vv, s);
-  }
   // the admitted P is read by copies queued on the iteration stream
+  void *held = ws;
+  if (srp != rp) {
+    (void)hipFreeAsync(ws, s);
+    held = srp;
+  }
   if (st) {
-    (void)hipFreeAsync(srp, s);
-    (void)hipFreeAsync(scc, s);
-    (void)hipFreeAsync(svv, s);
+    if (held) (void)hipFreeAsync(held, s);
   } else {
-    SGT_TRY(defer_free(b, srp, scc, svv));
+    SGT_TRY(defer_free(b, held));
   }
   return st;
 }
@@ -1152,16 +1151,19 @@ int sgtsne_batch_add_points_async(sgtsne_batch *b, const float *X, int n, int di
     }
   };
   // temporaries come from the stream-ordered pool (see sgtsne_batch_add)
-  chk(hipMallocAsync((void **)&f.Xf, nx * sizeof(float), s), "hipMallocAsync");
-  chk(hipMallocAsync((void **)&f.Xd, nx * sizeof(double), s), "hipMallocAsync");
-  chk(hipMallocAsync((void **)&f.Dd, (size_t)n * (k + 1) * sizeof(double), s), "hipMallocAsync");
-  chk(hipMallocAsync((void **)&f.Id, (size_t)n * (k + 1) * sizeof(int32_t), s), "hipMallocAsync");
-  chk(hipMallocAsync((void **)&f.rp, ((size_t)n + 1) * sizeof(int32_t), s), "hipMallocAsync");
-  chk(hipMallocAsync((void **)&f.cc, (size_t)n * k * sizeof(int32_t), s), "hipMallocAsync");
-  chk(hipMallocAsync((void **)&f.vv, (size_t)n * k * sizeof(float), s), "hipMallocAsync");
-  chk(hipMemcpyAsync(f.Xf, X, nx * sizeof(float), hipMemcpyHostToDevice, s), "copy of X");
-  if (!st) st = launch_to_double(s, f.Xf, f.Xd, (int64_t)nx);
-  if (!st) st = knn_begin(s, f.Xd, n, dim, k, f.Id, f.Dd, SGTSNE_KNN_AUTO, f.counts, &f.knn);
+  for (int pass = 0; pass < 2; ++pass) {
+    Carve c{static_cast<char *>(f.ws)};
+    f.Xf = c.take<float>(nx);
+    f.Dd = c.take<double>((size_t)n * (k + 1));
+    f.Id = c.take<int32_t>((size_t)n * (k + 1));
+    f.rp = c.take<int32_t>((size_t)n + 1);
+    f.cc = c.take<int32_t>((size_t)n * k);
+    f.vv = c.take<float>((size_t)n * k);
+    if (pass == 0) chk(hipMallocAsync(&f.ws, c.off, s), "hipMallocAsync");
+    if (st) break;
+  }
+  if (!st) chk(hipMemcpyAsync(f.Xf, X, nx * sizeof(float), hipMemcpyHostToDevice, s), "copy of X");
+  if (!st) st = knn_begin(s, f.Xf, n, dim, k, f.Id, f.Dd, SGTSNE_KNN_AUTO, f.counts, &f.knn);
   chk(hipEventRecord(f.ev, s), "event record");
   if (st) {
     fe_release(b, f);

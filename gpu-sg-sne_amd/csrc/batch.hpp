@@ -87,6 +87,5 @@ int launch_knn_csr(hipStream_t s, int n, int k, const int32_t *I, int32_t *rowpt
 int launch_gather_i32(hipStream_t s, int n, const int32_t *order, const int32_t *in, int32_t *out);
 int launch_iota(hipStream_t s, int n, int32_t *out);
 int launch_invert(hipStream_t s, int n, const int32_t *order, int32_t *inv);
-int launch_to_double(hipStream_t s, const float *in, double *out, int64_t m);
 
 }  // namespace sgt

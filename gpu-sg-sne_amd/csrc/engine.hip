@@ -1480,31 +1480,38 @@ int sgtsne_knn(const float *X, int n, int dim, int k, int method, int32_t *I, do
   SGT_CHECK(n > k && k >= 1 && dim >= 1, SGTSNE_ERR_ARG, "need n > k >= 1 and dim >= 1");
   hipStream_t s = nullptr;
   SGT_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
-  const size_t nx = (size_t)n * dim;
-  std::vector<double> xd(nx);
-  for (size_t t = 0; t < nx; t++) xd[t] = (double)X[t];
-  double *Xd = nullptr, *Dd = nullptr;
+  const size_t nx = (size_t)n * dim, no = (size_t)n * (k + 1);
+  float *Xd = nullptr;
+  double *Dd = nullptr;
   int32_t *Id = nullptr;
-  int st = alloc_dev((void **)&Xd, nx * sizeof(double));
-  if (!st) st = alloc_dev((void **)&Dd, (size_t)n * (k + 1) * sizeof(double));
-  if (!st) st = alloc_dev((void **)&Id, (size_t)n * (k + 1) * sizeof(int32_t));
-  if (!st && hipMemcpyAsync(Xd, xd.data(), nx * sizeof(double), hipMemcpyHostToDevice, s) != hipSuccess) {
+  void *ws = nullptr;
+  int st = SGTSNE_OK;
+  for (int pass = 0; pass < 2 && !st; ++pass) {
+    Carve c{static_cast<char *>(ws)};
+    Xd = c.take<float>(nx);
+    Dd = c.take<double>(no);
+    Id = c.take<int32_t>(no);
+    if (pass == 0 && hipMallocAsync(&ws, c.off, s) != hipSuccess) {
+      set_error("hipMallocAsync(%zu) failed", c.off);
+      ws = nullptr;
+      st = SGTSNE_ERR_NOMEM;
+    }
+  }
+  if (!st && hipMemcpyAsync(Xd, X, nx * sizeof(float), hipMemcpyHostToDevice, s) != hipSuccess) {
     set_error("copy of X failed");
     st = SGTSNE_ERR_HIP;
   }
   if (!st) st = launch_knn(s, Xd, n, dim, k, Id, Dd, method, fallback_rows);
-  if (!st && (hipMemcpyAsync(I, Id, (size_t)n * (k + 1) * sizeof(int32_t), hipMemcpyDeviceToHost, s) != hipSuccess ||
-              hipMemcpyAsync(D, Dd, (size_t)n * (k + 1) * sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess)) {
+  if (!st && (hipMemcpyAsync(I, Id, no * sizeof(int32_t), hipMemcpyDeviceToHost, s) != hipSuccess ||
+              hipMemcpyAsync(D, Dd, no * sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess)) {
     set_error("copy of kNN result failed");
     st = SGTSNE_ERR_HIP;
   }
+  if (ws) (void)hipFreeAsync(ws, s);
   if (hipStreamSynchronize(s) != hipSuccess && !st) {
     set_error("kNN kernel failed");
     st = SGTSNE_ERR_HIP;
   }
-  free_dev(Xd);
-  free_dev(Dd);
-  free_dev(Id);
   (void)hipStreamDestroy(s);
   return st;
 }
@@ -1572,32 +1579,43 @@ int sgtsne_perplexity_equalize(const int32_t *I, const double *D, int n, int k, 
   SGT_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
   double *Dd = nullptr;
   float *vd = nullptr;
-  int st = alloc_dev((void **)&Dd, (size_t)n * (k + 1) * sizeof(double));
-  if (!st) st = alloc_dev((void **)&vd, (size_t)n * k * sizeof(float));
+  void *ws = nullptr;
+  int st = SGTSNE_OK;
+  for (int pass = 0; pass < 2 && !st; ++pass) {
+    Carve c{static_cast<char *>(ws)};
+    Dd = c.take<double>((size_t)n * (k + 1));
+    vd = c.take<float>((size_t)n * k);
+    if (pass == 0 && hipMallocAsync(&ws, c.off, s) != hipSuccess) {
+      set_error("hipMallocAsync(%zu) failed", c.off);
+      ws = nullptr;
+      st = SGTSNE_ERR_NOMEM;
+    }
+  }
   if (!st && hipMemcpyAsync(Dd, D, (size_t)n * (k + 1) * sizeof(double), hipMemcpyHostToDevice, s) != hipSuccess) {
     set_error("copy of D failed");
     st = SGTSNE_ERR_HIP;
   }
   if (!st) st = launch_perplexity(s, Dd, n, k, u, vd, nullptr);
+  // kNN ids -> CSR without the self column (CU/perplexity_search.cu:100-112),
+  // while the device works
+  if (!st) {
+    for (int i = 0; i < n; i++) {
+      rowptr[i] = i * k;
+      std::memcpy(col + (size_t)i * k, I + (size_t)i * (k + 1) + 1, sizeof(int32_t) * (size_t)k);
+    }
+    rowptr[n] = n * k;
+  }
   if (!st && hipMemcpyAsync(val, vd, (size_t)n * k * sizeof(float), hipMemcpyDeviceToHost, s) != hipSuccess) {
     set_error("copy of P failed");
     st = SGTSNE_ERR_HIP;
   }
+  if (ws) (void)hipFreeAsync(ws, s);
   if (hipStreamSynchronize(s) != hipSuccess && !st) {
     set_error("perplexity kernel failed");
     st = SGTSNE_ERR_HIP;
   }
-  free_dev(Dd);
-  free_dev(vd);
   (void)hipStreamDestroy(s);
-  SGT_TRY(st);
-  // kNN ids -> CSR without the self column (CU/perplexity_search.cu:100-112)
-  for (int i = 0; i < n; i++) {
-    rowptr[i] = i * k;
-    for (int e = 0; e < k; e++) col[(size_t)i * k + e] = I[(size_t)i * (k + 1) + e + 1];
-  }
-  rowptr[n] = n * k;
-  return SGTSNE_OK;
+  return st;
 }
 
 }  // extern "C"

@@ -149,26 +149,24 @@ int fft_length_for(int ng);
 
 // ---- P construction (kernels_prep.hip) ----
 void retain_pool_memory();
-int launch_knn_exact(hipStream_t s, const double *X, int n, int dim, int k, int32_t *I, double *D);
-int launch_knn(hipStream_t s, const double *X, int n, int dim, int k, int32_t *I, double *D, int method,
+int launch_knn(hipStream_t s, const float *X, int n, int dim, int k, int32_t *I, double *D, int method,
                int *fallback_rows);
 // launch_knn in two halves for callers that must not wait in between:
 // knn_begin queues everything up to the certificate and a copy of the count
 // of uncertified rows into *count_host (pinned memory for a copy that does
-// not block); knn_end, called once the stream has passed that copy, queues
+// not block; after a failure knn_release frees what it holds); knn_end, called once the stream has passed that copy, queues
 // the exact recomputation of those rows and releases the temporaries.
 struct KnnPending {
   bool open = false;  // knn_end still has work to queue
-  const double *X = nullptr;
+  const float *X = nullptr;
   int n = 0, dim = 0, k = 0;
   int32_t *I = nullptr;
   double *D = nullptr;
   int *fb = nullptr;  // device: [0] count, then the rows
   const int *count_host = nullptr;
-  void *bufs[32] = {};
-  int nbufs = 0;
+  void *ws = nullptr;  // every temporary, one block
 };
-int knn_begin(hipStream_t s, const double *X, int n, int dim, int k, int32_t *I, double *D, int method,
+int knn_begin(hipStream_t s, const float *X, int n, int dim, int k, int32_t *I, double *D, int method,
               int *count_host, KnnPending *kp);
 int knn_end(hipStream_t s, KnnPending *kp, int *fallback_rows);
 void knn_release(hipStream_t s, KnnPending *kp);  // frees the temporaries without finishing

@@ -497,11 +497,6 @@ __global__ void iota_kernel(int n, int32_t *__restrict__ out) {
   if (i < n) out[i] = i;
 }
 
-__global__ void to_double_kernel_b(const float *__restrict__ in, double *__restrict__ out, int64_t m) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < m) out[t] = (double)in[t];
-}
-
 __global__ void offset_copy_kernel(const int32_t *__restrict__ in, int32_t *__restrict__ out, int64_t count,
                                    int32_t delta) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -677,13 +672,6 @@ int launch_invert(hipStream_t s, int n, const int32_t *order, int32_t *inv) {
 int launch_iota(hipStream_t s, int n, int32_t *out) {
   if (n <= 0) return SGTSNE_OK;
   iota_kernel<<<div_up(n, 256), 256, 0, s>>>(n, out);
-  SGT_LAUNCH_CHECK();
-  return SGTSNE_OK;
-}
-
-int launch_to_double(hipStream_t s, const float *in, double *out, int64_t m) {
-  if (m <= 0) return SGTSNE_OK;
-  to_double_kernel_b<<<div_up(m, 256), 256, 0, s>>>(in, out, m);
   SGT_LAUNCH_CHECK();
   return SGTSNE_OK;
 }

@@ -91,3 +91,13 @@ def test_knn_filtered_wide_blocks(sg):
         d2[q] = np.inf
         near = np.sort(np.partition(d2, 19)[:20])
         assert I[q, 0] == q and np.allclose(D[q, 1:], near, rtol=1e-12) and np.allclose(d2[I[q, 1:]], near, rtol=1e-12)
+
+
+# candidate lists of 65..256 entries re-ranked by one wave, two and four to a
+# lane, rows read one, two and four floats at a time
+@pytest.mark.parametrize("n,dim,k", [(66, 18, 64), (400, 20, 112), (401, 17, 113), (500, 18, 200), (900, 20, 240), (250, 64, 240)])
+def test_knn_filtered_rerank_widths(sg, O, n, dim, k):
+    X = _points(n, dim, 5 * n + dim)
+    I, D, fb = sg.knn(X, k, sg.KNN_FILTERED)
+    Io, Do = O.knn_exact(X, k)
+    assert fb >= 0 and np.array_equal(I, Io) and np.array_equal(D, Do)
