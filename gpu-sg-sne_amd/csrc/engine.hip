@@ -1256,16 +1256,21 @@ int sgtsne_ctx_step(sgtsne_ctx *c, int iters) {
   return st;
 }
 
+// Queues the repulsive sums and Z of the current Y.
+static int repulsive_terms(sgtsne_ctx *c, GridParams &g) {
+  SGT_TRY(wait_published(c));  // the bounds of the current Y
+  SGT_TRY(make_grid(c, *c->hs, g));
+  int nz = 0;
+  SGT_TRY(repulsive(c, g, false, &nz));
+  return launch_finalize_z(c->stream, nz, c->n, c->rw, c->sc);
+}
+
 int sgtsne_ctx_terms(sgtsne_ctx *c, float *Fattr, float *Frep, double *Z, int *ng, int layout) {
   SGT_CHECK(c != nullptr, SGTSNE_ERR_ARG, "ctx is NULL");
   SGT_CHECK(c->have_P && c->have_Y, SGTSNE_ERR_STATE, "upload P and set Y first");
   SGT_TRY(attractive(c));
-  SGT_TRY(wait_published(c));  // the bounds of the current Y
   GridParams g{};
-  SGT_TRY(make_grid(c, *c->hs, g));
-  int nz = 0;
-  SGT_TRY(repulsive(c, g, false, &nz));
-  SGT_TRY(launch_finalize_z(c->stream, nz, c->n, c->rw, c->sc));
+  SGT_TRY(repulsive_terms(c, g));
   DevScalars s{};
   SGT_HIP(hipMemcpyAsync(&s, c->sc, sizeof(DevScalars), hipMemcpyDeviceToHost, c->stream));
   SGT_HIP(hipStreamSynchronize(c->stream));
@@ -1279,8 +1284,8 @@ int sgtsne_ctx_terms(sgtsne_ctx *c, float *Fattr, float *Frep, double *Z, int *n
 int sgtsne_ctx_kl(sgtsne_ctx *c, double alpha, double *kl) {
   SGT_CHECK(c != nullptr && kl != nullptr, SGTSNE_ERR_ARG, "bad arguments");
   SGT_CHECK(c->have_P && c->have_Y, SGTSNE_ERR_STATE, "upload P and set Y first");
-  // Z of the current Y
-  SGT_TRY(sgtsne_ctx_terms(c, nullptr, nullptr, nullptr, nullptr, SGTSNE_LAYOUT_AOS));
+  GridParams g{};
+  SGT_TRY(repulsive_terms(c, g));  // Z of the current Y
   SGT_TRY(launch_kl(c->stream, c->d, c->n, c->rowptr, c->col, c->val, c->Y, alpha, c->sc, c->rw, c->sc));
   SGT_HIP(hipStreamSynchronize(c->stream));
   DevScalars s{};
