@@ -28,6 +28,7 @@
 #include <cmath>
 #include <cstring>
 #include <deque>
+#include <list>
 #include <mutex>
 #include <random>
 #include <vector>
@@ -63,6 +64,113 @@ struct StageSpan {
 
 constexpr size_t kStageBytes = 16u << 20;  // pinned staging for host -> device updates
 constexpr int kMarks = 16;                 // tick marks kept
+
+// The device blocks of a batch that come and go with its jobs: the front end's
+// workspaces, each P + P^T and the jobs' grids.  A block given back is kept for
+// the next job: it is handed out again on the stream it was given back on, or on
+// any once that stream has passed it, for requests of at least half its size.
+// hipFreeAsync held the host 96 us on average here and hipMallocAsync 41
+// (5 pairs per job: more than half of the time to admit a job of a few thousand
+// points: 16 jobs of 500-8000 points admitted, 8 iterations and removed 22.9 ->
+// 12.0 ms, 6 of 2000-20,000 in 3-D 14.7 -> 9.4).  At most kIdleBytes stay idle beyond the next call; the rest goes
+// back to the device's pool.
+constexpr size_t kIdleBytes = (size_t)4 << 30;
+class BlockCache final : public ScratchSource {
+ public:
+  int take(hipStream_t s, size_t bytes, void **p) override {
+    std::lock_guard<std::mutex> lock(mu_);
+    *p = nullptr;
+    Block *best = nullptr;
+    for (Block &b : blocks_)
+      if (b.idle && b.cap >= bytes && b.cap / 2 <= bytes + kStep && (!best || b.cap < best->cap) && passed(b, s))
+        best = &b;
+    if (!best) {
+      trim_locked(kIdleBytes);
+      Block nb;
+      nb.cap = (bytes + bytes / 8 + kStep - 1) / kStep * kStep;  // room for slightly larger jobs
+      hipError_t e = hipMallocAsync(&nb.p, nb.cap, s);
+      if (e != hipSuccess) {  // give the idle blocks back and try once more
+        (void)hipGetLastError();
+        trim_locked(0);
+        nb.cap = bytes > 0 ? bytes : 1;
+        e = hipMallocAsync(&nb.p, nb.cap, s);
+      }
+      if (e == hipSuccess) {
+        e = hipEventCreateWithFlags(&nb.ev, hipEventDisableTiming);
+        if (e != hipSuccess) (void)hipFreeAsync(nb.p, s);
+      }
+      if (e != hipSuccess) {
+        set_error("hipMallocAsync(%zu) failed: %s", bytes, hipGetErrorString(e));
+        return SGTSNE_ERR_NOMEM;
+      }
+      blocks_.push_back(nb);
+      best = &blocks_.back();
+    }
+    if (best->idle) idle_ -= best->cap;
+    best->idle = false;
+    *p = best->p;
+    return SGTSNE_OK;
+  }
+  void give(hipStream_t s, void *p) override {
+    if (!p) return;
+    std::lock_guard<std::mutex> lock(mu_);
+    for (auto it = blocks_.begin(); it != blocks_.end(); ++it)
+      if (it->p == p && !it->idle) {
+        if (hipEventRecord(it->ev, s) != hipSuccess) {  // no way to tell when it is free: not kept
+          (void)hipGetLastError();
+          (void)hipFreeAsync(it->p, s);
+          (void)hipEventDestroy(it->ev);
+          blocks_.erase(it);
+          return;
+        }
+        it->idle = true;
+        it->s = s;
+        idle_ += it->cap;
+        return;
+      }
+  }
+  // Returns idle blocks beyond kIdleBytes to the device's pool.
+  void trim() {
+    std::lock_guard<std::mutex> lock(mu_);
+    trim_locked(kIdleBytes);
+  }
+  // Returns every block; the caller has drained the streams.
+  void clear(hipStream_t s) {
+    std::lock_guard<std::mutex> lock(mu_);
+    for (Block &b : blocks_) {
+      (void)hipFreeAsync(b.p, s);
+      (void)hipEventDestroy(b.ev);
+    }
+    blocks_.clear();
+    idle_ = 0;
+  }
+  hipStream_t release_stream = nullptr;  // for blocks whose own stream has passed them
+
+ private:
+  static constexpr size_t kStep = (size_t)1 << 18;
+  struct Block {
+    void *p = nullptr;
+    size_t cap = 0;
+    hipEvent_t ev = nullptr;   // recorded where the block was last given back
+    hipStream_t s = nullptr;
+    bool idle = false;
+  };
+  static bool passed(const Block &b, hipStream_t s) { return b.s == s || hipEventQuery(b.ev) == hipSuccess; }
+  void trim_locked(size_t keep) {
+    for (auto it = blocks_.begin(); idle_ > keep && it != blocks_.end();)
+      if (it->idle && hipEventQuery(it->ev) == hipSuccess) {
+        (void)hipFreeAsync(it->p, release_stream);
+        (void)hipEventDestroy(it->ev);
+        idle_ -= it->cap;
+        it = blocks_.erase(it);  // the oldest first
+      } else {
+        ++it;
+      }
+  }
+  std::mutex mu_;
+  std::list<Block> blocks_;
+  size_t idle_ = 0;
+};
 
 // One admission from points (sgtsne_batch_add_points_async) whose front end
 // is queued in three parts on the front-end stream; sgtsne_batch_add_poll
@@ -143,6 +251,7 @@ struct sgtsne_batch {
   std::vector<HostJob> hj;
   std::vector<int> arena;        // live slots in ascending off
   BatchItem *items_d = nullptr;
+  JobPatch *patch_d = nullptr;   // records on their way to jobs_d
   int items_cap = 0, nitems = 0;
   double *zpart = nullptr, *spart = nullptr, *mpart = nullptr;
   void *args_d = nullptr;
@@ -165,13 +274,7 @@ struct sgtsne_batch {
   hipGraphExec_t execs[2] = {nullptr, nullptr};
   hipEvent_t exec_done[2] = {nullptr, nullptr};  // after each one's last launch
   int cur = 0;
-  // memory released on the iteration stream, returned to the pool once the
-  // queued work that used it has passed its event
-  struct Deferred {
-    void *p;
-    hipEvent_t ev;
-  };
-  std::vector<Deferred> deferred;
+  BlockCache blocks;
   bool graph_valid = false;
   bool use_graph = true;
   int64_t graph_replays = 0, graph_updates = 0, graph_instantiations = 0;
@@ -302,44 +405,6 @@ void release_graph(sgtsne_batch *b) {
   b->graph_valid = false;
 }
 
-// Queues the release of a block once the iteration stream has
-// passed this point (see release_deferred).
-int defer_free(sgtsne_batch *b, void *p) {
-  hipEvent_t ev = nullptr;
-  SGT_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-  SGT_HIP(hipEventRecord(ev, b->stream));
-  b->deferred.push_back(sgtsne_batch::Deferred{p, ev});
-  return SGTSNE_OK;
-}
-
-// Returns to the pool the deferred blocks whose event has completed (all of
-// them with `all`, after the caller has drained the stream).
-void release_deferred(sgtsne_batch *b, bool all = false) {
-  for (auto it = b->deferred.begin(); it != b->deferred.end();) {
-    if (all || hipEventQuery(it->ev) == hipSuccess) {
-      if (it->p) (void)hipFreeAsync(it->p, b->copy);  // idle stream: the block is free at once
-      (void)hipEventDestroy(it->ev);
-      it = b->deferred.erase(it);
-    } else {
-      ++it;
-    }
-  }
-}
-
-// Writes the static part of slot j's record (everything before the dynamic
-// fields) so that a running job's iteration state is left alone; skipped
-// when the device already holds it (an admission at the tail of the arena
-// changes only the new job's record, so admitting J jobs makes J uploads,
-// not J^2 / 2).
-constexpr size_t kJobStatic = offsetof(BatchJob, iter);
-static_assert(kJobStatic == 10 * sizeof(int) + 6 * sizeof(float) + sizeof(double) + 6 * sizeof(void *),
-              "the static part of a job record has no padding bytes (it is compared with memcmp)");
-int write_static(sgtsne_batch *b, int j) {
-  if (std::memcmp(&b->jobs_h[j], &b->jobs_up[j], kJobStatic) == 0) return SGTSNE_OK;
-  std::memcpy(&b->jobs_up[j], &b->jobs_h[j], kJobStatic);
-  return upload(b, b->jobs_d + j, &b->jobs_h[j], kJobStatic);
-}
-
 // Host-side check of the tables a step reads, before they are uploaded: the
 // running jobs' point and nonzero ranges lie inside the arena and do not
 // overlap, and every work item covers at most kBatchChunk points of its own
@@ -372,6 +437,26 @@ int validate_tables(const sgtsne_batch *b, const std::vector<BatchItem> &items) 
   return SGTSNE_OK;
 }
 
+// Writes the static part of every record that changed (everything before the
+// dynamic fields, so that a running job's iteration state is left alone).  One
+// copy of the changed records and one kernel that puts each in its slot: a copy
+// of each record queued J^2 / 2 copies for J jobs added or removed in turn,
+// 2 ms of host time for 16.
+int write_static(sgtsne_batch *b) {
+  std::vector<JobPatch> up;
+  for (int j : b->arena)
+    if (std::memcmp(&b->jobs_h[j], &b->jobs_up[j], kJobStatic) != 0) {
+      std::memcpy(&b->jobs_up[j], &b->jobs_h[j], kJobStatic);
+      up.emplace_back();
+      up.back().job = j;
+      std::memcpy(up.back().rec, &b->jobs_h[j], kJobStatic);
+    }
+  if (up.empty()) return SGTSNE_OK;
+  // queued patches are applied in stream order, so one buffer serves them all
+  SGT_TRY(upload(b, b->patch_d, up.data(), up.size() * sizeof(JobPatch)));
+  return launch_bpatch(b->stream, b->jobs_d, b->max_jobs, b->patch_d, (int)up.size());
+}
+
 int rebuild_items(sgtsne_batch *b) {
   std::vector<BatchItem> items;
   for (int j : b->arena) {
@@ -390,7 +475,7 @@ int rebuild_items(sgtsne_batch *b) {
   // stream-ordered after the iterations already queued, which still read the
   // old table; staged, so nothing here waits for them
   SGT_TRY(upload(b, b->items_d, items.data(), items.size() * sizeof(BatchItem)));
-  for (int j : b->arena) SGT_TRY(write_static(b, j));
+  SGT_TRY(write_static(b));
   SGT_TRY(stage_commit(b));
   invalidate_graph(b);
   return SGTSNE_OK;
@@ -730,7 +815,7 @@ int admit(sgtsne_batch *b, int n, int64_t nnz, const int32_t *rp_d, const int32_
   h.max_iter = max_iter;
   h.ng_cap = ng_cap;
   h.gbytes = gbytes;
-  SGT_HIP(hipMallocAsync(&h.gmem, gbytes, b->stream));
+  SGT_TRY(b->blocks.take(b->stream, gbytes, &h.gmem));
   SGT_HIP(hipMemsetAsync(h.gmem, 0, vb, b->stream));  // the spread grid starts (and stays) zero
   char *gm = static_cast<char *>(h.gmem);
 
@@ -812,18 +897,12 @@ void destroy_all(sgtsne_batch *b) {
     f.ev = nullptr;
   }
   release_graph(b);
-  release_deferred(b, true);
   for (hipEvent_t &e : b->exec_done)
     if (e) {
       (void)hipEventDestroy(e);
       e = nullptr;
     }
-  // per-job grids come from the stream-ordered pool: release them the same way
-  for (auto &h : b->hj)
-    if (h.gmem) {
-      (void)hipFreeAsync(h.gmem, b->stream);
-      h.gmem = nullptr;
-    }
+  b->blocks.clear(b->stream);  // the jobs' grids among them
   if (b->stream) (void)hipStreamSynchronize(b->stream);
   bfree(b->rowptr);
   bfree(b->col);
@@ -835,6 +914,7 @@ void destroy_all(sgtsne_batch *b) {
   bfree(b->Frep);
   bfree(b->perm);
   bfree(b->jobs_d);
+  bfree(b->patch_d);
   bfree(b->items_d);
   bfree(b->zpart);
   bfree(b->spart);
@@ -915,9 +995,8 @@ void fe_release(sgtsne_batch *b, FrontEnd &f) {
   const hipStream_t s = b->prep;
   knn_release(s, &f.knn);
   sym_release(s, &f.sym);
-  void *bufs[] = {f.ws, f.srp};
-  for (void *q : bufs)
-    if (q) (void)hipFreeAsync(q, s);
+  b->blocks.give(s, f.ws);
+  b->blocks.give(s, f.srp);
   fe_clear(f);
 }
 
@@ -932,24 +1011,24 @@ int fe_advance(sgtsne_batch *b, FrontEnd &f, int *job) {
     if (!st) st = launch_perplexity(s, f.Dd, f.n, f.k, f.u, f.vv, nullptr);
     if (!st) st = launch_knn_csr(s, f.n, f.k, f.Id, f.rp, f.cc);
     if (!st && b->p.lambda != 1.0) st = launch_lambda_rescale(s, f.n, f.rp, f.vv, b->p.lambda, b->p.drop_leaf);
-    if (!st) st = sym_begin(s, f.n, (int64_t)f.n * f.k, f.rp, f.cc, f.vv, f.counts + 1, &f.sym);
+    if (!st) st = sym_begin(s, b->blocks, f.n, (int64_t)f.n * f.k, f.rp, f.cc, f.vv, f.counts + 1, &f.sym);
   } else if (f.stage == 2) {  // merged count known: P_sym's CSR
-    st = sym_end(s, &f.sym, &f.srp, &f.scc, &f.svv, &f.m, true);
-    // released in stream order, after the kernels just queued that read them
-    if (f.ws) (void)hipFreeAsync(f.ws, s);
+    st = sym_end(s, &f.sym, &f.srp, &f.scc, &f.svv, &f.m, &b->blocks);
+    // given back in stream order, after the kernels just queued that read it
+    b->blocks.give(s, f.ws);
     f.ws = nullptr;
   } else {  // P_sym built: admission
     std::lock_guard<std::mutex> lock(b->mu);
-    release_deferred(b);
+    b->blocks.trim();
     st = admit(b, f.n, f.m, f.srp, f.scc, f.svv, f.y_in, f.max_iter, f.ng_cap, job);
     if (st) {
       fe_release(b, f);
       return st;
     }
     // the admitted P is read by copies queued on the iteration stream
-    st = defer_free(b, f.srp);
+    b->blocks.give(b->stream, f.srp);
     fe_clear(f);
-    return st ? st : 1;
+    return 1;
   }
   if (!st && hipEventRecord(f.ev, s) != hipSuccess) {
     set_error("front end: event record failed");
@@ -1009,6 +1088,7 @@ int sgtsne_batch_create(sgtsne_batch **out, const sgtsne_params *params, int max
   chk(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking), "stream");
   chk(hipStreamCreateWithFlags(&b->prep, hipStreamNonBlocking), "stream");
   b->copy = b->prep;
+  b->blocks.release_stream = b->copy;
   for (hipEvent_t &e : b->marks) chk(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event");
   chk(hipHostMalloc((void **)&b->stage, kStageBytes, hipHostMallocDefault), "pinned staging");
   chk(hipHostMalloc((void **)&b->fe_host, sizeof(int) * 2 * kFrontEnds, hipHostMallocDefault), "pinned counts");
@@ -1025,6 +1105,7 @@ int sgtsne_batch_create(sgtsne_batch **out, const sgtsne_params *params, int max
     if (!st) st = balloc((void **)q, sizeof(float) * P * b->ds);
   if (!st) st = balloc((void **)&b->perm, sizeof(int32_t) * P);
   if (!st) st = balloc((void **)&b->jobs_d, sizeof(BatchJob) * max_jobs);
+  if (!st) st = balloc((void **)&b->patch_d, sizeof(JobPatch) * max_jobs);
   if (!st) st = balloc((void **)&b->items_d, sizeof(BatchItem) * b->items_cap);
   if (!st) st = balloc((void **)&b->zpart, sizeof(double) * 2 * b->items_cap);
   if (!st) st = balloc((void **)&b->spart, sizeof(double) * 4 * b->items_cap);
@@ -1074,15 +1155,15 @@ int sgtsne_batch_add(sgtsne_batch *b, int n, int64_t nnz, const int32_t *rowptr,
   const hipStream_t s = b->prep;
   int32_t *rp = nullptr, *cc = nullptr;
   float *vv = nullptr;
-  // temporaries come from the stream-ordered pool: no release here waits for
-  // the iterations queued on the other stream
+  // temporaries come from the batch's blocks: no release here waits for the
+  // iterations queued on the other stream
   void *ws = nullptr;
   for (int pass = 0; pass < 2; ++pass) {
     Carve c{static_cast<char *>(ws)};
     rp = c.take<int32_t>((size_t)n + 1);
     cc = c.take<int32_t>(nnz);
     vv = c.take<float>(nnz);
-    if (pass == 0) SGT_HIP(hipMallocAsync(&ws, c.off, s));
+    if (pass == 0) SGT_TRY(b->blocks.take(s, c.off, &ws));
   }
   int st = SGTSNE_OK;
   if (hipMemcpyAsync(rp, rowptr, sizeof(int32_t) * ((size_t)n + 1), hipMemcpyHostToDevice, s) != hipSuccess ||
@@ -1096,26 +1177,22 @@ int sgtsne_batch_add(sgtsne_batch *b, int n, int64_t nnz, const int32_t *rowptr,
   int64_t m = nnz;
   if (!st && symmetrize) {
     if (b->p.lambda != 1.0) st = launch_lambda_rescale(s, n, rp, vv, b->p.lambda, b->p.drop_leaf);
-    if (!st) st = gpu_symmetrize(s, n, nnz, rp, cc, vv, &srp, &scc, &svv, &m, true);
+    if (!st) st = gpu_symmetrize(s, n, nnz, rp, cc, vv, &srp, &scc, &svv, &m, &b->blocks);
   }
   if (!st && hipStreamSynchronize(s) != hipSuccess) {  // the caller's P is read, and m known
     set_error("preparation of P failed");
     st = SGTSNE_ERR_HIP;
   }
   std::lock_guard<std::mutex> lock(b->mu);
-  release_deferred(b);
+  b->blocks.trim();
   if (!st) st = admit(b, n, m, srp, scc, svv, y_in, max_iter, ng_cap, job);
   // the admitted P is read by copies queued on the iteration stream
   void *held = ws;
   if (srp != rp) {
-    (void)hipFreeAsync(ws, s);
+    b->blocks.give(s, ws);
     held = srp;
   }
-  if (st) {
-    if (held) (void)hipFreeAsync(held, s);
-  } else {
-    SGT_TRY(defer_free(b, held));
-  }
+  b->blocks.give(st ? s : b->stream, held);
   return st;
 }
 
@@ -1150,7 +1227,7 @@ int sgtsne_batch_add_points_async(sgtsne_batch *b, const float *X, int n, int di
       st = e == hipErrorOutOfMemory ? SGTSNE_ERR_NOMEM : SGTSNE_ERR_HIP;
     }
   };
-  // temporaries come from the stream-ordered pool (see sgtsne_batch_add)
+  // temporaries come from the batch's blocks (see sgtsne_batch_add)
   for (int pass = 0; pass < 2; ++pass) {
     Carve c{static_cast<char *>(f.ws)};
     f.Xf = c.take<float>(nx);
@@ -1159,11 +1236,11 @@ int sgtsne_batch_add_points_async(sgtsne_batch *b, const float *X, int n, int di
     f.rp = c.take<int32_t>((size_t)n + 1);
     f.cc = c.take<int32_t>((size_t)n * k);
     f.vv = c.take<float>((size_t)n * k);
-    if (pass == 0) chk(hipMallocAsync(&f.ws, c.off, s), "hipMallocAsync");
+    if (pass == 0) st = b->blocks.take(s, c.off, &f.ws);
     if (st) break;
   }
   if (!st) chk(hipMemcpyAsync(f.Xf, X, nx * sizeof(float), hipMemcpyHostToDevice, s), "copy of X");
-  if (!st) st = knn_begin(s, f.Xf, n, dim, k, f.Id, f.Dd, SGTSNE_KNN_AUTO, f.counts, &f.knn);
+  if (!st) st = knn_begin(s, b->blocks, f.Xf, n, dim, k, f.Id, f.Dd, SGTSNE_KNN_AUTO, f.counts, &f.knn);
   chk(hipEventRecord(f.ev, s), "event record");
   if (st) {
     fe_release(b, f);
@@ -1213,7 +1290,7 @@ int sgtsne_batch_step(sgtsne_batch *b, int iters) {
   SGT_TRY(check_batch(b));
   std::lock_guard<std::mutex> lock(b->mu);
   SGT_CHECK(iters >= 0, SGTSNE_ERR_ARG, "iters < 0");
-  release_deferred(b);
+  b->blocks.trim();
   if (b->arena.empty()) return SGTSNE_OK;
   if (!b->tune_pinned &&
       (b->tuned_points == 0 || b->used_points > 2 * b->tuned_points || 2 * b->used_points < b->tuned_points))
@@ -1351,8 +1428,8 @@ int sgtsne_batch_remove(sgtsne_batch *b, int job) {
   empty.status = BJ_EMPTY;
   SGT_TRY(upload(b, b->jobs_d + job, &empty, sizeof(BatchJob)));
   std::memcpy(&b->jobs_up[job], &empty, kJobStatic);
-  release_deferred(b);
-  SGT_TRY(defer_free(b, h.gmem));
+  b->blocks.trim();
+  b->blocks.give(b->stream, h.gmem);
   if (h.done_ev) (void)hipEventDestroy(h.done_ev);
   b->grid_used -= h.gbytes;
   b->arena.erase(std::find(b->arena.begin(), b->arena.end(), job));

@@ -53,9 +53,21 @@ struct BatchJob {
   GridParams g;
 };
 
+constexpr size_t kJobStatic = offsetof(BatchJob, iter);
+static_assert(kJobStatic == 10 * sizeof(int) + 6 * sizeof(float) + sizeof(double) + 6 * sizeof(void *),
+              "the static part has no padding (it is compared by memcmp)");
+
+// The static part of one job's record, and the slot it goes to.
+struct JobPatch {
+  char rec[kJobStatic];
+  int job, pad;
+};
+
 struct BatchItem {
   int job, begin, end, pad;
 };
+
+int launch_bpatch(hipStream_t s, BatchJob *jobs, int njobs, const JobPatch *patch, int count);
 
 // Bytes of one job's grid buffers at grid side ng_cap.
 size_t batch_grid_bytes(int d, int ng_cap, size_t *vfix_b, size_t *phi_b, size_t *w_b, size_t *k_b);

@@ -149,13 +149,23 @@ int fft_length_for(int ng);
 
 // ---- P construction (kernels_prep.hip) ----
 void retain_pool_memory();
+// Where the workspaces of the calls below come from: take() gives a block for
+// work queued on s from now on, give() takes it back once s has passed the
+// work queued so far.  Safe from several threads.
+struct ScratchSource {
+  virtual int take(hipStream_t s, size_t bytes, void **p) = 0;
+  virtual void give(hipStream_t s, void *p) = 0;
+  virtual ~ScratchSource() = default;
+};
+ScratchSource &stream_scratch();  // hipMallocAsync / hipFreeAsync
 int launch_knn(hipStream_t s, const float *X, int n, int dim, int k, int32_t *I, double *D, int method,
                int *fallback_rows);
 // launch_knn in two halves for callers that must not wait in between:
 // knn_begin queues everything up to the certificate and a copy of the count
 // of uncertified rows into *count_host (pinned memory for a copy that does
-// not block; after a failure knn_release frees what it holds); knn_end, called once the stream has passed that copy, queues
-// the exact recomputation of those rows and releases the temporaries.
+// not block; after a failure knn_release frees what it holds); knn_end, called
+// once the stream has passed that copy, queues the exact recomputation of
+// those rows and releases the temporaries.
 struct KnnPending {
   bool open = false;  // knn_end still has work to queue
   const float *X = nullptr;
@@ -164,10 +174,11 @@ struct KnnPending {
   double *D = nullptr;
   int *fb = nullptr;  // device: [0] count, then the rows
   const int *count_host = nullptr;
+  ScratchSource *src = nullptr;
   void *ws = nullptr;  // every temporary, one block
 };
-int knn_begin(hipStream_t s, const float *X, int n, int dim, int k, int32_t *I, double *D, int method,
-              int *count_host, KnnPending *kp);
+int knn_begin(hipStream_t s, ScratchSource &src, const float *X, int n, int dim, int k, int32_t *I, double *D,
+              int method, int *count_host, KnnPending *kp);
 int knn_end(hipStream_t s, KnnPending *kp, int *fallback_rows);
 void knn_release(hipStream_t s, KnnPending *kp);  // frees the temporaries without finishing
 int launch_perplexity(hipStream_t s, const double *D, int n, int k, double u, float *val,
@@ -178,24 +189,26 @@ int launch_rowids(hipStream_t s, int n, const int32_t *rowptr, int32_t *row);
 int gpu_symmetrize(hipStream_t s, int n, int64_t nnz, const int32_t *rowptr_d,
                    const int32_t *col_d, const float *val_d, int32_t **rowptr_out,
                    int32_t **col_out, float **val_out, int64_t *nnz_out,
-                   bool stream_ordered = false);
+                   ScratchSource *out_src = nullptr);
 // gpu_symmetrize in two halves (see KnnPending): sym_begin queues the merge of
 // P and P^T and a copy of the merged nonzero count into *runs_host; sym_end,
 // once the stream has passed that copy, queues the normalisation and the CSR
-// build into stream-ordered outputs, without waiting for them.
+// build, without waiting for them, into one block of out_src that starts at
+// rowptr (nullptr: three hipMalloc'ed arrays).
 struct SymPending {
   bool open = false;
   int n = 0;
+  ScratchSource *src = nullptr;
   void *ws = nullptr;  // the one block the pointers below lie in
   const int32_t *off = nullptr, *ucnt = nullptr, *rp = nullptr;
   const int32_t *mcol = nullptr;
   const double *mval = nullptr, *total = nullptr;
   const int *runs_host = nullptr;
 };
-int sym_begin(hipStream_t s, int n, int64_t nnz, const int32_t *rowptr_d, const int32_t *col_d,
+int sym_begin(hipStream_t s, ScratchSource &src, int n, int64_t nnz, const int32_t *rowptr_d, const int32_t *col_d,
               const float *val_d, int *runs_host, SymPending *sp);
 int sym_end(hipStream_t s, SymPending *sp, int32_t **rowptr_out, int32_t **col_out, float **val_out,
-            int64_t *nnz_out, bool stream_ordered);
+            int64_t *nnz_out, ScratchSource *out_src);
 void sym_release(hipStream_t s, SymPending *sp);
 int launch_build_ell(hipStream_t s, int n, int width, const int32_t *rowptr, const int32_t *col,
                      const float *val, int32_t *ecol, float *eval, int32_t *tail_cnt);

@@ -676,6 +676,22 @@ int launch_iota(hipStream_t s, int n, int32_t *out) {
   return SGTSNE_OK;
 }
 
+namespace {
+__global__ __launch_bounds__(64) void bpatch_kernel(BatchJob *jobs, const JobPatch *patch) {
+  static_assert(kJobStatic % sizeof(uint32_t) == 0 && kJobStatic / sizeof(uint32_t) <= 64, "one word per thread");
+  const JobPatch &p = patch[blockIdx.x];
+  if (threadIdx.x < kJobStatic / sizeof(uint32_t))
+    reinterpret_cast<uint32_t *>(jobs + p.job)[threadIdx.x] = reinterpret_cast<const uint32_t *>(p.rec)[threadIdx.x];
+}
+}  // namespace
+
+int launch_bpatch(hipStream_t s, BatchJob *jobs, int njobs, const JobPatch *patch, int count) {
+  SGT_CHECK(count >= 1 && count <= njobs, SGTSNE_ERR_STATE, "%d records for %d slots", count, njobs);
+  bpatch_kernel<<<count, 64, 0, s>>>(jobs, patch);
+  SGT_LAUNCH_CHECK();
+  return SGTSNE_OK;
+}
+
 int launch_offset_copy_i32(hipStream_t s, const int32_t *in, int32_t *out, int64_t count, int32_t delta) {
   if (count <= 0) return SGTSNE_OK;
   const int blocks = (int)std::min<int64_t>((count + 255) / 256, 8192);

@@ -1794,13 +1794,14 @@ namespace {
 // (11.5 ms).
 constexpr size_t kKnnSlabBytes = (size_t)1 << 29;
 
-int knn_exact_rows(hipStream_t s, const float *X, int n, int dim, int k, const int *qlist, int nq, int32_t *I,
+int knn_exact_rows(hipStream_t s, ScratchSource &src, const float *X, int n, int dim, int k, const int *qlist, int nq, int32_t *I,
                    double *D) {
   const int slab = (int)std::min<int64_t>(nq, std::max<int64_t>(128, (int64_t)(kKnnSlabBytes / 8 / n) / 128 * 128));
   const int mirror = !qlist && nq == n && slab == n;
   const bool few = qlist && nq <= 256;
-  double *dist = nullptr;
-  SGT_HIP(hipMallocAsync((void **)&dist, sizeof(double) * (size_t)slab * n, s));
+  void *block = nullptr;
+  SGT_TRY(src.take(s, sizeof(double) * (size_t)slab * n, &block));
+  double *dist = static_cast<double *>(block);
   for (int s0 = 0; s0 < nq; s0 += slab) {
     const int m = std::min(slab, nq - s0);
     if (few)
@@ -1815,20 +1816,21 @@ int knn_exact_rows(hipStream_t s, const float *X, int n, int dim, int k, const i
       knn_select_kernel<2 * kKnnMaxK><<<m, kKnnThreads, 0, s>>>(dist, n, k, qlist, s0, I, D);
     SGT_LAUNCH_CHECK();
   }
-  SGT_HIP(hipFreeAsync(dist, s));
+  src.give(s, block);
   return SGTSNE_OK;
 }
 
 }  // namespace
 
-int knn_begin(hipStream_t s, const float *X, int n, int dim, int k, int32_t *I, double *D, int method,
-              int *count_host, KnnPending *pend) {
+int knn_begin(hipStream_t s, ScratchSource &src, const float *X, int n, int dim, int k, int32_t *I, double *D,
+              int method, int *count_host, KnnPending *pend) {
   *pend = KnnPending{};
+  pend->src = &src;
   SGT_CHECK(n > k && k >= 1 && dim >= 1, SGTSNE_ERR_ARG, "kNN needs n > k >= 1 (n=%d k=%d)", n, k);
   SGT_CHECK(k <= kKnnMaxK, SGTSNE_ERR_ARG, "k too large");
   const bool filter_ok = k + kFiltSlack <= kRerank && dim <= kFiltMaxDp && n >= kFiltQ;
   if (method == SGTSNE_KNN_EXACT_FP64 || (method == SGTSNE_KNN_AUTO && !filter_ok))
-    return knn_exact_rows(s, X, n, dim, k, nullptr, n, I, D);  // nothing left for knn_end
+    return knn_exact_rows(s, src, X, n, dim, k, nullptr, n, I, D);  // nothing left for knn_end
   SGT_CHECK(filter_ok, SGTSNE_ERR_ARG, "the filtered kNN needs k <= %d, dim <= %d and n >= %d",
             kRerank - kFiltSlack, kFiltMaxDp, kFiltQ);
   const int kp = std::min(k + kFiltSlack, n - 1);
@@ -1852,8 +1854,8 @@ int knn_begin(hipStream_t s, const float *X, int n, int dim, int k, int32_t *I, 
   uint32_t *key0 = nullptr, *key1 = nullptr;
   void *tmp = nullptr;
   unsigned long long *rmax;
-  // one block for every temporary: each pair of stream-ordered calls holds the
-  // host for about 50 us
+  // one block for every temporary: a stream-ordered allocation and its release
+  // hold the host for 50 us and more
   for (int pass = 0; pass < 2; ++pass) {
     Carve c{static_cast<char *>(pend->ws)};
     rmax = c.take<unsigned long long>(1);
@@ -1885,7 +1887,7 @@ int knn_begin(hipStream_t s, const float *X, int n, int dim, int k, int32_t *I, 
       trad = c.take<double>(ntiles);
       tmp = c.take<char>(tb);
     }
-    if (pass == 0) SGT_HIP(hipMallocAsync(&pend->ws, c.off, s));
+    if (pass == 0) SGT_TRY(src.take(s, c.off, &pend->ws));
   }
   pend->open = true;  // from here on a failure releases the block
   SGT_HIP(hipMemsetAsync(rmax, 0, sizeof(unsigned long long), s));
@@ -1945,7 +1947,7 @@ int knn_begin(hipStream_t s, const float *X, int n, int dim, int k, int32_t *I, 
 }
 
 void knn_release(hipStream_t s, KnnPending *kp) {
-  if (kp->ws) (void)hipFreeAsync(kp->ws, s);
+  if (kp->ws) kp->src->give(s, kp->ws);
   *kp = KnnPending{};
 }
 
@@ -1956,7 +1958,7 @@ int knn_end(hipStream_t s, KnnPending *kp, int *fallback_rows) {
   }
   const int nfb = *kp->count_host;
   int st = SGTSNE_OK;
-  if (nfb > 0) st = knn_exact_rows(s, kp->X, kp->n, kp->dim, kp->k, kp->fb + 1, nfb, kp->I, kp->D);
+  if (nfb > 0) st = knn_exact_rows(s, *kp->src, kp->X, kp->n, kp->dim, kp->k, kp->fb + 1, nfb, kp->I, kp->D);
   if (fallback_rows) *fallback_rows = nfb;
   knn_release(s, kp);
   return st;
@@ -1967,7 +1969,7 @@ int launch_knn(hipStream_t s, const float *X, int n, int dim, int k, int32_t *I,
   if (fallback_rows) *fallback_rows = -1;
   int nfb = 0;
   KnnPending kp;
-  const int st = knn_begin(s, X, n, dim, k, I, D, method, &nfb, &kp);
+  const int st = knn_begin(s, stream_scratch(), X, n, dim, k, I, D, method, &nfb, &kp);
   if (st) {
     knn_release(s, &kp);
     return st;
@@ -2019,6 +2021,19 @@ void retain_pool_memory() {
   (void)hipMemPoolSetAttribute(pool, hipMemPoolReuseAllowInternalDependencies, &off);
 }
 
+ScratchSource &stream_scratch() {
+  struct Direct final : ScratchSource {
+    int take(hipStream_t s, size_t bytes, void **p) override {
+      *p = nullptr;
+      SGT_HIP(hipMallocAsync(p, bytes > 0 ? bytes : 1, s));
+      return SGTSNE_OK;
+    }
+    void give(hipStream_t s, void *p) override { (void)hipFreeAsync(p, s); }
+  };
+  static Direct direct;
+  return direct;
+}
+
 int device_exclusive_scan(hipStream_t s, const int32_t *in, int32_t *out, int n) {
   size_t tb = 0;
   SGT_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, in, out, n, s));
@@ -2029,9 +2044,10 @@ int device_exclusive_scan(hipStream_t s, const int32_t *in, int32_t *out, int n)
   return SGTSNE_OK;
 }
 
-int sym_begin(hipStream_t s, int n, int64_t nnz, const int32_t *rowptr_d, const int32_t *col_d,
+int sym_begin(hipStream_t s, ScratchSource &src, int n, int64_t nnz, const int32_t *rowptr_d, const int32_t *col_d,
               const float *val_d, int *runs_host, SymPending *sp) {
   *sp = SymPending{};
+  sp->src = &src;
   const int64_t m2 = 2 * nnz;
   SGT_CHECK(m2 < (int64_t)INT_MAX, SGTSNE_ERR_ARG, "2*nnz exceeds the int32 range");
   size_t tb = 0, tr = 0;
@@ -2053,7 +2069,7 @@ int sym_begin(hipStream_t s, int n, int64_t nnz, const int32_t *rowptr_d, const 
     rowsum = c.take<double>(n);
     total = c.take<double>(1);
     tmp = c.take<char>(std::max(tb, tr));
-    if (pass == 0) SGT_HIP(hipMallocAsync(&sp->ws, c.off, s));
+    if (pass == 0) SGT_TRY(src.take(s, c.off, &sp->ws));
   }
   sp->open = true;
   sp->n = n;
@@ -2084,28 +2100,25 @@ int sym_begin(hipStream_t s, int n, int64_t nnz, const int32_t *rowptr_d, const 
 }
 
 void sym_release(hipStream_t s, SymPending *sp) {
-  if (sp->ws) (void)hipFreeAsync(sp->ws, s);
+  if (sp->ws) sp->src->give(s, sp->ws);
   *sp = SymPending{};
 }
 
 int sym_end(hipStream_t s, SymPending *sp, int32_t **rowptr_out, int32_t **col_out, float **val_out,
-            int64_t *nnz_out, bool stream_ordered) {
+            int64_t *nnz_out, ScratchSource *out_src) {
   SGT_CHECK(sp->open, SGTSNE_ERR_STATE, "no symmetrisation pending");
   const int n = sp->n;
   const int runs = *sp->runs_host;
   int32_t *rp = nullptr, *cc = nullptr;
   float *vv = nullptr;
-  // the outputs come from the stream-ordered pool as one block, which starts at
-  // rowptr and which the caller releases with hipFreeAsync, or each from
-  // hipMalloc (released with hipFree)
-  if (stream_ordered) {
+  if (out_src) {
     void *block = nullptr;
     for (int pass = 0; pass < 2; ++pass) {
       Carve c{static_cast<char *>(block)};
       rp = c.take<int32_t>((size_t)n + 1);
       cc = c.take<int32_t>(runs);
       vv = c.take<float>(runs);
-      if (pass == 0) SGT_HIP(hipMallocAsync(&block, c.off, s));
+      if (pass == 0) SGT_TRY(out_src->take(s, c.off, &block));
     }
   } else {
     SGT_HIP(hipMalloc((void **)&rp, sizeof(int32_t) * ((size_t)n + 1)));
@@ -2125,12 +2138,12 @@ int sym_end(hipStream_t s, SymPending *sp, int32_t **rowptr_out, int32_t **col_o
 
 int gpu_symmetrize(hipStream_t s, int n, int64_t nnz, const int32_t *rowptr_d, const int32_t *col_d,
                    const float *val_d, int32_t **rowptr_out, int32_t **col_out, float **val_out,
-                   int64_t *nnz_out, bool stream_ordered) {
+                   int64_t *nnz_out, ScratchSource *out_src) {
   int runs = 0;
   SymPending sp;
-  SGT_TRY(sym_begin(s, n, nnz, rowptr_d, col_d, val_d, &runs, &sp));
+  SGT_TRY(sym_begin(s, out_src ? *out_src : stream_scratch(), n, nnz, rowptr_d, col_d, val_d, &runs, &sp));
   SGT_HIP(hipStreamSynchronize(s));
-  SGT_TRY(sym_end(s, &sp, rowptr_out, col_out, val_out, nnz_out, stream_ordered));
+  SGT_TRY(sym_end(s, &sp, rowptr_out, col_out, val_out, nnz_out, out_src));
   SGT_HIP(hipStreamSynchronize(s));
   return SGTSNE_OK;
 }
