@@ -241,6 +241,8 @@ struct sgtsne_batch {
   int32_t *rowptr = nullptr, *col = nullptr;
   float *val = nullptr;
   float *Y = nullptr, *uY = nullptr, *gains = nullptr, *Fattr = nullptr, *Frep = nullptr;
+  int32_t *sord = nullptr;  // 3-D: the order in which the rows are spread
+  int ord_left = 0;         // iterations until it is renewed (0: before the next spread)
   int32_t *perm = nullptr;  // device row -> the caller's index within its job
   int64_t used_points = 0, used_nnz = 0;
 
@@ -472,6 +474,7 @@ int rebuild_items(sgtsne_batch *b) {
   SGT_CHECK((int)items.size() <= b->items_cap, SGTSNE_ERR_ARG, "work items exceed capacity");
   SGT_TRY(validate_tables(b, items));
   b->nitems = (int)items.size();
+  b->ord_left = 0;
   // stream-ordered after the iterations already queued, which still read the
   // old table; staged, so nothing here waits for them
   SGT_TRY(upload(b, b->items_d, items.data(), items.size() * sizeof(BatchItem)));
@@ -498,7 +501,7 @@ int attractive(sgtsne_batch *b) {
 int enqueue_terms(sgtsne_batch *b) {
   const int zd = b->p.zeta_mode == SGTSNE_ZETA_DIRECT;
   SGT_TRY(attractive(b));
-  SGT_TRY(launch_bs2g(b->stream, b->d, b->jobs_d, b->items_d, b->nitems, b->Y,
+  SGT_TRY(launch_bs2g(b->stream, b->d, b->jobs_d, b->items_d, b->nitems, b->Y, b->sord,
                       std::min(b->nitems * (b->d == 3 ? 4 : 1), b->s2g_blocks), b->d == 3 ? 64512 : b->s2g_lds));
   SGT_TRY(launch_bconv(b->stream, b->d, zd, b->args_d, b->prefix_d, b->max_jobs, b->conv_blocks));
   SGT_TRY(launch_bg2s(b->stream, b->d, zd, b->jobs_d, b->items_d, b->nitems, b->Y, b->Frep, b->zpart,
@@ -562,10 +565,24 @@ int capture(sgtsne_batch *b) {
   return SGTSNE_OK;
 }
 
+// Lists the rows along the tiles of their grids when that is due; the list then
+// serves the next `iters` iterations.
+int renew_order(sgtsne_batch *b, int iters) {
+  if (b->d != 3 || b->ord_left > 0) return SGTSNE_OK;
+  SGT_TRY(launch_bspread_order(b->stream, b->jobs_d, b->max_jobs, b->Y, b->sord));
+  b->ord_left = iters;
+  return SGTSNE_OK;
+}
+
 int run_iterations(sgtsne_batch *b, int64_t count) {
   if (count <= 0 || b->nitems == 0) return SGTSNE_OK;
   if (b->use_graph && !b->graph_valid) SGT_TRY(capture(b));
+  // a job's first iteration only places its grid: the order follows it
+  bool fresh = false;
+  for (int j : b->arena) fresh = fresh || b->hj[j].t == 0;
   for (int64_t k = 0; k < count; ++k) {
+    SGT_TRY(renew_order(b, k == 0 && fresh ? 1 : kBatchOrderIters));
+    --b->ord_left;
     if (b->graph_valid) {
       SGT_HIP(hipGraphLaunch(b->exec, b->stream));
       b->graph_replays++;
@@ -743,6 +760,7 @@ int reorder_job(sgtsne_batch *b, int j) {
   SGT_TRY(launch_gather_i32(s, n, order, b->perm + h.off, itmp));
   SGT_HIP(hipMemcpyAsync(b->perm + h.off, itmp, sizeof(int32_t) * n, hipMemcpyDeviceToDevice, s));
   h.reorders++;
+  b->ord_left = 0;
   return SGTSNE_OK;
 }
 
@@ -912,6 +930,7 @@ void destroy_all(sgtsne_batch *b) {
   bfree(b->gains);
   bfree(b->Fattr);
   bfree(b->Frep);
+  bfree(b->sord);
   bfree(b->perm);
   bfree(b->jobs_d);
   bfree(b->patch_d);
@@ -1103,6 +1122,7 @@ int sgtsne_batch_create(sgtsne_batch **out, const sgtsne_params *params, int max
   float **pts[5] = {&b->Y, &b->uY, &b->gains, &b->Fattr, &b->Frep};
   for (float **q : pts)
     if (!st) st = balloc((void **)q, sizeof(float) * P * b->ds);
+  if (!st && b->d == 3) st = balloc((void **)&b->sord, sizeof(int32_t) * P);
   if (!st) st = balloc((void **)&b->perm, sizeof(int32_t) * P);
   if (!st) st = balloc((void **)&b->jobs_d, sizeof(BatchJob) * max_jobs);
   if (!st) st = balloc((void **)&b->patch_d, sizeof(JobPatch) * max_jobs);
@@ -1404,6 +1424,7 @@ int sgtsne_batch_terms(sgtsne_batch *b, int job, float *Fattr, float *Frep, doub
   SGT_HIP(hipMemcpyAsync(st_iter, &b->jobs_d[job].iter, 2 * sizeof(int), hipMemcpyDeviceToHost, b->stream));
   SGT_HIP(hipStreamSynchronize(b->stream));
   SGT_CHECK(st_iter[1] == BJ_RUN, SGTSNE_ERR_STATE, "job %d is not iterating (status %d)", job, st_iter[1]);
+  SGT_TRY(renew_order(b, kBatchOrderIters));
   SGT_TRY(enqueue_terms(b));
   SGT_TRY(launch_bzeta(b->stream, b->jobs_d, job, b->zpart, b->scal_d));
   double z = 0.0;

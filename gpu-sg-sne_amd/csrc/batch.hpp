@@ -75,8 +75,11 @@ size_t batch_pass_args_bytes();
 int batch_npasses(int d);
 
 // Per-iteration phases (all jobs, persistent work-groups over the items).
+// ord: the order in which the rows are spread (3-D; nullptr: as stored).
 int launch_bs2g(hipStream_t s, int d, const BatchJob *jobs, const BatchItem *items, int nitems, const float *Y,
-                int blocks, int lds_bytes);
+                const int32_t *ord, int blocks, int lds_bytes);
+constexpr int kBatchOrderIters = 16;
+int launch_bspread_order(hipStream_t s, const BatchJob *jobs, int njobs, const float *Y, int32_t *ord);
 int launch_bconv(hipStream_t s, int d, int zdirect, const void *args, const int *prefix, int njobs, int blocks);
 int launch_bg2s(hipStream_t s, int d, int zdirect, const BatchJob *jobs, const BatchItem *items, int nitems,
                 const float *Y, float *Frep, double *zpart, int blocks);
