@@ -45,7 +45,7 @@ __host__ __device__ inline size_t pass_lds_bytes(int nl, int L, int Lp) {
 }
 
 // Even lengths whose only prime factors are 2, 3 and 5.
-__host__ __device__ inline bool fft_smooth(int L) {
+constexpr bool fft_smooth(int L) {
   if (L < 2 || (L & 1)) return false;
   while (L % 2 == 0) L /= 2;
   while (L % 3 == 0) L /= 3;
@@ -53,22 +53,50 @@ __host__ __device__ inline bool fft_smooth(int L) {
   return L == 1;
 }
 
-// Smallest supported FFT length >= n.
+// Twiddle tables, one per supported length in increasing order, each holding
+// exp(-2 pi i t / L) for t < L.  off[h]: entries of the tables of lengths below
+// 2 h; len[h]: half the smallest supported length >= 2 h.  Worked out when this is
+// compiled: a walk over the lengths by each thread took 85 us of a context's
+// creation (4 now), and 1.5 of the 13 us in which a batch plans an iteration.
+struct FftTables {
+  int off[kMaxL / 2 + 2];
+  short len[kMaxL / 2 + 2];
+};
+constexpr FftTables make_fft_tables() {
+  FftTables t{};
+  for (int h = 1; h <= kMaxL / 2 + 1; ++h) t.off[h] = t.off[h - 1] + (fft_smooth(2 * (h - 1)) ? 2 * (h - 1) : 0);
+  int next = kMaxL / 2;
+  for (int h = kMaxL / 2; h >= 0; --h) {
+    if (fft_smooth(2 * h)) next = h;
+    t.len[h] = (short)next;
+  }
+  return t;
+}
+static_assert(fft_smooth(kMaxL), "the longest line is a supported length");
+constexpr FftTables kFftTabHost = make_fft_tables();
+static __constant__ const FftTables kFftTabDev = make_fft_tables();
+
+__host__ __device__ inline const FftTables &fft_tables() {
+#ifdef __HIP_DEVICE_COMPILE__
+  return kFftTabDev;
+#else
+  return kFftTabHost;
+#endif
+}
+
+// Smallest supported FFT length >= n (above kMaxL, which no pass takes: the
+// smallest even length of that form).
 __host__ __device__ inline int fft_length(int n) {
-  int L = n < 2 ? 2 : n + (n & 1);
+  const int h = n < 2 ? 1 : (n + 1) / 2;
+  if (h <= kMaxL / 2) return 2 * fft_tables().len[h];
+  int L = 2 * h;
   while (!fft_smooth(L)) L += 2;
   return L;
 }
 
-// Twiddle tables, one per supported length in increasing order, each holding
-// exp(-2 pi i t / L) for t < L; the table of L starts at fft_table_offset(L).
-__host__ __device__ inline int fft_table_offset(int L) {
-  int off = 0;
-  for (int m = 2; m < L; m += 2)
-    if (fft_smooth(m)) off += m;
-  return off;
-}
-__host__ __device__ inline int fft_table_size() { return fft_table_offset(kMaxL + 2); }
+// Start of the table of L <= kMaxL.
+__host__ __device__ inline int fft_table_offset(int L) { return fft_tables().off[L / 2]; }
+__host__ __device__ inline int fft_table_size() { return fft_tables().off[kMaxL / 2 + 1]; }
 
 // q = x / d for 0 <= x < 2^22, through a float reciprocal and one correction.
 __device__ __forceinline__ int fdiv(int x, int d, float inv) {

@@ -50,13 +50,13 @@ int run_two(hipStream_t s, const PassArgs &k, const PassArgs &a, int pairs) {
 __global__ void twiddle_kernel(float2 *tw, int total) {
   const int g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= total) return;
-  int off = 0, L = 2;
-  for (; L <= kMaxL; L += 2) {
-    if (!fft_smooth(L)) continue;
-    if (g < off + L) break;
-    off += L;
+  int lo = 1, hi = kMaxL / 2 + 1;  // off[lo] <= g < off[hi]; the last such lo is a supported length
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (fft_tables().off[mid] <= g) lo = mid;
+    else hi = mid;
   }
-  const int t = g - off;
+  const int t = g - fft_tables().off[lo], L = 2 * lo;
   double sn, cs;
   sincospi(-2.0 * (double)t / (double)L, &sn, &cs);
   tw[g] = make_float2((float)cs, (float)sn);
