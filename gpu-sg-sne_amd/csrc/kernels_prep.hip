@@ -630,7 +630,7 @@ __global__ __launch_bounds__(256) void knn_tile_kernel(const float *__restrict__
     if (h == 0 && l < dim) {
       const double c = (acc[0][l] + acc[1][l]) / (double)nv;
       cen[l] = c;
-      tcen[(size_t)tile * dim + l] = c;
+      tcen[(size_t)l * gridDim.x + tile] = c;  // by dimension: the filter reads it for many tiles at once
     }
   }
   float2 *out = reinterpret_cast<float2 *>(Xr + (size_t)tile * kFiltR * dp);
@@ -843,7 +843,7 @@ __global__ __launch_bounds__(256) void knn_filter_kernel(const float *__restrict
 // list's new threshold.  An entry dropped or turned away has kp entries at or
 // below it, so the list always holds kp smallest values, and the ties dropped
 // at the kp-th have that very value: what the certificate needs.  The waves
-// meet once a round (a tile, or two with QB = 1).  An insertion thus costs a
+// meet once a round (a tile; with QB = 1 two, with 16 waves four).  An insertion thus costs a
 // few instructions of one wave and a cut about 300 per ~100 insertions; the
 // binary heaps this replaces took one lane log2(kp) dependent LDS round trips
 // per insertion while both waves of the work-group waited.  20,011 points of 50
@@ -966,7 +966,7 @@ __global__ __launch_bounds__(64 * NW) void knn_filter_list_kernel(const RefTiles
                                                               float *__restrict__ hd, int *__restrict__ hi) {
   constexpr int NQ = 16 * QB;
   constexpr int TW = NW / 4;                 // tiles taken at once, one per four waves
-  constexpr int TPR = QB == 1 ? 2 : 1;       // tiles between the meetings of the waves
+  constexpr int TPR = NW == 16 ? 4 : QB == 1 ? 2 : 1;  // tiles between the meetings of the waves
   constexpr int CAP = kTrig + 64 * TPR;      // no list overflows in a round
   static_assert(NST % 2 == 0 && kF2Q % NQ == 0 && TPR % TW == 0, "steps come in pairs, work-groups lie in one frame");
   __shared__ float lkey[NQ][CAP];
@@ -975,7 +975,8 @@ __global__ __launch_bounds__(64 * NW) void knn_filter_list_kernel(const RefTiles
   __shared__ float lthr[NQ];  // -infinity for a slot without a query: nothing enters
   __shared__ int lqid[NQ];
   __shared__ int need[3];     // round r uses need[r % 3]
-  __shared__ unsigned long long skipm[4];
+  __shared__ unsigned long long gom[4];
+  __shared__ int list[256];   // the group's tiles to visit
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, j = lane & 15;
   const int q0 = blockIdx.x * NQ, frame = q0 / kF2Q;
   const int ntiles = rf.ntiles;
@@ -1061,10 +1062,11 @@ __global__ __launch_bounds__(64 * NW) void knn_filter_list_kernel(const RefTiles
       if (rt_ >= 0.0) {  // not padding only
         skip = false;
         if (thr < INFINITY) {
-          const double *tc = rf.tcen + (size_t)t * rf.dim;
+          const double *tc = rf.tcen + t;
           double d2 = 0.0;
+#pragma unroll 8
           for (int l = 0; l < rf.dim; ++l) {
-            const double v = cbb[l] - tc[l];
+            const double v = cbb[l] - tc[(size_t)l * ntiles];
             d2 = fma(v, v, d2);
           }
           const double dcm = sqrt(d2);
@@ -1074,43 +1076,20 @@ __global__ __launch_bounds__(64 * NW) void knn_filter_list_kernel(const RefTiles
         }
       }
     }
-    const unsigned long long sb = __ballot(skip);
-    if (lane == 0 && w < 4) skipm[w] = sb;
+    // the tiles to visit, in order
+    const unsigned long long go = __ballot(!skip);
+    if (lane == 0 && w < 4) gom[w] = go;
     __syncthreads();
-    unsigned long long t0 = ~skipm[0], t1 = ~skipm[1], t2 = ~skipm[2], t3 = ~skipm[3];
-    auto next_tile = [&]() {  // takes the next tile of the group, -1: none left
-      int i = -1;
-      if (t0) {
-        i = __builtin_ctzll(t0);
-        t0 &= t0 - 1;
-      } else if (t1) {
-        i = 64 + __builtin_ctzll(t1);
-        t1 &= t1 - 1;
-      } else if (t2) {
-        i = 128 + __builtin_ctzll(t2);
-        t2 &= t2 - 1;
-      } else if (t3) {
-        i = 192 + __builtin_ctzll(t3);
-        t3 &= t3 - 1;
-      }
-      return i < 0 ? -1 : visit(g0 + i);
-    };
-    // the next TW tiles; this wave's is the (w / 4)-th of them
-    int first, tile;
-    auto next_tiles = [&]() {
-      first = tile = next_tile();
-#pragma unroll
-      for (int u = 1; u < TW; ++u) {
-        const int t = next_tile();
-        if (w / 4 == u) tile = t;
-      }
-      if (tile >= 0) load(tile);
-    };
-    next_tiles();
-    while (first >= 0) {
+    const int m0 = __popcll(gom[0]), m1 = m0 + __popcll(gom[1]), m2 = m1 + __popcll(gom[2]), m = m2 + __popcll(gom[3]);
+    if (!skip)
+      list[(w == 0 ? 0 : w == 1 ? m0 : w == 2 ? m1 : m2) + __popcll(go & ((1ull << lane) - 1ull))] = visit(g0 + tid);
+    __syncthreads();
+    int k = w / 4;  // the next one of these four waves
+    if (k < m) load(list[k]);
+    for (int r0 = 0; r0 < m; r0 += TPR) {
 #pragma unroll 1
-      for (int u = 0; u < TPR / TW && first >= 0; ++u) {
-        const bool mine = tile >= 0;
+      for (int u = 0; u < TPR / TW; ++u, k += TW) {
+        if (k >= m) break;
         float bv[NST];
 #pragma unroll
         for (int h = 0; h < NST / 2; ++h) {
@@ -1118,8 +1097,7 @@ __global__ __launch_bounds__(64 * NW) void knn_filter_list_kernel(const RefTiles
           bv[2 * h + 1] = nb[h].y;
         }
         const int rid = nid;
-        next_tiles();
-        if (!mine) continue;
+        if (k + TW < m) load(list[k + TW]);
         // into the block's frame, with the squared norms of the references
         float rn = 0.0f;
 #pragma unroll
@@ -1149,24 +1127,30 @@ __global__ __launch_bounds__(64 * NW) void knn_filter_list_kernel(const RefTiles
           }
         if (__ballot(any)) {
 #pragma unroll
-          for (int b = 0; b < QB; ++b)
+          for (int b = 0; b < QB; ++b) {
+            // the 16 references that enter the list of this lane's v-th query;
+            // lane v of the 16 takes their places, for the four queries at once
+            unsigned gm[4];
+            int c = 0;
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-              const bool in = dd[b][v] < th[b][v] && rid != qq[b][v];
-              const unsigned gm = (unsigned)(__ballot(in) >> (16 * g)) & 0xFFFFu;  // this query's 16 references
-              const int c = __popc(gm), ql = 16 * b + 4 * g + v;
-              int base = 0;
-              if (j == 0 && c) {
-                base = atomicAdd(&lcnt[ql], c);
-                if (base + c > kTrig) need[round % 3] = 1;
-              }
-              base = __shfl(base, 16 * g, 64);
-              if (in) {
-                const int p = base + __popc(gm & ((1u << j) - 1u));
-                lkey[ql][p] = dd[b][v];
-                lid[ql][p] = rid;
+              gm[v] = (unsigned)(__ballot(dd[b][v] < th[b][v] && rid != qq[b][v]) >> (16 * g)) & 0xFFFFu;
+              if (j == v) c = __popc(gm[v]);
+            }
+            int base = 0;
+            if (c) {
+              base = atomicAdd(&lcnt[16 * b + 4 * g + j], c);
+              if (base + c > kTrig) need[round % 3] = 1;
+            }
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+              const int p = __shfl(base, 16 * g + v, 64) + __popc(gm[v] & ((1u << j) - 1u));
+              if ((gm[v] >> j) & 1u) {
+                lkey[16 * b + 4 * g + v][p] = dd[b][v];
+                lid[16 * b + 4 * g + v][p] = rid;
               }
             }
+          }
         }
       }
       __syncthreads();
@@ -1213,17 +1197,27 @@ struct BlockCentred {
 // 84.2 at 200,000, 1272 / 1148 at 1.3M.
 constexpr int kFiltWide = 1 << 19;
 
-// Points up to which the 16 queries are given eight waves instead of four: up to
-// there at most 2.5 work-groups per CU are in flight and the walk over the tiles
-// is bound by its latency.  With 4 / 8 waves: 118 / 95 us on average for 16 jobs
-// of 500-8000 points; whole kNN calls 1.53 / 1.46 ms at 10,000 points, 2.81 /
-// 2.88 at 20,000, 20.9 / 22.8 at 100,000, 61.7 / 71.4 at 200,000.
-constexpr int kFiltDeep = 10240;
+// Points up to which the 16 queries are given 16 waves (a work-group per CU; up to
+// 64 dimensions, beyond which 16 waves run out of registers) and eight instead
+// of four: the walk over the tiles is then bound by its latency.  The filter alone
+// with 8 / 16 waves: 51 / 40 us at 1000 points, 109 / 91 at 4000, 168 / 181 at
+// 6000; with 4 / 8: 404 / 354 us at 12,000, 580 / 501 at 20,011, 1495 / 1518 at
+// 50,000, 10.0 / 11.6 ms at 200,003.
+constexpr int kFiltDeeper = 1 << 12;
+constexpr int kFiltDeep = 1 << 15;
 
 template <int NST>
 int launch_filter(hipStream_t s, const float *Xc, const float *n32, int n, int kp, const BlockCentred &bc,
                   float *hd, int *hi) {
   if (kp <= kF2MaxKp) {
+    if constexpr (NST <= 16) {
+      if (n <= kFiltDeeper) {
+        knn_filter_list_kernel<NST, 1, 16><<<div_up(n, 16), 1024, 0, s>>>(bc.rf, bc.Xq, bc.qn32, bc.qorder, bc.delta,
+                                                                          n, kp, hd, hi);
+        SGT_LAUNCH_CHECK();
+        return SGTSNE_OK;
+      }
+    }
     if (n <= kFiltDeep)
       knn_filter_list_kernel<NST, 1, 8><<<div_up(n, 16), 512, 0, s>>>(bc.rf, bc.Xq, bc.qn32, bc.qorder, bc.delta, n,
                                                                       kp, hd, hi);
@@ -1438,24 +1432,27 @@ int launch_rerank(hipStream_t s, const float *X, int n, int dim, int k, int kp, 
   return SGTSNE_OK;
 }
 
-// ---- perplexity bisection (HY/sgtsne.cpp:201-254), 16 lanes per point ------
+// ---- perplexity bisection (HY/sgtsne.cpp:201-254), LANES lanes per point ----
 // The reference's bisection on beta, step for step: the entropy H of the
 // point's row at beta against log(u), beta doubled / halved until bracketed,
-// then bisected, until |H - log u| < 1e-5 (at most 200 steps).  Each of the 16
-// lanes of a point's group takes the neighbours m = lane, lane + 16, ...; a
-// step's two sums (sum_m exp(-beta d_m) and sum_m d_m exp(-beta d_m)) are
-// added over the group by a fixed butterfly (deterministic), so a step costs
-// about k / 16 exponentials per lane instead of 2 k on one thread.  As in the
-// reference, the values normalised at the end are those of the last
-// evaluated beta (recomputed from it).
-constexpr int kPerpLanes = 16;
-
+// then bisected, until |H - log u| < 1e-5 (at most 200 steps).  Each lane of a
+// point's group takes the neighbours m = lane, lane + LANES, ..., PER of them
+// held in registers (PER = 0: any number, read again at each step); a step's two
+// sums (sum_m exp(-beta d_m) and sum_m d_m exp(-beta d_m)) are added over the
+// group by a fixed butterfly (deterministic).  Bound by the FP64 exponentials,
+// for few points by the latency of a step.  As in the reference, the values
+// normalised at the end are those of the last evaluated beta (recomputed from
+// it).
+template <int LANES, int PER>
 __global__ __launch_bounds__(256) void perplexity_kernel2(const double *__restrict__ D, int n, int k, double u,
                                                           float *__restrict__ val, double *__restrict__ beta_out) {
-  const int i = (blockIdx.x * blockDim.x + threadIdx.x) / kPerpLanes;
-  const int l = threadIdx.x & (kPerpLanes - 1);
+  const int i = (blockIdx.x * blockDim.x + threadIdx.x) / LANES;
+  const int l = threadIdx.x & (LANES - 1);
   if (i >= n) return;  // whole groups leave together
   const double *dist = D + (size_t)i * (k + 1) + 1;
+  double dm[PER > 0 ? PER : 1];
+#pragma unroll
+  for (int m = 0; m < PER; ++m) dm[m] = l + m * LANES < k ? dist[l + m * LANES] : 0.0;
   const double tol = 1e-5;
   const double logu = log(u);
   double beta = 1.0, min_beta = -DBL_MAX, max_beta = DBL_MAX;
@@ -1465,15 +1462,25 @@ __global__ __launch_bounds__(256) void perplexity_kernel2(const double *__restri
   while (!found && iter < 200) {  // uniform over the group
     beta_eval = beta;
     double sp = 0.0, sh = 0.0;
-    for (int m = l; m < k; m += kPerpLanes) {
-      const double e = exp(-beta * dist[m]);
-      sp += e;
-      sh += dist[m] * e;
+    if constexpr (PER > 0) {
+#pragma unroll
+      for (int m = 0; m < PER; ++m)
+        if (l + m * LANES < k) {
+          const double e = exp(-beta * dm[m]);
+          sp += e;
+          sh += dm[m] * e;
+        }
+    } else {
+      for (int m = l; m < k; m += LANES) {
+        const double e = exp(-beta * dist[m]);
+        sp += e;
+        sh += dist[m] * e;
+      }
     }
 #pragma unroll
-    for (int o = kPerpLanes / 2; o > 0; o >>= 1) {
-      sp += __shfl_xor(sp, o, kPerpLanes);
-      sh += __shfl_xor(sh, o, kPerpLanes);
+    for (int o = LANES / 2; o > 0; o >>= 1) {
+      sp += __shfl_xor(sp, o, LANES);
+      sh += __shfl_xor(sh, o, LANES);
     }
     sum_P = DBL_MIN + sp;
     const double H = (beta * sh) / sum_P + log(sum_P);
@@ -1489,7 +1496,7 @@ __global__ __launch_bounds__(256) void perplexity_kernel2(const double *__restri
     }
     ++iter;
   }
-  for (int m = l; m < k; m += kPerpLanes) val[(size_t)i * k + m] = (float)(exp(-beta_eval * dist[m]) / sum_P);
+  for (int m = l; m < k; m += LANES) val[(size_t)i * k + m] = (float)(exp(-beta_eval * dist[m]) / sum_P);
   if (beta_out && l == 0) beta_out[i] = beta;
 }
 
@@ -2083,7 +2090,12 @@ int launch_knn(hipStream_t s, const float *X, int n, int dim, int k, int32_t *I,
 
 int launch_perplexity(hipStream_t s, const double *D, int n, int k, double u, float *val,
                       double *beta_out) {
-  perplexity_kernel2<<<(int)div_up((int64_t)n * kPerpLanes, 256), 256, 0, s>>>(D, n, k, u, val, beta_out);
+  // 64 lanes per point would gain 4 us up to 1000 points (27 us) and lose above
+  // 1500; held in registers: 40 -> 29 us at 4000 points, 80 -> 70 at 16,000
+  const int blocks = div_up(n, 16);
+  if (k <= 96) perplexity_kernel2<16, 6><<<blocks, 256, 0, s>>>(D, n, k, u, val, beta_out);
+  else if (k <= 160) perplexity_kernel2<16, 10><<<blocks, 256, 0, s>>>(D, n, k, u, val, beta_out);
+  else perplexity_kernel2<16, 0><<<blocks, 256, 0, s>>>(D, n, k, u, val, beta_out);
   SGT_LAUNCH_CHECK();
   return SGTSNE_OK;
 }

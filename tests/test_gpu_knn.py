@@ -103,11 +103,11 @@ def test_knn_filtered_rerank_widths(sg, O, n, dim, k):
     assert fb >= 0 and np.array_equal(I, Io) and np.array_equal(D, Do)
 
 
-# both sides of the 10,240 points up to which the filter gives a query block
-# eight waves
-@pytest.mark.parametrize("n", [10240, 10241])
-def test_knn_filtered_wave_counts(sg, n):
-    X = _points(n, 12, n)
+# both sides of the points up to which the filter gives a query block 16 waves
+# (where the dimensions leave the registers) and eight
+@pytest.mark.parametrize("n,dim", [(4096, 64), (4096, 65), (4097, 64), (32768, 12), (32769, 12)])
+def test_knn_filtered_wave_counts(sg, n, dim):
+    X = _points(n, dim, n)
     I, D, fb = sg.knn(X, 30, sg.KNN_FILTERED)
     Ie, De, _ = sg.knn(X, 30, sg.KNN_EXACT_FP64)
     assert fb >= 0 and np.array_equal(I, Ie) and np.array_equal(D, De)
