@@ -1203,7 +1203,10 @@ int launch_s2g(hipStream_t s, const GridParams &g, int n, const float *Y, float 
     const int e = std::min(60, std::max(1, 61 - std::ilogb(bound)));
     unsigned long long *Vf = reinterpret_cast<unsigned long long *>(scratch);
     SGT_TRY(launch_fill(s, scratch, 2 * cells, 0.0f));
-    const int unit = g.d == 3 ? kFixUnit3 : 1024;
+    // runs long enough to share cells, short enough for two work-groups per CU:
+    // 60,000 points late in a 2-D run with runs of 1024 / 128 / 64: 29.9 / 9.4 /
+    // 14.0 us; 200,003 points in 3-D with 256 / 128: 68 / 72 us
+    const int unit = std::min(g.d == 3 ? kFixUnit3 : 1024, std::max(64, div_up(n, 64 * 512) * 64));
     const int lds_b = 64512;  // two work-groups per CU
     const int blocks = (int)std::min<int64_t>(div_up(n, unit), 2048);
     if (g.d == 2)
