@@ -502,7 +502,7 @@ int enqueue_terms(sgtsne_batch *b) {
   const int zd = b->p.zeta_mode == SGTSNE_ZETA_DIRECT;
   SGT_TRY(attractive(b));
   SGT_TRY(launch_bs2g(b->stream, b->d, b->jobs_d, b->items_d, b->nitems, b->Y, b->sord,
-                      std::min(b->nitems * (b->d == 3 ? 4 : 1), b->s2g_blocks), b->d == 3 ? 64512 : b->s2g_lds));
+                      b->s2g_blocks, b->d == 3 ? 64512 : b->s2g_lds));
   SGT_TRY(launch_bconv(b->stream, b->d, zd, b->args_d, b->prefix_d, b->max_jobs, b->conv_blocks));
   SGT_TRY(launch_bg2s(b->stream, b->d, zd, b->jobs_d, b->items_d, b->nitems, b->Y, b->Frep, b->zpart,
                       std::min(b->nitems, b->pt_blocks)));

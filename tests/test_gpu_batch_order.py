@@ -31,11 +31,11 @@ def _ring(sg, O, n):
             O.CSR(n, rp.astype(np.int64), cols.ravel().astype(np.int32), val.astype(np.float32).astype(np.float64)))
 
 
-def _check(B, O, jobs):
+def _check(B, O, jobs, h=1.2):
     for j, So in jobs:
         Y = B.get_Y(j).astype(np.float64)
         Fa, Fr, Z, _ = B.terms(j)
-        Fro, Zo, _ = O.repulsive_interp(Y.copy(), 1.2, O.ZETA_DIRECT)
+        Fro, Zo, _ = O.repulsive_interp(Y.copy(), h, O.ZETA_DIRECT)
         assert np.linalg.norm(Fa - O.attractive(So, Y)) <= TOL * np.linalg.norm(O.attractive(So, Y))
         assert np.linalg.norm(Fr - Fro) <= TOL * np.linalg.norm(Fro)
         assert abs(Z - Zo) <= TOL * Zo
@@ -63,3 +63,18 @@ def test_batch_order_follows_the_jobs(sg, O, sizes, extent):
                            max_iter=100, ng_cap=128), So))
         B.step(2)
         _check(B, O, jobs)
+
+
+# 1-D and 2-D jobs are spread in eighths of an item of 1024 points: items that
+# eight does not divide, one of a single point, and one shorter than eight parts
+@pytest.mark.parametrize("d,h", [(1, 0.5), (2, 0.7)])
+@pytest.mark.parametrize("sizes", [(300, 1025, 1031), (1023, 1024, 2049)])
+def test_batch_spread_in_eighths(sg, O, d, h, sizes):
+    rng = np.random.default_rng(sum(sizes) + d)
+    with sg.Batch(sg.tsneparams(d=d), 4, 8000, 200_000) as B:
+        jobs = []
+        for n in sizes:
+            S, So = _ring(sg, O, n)
+            jobs.append((B.add(S, symmetrize=False, y_in=rng.uniform(-15, 15, (n, d)).astype(np.float32), max_iter=100), So))
+        B.step(1)
+        _check(B, O, jobs, h)
