@@ -70,10 +70,10 @@ constexpr int kMarks = 16;                 // tick marks kept
 // the next job: it is handed out again on the stream it was given back on, or on
 // any once that stream has passed it, for requests of at least half its size.
 // hipFreeAsync held the host 96 us on average here and hipMallocAsync 41
-// (5 pairs per job: more than half of the time to admit a job of a few thousand
-// points: 16 jobs of 500-8000 points admitted, 8 iterations and removed 22.9 ->
-// 12.0 ms, 6 of 2000-20,000 in 3-D 14.7 -> 9.4).  At most kIdleBytes stay idle beyond the next call; the rest goes
-// back to the device's pool.
+// (5 pairs per job, more than half of the time to admit one of a few thousand
+// points): 16 jobs of 500-8000 points admitted, 8 iterations and removed 22.9 ->
+// 12.0 ms, 6 of 2000-20,000 in 3-D 14.7 -> 9.4.  At most kIdleBytes stay idle
+// beyond the next call; the rest goes back to the device's pool.
 constexpr size_t kIdleBytes = (size_t)4 << 30;
 class BlockCache final : public ScratchSource {
  public:

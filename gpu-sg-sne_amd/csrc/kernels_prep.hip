@@ -310,9 +310,9 @@ __global__ __launch_bounds__(kKnnThreads) void knn_select_kernel(const double *_
 // A rigorous bound on the approximation error then certifies, per query, that
 // no point outside the candidate list can be among the exact k nearest; the
 // candidates' distances are recomputed with exactly the arithmetic of
-// knn_kernel and the k smallest (distance, index) keys are kept, so a
-// certified row equals knn_kernel's row bit for bit.  Rows that cannot be
-// certified (ties or near-ties wider than the slack) go through knn_kernel.
+// the FP64 kernels and the k smallest (distance, index) keys are kept, so a
+// certified row equals their row bit for bit.  Rows that cannot be
+// certified (ties or near-ties wider than the slack) go through them.
 constexpr int kFiltQ = 64;        // queries per work-group, 16 per wave
 constexpr int kFiltR = 64;        // references per tile, 4 blocks of 16
 constexpr int kFiltMaxDp = 128;   // padded dimensions (A operands held in registers)
@@ -1262,7 +1262,7 @@ int launch_filter_for(hipStream_t s, int nst, const float *Xc, const float *n32,
 }
 
 // One wave per query: certify the candidate list, recompute the
-// candidates' distances as knn_kernel does (diff = x_q - x_c in FP64,
+// candidates' distances as knn_dist_kernel does (diff = x_q - x_c in FP64,
 // acc = fma(diff, diff, acc) over the dimensions in order) and write the row.
 //
 // The filter compares a = fl32(x_q - c) with b = fl32(fl32(x_c - mu) -
@@ -1950,7 +1950,7 @@ int knn_begin(hipStream_t s, ScratchSource &src, const float *X, int n, int dim,
             kRerank - kFiltSlack, kFiltMaxDp, kFiltQ);
   const int kp = std::min(k + kFiltSlack, n - 1);
   const int nst = filter_steps(dim, kp), dp = 4 * nst;
-  const bool blocked = kp <= kF2MaxKp;  // the LDS-heap filter centres each query block
+  const bool blocked = kp <= kF2MaxKp;  // the list filter centres each query block
   const int nb = div_up(n, kF2Q);
   // point order: cell (nearest of P pivots), then the Morton code of a 3-D
   // projection of the centred points; the query blocks and the reference
