@@ -94,7 +94,7 @@ def test_knn_filtered_wide_blocks(sg):
 
 
 # candidate lists of 65..256 entries re-ranked by one wave, two and four to a
-# lane, rows read one, two and four floats at a time
+# lane, rows staged 16 dimensions at a time with a remainder
 @pytest.mark.parametrize("n,dim,k", [(66, 18, 64), (400, 20, 112), (401, 17, 113), (500, 18, 200), (900, 20, 240), (250, 64, 240)])
 def test_knn_filtered_rerank_widths(sg, O, n, dim, k):
     X = _points(n, dim, 5 * n + dim)
