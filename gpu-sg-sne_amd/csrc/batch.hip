@@ -195,7 +195,8 @@ struct FrontEnd {
   KnnPending knn;
   SymPending sym;
   hipEvent_t ev = nullptr;  // after the queued part (kept across uses of the slot)
-  int *counts = nullptr;    // pinned: [0] uncertified kNN rows, [1] nonzeros of P + P^T
+  // pinned: [0] uncertified kNN rows, [1] nonzeros of P + P^T, [2] 1: a point without k neighbours
+  int *counts = nullptr;
 };
 
 }  // namespace
@@ -1028,10 +1029,16 @@ int fe_advance(sgtsne_batch *b, FrontEnd &f, int *job) {
   if (f.stage == 1) {  // kNN rows certified: the uncertified ones, P, and the merge of P and P^T
     st = knn_end(s, &f.knn, nullptr);
     if (!st) st = launch_perplexity(s, f.Dd, f.n, f.k, f.u, f.vv, nullptr);
-    if (!st) st = launch_knn_csr(s, f.n, f.k, f.Id, f.rp, f.cc);
+    f.counts[2] = 0;
+    if (!st) st = launch_knn_csr(s, f.n, f.k, f.Id, f.rp, f.cc, f.counts + 2);
     if (!st && b->p.lambda != 1.0) st = launch_lambda_rescale(s, f.n, f.rp, f.vv, b->p.lambda, b->p.drop_leaf);
     if (!st) st = sym_begin(s, b->blocks, f.n, (int64_t)f.n * f.k, f.rp, f.cc, f.vv, f.counts + 1, &f.sym);
   } else if (f.stage == 2) {  // merged count known: P_sym's CSR
+    if (f.counts[2]) {
+      set_error("a point has fewer than %d neighbours at a distance (a NaN coordinate)", f.k);
+      fe_release(b, f);
+      return SGTSNE_ERR_NUMERIC;
+    }
     st = sym_end(s, &f.sym, &f.srp, &f.scc, &f.svv, &f.m, &b->blocks);
     // given back in stream order, after the kernels just queued that read it
     b->blocks.give(s, f.ws);
@@ -1110,10 +1117,10 @@ int sgtsne_batch_create(sgtsne_batch **out, const sgtsne_params *params, int max
   b->blocks.release_stream = b->copy;
   for (hipEvent_t &e : b->marks) chk(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event");
   chk(hipHostMalloc((void **)&b->stage, kStageBytes, hipHostMallocDefault), "pinned staging");
-  chk(hipHostMalloc((void **)&b->fe_host, sizeof(int) * 2 * kFrontEnds, hipHostMallocDefault), "pinned counts");
+  chk(hipHostMalloc((void **)&b->fe_host, sizeof(int) * 3 * kFrontEnds, hipHostMallocDefault), "pinned counts");
   for (int i = 0; i < kFrontEnds; ++i) {
     chk(hipEventCreateWithFlags(&b->fe[i].ev, hipEventDisableTiming), "event");
-    b->fe[i].counts = b->fe_host ? b->fe_host + 2 * i : nullptr;
+    b->fe[i].counts = b->fe_host ? b->fe_host + 3 * i : nullptr;
   }
   const size_t P = (size_t)max_points;
   if (!st) st = balloc((void **)&b->rowptr, sizeof(int32_t) * (P + 1));

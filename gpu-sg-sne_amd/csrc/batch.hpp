@@ -98,7 +98,9 @@ int launch_bmorton(hipStream_t s, int d, const BatchJob *jobs, int job, int off,
 int launch_offset_copy_i32(hipStream_t s, const int32_t *in, int32_t *out, int64_t count, int32_t delta);
 // Z of one job from the item partials of the last gather (one wavefront).
 int launch_bzeta(hipStream_t s, const BatchJob *jobs, int job, const double *zpart, double *out);
-int launch_knn_csr(hipStream_t s, int n, int k, const int32_t *I, int32_t *rowptr, int32_t *col);
+// bad: pinned, set to 1 when a row holds an id that is no point's (such an id is
+// replaced by the row's own).
+int launch_knn_csr(hipStream_t s, int n, int k, const int32_t *I, int32_t *rowptr, int32_t *col, int *bad);
 int launch_gather_i32(hipStream_t s, int n, const int32_t *order, const int32_t *in, int32_t *out);
 int launch_iota(hipStream_t s, int n, int32_t *out);
 int launch_invert(hipStream_t s, int n, const int32_t *order, int32_t *inv);

@@ -543,13 +543,20 @@ __global__ void bmorton_kernel(int d, const BatchJob *__restrict__ jobs, int job
 
 // kNN ids [n][k+1] (self first) -> CSR columns without the self column
 // (CU/perplexity_search.cu:100-112); rowptr[i] = i k.
+// kNN rows -> CSR without the self column.  A row left short (a point with a NaN
+// coordinate has no distances) ends in ids that are no point's; P + P^T writes at
+// its columns, so such an id becomes the row's own and *bad (pinned) tells the
+// host to refuse the job.
 __global__ void knn_csr_kernel(int n, int k, const int32_t *__restrict__ I, int32_t *__restrict__ rowptr,
-                               int32_t *__restrict__ col) {
+                               int32_t *__restrict__ col, int *bad) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t <= n) rowptr[t] = (int32_t)(t * k);
   if (t < (int64_t)n * k) {
     const int64_t i = t / k, e = t - i * k;
-    col[t] = I[i * (k + 1) + e + 1];
+    const int32_t c = I[i * (k + 1) + e + 1];
+    const bool ok = c >= 0 && c < n;
+    col[t] = ok ? c : (int32_t)i;
+    if (!ok) *bad = 1;
   }
 }
 
@@ -736,8 +743,8 @@ int launch_bzeta(hipStream_t s, const BatchJob *jobs, int job, const double *zpa
   return SGTSNE_OK;
 }
 
-int launch_knn_csr(hipStream_t s, int n, int k, const int32_t *I, int32_t *rowptr, int32_t *col) {
-  knn_csr_kernel<<<div_up((int64_t)n * k + 1, 256), 256, 0, s>>>(n, k, I, rowptr, col);
+int launch_knn_csr(hipStream_t s, int n, int k, const int32_t *I, int32_t *rowptr, int32_t *col, int *bad) {
+  knn_csr_kernel<<<div_up((int64_t)n * k + 1, 256), 256, 0, s>>>(n, k, I, rowptr, col, bad);
   SGT_LAUNCH_CHECK();
   return SGTSNE_OK;
 }

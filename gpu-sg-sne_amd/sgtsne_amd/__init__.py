@@ -27,6 +27,7 @@ LAYOUT_SOA = 0
 LAYOUT_AOS = 1
 ZETA_DIRECT = 0
 ZETA_ALGEBRAIC = 1
+ERR_NUMERIC = -4
 ERR_FULL = -8
 JOB_RUNNING = 0
 JOB_DONE = 1
@@ -458,6 +459,10 @@ class Full(SgtsneError):
     """No room in the batch right now (slots, arena or grid budget)."""
 
 
+class Numeric(SgtsneError):
+    """A job's points have no k neighbours each (NaN coordinates)."""
+
+
 class Batch:
     """Many embedding jobs advanced together on the device (sgtsne_batch_*).
 
@@ -502,6 +507,8 @@ class Batch:
     def _admit(self, status, job, n):
         if status == ERR_FULL:
             raise Full(lib().sgtsne_last_error().decode(errors="replace"))
+        if status == ERR_NUMERIC:
+            raise Numeric(f"sgtsne error {status}: {lib().sgtsne_last_error().decode(errors='replace')}")
         _check(status)
         self.n[job.value] = n
         return job.value

@@ -38,7 +38,7 @@ import time
 
 import numpy as np
 
-from . import Batch, Full, tsneparams
+from . import Batch, Full, Numeric, tsneparams
 from .synth import random_init
 
 _POINT_BYTES = {2: 6 * 2 * 4 + 4, 3: 6 * 4 * 4 + 4}
@@ -165,6 +165,10 @@ class Server:
                 else:
                     keep.append(r)
                 continue
+            except Numeric:
+                r.done, r.Y = now_fn(), None  # its points are not numbers: rejected
+                self.finished.append(r)
+                continue
             self._register(r, fp, job, now_fn)
             admitted += 1
         self.queue = collections.deque(sorted(keep, key=lambda q: (q.arrival, q.rid)))
@@ -214,6 +218,13 @@ class Server:
                     self.finished.append(r)
                 else:
                     self.queue.append(r)  # retried once jobs retire
+                moved = True
+                continue
+            except Numeric:
+                self.fronts[d] = None
+                self.used[d] -= fp
+                r.done, r.Y = now_fn(), None  # its points are not numbers: rejected
+                self.finished.append(r)
                 moved = True
                 continue
             if job is None:

@@ -26,7 +26,7 @@ extern "C" {
 #define SGTSNE_ERR_ARG (-1)       /* invalid argument / size              */
 #define SGTSNE_ERR_HIP (-2)       /* HIP runtime error                     */
 #define SGTSNE_ERR_NOMEM (-3)     /* device or host allocation failed      */
-#define SGTSNE_ERR_NUMERIC (-4)   /* non-finite embedding (out of grid)    */
+#define SGTSNE_ERR_NUMERIC (-4)   /* non-finite embedding or points        */
 #define SGTSNE_ERR_STATE (-5)     /* call order (e.g. step before upload)  */
 #define SGTSNE_ERR_NODEV (-6)     /* no gfx950 device visible              */
 #define SGTSNE_ERR_FULL (-8)      /* no room: job slots, arena or grid budget
@@ -360,7 +360,8 @@ int sgtsne_batch_add(sgtsne_batch *batch, int n, int64_t nnz, const int32_t *row
 /* Admits a job from its points X [n][dim]: exact kNN (k), perplexity u and
  * P + P^T on the device (perplexityEqualization, CU/perplexity_search.cu:114-141,
  * then as sgtsne_batch_add).  Runs on a stream of its own, so it overlaps
- * iterations already queued by sgtsne_batch_step. */
+ * iterations already queued by sgtsne_batch_step.  SGTSNE_ERR_NUMERIC, and no
+ * job, when a point has fewer than k neighbours (a NaN coordinate). */
 int sgtsne_batch_add_points(sgtsne_batch *batch, const float *X, int n, int dim, int k, double u, const float *y_in,
                             int max_iter, int ng_cap, int *job);
 

@@ -264,3 +264,25 @@ def test_server_refuses_unvalidated_queue_depths():
     for kw in ({"tick": 20}, {"depth": 6}, {"depth": {2: 3, 3: 4}}):
         with pytest.raises(ValueError, match="supported"):
             serving.Server(**kw)
+
+
+@pytest.mark.parametrize("front", ["async", "sync"])
+def test_server_rejects_points_that_are_not_numbers(front):
+    # the engine refuses such a job after its front end: that request ends
+    # without an embedding, and the others are served
+    log = []
+    srv, eng = _server(log, front=front, max_iter=30)
+    e2 = eng[2]
+    orig = e2.add_points
+
+    def add_points(X, *a, **kw):
+        if X.shape[0] == 601:
+            e2.front = None
+            raise serving.Numeric("a point has no neighbours")
+        return orig(X, *a, **kw)
+
+    e2.add_points = add_points
+    with srv:
+        got = srv.run([(0.0, n, 2, i) for i, n in enumerate((500, 601, 700))], lambda n, s: np.zeros((n, 4), np.float32))
+    assert [r.Y is None for r in got] == [False, True, False]
+    assert srv.used == {2: 0, 3: 0} and not any(srv.fronts.values())
