@@ -1917,7 +1917,7 @@ int knn_exact_rows(hipStream_t s, ScratchSource &src, const float *X, int n, int
   void *block = nullptr;
   SGT_TRY(src.take(s, sizeof(double) * (size_t)slab * n, &block));
   double *dist = static_cast<double *>(block);
-  for (int s0 = 0; s0 < nq; s0 += slab) {
+  auto rows = [&](int s0) -> int {
     const int m = std::min(slab, nq - s0);
     if (few)
       knn_dist_kernel<2, 4><<<dim3(div_up(n, 64), div_up(m, 32)), kKnnThreads, 0, s>>>(X, n, dim, qlist, s0, m, 0, dist);
@@ -1930,9 +1930,12 @@ int knn_exact_rows(hipStream_t s, ScratchSource &src, const float *X, int n, int
     else
       knn_select_kernel<2 * kKnnMaxK><<<m, kKnnThreads, 0, s>>>(dist, n, k, qlist, s0, I, D);
     SGT_LAUNCH_CHECK();
-  }
+    return SGTSNE_OK;
+  };
+  int st = SGTSNE_OK;
+  for (int s0 = 0; s0 < nq && !st; s0 += slab) st = rows(s0);
   src.give(s, block);
-  return SGTSNE_OK;
+  return st;
 }
 
 }  // namespace
@@ -2210,6 +2213,17 @@ int sym_begin(hipStream_t s, ScratchSource &src, int n, int64_t nnz, const int32
   return SGTSNE_OK;
 }
 
+// Gives back the arrays of sym_end.
+static void sym_free(hipStream_t s, int32_t *rp, int32_t *cc, float *vv, ScratchSource *out_src) {
+  if (out_src) {
+    out_src->give(s, rp);  // one block, which starts at rowptr
+    return;
+  }
+  if (rp) (void)hipFree(rp);
+  if (cc) (void)hipFree(cc);
+  if (vv) (void)hipFree(vv);
+}
+
 void sym_release(hipStream_t s, SymPending *sp) {
   if (sp->ws) sp->src->give(s, sp->ws);
   *sp = SymPending{};
@@ -2231,14 +2245,21 @@ int sym_end(hipStream_t s, SymPending *sp, int32_t **rowptr_out, int32_t **col_o
       vv = c.take<float>(runs);
       if (pass == 0) SGT_TRY(out_src->take(s, c.off, &block));
     }
-  } else {
-    SGT_HIP(hipMalloc((void **)&rp, sizeof(int32_t) * ((size_t)n + 1)));
-    SGT_HIP(hipMalloc((void **)&cc, sizeof(int32_t) * (size_t)(runs > 0 ? runs : 1)));
-    SGT_HIP(hipMalloc((void **)&vv, sizeof(float) * (size_t)(runs > 0 ? runs : 1)));
+  } else if (hipMalloc((void **)&rp, sizeof(int32_t) * ((size_t)n + 1)) != hipSuccess ||
+             hipMalloc((void **)&cc, sizeof(int32_t) * (size_t)(runs > 0 ? runs : 1)) != hipSuccess ||
+             hipMalloc((void **)&vv, sizeof(float) * (size_t)(runs > 0 ? runs : 1)) != hipSuccess) {
+    (void)hipGetLastError();
+    sym_free(s, rp, cc, vv, nullptr);
+    set_error("no memory for P + P^T (%d nonzeros)", runs);
+    return SGTSNE_ERR_NOMEM;
   }
   sym_finish_kernel<<<std::min(div_up(n, 4), 16384), 256, 0, s>>>(n, sp->off, sp->rp, sp->mcol, sp->mval, sp->total,
                                                                   rp, cc, vv);
-  SGT_LAUNCH_CHECK();
+  if (const hipError_t e = hipGetLastError(); e != hipSuccess) {
+    sym_free(s, rp, cc, vv, out_src);
+    set_error("P + P^T failed: %s", hipGetErrorString(e));
+    return SGTSNE_ERR_HIP;
+  }
   sym_release(s, sp);
   *rowptr_out = rp;
   *col_out = cc;
@@ -2252,10 +2273,27 @@ int gpu_symmetrize(hipStream_t s, int n, int64_t nnz, const int32_t *rowptr_d, c
                    int64_t *nnz_out, ScratchSource *out_src) {
   int runs = 0;
   SymPending sp;
-  SGT_TRY(sym_begin(s, out_src ? *out_src : stream_scratch(), n, nnz, rowptr_d, col_d, val_d, &runs, &sp));
-  SGT_HIP(hipStreamSynchronize(s));
-  SGT_TRY(sym_end(s, &sp, rowptr_out, col_out, val_out, nnz_out, out_src));
-  SGT_HIP(hipStreamSynchronize(s));
+  int32_t *rp = nullptr, *cc = nullptr;
+  float *vv = nullptr;
+  auto wait = [&]() -> int {
+    SGT_HIP(hipStreamSynchronize(s));
+    return SGTSNE_OK;
+  };
+  int st = sym_begin(s, out_src ? *out_src : stream_scratch(), n, nnz, rowptr_d, col_d, val_d, &runs, &sp);
+  if (!st) st = wait();
+  if (!st) st = sym_end(s, &sp, &rp, &cc, &vv, nnz_out, out_src);
+  if (st) {
+    sym_release(s, &sp);
+    return st;
+  }
+  st = wait();
+  if (st) {
+    sym_free(s, rp, cc, vv, out_src);
+    return st;
+  }
+  *rowptr_out = rp;
+  *col_out = cc;
+  *val_out = vv;
   return SGTSNE_OK;
 }
 
