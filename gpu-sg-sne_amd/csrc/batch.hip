@@ -91,7 +91,7 @@ class BlockCache final : public ScratchSource {
       hipError_t e = hipMallocAsync(&nb.p, nb.cap, s);
       if (e != hipSuccess) {  // give the idle blocks back and try once more
         (void)hipGetLastError();
-        trim_locked(0);
+        reclaim_locked();
         nb.cap = bytes > 0 ? bytes : 1;
         e = hipMallocAsync(&nb.p, nb.cap, s);
       }
@@ -100,6 +100,7 @@ class BlockCache final : public ScratchSource {
         if (e != hipSuccess) (void)hipFreeAsync(nb.p, s);
       }
       if (e != hipSuccess) {
+        (void)hipGetLastError();  // reported here, not by the next launch
         set_error("hipMallocAsync(%zu) failed: %s", bytes, hipGetErrorString(e));
         return SGTSNE_ERR_NOMEM;
       }
@@ -166,6 +167,19 @@ class BlockCache final : public ScratchSource {
       } else {
         ++it;
       }
+  }
+  // Every idle block back to the device, for any stream: the pool hands what one
+  // stream freed to another only by an order the caller made
+  // (retain_pool_memory), so the frees are waited for and the pool is trimmed.
+  void reclaim_locked() {
+    for (Block &b : blocks_)
+      if (b.idle) (void)hipEventSynchronize(b.ev);
+    trim_locked(0);
+    (void)hipStreamSynchronize(release_stream);
+    int dev = 0;
+    hipMemPool_t pool = nullptr;
+    if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetDefaultMemPool(&pool, dev) == hipSuccess)
+      (void)hipMemPoolTrimTo(pool, 0);
   }
   std::mutex mu_;
   std::list<Block> blocks_;
