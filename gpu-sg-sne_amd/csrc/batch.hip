@@ -302,6 +302,7 @@ namespace {
 int balloc(void **p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes > 0 ? bytes : 1);
   if (e != hipSuccess) {
+    (void)hipGetLastError();
     set_error("hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
     return SGTSNE_ERR_NOMEM;
   }
@@ -1264,6 +1265,7 @@ int sgtsne_batch_add_points_async(sgtsne_batch *b, const float *X, int n, int di
   int st = SGTSNE_OK;
   auto chk = [&](hipError_t e, const char *what) {
     if (st == SGTSNE_OK && e != hipSuccess) {
+      (void)hipGetLastError();
       set_error("front end: %s failed: %s", what, hipGetErrorString(e));
       st = e == hipErrorOutOfMemory ? SGTSNE_ERR_NOMEM : SGTSNE_ERR_HIP;
     }

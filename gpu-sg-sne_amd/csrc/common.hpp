@@ -17,6 +17,7 @@ void set_error(const char *fmt, ...);
   do {                                                                                 \
     hipError_t e_ = (call);                                                            \
     if (e_ != hipSuccess) {                                                            \
+      (void)hipGetLastError(); /* reported here, not by a later launch check */        \
       ::sgt::set_error("%s:%d: %s failed: %s", __FILE__, __LINE__, #call,              \
                        hipGetErrorString(e_));                                         \
       return SGTSNE_ERR_HIP;                                                           \

@@ -154,6 +154,7 @@ constexpr int kSpreadOrderIters = 16;
 int alloc_dev(void **p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes > 0 ? bytes : 1);
   if (e != hipSuccess) {
+    (void)hipGetLastError();
     set_error("hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
     return SGTSNE_ERR_NOMEM;
   }
@@ -1497,6 +1498,7 @@ int sgtsne_knn(const float *X, int n, int dim, int k, int method, int32_t *I, do
     Dd = c.take<double>(no);
     Id = c.take<int32_t>(no);
     if (pass == 0 && hipMallocAsync(&ws, c.off, s) != hipSuccess) {
+      (void)hipGetLastError();
       set_error("hipMallocAsync(%zu) failed", c.off);
       ws = nullptr;
       st = SGTSNE_ERR_NOMEM;
@@ -1591,6 +1593,7 @@ int sgtsne_perplexity_equalize(const int32_t *I, const double *D, int n, int k, 
     Dd = c.take<double>((size_t)n * (k + 1));
     vd = c.take<float>((size_t)n * k);
     if (pass == 0 && hipMallocAsync(&ws, c.off, s) != hipSuccess) {
+      (void)hipGetLastError();
       set_error("hipMallocAsync(%zu) failed", c.off);
       ws = nullptr;
       st = SGTSNE_ERR_NOMEM;
