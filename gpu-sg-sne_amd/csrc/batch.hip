@@ -1047,7 +1047,7 @@ int fe_advance(sgtsne_batch *b, FrontEnd &f, int *job) {
     f.counts[2] = 0;
     if (!st) st = launch_knn_csr(s, f.n, f.k, f.Id, f.rp, f.cc, f.counts + 2);
     if (!st && b->p.lambda != 1.0) st = launch_lambda_rescale(s, f.n, f.rp, f.vv, b->p.lambda, b->p.drop_leaf);
-    if (!st) st = sym_begin(s, b->blocks, f.n, (int64_t)f.n * f.k, f.rp, f.cc, f.vv, f.counts + 1, &f.sym);
+    if (!st) st = sym_begin(s, b->blocks, f.n, (int64_t)f.n * f.k, f.rp, f.cc, f.vv, 2 * f.k, f.counts + 1, &f.sym);
   } else if (f.stage == 2) {  // merged count known: P_sym's CSR
     if (f.counts[2]) {
       set_error("a point has fewer than %d neighbours at a distance (a NaN coordinate)", f.k);

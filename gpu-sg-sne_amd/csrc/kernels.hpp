@@ -194,19 +194,27 @@ int gpu_symmetrize(hipStream_t s, int n, int64_t nnz, const int32_t *rowptr_d,
 // P and P^T and a copy of the merged nonzero count into *runs_host; sym_end,
 // once the stream has passed that copy, queues the normalisation and the CSR
 // build, without waiting for them, into one block of out_src that starts at
-// rowptr (nullptr: three hipMalloc'ed arrays).
+// rowptr (nullptr: three hipMalloc'ed arrays).  max_row: the longest row of P when no
+// row holds a column twice, else 0 (any P).
+struct SymLong {  // its long rows, as the merge lists them
+  int *cnt = nullptr;            // [0] rows sorted by a work-group, [1] hubs
+  int32_t *mid = nullptr, *hub = nullptr;
+  double *part = nullptr;        // of each part of each hub: its sum,
+  int32_t *end = nullptr;        // and where it ends in the merged row
+};
 struct SymPending {
   bool open = false;
   int n = 0;
   ScratchSource *src = nullptr;
   void *ws = nullptr;  // the one block the pointers below lie in
-  const int32_t *off = nullptr, *ucnt = nullptr, *rp = nullptr;
+  const int32_t *off = nullptr, *rp = nullptr;
   const int32_t *mcol = nullptr;
   const double *mval = nullptr, *total = nullptr;
+  SymLong rows;
   const int *runs_host = nullptr;
 };
 int sym_begin(hipStream_t s, ScratchSource &src, int n, int64_t nnz, const int32_t *rowptr_d, const int32_t *col_d,
-              const float *val_d, int *runs_host, SymPending *sp);
+              const float *val_d, int max_row, int *runs_host, SymPending *sp);
 int sym_end(hipStream_t s, SymPending *sp, int32_t **rowptr_out, int32_t **col_out, float **val_out,
             int64_t *nnz_out, ScratchSource *out_src);
 void sym_release(hipStream_t s, SymPending *sp);

@@ -1536,7 +1536,6 @@ __global__ void rowids_kernel(int n, const int32_t *__restrict__ rowptr, int32_t
   for (int t = rowptr[i]; t < rowptr[i + 1]; ++t) row[t] = i;
 }
 
-// ---- P + P^T ----------------------------------------------------------------
 // ---- P + P^T, row by row -----------------------------------------------------------
 // Row i of the merge holds row i of P and, after it, the entries of column i:
 // every entry of P takes its place in its column's row from a counter (which
@@ -1548,21 +1547,67 @@ __global__ void rowids_kernel(int n, const int32_t *__restrict__ rowptr, int32_t
 // moved 32 bytes in each of 6 passes and took about 25 launches for a small
 // job.  16 jobs of 500-8000 points admitted to a batch: 48.9 -> 32.9 ms; a whole
 // call on 1203 points 1.89 -> 1.52 ms.
-constexpr int kSymRow = 1024;      // longest row one wave sorts
-constexpr int kSymRowLds = 8192;   // longest row sorted in LDS; longer ones in place
+//
+// Rows by their length: up to kSymRow entries one wave each; up to kSymRowLds a
+// work-group each, from a list of them, so that they spread over the device
+// wherever they lie; longer ones (hubs) in ranges of kSymCols columns, a work-group
+// each, whose sums are kept by column.
+constexpr int kSymRow = 1024;
+constexpr int kSymRowLds = 8192;
+constexpr int kSymCols = 8192;       // columns of a hub's range (FP64 sums: 64 KB of LDS)
+constexpr int kSymBelow = 1 << 19;   // columns of one bitmap of those below a range (64 KB)
 
-__global__ void sym_len_kernel(int n, const int32_t *__restrict__ rowptr, int32_t *__restrict__ cnt) {
+__global__ void sym_len_kernel(int n, const int32_t *__restrict__ rowptr, int32_t *__restrict__ cnt, int *lcnt) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i <= n) cnt[i] = i < n ? rowptr[i + 1] - rowptr[i] : 0;
+  if (i < 2) lcnt[i] = 0;
 }
 
-// pos[t] = place of entry t in the merged row of its column (one wave per row).
-__global__ __launch_bounds__(256) void sym_place_kernel(int n, const int32_t *__restrict__ rowptr,
-                                                        const int32_t *__restrict__ col, int32_t *__restrict__ cnt,
-                                                        int32_t *__restrict__ pos) {
-  const int lane = threadIdx.x & 63, nw = (gridDim.x * blockDim.x) >> 6;
-  for (int i = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; i < n; i += nw)
-    for (int t = rowptr[i] + lane; t < rowptr[i + 1]; t += 64) pos[t] = atomicAdd(&cnt[col[t]], 1);
+// pos[t] = place of entry t in the merged row of its column.  A work-group takes
+// kPlaceRun entries and counts equal columns in LDS first (a hash table; an entry
+// whose slot another column holds goes to the counter itself), so that a hub's
+// counter is increased once per work-group: the 900,000 entries of one column
+// took 10.2 ms one by one.
+constexpr int kPlaceRun = 2048, kPlaceSlots = 4096;
+
+__global__ __launch_bounds__(256) void sym_place_kernel(int64_t nnz, const int32_t *__restrict__ col,
+                                                        int32_t *__restrict__ cnt, int32_t *__restrict__ pos) {
+  constexpr int U = kPlaceRun / 256;
+  __shared__ int tag[kPlaceSlots], num[kPlaceSlots];
+  const int tid = threadIdx.x;
+  for (int64_t t0 = (int64_t)blockIdx.x * kPlaceRun; t0 < nnz; t0 += (int64_t)gridDim.x * kPlaceRun) {
+    for (int i = tid; i < kPlaceSlots; i += 256) {
+      tag[i] = -1;
+      num[i] = 0;
+    }
+    __syncthreads();
+    int at[U], slot[U];  // place within the slot's column (slot >= 0) or in the row
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t t = t0 + u * 256 + tid;
+      if (t < nnz) {
+        const int c = col[t];
+        slot[u] = (int)(((unsigned)c * 2654435761u) >> 20);
+        const int held = atomicCAS(&tag[slot[u]], -1, c);
+        if (held == -1 || held == c) {
+          at[u] = atomicAdd(&num[slot[u]], 1);
+        } else {
+          at[u] = atomicAdd(&cnt[c], 1);
+          slot[u] = -1;
+        }
+      }
+    }
+    __syncthreads();
+    for (int i = tid; i < kPlaceSlots; i += 256)
+      if (num[i]) num[i] = atomicAdd(&cnt[tag[i]], num[i]);  // now the first place
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t t = t0 + u * 256 + tid;
+      if (t < nnz) pos[t] = slot[u] >= 0 ? num[slot[u]] + at[u] : at[u];
+    }
+    __syncthreads();
+  }
 }
 
 __device__ __forceinline__ unsigned long long sym_entry(int col, float v) {
@@ -1587,11 +1632,10 @@ __global__ __launch_bounds__(256) void sym_scatter_kernel(int n, const int32_t *
   }
 }
 
-// Ascending sort of len words (LDS or memory) by the whole work-group: a
-// bitonic network whose merges start with a mirrored step, so every exchange
-// is ascending and the places past len need no padding.
-template <class P>
-__device__ void sort_words(P x, int len) {
+// Ascending sort of len words (LDS) by the whole work-group: a bitonic network
+// whose merges start with a mirrored step, so every exchange is ascending and
+// the places past len need no padding.
+__device__ void sort_words(unsigned long long *x, int len) {
   auto exchange = [&](int i, int j) {
     if (j < len) {
       const unsigned long long a = x[i], b = x[j];
@@ -1621,12 +1665,11 @@ __device__ void sort_words(P x, int len) {
   __syncthreads();
 }
 
-// Merges one sorted row (x, in LDS or memory): its columns and summed values to
-// mcol / mval at the row's place (mval may be x itself: a round's words are read
-// before its results, none of them further on, are written).  Every thread of
-// the work-group calls it; wsum holds 2 + 2 * waves words.
-template <class P>
-__device__ void merge_row(P x, int len, int32_t *mcol, double *mval, int32_t *ucnt, double *rowsum, double *wsum) {
+// Merges one sorted row (x, in LDS): its columns and summed values to mcol / mval
+// at the row's place.  Every thread of the work-group calls it; wsum holds 2 + 2 *
+// waves words.
+__device__ void merge_row(const unsigned long long *x, int len, int32_t *mcol, double *mval, int32_t *ucnt, double *rowsum,
+                          double *wsum) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
   int *wcnt = reinterpret_cast<int *>(wsum + nw);
   double sum = 0.0;
@@ -1643,7 +1686,7 @@ __device__ void merge_row(P x, int len, int32_t *mcol, double *mval, int32_t *uc
       for (int j = i; j < len && (unsigned)(x[j] >> 32) == c; ++j) v += (double)__uint_as_float((unsigned)x[j]);
     const unsigned long long m = __ballot(head);
     if (lane == 0) wcnt[w] = __popcll(m);
-    __syncthreads();  // the round's words are read
+    __syncthreads();
     int at = done + __popcll(m & ((1ull << lane) - 1ull));
     for (int k = 0; k < nw; ++k) {
       if (k < w) at += wcnt[k];
@@ -1668,70 +1711,199 @@ __device__ void merge_row(P x, int len, int32_t *mcol, double *mval, int32_t *uc
   __syncthreads();
 }
 
-// Rows of up to kSymRow entries, one wave each.
+// Rows of up to kSymRow entries, one wave each; the others are listed.
 __global__ __launch_bounds__(64) void sym_merge_kernel(int n, const int32_t *__restrict__ off,
-                                                       unsigned long long *__restrict__ ent,
-                                                       int32_t *__restrict__ mcol, int32_t *__restrict__ ucnt,
-                                                       double *__restrict__ rowsum) {
+                                                       const unsigned long long *__restrict__ ent,
+                                                       int32_t *__restrict__ mcol, double *__restrict__ mval,
+                                                       int32_t *__restrict__ ucnt, double *__restrict__ rowsum,
+                                                       SymLong L) {
   __shared__ unsigned long long x[kSymRow];
   __shared__ double wsum[4];
   for (int r = blockIdx.x; r < n; r += gridDim.x) {
     const int o = off[r], len = off[r + 1] - o;
-    if (len > kSymRow) continue;
+    if (len > kSymRow) {
+      if (threadIdx.x == 0) {
+        if (len <= kSymRowLds) L.mid[atomicAdd(L.cnt, 1)] = r;
+        else L.hub[atomicAdd(L.cnt + 1, 1)] = r;
+      }
+      continue;
+    }
     for (int i = threadIdx.x; i < len; i += 64) x[i] = ent[o + i];
     sort_words(x, len);
-    merge_row(x, len, mcol + o, reinterpret_cast<double *>(ent) + o, ucnt + r, rowsum + r, wsum);
+    merge_row(x, len, mcol + o, mval + o, ucnt + r, rowsum + r, wsum);
   }
 }
 
-// The longer rows, a 1024-thread work-group each: in LDS, or in place when they
-// do not fit.
-__global__ __launch_bounds__(1024) void sym_merge_long_kernel(int n, const int32_t *__restrict__ off,
-                                                              unsigned long long *__restrict__ ent,
-                                                              int32_t *__restrict__ mcol, int32_t *__restrict__ ucnt,
-                                                              double *__restrict__ rowsum) {
+// The listed rows of up to kSymRowLds entries, a work-group each, bound by the
+// barriers of the sort: a job of 20,000 points with rows of 1200 added to a batch 7.1
+// ms (28 when a work-group walked the long rows of its 1024 neighbours).
+__global__ __launch_bounds__(1024) void sym_merge_mid_kernel(const int32_t *__restrict__ off,
+                                                             const unsigned long long *__restrict__ ent,
+                                                             int32_t *__restrict__ mcol, double *__restrict__ mval,
+                                                             int32_t *__restrict__ ucnt, double *__restrict__ rowsum,
+                                                             SymLong L) {
   extern __shared__ unsigned long long xl[];
   __shared__ double wsum[32];
-  __shared__ int list[1024];
-  __shared__ int cnt;
-  for (int b = blockIdx.x * 1024; b < n; b += gridDim.x * 1024) {
-    if (threadIdx.x == 0) cnt = 0;
-    __syncthreads();
-    const int r = b + threadIdx.x;
-    if (r < n && off[r + 1] - off[r] > kSymRow) list[atomicAdd(&cnt, 1)] = r;
-    __syncthreads();
-    const int m = cnt;
-    for (int q = 0; q < m; ++q) {
-      const int row = list[q], o = off[row], len = off[row + 1] - o;
-      double *mval = reinterpret_cast<double *>(ent) + o;
-      if (len <= kSymRowLds) {
-        for (int i = threadIdx.x; i < len; i += 1024) xl[i] = ent[o + i];
-        sort_words(xl, len);
-        merge_row(xl, len, mcol + o, mval, ucnt + row, rowsum + row, wsum);
-      } else {
-        volatile unsigned long long *x = ent + o;
-        sort_words(x, len);
-        merge_row(x, len, mcol + o, mval, ucnt + row, rowsum + row, wsum);
+  const int rows = L.cnt[0];
+  for (int q = blockIdx.x; q < rows; q += gridDim.x) {
+    const int row = L.mid[q], o = off[row], len = off[row + 1] - o;
+    for (int i = threadIdx.x; i < len; i += 1024) xl[i] = ent[o + i];
+    sort_words(xl, len);
+    merge_row(xl, len, mcol + o, mval + o, ucnt + row, rowsum + row, wsum);
+  }
+}
+
+// Sum over the work-group's 16 waves of a count each thread holds, and the sum
+// over the threads before this one.
+__device__ int block_scan(int v, int *wcnt, int *before) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int inc = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int u = __shfl_up(inc, o, 64);
+    if (lane >= o) inc += u;
+  }
+  if (lane == 63) wcnt[w] = inc;
+  __syncthreads();
+  int all = 0, base = 0;
+  for (int k = 0; k < 16; ++k) {
+    if (k < w) base += wcnt[k];
+    all += wcnt[k];
+  }
+  __syncthreads();
+  *before = base + inc - v;
+  return all;
+}
+
+// Ranges of kSymCols columns that one work-group of a hub takes in turn, and the
+// work-groups of a hub (at most kHubParts).
+constexpr int kHubParts = 256;
+__host__ __device__ inline int hub_run(int n) { return (n / kSymCols + kHubParts) / kHubParts; }
+__host__ __device__ inline int hub_parts(int n) { return (n - 1) / (kSymCols * hub_run(n)) + 1; }
+
+// The hubs: a work-group takes a range of kSymCols columns of one row, reads the
+// whole row, adds the values of its columns in LDS by column and counts the
+// distinct columns below the range (a bitmap), which is where its part of the
+// merged row starts.  No sort, and no limit on the length of a row.  A column has
+// two entries (P_ij and P_ji), whose sum does not depend on their order, unless P
+// holds an entry more than once: then the FP64 sums are exact, in any order, for
+// values within 2^29 of each other.  Bound by the reads of the row, once per range.
+// A job of 1M points with a hub of 900,000 added to a batch: 141 ms with the row
+// sorted in memory by one work-group, 15 so (its hub 0.75); 200,000 points with
+// eight hubs of 100,000: 79 and 3.5.
+__global__ __launch_bounds__(1024) void sym_merge_hub_kernel(int n, const int32_t *__restrict__ off,
+                                                             const unsigned long long *__restrict__ ent,
+                                                             int32_t *__restrict__ mcol, double *__restrict__ mval,
+                                                             int32_t *__restrict__ ucnt, SymLong L) {
+  extern __shared__ double acc[];  // [kSymCols], then the two bitmaps
+  unsigned *mine = reinterpret_cast<unsigned *>(acc + kSymCols), *below = mine + kSymCols / 32;
+  __shared__ int wcnt[16];
+  __shared__ double wsum[16];
+  constexpr int PER = kSymCols / 1024;  // columns of a thread
+  static_assert(PER == 8, "a thread's columns are one byte of the bitmap");
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int parts = hub_parts(n), run = hub_run(n);
+  const int64_t items = (int64_t)L.cnt[1] * parts;
+  for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {
+    const int row = L.hub[it / parts], j = (int)(it % parts);
+    const int o = off[row], len = off[row + 1] - o;
+    int start = 0;  // distinct columns below the range
+    double part = 0.0;
+    for (int r = 0; r < run; ++r) {
+      const unsigned c0 = ((unsigned)j * run + r) * kSymCols;
+      if (c0 >= (unsigned)n) break;
+      for (int i = tid; i < kSymCols; i += 1024) acc[i] = 0.0;
+      if (tid < kSymCols / 32) mine[tid] = 0;
+      // the first range counts those below it, one bitmap's columns at a time;
+      // each range's own columns are added in the first pass
+      const unsigned c1 = r == 0 ? c0 : 0;
+      for (unsigned lo = 0;; lo += kSymBelow) {
+        const unsigned hi = min(c1, lo + kSymBelow);
+        for (unsigned i = tid; i < (hi - lo + 31) / 32; i += 1024) below[i] = 0;
+        __syncthreads();
+#pragma unroll 4
+        for (int i = tid; i < len; i += 1024) {
+          const unsigned long long x = ent[o + i];
+          const unsigned c = (unsigned)(x >> 32);
+          if (c - c0 < (unsigned)kSymCols) {
+            if (lo == 0) {
+              atomicAdd(&acc[c - c0], (double)__uint_as_float((unsigned)x));
+              atomicOr(&mine[(c - c0) / 32], 1u << (c % 32));
+            }
+          } else if (c - lo < hi - lo) {
+            atomicOr(&below[(c - lo) / 32], 1u << (c % 32));
+          }
+        }
+        __syncthreads();
+        int cnt = 0, before;
+        for (unsigned i = tid; i < (hi - lo + 31) / 32; i += 1024) cnt += __popc(below[i]);
+        start += block_scan(cnt, wcnt, &before);
+        if (hi == c1) break;
       }
+      const unsigned bits = (mine[tid / 4] >> (8 * (tid % 4))) & 0xFFu;
+      int at;
+      const int total = block_scan(__popc(bits), wcnt, &at);
+      at += o + start;
+#pragma unroll
+      for (int e = 0; e < PER; ++e)
+        if ((bits >> e) & 1u) {
+          const double v = acc[tid * PER + e];
+          mcol[at] = (int32_t)(c0 + tid * PER + e);
+          mval[at++] = v;
+          part += v;
+        }
+      start += total;
+      __syncthreads();  // the sums are read
+    }
+    part = wave_sum(part);
+    if (lane == 0) wsum[w] = part;
+    __syncthreads();
+    if (tid == 0) {
+      for (int k = 1; k < 16; ++k) part += wsum[k];
+      L.part[it] = part;
+      L.end[it] = start;
+      if (j == parts - 1) ucnt[row] = start;
     }
     __syncthreads();
   }
 }
 
-// The merged rows, normalised by the sum of all of them, side by side.
+// A hub's sum from its parts, one wave each.
+__global__ __launch_bounds__(64) void sym_hub_sum_kernel(int n, double *__restrict__ rowsum, SymLong L) {
+  const int parts = hub_parts(n);
+  for (int h = blockIdx.x; h < L.cnt[1]; h += gridDim.x) {
+    double s = 0.0;
+    for (int j = threadIdx.x; j < parts; j += 64) s += L.part[(int64_t)h * parts + j];
+    s = wave_sum(s);
+    if (threadIdx.x == 0) rowsum[L.hub[h]] = s;
+  }
+}
+
+// The merged rows, normalised by the sum of all of them, side by side: a wave for
+// each row, a work-group for each part of a hub.
 __global__ __launch_bounds__(256) void sym_finish_kernel(int n, const int32_t *__restrict__ off,
                                                          const int32_t *__restrict__ rp,
                                                          const int32_t *__restrict__ mcol,
                                                          const double *__restrict__ mval,
                                                          const double *__restrict__ total,
                                                          int32_t *__restrict__ rowptr, int32_t *__restrict__ col,
-                                                         float *__restrict__ val) {
+                                                         float *__restrict__ val, SymLong L) {
   const int lane = threadIdx.x & 63, nw = (gridDim.x * blockDim.x) >> 6;
   const double tot = *total;
+  const int parts = hub_parts(n);
+  const int64_t items = (int64_t)L.cnt[1] * parts;
+  for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {
+    const int row = L.hub[it / parts], o = off[row], p = rp[row];
+    for (int e = (it % parts ? L.end[it - 1] : 0) + threadIdx.x; e < L.end[it]; e += blockDim.x) {
+      col[p + e] = mcol[o + e];
+      val[p + e] = (float)(mval[o + e] / tot);
+    }
+  }
   for (int i = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; i < n; i += nw) {
     const int o = off[i], p = rp[i], m = rp[i + 1] - p;
     if (lane == 0) rowptr[i] = p;
     if (i == n - 1 && lane == 0) rowptr[n] = rp[n];
+    if (off[i + 1] - o > kSymRowLds) continue;
     for (int e = lane; e < m; e += 64) {
       col[p + e] = mcol[o + e];
       val[p + e] = (float)(mval[o + e] / tot);
@@ -2159,7 +2331,7 @@ int device_exclusive_scan(hipStream_t s, const int32_t *in, int32_t *out, int n)
 }
 
 int sym_begin(hipStream_t s, ScratchSource &src, int n, int64_t nnz, const int32_t *rowptr_d, const int32_t *col_d,
-              const float *val_d, int *runs_host, SymPending *sp) {
+              const float *val_d, int max_row, int *runs_host, SymPending *sp) {
   *sp = SymPending{};
   sp->src = &src;
   const int64_t m2 = 2 * nnz;
@@ -2167,9 +2339,15 @@ int sym_begin(hipStream_t s, ScratchSource &src, int n, int64_t nnz, const int32
   size_t tb = 0, tr = 0;
   SGT_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, (int32_t *)nullptr, (int32_t *)nullptr, n + 1, s));
   SGT_HIP(hipcub::DeviceReduce::Sum(nullptr, tr, (double *)nullptr, (double *)nullptr, n, s));
+  // the longest merged row: its own entries and, from each other row, one per
+  // column (any number if P may hold an entry more than once)
+  const int64_t longest = std::min<int64_t>(m2, max_row > 0 ? (int64_t)n + max_row : m2);
+  const bool mids = longest > kSymRow, hubs = longest > kSymRowLds;
+  const int64_t nhub = hubs ? m2 / kSymRowLds : 0, parts = hub_parts(n);
   int32_t *cnt, *off, *pos, *mcol, *ucnt, *rp;
   unsigned long long *ent;
-  double *rowsum, *total;
+  double *mval, *rowsum, *total;
+  SymLong &L = sp->rows;
   void *tmp;
   for (int pass = 0; pass < 2; ++pass) {  // sizes, then the pieces of the block
     Carve c{static_cast<char *>(sp->ws)};
@@ -2178,6 +2356,12 @@ int sym_begin(hipStream_t s, ScratchSource &src, int n, int64_t nnz, const int32
     pos = c.take<int32_t>(nnz);
     ent = c.take<unsigned long long>(m2);
     mcol = c.take<int32_t>(m2);
+    mval = c.take<double>(m2);
+    L.cnt = c.take<int>(2);
+    L.mid = c.take<int32_t>(mids ? m2 / kSymRow : 0);
+    L.hub = c.take<int32_t>(nhub);
+    L.part = c.take<double>(nhub * parts);
+    L.end = c.take<int32_t>(nhub * parts);
     ucnt = c.take<int32_t>((size_t)n + 1);
     rp = c.take<int32_t>((size_t)n + 1);
     rowsum = c.take<double>(n);
@@ -2188,25 +2372,33 @@ int sym_begin(hipStream_t s, ScratchSource &src, int n, int64_t nnz, const int32
   sp->open = true;
   sp->n = n;
   sp->off = off;
-  sp->ucnt = ucnt;
   sp->rp = rp;
   sp->mcol = mcol;
-  sp->mval = reinterpret_cast<const double *>(ent);
+  sp->mval = mval;
   sp->total = total;
   sp->runs_host = runs_host;
   const int wblocks = std::min(div_up(n, 4), 16384);  // four waves of a row each
-  sym_len_kernel<<<div_up((int64_t)n + 1, 256), 256, 0, s>>>(n, rowptr_d, cnt);
+  sym_len_kernel<<<div_up((int64_t)n + 1, 256), 256, 0, s>>>(n, rowptr_d, cnt, L.cnt);
   SGT_LAUNCH_CHECK();
-  sym_place_kernel<<<wblocks, 256, 0, s>>>(n, rowptr_d, col_d, cnt, pos);
+  if (nnz > 0) sym_place_kernel<<<(int)std::min<int64_t>((nnz + kPlaceRun - 1) / kPlaceRun, 65536), 256, 0, s>>>(nnz, col_d, cnt, pos);
   SGT_LAUNCH_CHECK();
   SGT_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, tb, cnt, off, n + 1, s));
   sym_scatter_kernel<<<wblocks, 256, 0, s>>>(n, rowptr_d, col_d, val_d, off, pos, ent);
   SGT_LAUNCH_CHECK();
-  sym_merge_kernel<<<std::min(n, 65536), 64, 0, s>>>(n, off, ent, mcol, ucnt, rowsum);
+  sym_merge_kernel<<<std::min(n, 65536), 64, 0, s>>>(n, off, ent, mcol, mval, ucnt, rowsum, L);
   SGT_LAUNCH_CHECK();
-  sym_merge_long_kernel<<<std::min(div_up(n, 1024), 512), 1024, sizeof(unsigned long long) * kSymRowLds, s>>>(
-      n, off, ent, mcol, ucnt, rowsum);
-  SGT_LAUNCH_CHECK();
+  if (mids) {  // two work-groups per CU
+    sym_merge_mid_kernel<<<(int)std::min<int64_t>(m2 / kSymRow, 512), 1024, sizeof(unsigned long long) * kSymRowLds, s>>>(
+        off, ent, mcol, mval, ucnt, rowsum, L);
+    SGT_LAUNCH_CHECK();
+  }
+  if (hubs) {  // one per CU
+    sym_merge_hub_kernel<<<(int)std::min<int64_t>(nhub * parts, 256), 1024,
+                           sizeof(double) * kSymCols + (kSymCols + kSymBelow) / 8, s>>>(n, off, ent, mcol, mval, ucnt, L);
+    SGT_LAUNCH_CHECK();
+    sym_hub_sum_kernel<<<(int)std::min<int64_t>(nhub, 256), 64, 0, s>>>(n, rowsum, L);
+    SGT_LAUNCH_CHECK();
+  }
   SGT_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, tb, ucnt, rp, n + 1, s));  // ucnt[n] is not read into rp
   SGT_HIP(hipcub::DeviceReduce::Sum(tmp, tr, rowsum, total, n, s));
   SGT_HIP(hipMemcpyAsync(runs_host, rp + n, sizeof(int), hipMemcpyDeviceToHost, s));
@@ -2254,7 +2446,7 @@ int sym_end(hipStream_t s, SymPending *sp, int32_t **rowptr_out, int32_t **col_o
     return SGTSNE_ERR_NOMEM;
   }
   sym_finish_kernel<<<std::min(div_up(n, 4), 16384), 256, 0, s>>>(n, sp->off, sp->rp, sp->mcol, sp->mval, sp->total,
-                                                                  rp, cc, vv);
+                                                                  rp, cc, vv, sp->rows);
   if (const hipError_t e = hipGetLastError(); e != hipSuccess) {
     sym_free(s, rp, cc, vv, out_src);
     set_error("P + P^T failed: %s", hipGetErrorString(e));
@@ -2279,7 +2471,7 @@ int gpu_symmetrize(hipStream_t s, int n, int64_t nnz, const int32_t *rowptr_d, c
     SGT_HIP(hipStreamSynchronize(s));
     return SGTSNE_OK;
   };
-  int st = sym_begin(s, out_src ? *out_src : stream_scratch(), n, nnz, rowptr_d, col_d, val_d, &runs, &sp);
+  int st = sym_begin(s, out_src ? *out_src : stream_scratch(), n, nnz, rowptr_d, col_d, val_d, 0, &runs, &sp);
   if (!st) st = wait();
   if (!st) st = sym_end(s, &sp, &rp, &cc, &vv, nnz_out, out_src);
   if (st) {
