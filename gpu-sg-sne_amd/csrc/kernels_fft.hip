@@ -93,103 +93,128 @@ int run_kind(hipStream_t s, int kind, const PassArgs &a, int pairs, bool node_ma
 // transforms are a chain of three (3-D: five) launches whose work is a few
 // thousand operations per line; the sum over all pairs of nodes is 262,144
 // multiply-adds on a 16 x 16 grid and 84 million on a 16-cube, one launch
-// spread over the device.  FP32 sums in a fixed order: at most 32 terms per
-// thread, then the threads' partials in a fixed order.  16 x 16 grid: 25.5 us of
-// transforms -> 4.4; 16-cube: 58 -> 16.  Potentials come node-major; channel 3 (2-D) or 4 (3-D) is the charge with K1.
+// spread over the device.  Kernel values and sums in FP64 (which issues at the
+// rate of FP32 here), in a fixed order: early in a run the charges y_i nearly
+// cancel, and FP32 sums of them could be further off than the transforms.  Frep
+// against 64 bits, mean over 700-30,000 points, transforms / FP32 sums / these:
+// 2-D 2.89e-7 / 2.80e-7 / 2.63e-7, 3-D 3.52e-7 / 3.39e-7 / 3.32e-7.
+// 16 x 16 grid: 25.5 us of transforms -> 4.4; 16-cube: 58 -> 12.
+// Potentials come node-major; channel 3 (2-D) or 4 (3-D) is the charge with K1.
 constexpr int kDirect2 = 32, kDirect3 = 16;  // largest sides
+constexpr int kDirectX = 16;                 // outputs of a 2-D work-group
 
-// One work-group per grid row y; thread (x, j) adds the nodes of row y' = j.
+// A work-group per grid row y and kDirectX of its nodes x; thread (x, j) adds the
+// nodes of row y' = j.
 template <int XP>
-__global__ __launch_bounds__(XP *XP) void conv_direct2_kernel(int ng, float hsq, const float *__restrict__ V,
-                                                             float4 *__restrict__ Phi) {
+__global__ __launch_bounds__(kDirectX *XP) void conv_direct2_kernel(int ng, double hsq, const float *__restrict__ V,
+                                                                   float4 *__restrict__ Phi) {
   __shared__ float4 vs[XP][XP];    // charges of (x', y')
-  __shared__ float2 ks[XP][XP];    // K2, K1 at (|x - x'|, |y - y'|)
-  __shared__ float4 red[XP][XP];
-  const int x = threadIdx.x % XP, j = threadIdx.x / XP, y = blockIdx.x, G = ng * ng;
-  const bool in = x < ng && j < ng;
-  const int e = j * ng + x;
-  vs[j][x] = in ? make_float4(V[e], V[G + e], V[2 * G + e], 0.0f) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  const float dy = (float)(y - j), r2 = (float)x * (float)x + dy * dy;
-  const float k1 = 1.0f / (1.0f + hsq * r2);
-  ks[j][x] = make_float2(k1 * k1, k1);
+  __shared__ double2 ks[XP][XP];   // K2, K1 at (|x - x'|, |y - y'|)
+  __shared__ double4 red[XP][kDirectX];
+  const int xl = threadIdx.x % kDirectX, j = threadIdx.x / kDirectX, x = blockIdx.y * kDirectX + xl, y = blockIdx.x;
+  const int G = ng * ng;
+#pragma unroll
+  for (int t = threadIdx.x; t < XP * XP; t += kDirectX * XP) {
+    const int xx = t % XP, jj = t / XP, e = jj * ng + xx;
+    vs[jj][xx] = xx < ng && jj < ng ? make_float4(V[e], V[G + e], V[2 * G + e], 0.0f) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const double k1 = 1.0 / (1.0 + hsq * (double)(xx * xx + (y - jj) * (y - jj)));
+    ks[jj][xx] = make_double2(k1 * k1, k1);
+  }
   __syncthreads();
-  float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  double4 acc = make_double4(0.0, 0.0, 0.0, 0.0);
 #pragma unroll 8
   for (int xp = 0; xp < ng; ++xp) {
     const float4 v = vs[j][xp];
-    const float2 k = ks[j][abs(x - xp)];
-    acc.x = fmaf(k.x, v.x, acc.x);
-    acc.y = fmaf(k.x, v.y, acc.y);
-    acc.z = fmaf(k.x, v.z, acc.z);
-    acc.w = fmaf(k.y, v.x, acc.w);
+    const double2 k = ks[j][abs(x - xp)];
+    acc.x = fma(k.x, (double)v.x, acc.x);
+    acc.y = fma(k.x, (double)v.y, acc.y);
+    acc.z = fma(k.x, (double)v.z, acc.z);
+    acc.w = fma(k.y, (double)v.x, acc.w);
   }
-  red[j][x] = acc;
+  red[j][xl] = acc;
   __syncthreads();
   // rows y' added in order, eight of them per thread, then the eighths
   if (j < XP / 8) {
-    float4 s = red[8 * j][x];
+    double4 s = red[8 * j][xl];
 #pragma unroll
     for (int k = 1; k < 8; ++k) {
-      const float4 t = red[8 * j + k][x];
+      const double4 t = red[8 * j + k][xl];
       s.x += t.x;
       s.y += t.y;
       s.z += t.z;
       s.w += t.w;
     }
-    red[8 * j][x] = s;
+    red[8 * j][xl] = s;
   }
   __syncthreads();
   if (j == 0 && x < ng) {
-    float4 s = red[0][x];
+    double4 s = red[0][xl];
 #pragma unroll
     for (int k = 1; k < XP / 8; ++k) {
-      const float4 t = red[8 * k][x];
+      const double4 t = red[8 * k][xl];
       s.x += t.x;
       s.y += t.y;
       s.z += t.z;
       s.w += t.w;
     }
-    Phi[y * ng + x] = s;
+    Phi[y * ng + x] = make_float4((float)s.x, (float)s.y, (float)s.z, (float)s.w);
   }
 }
 
 // One work-group per row (y, z); thread (y', z') adds the 16 nodes of its row
 // to the 16 outputs in registers, and the threads' sums are added across each
-// wave and then over the four waves.
-__global__ __launch_bounds__(256) void conv_direct3_kernel(int ng, float hsq, const float *__restrict__ V,
+// wave and then over the four waves.  Bound by the loads: a lane's row is lines of
+// its own, so it is read in 16-byte vectors (11.8 us with them, 18.7 without).
+__global__ __launch_bounds__(256) void conv_direct3_kernel(int ng, double hsq, const float *__restrict__ V,
                                                            float *__restrict__ Phi) {
   constexpr int S = kDirect3, C = 5;
-  __shared__ float red[4][S * C];
+  __shared__ double red[4][S * C];
   const int yp = threadIdx.x % S, zp = threadIdx.x / S;
   const int y = blockIdx.x % ng, z = blockIdx.x / ng, G = ng * ng * ng;
   const bool in = yp < ng && zp < ng;
-  float k1[S];
-  const float dy = (float)(y - yp), dz = (float)(z - zp), r0 = dy * dy + dz * dz;
+  double k1[S];
+  const int r0 = (y - yp) * (y - yp) + (z - zp) * (z - zp);
 #pragma unroll
-  for (int d = 0; d < S; ++d) k1[d] = 1.0f / (1.0f + hsq * ((float)(d * d) + r0));
-  float acc[S][C];
+  for (int d = 0; d < S; ++d) k1[d] = 1.0 / (1.0 + hsq * (double)(d * d + r0));
+  double acc[S][C];
 #pragma unroll
   for (int x = 0; x < S; ++x)
 #pragma unroll
-    for (int c = 0; c < C; ++c) acc[x][c] = 0.0f;
+    for (int c = 0; c < C; ++c) acc[x][c] = 0.0;
   const float *row = V + (zp * ng + yp) * ng;
+  float vr[4][S];
+  if (ng % 4 == 0) {  // rows of whole 16-byte vectors (every lane reads lines of its own)
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int h = 0; h < S / 4; ++h) {
+        const float4 q = in && 4 * h < ng ? reinterpret_cast<const float4 *>(row + c * G)[h] : make_float4(0.f, 0.f, 0.f, 0.f);
+        vr[c][4 * h] = q.x;
+        vr[c][4 * h + 1] = q.y;
+        vr[c][4 * h + 2] = q.z;
+        vr[c][4 * h + 3] = q.w;
+      }
+  } else {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int xp = 0; xp < S; ++xp) vr[c][xp] = in && xp < ng ? row[c * G + xp] : 0.0f;
+  }
 #pragma unroll
   for (int xp = 0; xp < S; ++xp) {
-    float v[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) v[c] = in && xp < ng ? row[c * G + xp] : 0.0f;
+    const float v[4] = {vr[0][xp], vr[1][xp], vr[2][xp], vr[3][xp]};
 #pragma unroll
     for (int x = 0; x < S; ++x) {
-      const float k = k1[x > xp ? x - xp : xp - x], kk = k * k;
+      const double k = k1[x > xp ? x - xp : xp - x], kk = k * k;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) acc[x][c] = fmaf(kk, v[c], acc[x][c]);
-      acc[x][4] = fmaf(k, v[0], acc[x][4]);
+      for (int c = 0; c < 4; ++c) acc[x][c] = fma(kk, (double)v[c], acc[x][c]);
+      acc[x][4] = fma(k, (double)v[0], acc[x][4]);
     }
   }
   // across the wave: halves exchanged until 16 groups of four lanes hold 5 sums
   // each (85 shuffles; 80 butterflies would be 480), then added over the four
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  float a[S * C];
+  double a[S * C];
 #pragma unroll
   for (int x = 0; x < S; ++x)
 #pragma unroll
@@ -199,7 +224,7 @@ __global__ __launch_bounds__(256) void conv_direct3_kernel(int ng, float hsq, co
     const bool up = lane & o;
 #pragma unroll
     for (int i = 0; i < half; ++i) {
-      const float keep = up ? a[i + half] : a[i], send = up ? a[i] : a[i + half];
+      const double keep = up ? a[i + half] : a[i], send = up ? a[i] : a[i + half];
       a[i] = keep + __shfl_xor(send, o, 64);
     }
   }
@@ -213,9 +238,9 @@ __global__ __launch_bounds__(256) void conv_direct3_kernel(int ng, float hsq, co
   for (int o = threadIdx.x; o < S * C; o += blockDim.x) {
     const int x = o / C, c = o - x * C;
     if (x >= ng) continue;
-    const float s = (red[0][o] + red[1][o]) + (red[2][o] + red[3][o]);
+    const double s = (red[0][o] + red[1][o]) + (red[2][o] + red[3][o]);
     const int e = (z * ng + y) * ng + x;
-    Phi[c < 4 ? 4 * e + c : 4 * G + e] = s;
+    Phi[c < 4 ? 4 * e + c : 4 * G + e] = (float)s;
   }
 }
 
@@ -246,11 +271,11 @@ int launch_conv(hipStream_t s, const GridParams &g, int zdirect, const float *V,
                 const ConvBuffers &b, bool node_major) {
   SGT_CHECK(g.L <= kMaxL && g.L >= 2 * g.ng - 1 && fft_smooth(g.L), SGTSNE_ERR_ARG,
             "FFT length %d invalid for ng %d", g.L, g.ng);
-  const float hsq = (float)(g.hgrid * g.hgrid);
+  const double hsq = (double)g.hgrid * (double)g.hgrid;
   if (node_major && g.d == 2 && g.ng <= kDirect2) {
     float4 *Phi4 = reinterpret_cast<float4 *>(Phi);
-    if (g.ng <= 16) conv_direct2_kernel<16><<<g.ng, 256, 0, s>>>(g.ng, hsq, V, Phi4);
-    else conv_direct2_kernel<32><<<g.ng, 1024, 0, s>>>(g.ng, hsq, V, Phi4);
+    if (g.ng <= 16) conv_direct2_kernel<16><<<g.ng, 16 * kDirectX, 0, s>>>(g.ng, hsq, V, Phi4);
+    else conv_direct2_kernel<32><<<dim3(g.ng, 2), 32 * kDirectX, 0, s>>>(g.ng, hsq, V, Phi4);
     SGT_LAUNCH_CHECK();
     return SGTSNE_OK;
   }
