@@ -256,7 +256,8 @@ struct sgtsne_batch {
   int32_t *rowptr = nullptr, *col = nullptr;
   float *val = nullptr;
   float *Y = nullptr, *uY = nullptr, *gains = nullptr, *Fattr = nullptr, *Frep = nullptr;
-  int32_t *sord = nullptr;  // 3-D: the order in which the rows are spread
+  int32_t *sord = nullptr;  // 3-D: the order in which the rows are spread,
+  int *sord_cnt = nullptr;  // and the counts it is made from
   int ord_left = 0;         // iterations until it is renewed (0: before the next spread)
   int32_t *perm = nullptr;  // device row -> the caller's index within its job
   int64_t used_points = 0, used_nnz = 0;
@@ -585,7 +586,7 @@ int capture(sgtsne_batch *b) {
 // serves the next `iters` iterations.
 int renew_order(sgtsne_batch *b, int iters) {
   if (b->d != 3 || b->ord_left > 0) return SGTSNE_OK;
-  SGT_TRY(launch_bspread_order(b->stream, b->jobs_d, b->max_jobs, b->Y, b->sord));
+  SGT_TRY(launch_bspread_order(b->stream, b->jobs_d, b->max_jobs, b->items_d, b->nitems, b->Y, b->sord_cnt, b->sord));
   b->ord_left = iters;
   return SGTSNE_OK;
 }
@@ -947,6 +948,7 @@ void destroy_all(sgtsne_batch *b) {
   bfree(b->Fattr);
   bfree(b->Frep);
   bfree(b->sord);
+  bfree(b->sord_cnt);
   bfree(b->perm);
   bfree(b->jobs_d);
   bfree(b->patch_d);
@@ -1144,7 +1146,10 @@ int sgtsne_batch_create(sgtsne_batch **out, const sgtsne_params *params, int max
   float **pts[5] = {&b->Y, &b->uY, &b->gains, &b->Fattr, &b->Frep};
   for (float **q : pts)
     if (!st) st = balloc((void **)q, sizeof(float) * P * b->ds);
+  const size_t ob = sizeof(int) * 2 * kBatchOrderBins * (size_t)max_jobs;
   if (!st && b->d == 3) st = balloc((void **)&b->sord, sizeof(int32_t) * P);
+  if (!st && b->d == 3) st = balloc((void **)&b->sord_cnt, ob);
+  if (!st && b->d == 3) chk(hipMemsetAsync(b->sord_cnt, 0, ob, b->stream), "memset");
   if (!st) st = balloc((void **)&b->perm, sizeof(int32_t) * P);
   if (!st) st = balloc((void **)&b->jobs_d, sizeof(BatchJob) * max_jobs);
   if (!st) st = balloc((void **)&b->patch_d, sizeof(JobPatch) * max_jobs);

@@ -79,7 +79,10 @@ int batch_npasses(int d);
 int launch_bs2g(hipStream_t s, int d, const BatchJob *jobs, const BatchItem *items, int nitems, const float *Y,
                 const int32_t *ord, int blocks, int lds_bytes);
 constexpr int kBatchOrderIters = 16;
-int launch_bspread_order(hipStream_t s, const BatchJob *jobs, int njobs, const float *Y, int32_t *ord);
+constexpr int kBatchOrderBins = 4096;
+// cnt: 2 kBatchOrderBins ints per job slot, zero before the first call.
+int launch_bspread_order(hipStream_t s, const BatchJob *jobs, int njobs, const BatchItem *items, int nitems,
+                         const float *Y, int *cnt, int32_t *ord);
 int launch_bconv(hipStream_t s, int d, int zdirect, const void *args, const int *prefix, int njobs, int blocks);
 int launch_bg2s(hipStream_t s, int d, int zdirect, const BatchJob *jobs, const BatchItem *items, int nitems,
                 const float *Y, float *Frep, double *zpart, int blocks);
