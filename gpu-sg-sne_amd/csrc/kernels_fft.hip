@@ -93,11 +93,12 @@ int run_kind(hipStream_t s, int kind, const PassArgs &a, int pairs, bool node_ma
 // transforms are a chain of three (3-D: five) launches whose work is a few
 // thousand operations per line; the sum over all pairs of nodes is 262,144
 // multiply-adds on a 16 x 16 grid and 84 million on a 16-cube, one launch
-// spread over the device.  Kernel values and sums in FP64 (which issues at the
-// rate of FP32 here), in a fixed order: early in a run the charges y_i nearly
-// cancel, and FP32 sums of them could be further off than the transforms.  Frep
-// against 64 bits, mean over 700-30,000 points, transforms / FP32 sums / these:
-// 2-D 2.89e-7 / 2.80e-7 / 2.63e-7, 3-D 3.52e-7 / 3.39e-7 / 3.32e-7.
+// spread over the device.  Sums in FP64 (which issues at the rate of FP32 here)
+// of the transforms' FP32 kernel values and charges, in a fixed order: early in a
+// run the charges y_i nearly cancel, and FP32 sums of them could be further off
+// than the transforms.  Frep against 64 bits, mean over 700-30,000 points,
+// transforms / FP32 sums / these: 2-D 2.89e-7 / 2.80e-7 / 2.64e-7, 3-D 3.52e-7 /
+// 3.39e-7 / 3.33e-7 (with FP64 kernel values too 2.63e-7 and 3.32e-7).
 // 16 x 16 grid: 25.5 us of transforms -> 4.4; 16-cube: 58 -> 12.
 // Potentials come node-major; channel 3 (2-D) or 4 (3-D) is the charge with K1.
 constexpr int kDirect2 = 32, kDirect3 = 16;  // largest sides
@@ -106,7 +107,7 @@ constexpr int kDirectX = 16;                 // outputs of a 2-D work-group
 // A work-group per grid row y and kDirectX of its nodes x; thread (x, j) adds the
 // nodes of row y' = j.
 template <int XP>
-__global__ __launch_bounds__(kDirectX *XP) void conv_direct2_kernel(int ng, double hsq, const float *__restrict__ V,
+__global__ __launch_bounds__(kDirectX *XP) void conv_direct2_kernel(int ng, float hsq, const float *__restrict__ V,
                                                                    float4 *__restrict__ Phi) {
   __shared__ float4 vs[XP][XP];    // charges of (x', y')
   __shared__ double2 ks[XP][XP];   // K2, K1 at (|x - x'|, |y - y'|)
@@ -117,8 +118,8 @@ __global__ __launch_bounds__(kDirectX *XP) void conv_direct2_kernel(int ng, doub
   for (int t = threadIdx.x; t < XP * XP; t += kDirectX * XP) {
     const int xx = t % XP, jj = t / XP, e = jj * ng + xx;
     vs[jj][xx] = xx < ng && jj < ng ? make_float4(V[e], V[G + e], V[2 * G + e], 0.0f) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    const double k1 = 1.0 / (1.0 + hsq * (double)(xx * xx + (y - jj) * (y - jj)));
-    ks[jj][xx] = make_double2(k1 * k1, k1);
+    const float k1 = 1.0f / (1.0f + hsq * (float)(xx * xx + (y - jj) * (y - jj)));
+    ks[jj][xx] = make_double2((double)(k1 * k1), (double)k1);
   }
   __syncthreads();
   double4 acc = make_double4(0.0, 0.0, 0.0, 0.0);
@@ -165,17 +166,17 @@ __global__ __launch_bounds__(kDirectX *XP) void conv_direct2_kernel(int ng, doub
 // to the 16 outputs in registers, and the threads' sums are added across each
 // wave and then over the four waves.  Bound by the loads: a lane's row is lines of
 // its own, so it is read in 16-byte vectors (11.8 us with them, 18.7 without).
-__global__ __launch_bounds__(256) void conv_direct3_kernel(int ng, double hsq, const float *__restrict__ V,
+__global__ __launch_bounds__(256) void conv_direct3_kernel(int ng, float hsq, const float *__restrict__ V,
                                                            float *__restrict__ Phi) {
   constexpr int S = kDirect3, C = 5;
   __shared__ double red[4][S * C];
   const int yp = threadIdx.x % S, zp = threadIdx.x / S;
   const int y = blockIdx.x % ng, z = blockIdx.x / ng, G = ng * ng * ng;
   const bool in = yp < ng && zp < ng;
-  double k1[S];
+  float k1[S];
   const int r0 = (y - yp) * (y - yp) + (z - zp) * (z - zp);
 #pragma unroll
-  for (int d = 0; d < S; ++d) k1[d] = 1.0 / (1.0 + hsq * (double)(d * d + r0));
+  for (int d = 0; d < S; ++d) k1[d] = 1.0f / (1.0f + hsq * (float)(d * d + r0));
   double acc[S][C];
 #pragma unroll
   for (int x = 0; x < S; ++x)
@@ -205,10 +206,10 @@ __global__ __launch_bounds__(256) void conv_direct3_kernel(int ng, double hsq, c
     const float v[4] = {vr[0][xp], vr[1][xp], vr[2][xp], vr[3][xp]};
 #pragma unroll
     for (int x = 0; x < S; ++x) {
-      const double k = k1[x > xp ? x - xp : xp - x], kk = k * k;
+      const float k = k1[x > xp ? x - xp : xp - x], kk = k * k;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) acc[x][c] = fma(kk, (double)v[c], acc[x][c]);
-      acc[x][4] = fma(k, (double)v[0], acc[x][4]);
+      for (int c = 0; c < 4; ++c) acc[x][c] = fma((double)kk, (double)v[c], acc[x][c]);
+      acc[x][4] = fma((double)k, (double)v[0], acc[x][4]);
     }
   }
   // across the wave: halves exchanged until 16 groups of four lanes hold 5 sums
@@ -271,7 +272,7 @@ int launch_conv(hipStream_t s, const GridParams &g, int zdirect, const float *V,
                 const ConvBuffers &b, bool node_major) {
   SGT_CHECK(g.L <= kMaxL && g.L >= 2 * g.ng - 1 && fft_smooth(g.L), SGTSNE_ERR_ARG,
             "FFT length %d invalid for ng %d", g.L, g.ng);
-  const double hsq = (double)g.hgrid * (double)g.hgrid;
+  const float hsq = (float)(g.hgrid * g.hgrid);
   if (node_major && g.d == 2 && g.ng <= kDirect2) {
     float4 *Phi4 = reinterpret_cast<float4 *>(Phi);
     if (g.ng <= 16) conv_direct2_kernel<16><<<g.ng, 16 * kDirectX, 0, s>>>(g.ng, hsq, V, Phi4);
