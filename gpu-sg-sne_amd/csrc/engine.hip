@@ -129,6 +129,7 @@ struct sgtsne_ctx {
   // timing
   bool timing = true;
   bool stamped = false;  // the last publication carries an iteration's phase times
+  unsigned long long open_update = 0;  // start of the update whose end is still to come
   double ms_per_tick = 1e-5;  // of the device clock
   double acc_ms[7] = {0, 0, 0, 0, 0, 0, 0};
   double *time_info = nullptr;  // optional per-iteration output (sgtsne_run)
@@ -412,19 +413,30 @@ int wait_published(sgtsne_ctx *c) {
   }
 }
 
-// Adds the phase times of iteration `it`, published with its centring.
+// Ends the last phase (update and centring) of the iteration harvested last.
+void close_timing(sgtsne_ctx *c, unsigned long long end) {
+  if (!c->open_update) return;
+  const double t = (double)(end - c->open_update) * c->ms_per_tick;
+  c->open_update = 0;
+  c->acc_ms[4] += t;
+  c->acc_ms[5] += t;
+}
+
+// Adds the phase times of iteration `it`, published with its centring; that
+// phase itself ends after the publication, where the next iteration begins.
 void harvest_timing(sgtsne_ctx *c, int it) {
   if (!c->stamped) return;
   c->stamped = false;
-  double t[5];  // attr (and any wait for the host), s2g, conv, g2s, update(+centre)
-  for (int k = 0; k < 5; k++) t[k] = (double)(c->hs->stamp[k + 1] - c->hs->stamp[k]) * c->ms_per_tick;
+  close_timing(c, c->hs->stamp[0]);
+  double t[4];  // attr (and any wait for the host), s2g, conv, g2s
+  for (int k = 0; k < 4; k++) t[k] = (double)(c->hs->stamp[k + 1] - c->hs->stamp[k]) * c->ms_per_tick;
   c->acc_ms[0] += t[0];
   c->acc_ms[1] += t[1];
   c->acc_ms[2] += t[2];
   c->acc_ms[3] += t[3];
-  c->acc_ms[4] += t[4];
-  c->acc_ms[5] += t[0] + t[1] + t[2] + t[3] + t[4];
+  c->acc_ms[5] += t[0] + t[1] + t[2] + t[3];
   c->acc_ms[6] += 1;
+  c->open_update = c->hs->stamp[4];
   if (c->time_info) {
     double *ti = c->time_info + 7 * (size_t)(it - c->time_info_base);
     ti[0] = t[0];
@@ -598,8 +610,10 @@ int iterate(sgtsne_ctx *c) {
       (c->p.format == SGTSNE_FORMAT_CSR_SEG || c->p.format == SGTSNE_FORMAT_CSR))
     for (int r : kSpatialReorderIters)
       if (it == r) {
+        SGT_HIP(hipStreamSynchronize(c->stream));
         SGT_TRY(wait_published(c));
         harvest_timing(c, it - 1);
+        close_timing(c, c->hs->end);
         SGT_TRY(spatial_reorder(c));
         if (c->timing) SGT_TRY(launch_stamp(c->stream, c->sc, STAMP_END));  // not part of the iteration
       }
@@ -1248,11 +1262,15 @@ int sgtsne_ctx_step(sgtsne_ctx *c, int iters) {
   SGT_CHECK(c->have_P && c->have_Y, SGTSNE_ERR_STATE, "upload P and set Y before stepping");
   for (auto &v : c->acc_ms) v = 0.0;
   c->stamped = false;
+  c->open_update = 0;
   int st = SGTSNE_OK;
   if (c->timing && iters > 0) st = launch_stamp(c->stream, c->sc, STAMP_END);
   for (int k = 0; k < iters && st == SGTSNE_OK; k++) st = iterate(c);
   SGT_HIP(hipStreamSynchronize(c->stream));
-  if (st == SGTSNE_OK) harvest_timing(c, c->iter - 1);
+  if (st == SGTSNE_OK) {
+    harvest_timing(c, c->iter - 1);
+    close_timing(c, c->hs->end);
+  }
   c->stamped = false;
   return st;
 }

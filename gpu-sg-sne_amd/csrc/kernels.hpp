@@ -28,8 +28,9 @@ enum StampAt { STAMP_S2G = 0, STAMP_CONV = 1, STAMP_G2S = 2, STAMP_UPDATE = 3, S
 // queuing a copy and waiting for an event.
 struct HostScalars {
   double minv[4], maxv[4];
-  unsigned long long stamp[6];  // iteration start, the five above
+  unsigned long long stamp[5];  // iteration start, then the spread's, convolution's, gather's and update's
   unsigned long long seq;
+  unsigned long long end;       // end of the centring: not before the stream has passed it
 };
 
 // Partial-reduction workspace: one slot per block plus a ticket counter.

@@ -871,11 +871,8 @@ __global__ __launch_bounds__(kUpdBlock) void center_kernel(int n, float *__restr
       sc->maxv[a] = (double)(v.mx[a] - m[a]);
     }
     if (stamp) {
-      const unsigned long long t = wall_clock64();
       hs->stamp[0] = sc->stamp[STAMP_END];  // this iteration began where the last one ended
       for (int k = 0; k < 4; ++k) hs->stamp[1 + k] = sc->stamp[k];
-      hs->stamp[5] = t;
-      sc->stamp[STAMP_END] = t;
     }
     publish(hs, sc, seq);
   }
@@ -885,6 +882,13 @@ __global__ __launch_bounds__(kUpdBlock) void center_kernel(int n, float *__restr
 #pragma unroll
     for (int a = 0; a < D; ++a) y[a] -= m[a];
     store_pt<D>(Y, i, y);
+  }
+  // the end of the iteration: all the work-groups are in flight at once with the
+  // same work, so the first one's end is the kernel's within its last wave
+  if (stamp && blockIdx.x == 0 && threadIdx.x == 0) {
+    const unsigned long long t = wall_clock64();
+    sc->stamp[STAMP_END] = t;
+    hs->end = t;
   }
 }
 

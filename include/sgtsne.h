@@ -225,8 +225,10 @@ int sgtsne_ctx_repulsive_exact(sgtsne_ctx *ctx, float *Frep, double *Z, int layo
 
 /* Per-phase device time of the last sgtsne_ctx_step call, ms summed over
  * its iterations, from the device clock at the start of each phase's first
- * kernel: [0] attractive (with any wait for the host to size the grid), [1] S2G (incl. binning), [2] G2G (FFT
- * convolution), [3] G2S + forces, [4] update, [5] total, [6] iterations. */
+ * kernel and at the end of the centring: [0] attractive (with any wait for the
+ * host to size the grid, which small jobs have), [1] S2G (incl. binning), [2]
+ * G2G (convolution), [3] G2S + forces, [4] update and centring, [5] total,
+ * [6] iterations. */
 int sgtsne_ctx_timing(sgtsne_ctx *ctx, double *out7);
 
 /* Choice of the attractive-kernel autotuner (run at upload for the default
