@@ -2070,7 +2070,9 @@ __global__ void gather_points_kernel(int n, int ds, const int32_t *__restrict__ 
 namespace {
 
 // Exact kNN of the query slots [0, nq) (points qlist[slot], or all points),
-// in slabs of slots whose distances to every point take at most about 512 MB.
+// in slabs of slots whose distances to every point take 512 MB, or of 128 slots
+// where those take more (1.3 GB at 1.3M points: whole tiles, and work-groups
+// enough for the selection); when there is no memory for that, of fewer.
 // All points of a matrix that fits one slab (n <= 8192): mirrored tiles of 128
 // x 128.  Lists of up to 256 slots (rows the certificate left) take tiles of
 // 32 x 64, which spread a few rows over the device: 128 x 128 tiles would
@@ -2078,16 +2080,21 @@ namespace {
 // for the distances (20 G pair-dimensions/s of the 39 G/s FP64 issue allows)
 // and 0.17 ms for the selection (one work-group per 64 queries with serial
 // heaps: 37.1 ms); the 82 uncertified rows of a 20,011-point 50-D job 0.08 ms
-// (11.5 ms).
+// (11.5 ms).  Slabs of up to 64 slots take the small tiles too.
 constexpr size_t kKnnSlabBytes = (size_t)1 << 29;
 
 int knn_exact_rows(hipStream_t s, ScratchSource &src, const float *X, int n, int dim, int k, const int *qlist, int nq, int32_t *I,
                    double *D) {
-  const int slab = (int)std::min<int64_t>(nq, std::max<int64_t>(128, (int64_t)(kKnnSlabBytes / 8 / n) / 128 * 128));
-  const int mirror = !qlist && nq == n && slab == n;
-  const bool few = qlist && nq <= 256;
+  int slab = (int)std::min<int64_t>(nq, std::max<int64_t>(128, (int64_t)(kKnnSlabBytes / 8 / n) / 128 * 128));
   void *block = nullptr;
-  SGT_TRY(src.take(s, sizeof(double) * (size_t)slab * n, &block));
+  for (;;) {
+    const int st = src.take(s, sizeof(double) * (size_t)slab * n, &block);
+    if (st == SGTSNE_OK) break;
+    if (slab == 1) return st;
+    slab = slab > 64 ? (slab / 2 + 31) / 32 * 32 : slab / 2;
+  }
+  const int mirror = !qlist && nq == n && slab == n;
+  const bool few = slab <= 64 || (qlist && nq <= 256);
   double *dist = static_cast<double *>(block);
   auto rows = [&](int s0) -> int {
     const int m = std::min(slab, nq - s0);
