@@ -68,26 +68,33 @@ constexpr int kMarks = 16;                 // tick marks kept
 // The device blocks of a batch that come and go with its jobs: the front end's
 // workspaces, each P + P^T and the jobs' grids.  A block given back is kept for
 // the next job: it is handed out again on the stream it was given back on, or on
-// any once that stream has passed it, for requests of at least half its size.
+// any once that stream has passed it, for requests of at least half its size (from
+// kLargeBytes on, of eight ninths; a job's grid, which admission counts, only for
+// a grid of its size).
 // hipFreeAsync held the host 96 us on average here and hipMallocAsync 41
 // (5 pairs per job, more than half of the time to admit one of a few thousand
 // points): 16 jobs of 500-8000 points admitted, 8 iterations and removed 22.9 ->
-// 12.0 ms, 6 of 2000-20,000 in 3-D 14.7 -> 9.4.  At most kIdleBytes stay idle
-// beyond the next call; the rest goes back to the device's pool.
+// 12.0 ms, 6 of 2000-20,000 in 3-D 14.7 -> 9.4.  At most an eighth of the batch's
+// grid budget, and no more than kIdleBytes, stays idle beyond the next call; the
+// rest goes back to the device's pool.
 constexpr size_t kIdleBytes = (size_t)4 << 30;
+constexpr size_t kLargeBytes = (size_t)64 << 20;
 class BlockCache final : public ScratchSource {
  public:
-  int take(hipStream_t s, size_t bytes, void **p) override {
+  int take(hipStream_t s, size_t bytes, void **p) override { return take(s, bytes, false, p); }
+  // exact: a block of that size (in whole steps)
+  int take(hipStream_t s, size_t bytes, bool exact, void **p) {
     std::lock_guard<std::mutex> lock(mu_);
     *p = nullptr;
+    const size_t room = exact ? bytes : bytes + bytes / 8;  // of a new block: for slightly larger jobs
+    const size_t most = exact || bytes >= kLargeBytes ? room + kStep : 2 * (bytes + kStep);
     Block *best = nullptr;
     for (Block &b : blocks_)
-      if (b.idle && b.cap >= bytes && b.cap / 2 <= bytes + kStep && (!best || b.cap < best->cap) && passed(b, s))
-        best = &b;
+      if (b.idle && b.cap >= bytes && b.cap <= most && (!best || b.cap < best->cap) && passed(b, s)) best = &b;
     if (!best) {
-      trim_locked(kIdleBytes);
+      trim_locked(idle_limit);
       Block nb;
-      nb.cap = (bytes + bytes / 8 + kStep - 1) / kStep * kStep;  // room for slightly larger jobs
+      nb.cap = (room + kStep - 1) / kStep * kStep;
       hipError_t e = hipMallocAsync(&nb.p, nb.cap, s);
       if (e != hipSuccess) {  // give the idle blocks back and try once more
         (void)hipGetLastError();
@@ -130,10 +137,10 @@ class BlockCache final : public ScratchSource {
         return;
       }
   }
-  // Returns idle blocks beyond kIdleBytes to the device's pool.
+  // Returns idle blocks beyond the limit to the device's pool.
   void trim() {
     std::lock_guard<std::mutex> lock(mu_);
-    trim_locked(kIdleBytes);
+    trim_locked(idle_limit);
   }
   // Returns every block; the caller has drained the streams.
   void clear(hipStream_t s) {
@@ -146,6 +153,7 @@ class BlockCache final : public ScratchSource {
     idle_ = 0;
   }
   hipStream_t release_stream = nullptr;  // for blocks whose own stream has passed them
+  size_t idle_limit = kIdleBytes;
 
  private:
   static constexpr size_t kStep = (size_t)1 << 18;
@@ -850,7 +858,7 @@ int admit(sgtsne_batch *b, int n, int64_t nnz, const int32_t *rp_d, const int32_
   h.max_iter = max_iter;
   h.ng_cap = ng_cap;
   h.gbytes = gbytes;
-  SGT_TRY(b->blocks.take(b->stream, gbytes, &h.gmem));
+  SGT_TRY(b->blocks.take(b->stream, gbytes, true, &h.gmem));
   SGT_HIP(hipMemsetAsync(h.gmem, 0, vb, b->stream));  // the spread grid starts (and stays) zero
   char *gm = static_cast<char *>(h.gmem);
 
@@ -1132,6 +1140,7 @@ int sgtsne_batch_create(sgtsne_batch **out, const sgtsne_params *params, int max
   chk(hipStreamCreateWithFlags(&b->prep, hipStreamNonBlocking), "stream");
   b->copy = b->prep;
   b->blocks.release_stream = b->copy;
+  b->blocks.idle_limit = std::min(kIdleBytes, b->grid_budget / 8);
   for (hipEvent_t &e : b->marks) chk(hipEventCreateWithFlags(&e, hipEventDisableTiming), "event");
   chk(hipHostMalloc((void **)&b->stage, kStageBytes, hipHostMallocDefault), "pinned staging");
   chk(hipHostMalloc((void **)&b->fe_host, sizeof(int) * 3 * kFrontEnds, hipHostMallocDefault), "pinned counts");

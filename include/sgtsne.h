@@ -345,7 +345,9 @@ int sgtsne_locality_order(int n, const int32_t *rowptr, const int32_t *col, int3
 int sgtsne_copy_probe(int64_t bytes, int reps, double *ms_per_copy);
 
 /* Capacity: job slots (<= 1024), points and P_sym nonzeros of the arena, and
- * the byte budget of the per-job grid buffers (<= 0: 64 GiB). */
+ * the byte budget of the per-job grid buffers (<= 0: 64 GiB).  Beside the jobs
+ * the batch keeps device blocks of jobs that have left, and of their front ends,
+ * for the next ones: at most an eighth of that budget and 4 GiB. */
 int sgtsne_batch_create(sgtsne_batch **batch, const sgtsne_params *params, int max_jobs, int64_t max_points,
                         int64_t max_nnz, int64_t grid_budget_bytes);
 int sgtsne_batch_destroy(sgtsne_batch *batch);
