@@ -69,8 +69,8 @@ constexpr int kMarks = 16;                 // tick marks kept
 // workspaces, each P + P^T and the jobs' grids.  A block given back is kept for
 // the next job: it is handed out again on the stream it was given back on, or on
 // any once that stream has passed it, for requests of at least half its size (from
-// kLargeBytes on, of eight ninths; a job's grid, which admission counts, only for
-// a grid of its size).
+// kLargeBytes on, of eight ninths, and for a job's grid, which admission counts,
+// of a grid's size).
 // hipFreeAsync held the host 96 us on average here and hipMallocAsync 41
 // (5 pairs per job, more than half of the time to admit one of a few thousand
 // points): 16 jobs of 500-8000 points admitted, 8 iterations and removed 22.9 ->
@@ -82,12 +82,12 @@ constexpr size_t kLargeBytes = (size_t)64 << 20;
 class BlockCache final : public ScratchSource {
  public:
   int take(hipStream_t s, size_t bytes, void **p) override { return take(s, bytes, false, p); }
-  // exact: a block of that size (in whole steps)
-  int take(hipStream_t s, size_t bytes, bool exact, void **p) {
+  int take(hipStream_t s, size_t bytes, bool grid, void **p) {
     std::lock_guard<std::mutex> lock(mu_);
     *p = nullptr;
-    const size_t room = exact ? bytes : bytes + bytes / 8;  // of a new block: for slightly larger jobs
-    const size_t most = exact || bytes >= kLargeBytes ? room + kStep : 2 * (bytes + kStep);
+    const bool large = bytes >= kLargeBytes;
+    const size_t room = large && grid ? bytes : bytes + bytes / 8;  // of a new block: for slightly larger jobs
+    const size_t most = large ? room + kStep : 2 * (bytes + kStep);
     Block *best = nullptr;
     for (Block &b : blocks_)
       if (b.idle && b.cap >= bytes && b.cap <= most && (!best || b.cap < best->cap) && passed(b, s)) best = &b;
