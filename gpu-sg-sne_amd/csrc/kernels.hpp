@@ -200,7 +200,7 @@ int gpu_symmetrize(hipStream_t s, int n, int64_t nnz, const int32_t *rowptr_d,
 struct SymLong {  // its long rows, as the merge lists them
   int *cnt = nullptr;            // [0] rows sorted by a work-group, [1] hubs
   int32_t *mid = nullptr, *hub = nullptr;
-  double *part = nullptr;        // of each part of each hub: its sum,
+  double *part = nullptr;        // of each part of each hub: its sum (after the rows' sums),
   int32_t *end = nullptr;        // and where it ends in the merged row
 };
 struct SymPending {

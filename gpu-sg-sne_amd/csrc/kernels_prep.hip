@@ -1557,10 +1557,12 @@ constexpr int kSymRowLds = 8192;
 constexpr int kSymCols = 8192;       // columns of a hub's range (FP64 sums: 64 KB of LDS)
 constexpr int kSymBelow = 1 << 19;   // columns of one bitmap of those below a range (64 KB)
 
-__global__ void sym_len_kernel(int n, const int32_t *__restrict__ rowptr, int32_t *__restrict__ cnt, int *lcnt) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void sym_len_kernel(int n, const int32_t *__restrict__ rowptr, int32_t *__restrict__ cnt, SymLong L,
+                               int64_t parts) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i <= n) cnt[i] = i < n ? rowptr[i + 1] - rowptr[i] : 0;
-  if (i < 2) lcnt[i] = 0;
+  if (i < 2) L.cnt[i] = 0;
+  if (i < parts) L.part[i] = 0.0;
 }
 
 // pos[t] = place of entry t in the merged row of its column.  A work-group takes
@@ -1723,8 +1725,12 @@ __global__ __launch_bounds__(64) void sym_merge_kernel(int n, const int32_t *__r
     const int o = off[r], len = off[r + 1] - o;
     if (len > kSymRow) {
       if (threadIdx.x == 0) {
-        if (len <= kSymRowLds) L.mid[atomicAdd(L.cnt, 1)] = r;
-        else L.hub[atomicAdd(L.cnt + 1, 1)] = r;
+        if (len <= kSymRowLds) {
+          L.mid[atomicAdd(L.cnt, 1)] = r;
+        } else {
+          L.hub[atomicAdd(L.cnt + 1, 1)] = r;
+          rowsum[r] = 0.0;  // its sum is in its parts
+        }
       }
       continue;
     }
@@ -1865,17 +1871,6 @@ __global__ __launch_bounds__(1024) void sym_merge_hub_kernel(int n, const int32_
       if (j == parts - 1) ucnt[row] = start;
     }
     __syncthreads();
-  }
-}
-
-// A hub's sum from its parts, one wave each.
-__global__ __launch_bounds__(64) void sym_hub_sum_kernel(int n, double *__restrict__ rowsum, SymLong L) {
-  const int parts = hub_parts(n);
-  for (int h = blockIdx.x; h < L.cnt[1]; h += gridDim.x) {
-    double s = 0.0;
-    for (int j = threadIdx.x; j < parts; j += 64) s += L.part[(int64_t)h * parts + j];
-    s = wave_sum(s);
-    if (threadIdx.x == 0) rowsum[L.hub[h]] = s;
   }
 }
 
@@ -2345,12 +2340,12 @@ int sym_begin(hipStream_t s, ScratchSource &src, int n, int64_t nnz, const int32
   SGT_CHECK(m2 < (int64_t)INT_MAX, SGTSNE_ERR_ARG, "2*nnz exceeds the int32 range");
   size_t tb = 0, tr = 0;
   SGT_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, (int32_t *)nullptr, (int32_t *)nullptr, n + 1, s));
-  SGT_HIP(hipcub::DeviceReduce::Sum(nullptr, tr, (double *)nullptr, (double *)nullptr, n, s));
   // the longest merged row: its own entries and, from each other row, one per
   // column (any number if P may hold an entry more than once)
   const int64_t longest = std::min<int64_t>(m2, max_row > 0 ? (int64_t)n + max_row : m2);
   const bool mids = longest > kSymRow, hubs = longest > kSymRowLds;
   const int64_t nhub = hubs ? m2 / kSymRowLds : 0, parts = hub_parts(n);
+  SGT_HIP(hipcub::DeviceReduce::Sum(nullptr, tr, (double *)nullptr, (double *)nullptr, (int)(n + nhub * parts), s));
   int32_t *cnt, *off, *pos, *mcol, *ucnt, *rp;
   unsigned long long *ent;
   double *mval, *rowsum, *total;
@@ -2367,11 +2362,11 @@ int sym_begin(hipStream_t s, ScratchSource &src, int n, int64_t nnz, const int32
     L.cnt = c.take<int>(2);
     L.mid = c.take<int32_t>(mids ? m2 / kSymRow : 0);
     L.hub = c.take<int32_t>(nhub);
-    L.part = c.take<double>(nhub * parts);
     L.end = c.take<int32_t>(nhub * parts);
     ucnt = c.take<int32_t>((size_t)n + 1);
     rp = c.take<int32_t>((size_t)n + 1);
-    rowsum = c.take<double>(n);
+    rowsum = c.take<double>((size_t)n + nhub * parts);
+    L.part = rowsum + n;
     total = c.take<double>(1);
     tmp = c.take<char>(std::max(tb, tr));
     if (pass == 0) SGT_TRY(src.take(s, c.off, &sp->ws));
@@ -2385,7 +2380,7 @@ int sym_begin(hipStream_t s, ScratchSource &src, int n, int64_t nnz, const int32
   sp->total = total;
   sp->runs_host = runs_host;
   const int wblocks = std::min(div_up(n, 4), 16384);  // four waves of a row each
-  sym_len_kernel<<<div_up((int64_t)n + 1, 256), 256, 0, s>>>(n, rowptr_d, cnt, L.cnt);
+  sym_len_kernel<<<div_up(std::max<int64_t>((int64_t)n + 1, nhub * parts), 256), 256, 0, s>>>(n, rowptr_d, cnt, L, nhub * parts);
   SGT_LAUNCH_CHECK();
   if (nnz > 0) sym_place_kernel<<<(int)std::min<int64_t>((nnz + kPlaceRun - 1) / kPlaceRun, 65536), 256, 0, s>>>(nnz, col_d, cnt, pos);
   SGT_LAUNCH_CHECK();
@@ -2403,11 +2398,9 @@ int sym_begin(hipStream_t s, ScratchSource &src, int n, int64_t nnz, const int32
     sym_merge_hub_kernel<<<(int)std::min<int64_t>(nhub * parts, 256), 1024,
                            sizeof(double) * kSymCols + (kSymCols + kSymBelow) / 8, s>>>(n, off, ent, mcol, mval, ucnt, L);
     SGT_LAUNCH_CHECK();
-    sym_hub_sum_kernel<<<(int)std::min<int64_t>(nhub, 256), 64, 0, s>>>(n, rowsum, L);
-    SGT_LAUNCH_CHECK();
   }
   SGT_HIP(hipcub::DeviceScan::ExclusiveSum(tmp, tb, ucnt, rp, n + 1, s));  // ucnt[n] is not read into rp
-  SGT_HIP(hipcub::DeviceReduce::Sum(tmp, tr, rowsum, total, n, s));
+  SGT_HIP(hipcub::DeviceReduce::Sum(tmp, tr, rowsum, total, (int)(n + nhub * parts), s));  // rows, then hubs' parts
   SGT_HIP(hipMemcpyAsync(runs_host, rp + n, sizeof(int), hipMemcpyDeviceToHost, s));
   return SGTSNE_OK;
 }
