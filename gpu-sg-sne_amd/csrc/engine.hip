@@ -1498,6 +1498,42 @@ int sgtsne_copy_probe(int64_t bytes, int reps, double *ms_per_copy) {
   return st;
 }
 
+}  // extern "C"
+
+namespace {
+
+// The arrays of one call on a stream of its own: a block of the device's pool,
+// which keeps it for the next call (retain_pool_memory), or from kPooledBytes on
+// one by hipMalloc, whose time such a call does not notice, given back at its end.
+struct CallBlock {
+  static constexpr size_t kPooledBytes = (size_t)256 << 20;
+  void *p = nullptr;
+  bool pooled = false;
+  int take(hipStream_t s, size_t bytes) {
+    pooled = bytes < kPooledBytes;
+    if (!pooled) return alloc_dev(&p, bytes);
+    if (hipMallocAsync(&p, bytes, s) != hipSuccess) {
+      (void)hipGetLastError();
+      set_error("hipMallocAsync(%zu) failed", bytes);
+      p = nullptr;
+      return SGTSNE_ERR_NOMEM;
+    }
+    return SGTSNE_OK;
+  }
+  void release(hipStream_t s) {  // after the work queued on s so far
+    if (p && pooled) (void)hipFreeAsync(p, s);
+    if (p && !pooled) {
+      (void)hipStreamSynchronize(s);
+      (void)hipFree(p);
+    }
+    p = nullptr;
+  }
+};
+
+}  // namespace
+
+extern "C" {
+
 int sgtsne_knn(const float *X, int n, int dim, int k, int method, int32_t *I, double *D, int *fallback_rows) {
   SGT_CHECK(X && I && D, SGTSNE_ERR_ARG, "NULL argument");
   SGT_CHECK(method >= SGTSNE_KNN_AUTO && method <= SGTSNE_KNN_FILTERED, SGTSNE_ERR_ARG, "unknown kNN method %d", method);
@@ -1508,19 +1544,14 @@ int sgtsne_knn(const float *X, int n, int dim, int k, int method, int32_t *I, do
   float *Xd = nullptr;
   double *Dd = nullptr;
   int32_t *Id = nullptr;
-  void *ws = nullptr;
+  CallBlock ws;
   int st = SGTSNE_OK;
   for (int pass = 0; pass < 2 && !st; ++pass) {
-    Carve c{static_cast<char *>(ws)};
+    Carve c{static_cast<char *>(ws.p)};
     Xd = c.take<float>(nx);
     Dd = c.take<double>(no);
     Id = c.take<int32_t>(no);
-    if (pass == 0 && hipMallocAsync(&ws, c.off, s) != hipSuccess) {
-      (void)hipGetLastError();
-      set_error("hipMallocAsync(%zu) failed", c.off);
-      ws = nullptr;
-      st = SGTSNE_ERR_NOMEM;
-    }
+    if (pass == 0) st = ws.take(s, c.off);
   }
   if (!st && hipMemcpyAsync(Xd, X, nx * sizeof(float), hipMemcpyHostToDevice, s) != hipSuccess) {
     set_error("copy of X failed");
@@ -1532,7 +1563,7 @@ int sgtsne_knn(const float *X, int n, int dim, int k, int method, int32_t *I, do
     set_error("copy of kNN result failed");
     st = SGTSNE_ERR_HIP;
   }
-  if (ws) (void)hipFreeAsync(ws, s);
+  ws.release(s);
   if (hipStreamSynchronize(s) != hipSuccess && !st) {
     set_error("kNN kernel failed");
     st = SGTSNE_ERR_HIP;
@@ -1604,18 +1635,13 @@ int sgtsne_perplexity_equalize(const int32_t *I, const double *D, int n, int k, 
   SGT_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
   double *Dd = nullptr;
   float *vd = nullptr;
-  void *ws = nullptr;
+  CallBlock ws;
   int st = SGTSNE_OK;
   for (int pass = 0; pass < 2 && !st; ++pass) {
-    Carve c{static_cast<char *>(ws)};
+    Carve c{static_cast<char *>(ws.p)};
     Dd = c.take<double>((size_t)n * (k + 1));
     vd = c.take<float>((size_t)n * k);
-    if (pass == 0 && hipMallocAsync(&ws, c.off, s) != hipSuccess) {
-      (void)hipGetLastError();
-      set_error("hipMallocAsync(%zu) failed", c.off);
-      ws = nullptr;
-      st = SGTSNE_ERR_NOMEM;
-    }
+    if (pass == 0) st = ws.take(s, c.off);
   }
   if (!st && hipMemcpyAsync(Dd, D, (size_t)n * (k + 1) * sizeof(double), hipMemcpyHostToDevice, s) != hipSuccess) {
     set_error("copy of D failed");
@@ -1635,7 +1661,7 @@ int sgtsne_perplexity_equalize(const int32_t *I, const double *D, int n, int k, 
     set_error("copy of P failed");
     st = SGTSNE_ERR_HIP;
   }
-  if (ws) (void)hipFreeAsync(ws, s);
+  ws.release(s);
   if (hipStreamSynchronize(s) != hipSuccess && !st) {
     set_error("perplexity kernel failed");
     st = SGTSNE_ERR_HIP;

@@ -18,6 +18,6 @@ def _run(sg, tmp_path, name):
     assert r.returncode == 0, r.stdout + r.stderr
 
 
-@pytest.mark.parametrize("name", ["lost_blocks", "block_cache_oom", "sticky_error", "exact_rows_memory", "block_cache_bounds"])
+@pytest.mark.parametrize("name", ["lost_blocks", "block_cache_oom", "sticky_error", "exact_rows_memory", "block_cache_bounds", "pool_kept"])
 def test_host_program(sg, tmp_path, name):
     _run(sg, tmp_path, name)
