@@ -434,7 +434,8 @@ def run_config(sg, P, d, steps, warmup, fmt="CSR_SEG", reorder=2, cpu_seconds=15
     roof_c = {"bound": "hbm", "achieved": round(ach_c, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
               "frac": round(ach_c / HBM_PEAK_GBS, 5), "bytes_per_iteration": bytes_c, "grid_side": grid,
               "ms_per_iteration": round(t_c * 1e3, 5),
-              "kernels": "spread + grid reduce, FFT convolution passes, gather + forces + Z partials"}
+              "kernels": "spread + grid reduce, convolution (direct sum on grids of side <= 32 in 2-D, 16 in 3-D, else FFT "
+                         "passes), gather + forces + Z partials"}
 
     out = {"n": n, "d": d, "format": fmt.lower(), "nnz_sym": nnz, "ms_per_iter": round(ms_per_step, 4),
            "timed_iterations": [it0, it0 + steps - 1], "phases_ms": {k2: round(v, 5) for k2, v in phases.items()},

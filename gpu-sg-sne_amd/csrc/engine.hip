@@ -1081,10 +1081,8 @@ int sgtsne_ctx_create(sgtsne_ctx **out, const sgtsne_params *params) {
   }
   c->rw.max_blocks = 65536 + 4096;
   if ((st = alloc_dev((void **)&c->rw.part, sizeof(double) * 8 * c->rw.max_blocks))) return fail(st);
-  if ((st = alloc_dev((void **)&c->rw.ticket, sizeof(unsigned) * 4))) return fail(st);
   if ((st = alloc_dev((void **)&c->sc, sizeof(DevScalars)))) return fail(st);
-  if (hipMemset(c->rw.ticket, 0, sizeof(unsigned) * 4) != hipSuccess ||
-      hipMemset(c->sc, 0, sizeof(DevScalars)) != hipSuccess) {
+  if (hipMemset(c->sc, 0, sizeof(DevScalars)) != hipSuccess) {
     set_error("hipMemset failed");
     return fail(SGTSNE_ERR_HIP);
   }
@@ -1115,7 +1113,6 @@ int sgtsne_ctx_destroy(sgtsne_ctx *c) {
   free_spread_order(c);
   free_dev(c->perm_d);
   free_dev(c->rw.part);
-  free_dev(c->rw.ticket);
   free_dev(c->sc);
   free_dev(c->V);
   free_dev(c->Phi);

@@ -33,10 +33,9 @@ struct HostScalars {
   unsigned long long end;       // end of the centring: not before the stream has passed it
 };
 
-// Partial-reduction workspace: one slot per block plus a ticket counter.
+// Partial-reduction workspace: one slot per block.
 struct RedWork {
   double *part;       // [max_blocks * 8]
-  unsigned *ticket;   // single counter, reset by the last block
   int max_blocks;
 };
 
@@ -111,8 +110,8 @@ constexpr int kSpreadBins = 32768;
 bool s2g_takes_order(const GridParams &g, int mode);
 int launch_spread_order(hipStream_t s, const GridParams &g, int n, const float *Y, int2 *key, int *cnt, int32_t *ord);
 int64_t s2g_scratch_need(const GridParams &g, int n, int mode = 0);
-// Frep and the partials of Z; *nz receives how many there are: launch_update
-// adds them up itself, launch_finalize_z puts their sum into sc->Z for others.
+// Frep and the partials of Z; *nz receives how many there are:
+// launch_update_center adds them up itself, launch_finalize_z puts their sum into sc->Z for others.
 int launch_g2s_force(hipStream_t s, const GridParams &g, int n, const float *Y, const float *Phi,
                      float *Frep, int zdirect, RedWork rw, int *nz, DevScalars *stamp = nullptr,
                      const int32_t *ord = nullptr);

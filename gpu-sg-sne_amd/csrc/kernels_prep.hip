@@ -566,9 +566,6 @@ __global__ __launch_bounds__(256) void knn_cell_kernel(const float *__restrict__
   if (threadIdx.x < kKnnMaxCells && hist[threadIdx.x]) atomicAdd(&cnt[threadIdx.x], hist[threadIdx.x]);
 }
 
-// Sort keys: the cell in the top 6 bits (when cells are given), then the
-// Morton code of a 3-D projection of the centred point.
-
 // One work-group per reference tile of kFiltR slots.  The sorted points of each
 // cell start a fresh tile; the slots left over are padding (id -1).  Slot ids,
 // the id -> slot map, the tile's centred points and its bounding sphere: centre =
@@ -831,7 +828,7 @@ __global__ __launch_bounds__(256) void knn_filter_kernel(const float *__restrict
 // The same filter with the candidate lists in LDS (lists of up to kF2MaxKp).
 // A work-group of four waves owns NQ = 16 QB queries of one frame.  The
 // references come in tiles of 64, 16 to a wave, stored in the order the matrix
-// instructions take them (knn_ref_scatter_kernel), so a wave reads its B
+// instructions take them (knn_tile_kernel), so a wave reads its B
 // operands straight from memory, coalesced, the next tile's in flight, and
 // nothing is staged or transposed in LDS.
 //
@@ -1180,7 +1177,6 @@ __global__ __launch_bounds__(64 * NW) void knn_filter_list_kernel(const RefTiles
   }
 }
 
-// Step counts (dimensions / 4, rounded up) the filters are built for.
 // The block-centred arrays of the LDS-list filter (kp <= kF2MaxKp).
 struct BlockCentred {
   const float *Xq;         // queries in slot order, centred at their block's mean
@@ -2072,7 +2068,8 @@ namespace {
 // x 128.  Lists of up to 256 slots (rows the certificate left) take tiles of
 // 32 x 64, which spread a few rows over the device: 128 x 128 tiles would
 // leave n / 128 work-groups.  Measured: 6007 points of 784 dimensions 1.40 ms
-// for the distances (20 G pair-dimensions/s of the 39 G/s FP64 issue allows)
+// for the distances (10 T pair-dimensions/s, of two FP64 operations each: half of
+// the 39 T operations/s that FP64 issue allows)
 // and 0.17 ms for the selection (one work-group per 64 queries with serial
 // heaps: 37.1 ms); the 82 uncertified rows of a 20,011-point 50-D job 0.08 ms
 // (11.5 ms).  Slabs of up to 64 slots take the small tiles too.
