@@ -111,7 +111,8 @@ __global__ __launch_bounds__(kDirectX *XP) void conv_direct2_kernel(int ng, floa
                                                                    float4 *__restrict__ Phi) {
   __shared__ float4 vs[XP][XP];    // charges of (x', y')
   __shared__ double2 ks[XP][XP];   // K2, K1 at (|x - x'|, |y - y'|)
-  __shared__ double4 red[XP][kDirectX];
+  constexpr int WAVES = kDirectX * XP / 64;
+  __shared__ double4 red[WAVES][kDirectX];
   const int xl = threadIdx.x % kDirectX, j = threadIdx.x / kDirectX, x = blockIdx.y * kDirectX + xl, y = blockIdx.x;
   const int G = ng * ng;
 #pragma unroll
@@ -132,33 +133,26 @@ __global__ __launch_bounds__(kDirectX *XP) void conv_direct2_kernel(int ng, floa
     acc.z = fma(k.x, (double)v.z, acc.z);
     acc.w = fma(k.y, (double)v.x, acc.w);
   }
-  red[j][xl] = acc;
-  __syncthreads();
-  // rows y' added in order, eight of them per thread, then the eighths
-  if (j < XP / 8) {
-    double4 s = red[8 * j][xl];
+  // a wave's four rows y' added across it, then the waves' sums in order
 #pragma unroll
-    for (int k = 1; k < 8; ++k) {
-      const double4 t = red[8 * j + k][xl];
-      s.x += t.x;
-      s.y += t.y;
-      s.z += t.z;
-      s.w += t.w;
-    }
-    red[8 * j][xl] = s;
+  for (int o = kDirectX; o < 64; o <<= 1) {
+    acc.x += __shfl_xor(acc.x, o, 64);
+    acc.y += __shfl_xor(acc.y, o, 64);
+    acc.z += __shfl_xor(acc.z, o, 64);
+    acc.w += __shfl_xor(acc.w, o, 64);
   }
+  if ((threadIdx.x & 63) < kDirectX) red[threadIdx.x >> 6][xl] = acc;
   __syncthreads();
   if (j == 0 && x < ng) {
-    double4 s = red[0][xl];
 #pragma unroll
-    for (int k = 1; k < XP / 8; ++k) {
-      const double4 t = red[8 * k][xl];
-      s.x += t.x;
-      s.y += t.y;
-      s.z += t.z;
-      s.w += t.w;
+    for (int k = 1; k < WAVES; ++k) {
+      const double4 t = red[k][xl];
+      acc.x += t.x;
+      acc.y += t.y;
+      acc.z += t.z;
+      acc.w += t.w;
     }
-    Phi[y * ng + x] = make_float4((float)s.x, (float)s.y, (float)s.z, (float)s.w);
+    Phi[y * ng + x] = make_float4((float)acc.x, (float)acc.y, (float)acc.z, (float)acc.w);
   }
 }
 
