@@ -604,16 +604,21 @@ int spatial_reorder(sgtsne_ctx *c) {
   return SGTSNE_OK;
 }
 
-int iterate(sgtsne_ctx *c) {
+// last: the host reads the iteration's end (the stream drains behind it).
+int iterate(sgtsne_ctx *c, bool last) {
   const int it = c->iter;
   if (c->p.reorder >= 2 && c->n >= kSpatialReorderMin &&
       (c->p.format == SGTSNE_FORMAT_CSR_SEG || c->p.format == SGTSNE_FORMAT_CSR))
     for (int r : kSpatialReorderIters)
       if (it == r) {
-        SGT_HIP(hipStreamSynchronize(c->stream));
         SGT_TRY(wait_published(c));
         harvest_timing(c, it - 1);
-        close_timing(c, c->hs->end);
+        if (c->open_update) {  // its end, from the device: the re-order belongs to no iteration
+          unsigned long long end = 0;
+          SGT_HIP(hipMemcpyAsync(&end, &c->sc->stamp[STAMP_END], sizeof(end), hipMemcpyDeviceToHost, c->stream));
+          SGT_HIP(hipStreamSynchronize(c->stream));
+          close_timing(c, end);
+        }
         SGT_TRY(spatial_reorder(c));
         if (c->timing) SGT_TRY(launch_stamp(c->stream, c->sc, STAMP_END));  // not part of the iteration
       }
@@ -661,7 +666,8 @@ int iterate(sgtsne_ctx *c) {
     SGT_TRY(st);
   }
   SGT_TRY(launch_update_center(c->stream, c->d, c->n, c->Y, c->uY, c->gains, c->Fattr, c->Frep, (float)alpha,
-                               (float)momentum, (float)eta, nz, c->rw, c->sc, c->hs, ++c->seq, c->timing));
+                               (float)momentum, (float)eta, nz, c->rw, c->sc, c->hs, ++c->seq,
+                               !c->timing ? 0 : last ? 2 : 1));
   c->stamped = c->timing;
   c->iter++;
   return SGTSNE_OK;
@@ -1262,7 +1268,7 @@ int sgtsne_ctx_step(sgtsne_ctx *c, int iters) {
   c->open_update = 0;
   int st = SGTSNE_OK;
   if (c->timing && iters > 0) st = launch_stamp(c->stream, c->sc, STAMP_END);
-  for (int k = 0; k < iters && st == SGTSNE_OK; k++) st = iterate(c);
+  for (int k = 0; k < iters && st == SGTSNE_OK; k++) st = iterate(c, k == iters - 1);
   SGT_HIP(hipStreamSynchronize(c->stream));
   if (st == SGTSNE_OK) {
     harvest_timing(c, c->iter - 1);

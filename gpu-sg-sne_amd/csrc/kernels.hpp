@@ -30,7 +30,7 @@ struct HostScalars {
   double minv[4], maxv[4];
   unsigned long long stamp[5];  // iteration start, then the spread's, convolution's, gather's and update's
   unsigned long long seq;
-  unsigned long long end;       // end of the centring: not before the stream has passed it
+  unsigned long long end;       // end of the centring that was asked for it, once the stream has passed it
 };
 
 // Partial-reduction workspace: one slot per block.
@@ -118,10 +118,11 @@ int launch_g2s_force(hipStream_t s, const GridParams &g, int n, const float *Y, 
 int launch_finalize_z(hipStream_t s, int nz, int n, RedWork rw, DevScalars *sc);
 int launch_finalize_kl(hipStream_t s, int nblocks, RedWork rw, DevScalars *sc);
 // The update of Y from the forces and the nz partials of Z, then the centring
-// of the new Y with its min / max into sc and hs (two kernels).
+// of the new Y with its min / max into sc and hs (two kernels).  stamp: 1 with the
+// phase times, 2 with the iteration's end in hs too.
 int launch_update_center(hipStream_t s, int d, int n, float *Y, float *uY, float *gains, const float *Fattr,
                          const float *Frep, float alpha, float momentum, float eta, int nz, RedWork rw,
-                         DevScalars *sc, HostScalars *hs, unsigned long long seq, bool stamp);
+                         DevScalars *sc, HostScalars *hs, unsigned long long seq, int stamp);
 // Device clock now, into sc->stamp[at].
 int launch_stamp(hipStream_t s, DevScalars *sc, int at);
 int launch_rep_exact(hipStream_t s, int d, int n, const float *Y, float *Frep, RedWork rw,

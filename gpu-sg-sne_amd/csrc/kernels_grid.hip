@@ -884,11 +884,12 @@ __global__ __launch_bounds__(kUpdBlock) void center_kernel(int n, float *__restr
     store_pt<D>(Y, i, y);
   }
   // the end of the iteration: all the work-groups are in flight at once with the
-  // same work, so the first one's end is the kernel's within its last wave
-  if (stamp && blockIdx.x == 0 && threadIdx.x == 0) {
+  // same work, so the last one's end is about the kernel's (the first one also
+  // publishes).  To the host only where it asks for it.
+  if (stamp && blockIdx.x == gridDim.x - 1 && threadIdx.x == blockDim.x - 64) {
     const unsigned long long t = wall_clock64();
     sc->stamp[STAMP_END] = t;
-    hs->end = t;
+    if (stamp > 1) hs->end = t;
   }
 }
 
@@ -1346,7 +1347,7 @@ int launch_get_points(hipStream_t s, int d, int n, const float *in, int layout, 
 
 int launch_update_center(hipStream_t s, int d, int n, float *Y, float *uY, float *gains, const float *Fattr,
                          const float *Frep, float alpha, float momentum, float eta, int nz, RedWork rw,
-                         DevScalars *sc, HostScalars *hs, unsigned long long seq, bool stamp) {
+                         DevScalars *sc, HostScalars *hs, unsigned long long seq, int stamp) {
   const int tpb = upd_threads(n), blocks = upd_blocks(n);
   SGT_CHECK(nz >= 1 && nz <= 2048 && rw.max_blocks >= 2048 + kMaxBoxParts, SGTSNE_ERR_STATE, "%d partials of Z", nz);
   BoxPart *box = box_parts(rw);
