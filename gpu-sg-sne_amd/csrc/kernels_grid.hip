@@ -884,9 +884,10 @@ __global__ __launch_bounds__(kUpdBlock) void center_kernel(int n, float *__restr
     store_pt<D>(Y, i, y);
   }
   // the end of the iteration: all the work-groups are in flight at once with the
-  // same work, so the last one's end is about the kernel's (the first one also
-  // publishes).  To the host only where it asks for it.
-  if (stamp && blockIdx.x == gridDim.x - 1 && threadIdx.x == blockDim.x - 64) {
+  // same work, so the first one's end is the kernel's within its last wave (and its
+  // first thread has read the last iteration's).  To the host only where it asks
+  // for it.
+  if (stamp && blockIdx.x == 0 && threadIdx.x == 0) {
     const unsigned long long t = wall_clock64();
     sc->stamp[STAMP_END] = t;
     if (stamp > 1) hs->end = t;
