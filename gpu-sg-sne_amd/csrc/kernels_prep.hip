@@ -302,6 +302,178 @@ __global__ __launch_bounds__(kKnnThreads) void knn_select_kernel(const double *_
   }
 }
 
+// ---- exact kNN without a block of distances ---------------------------------
+// Work-group tile: 64 queries x 32 references; 256 threads each own a 4x2
+// micro-tile of (query, reference) distances, summed as in knn_dist_kernel.
+// Candidates below a query's current worst key (distance, index) are queued in
+// LDS and merged by one thread per query into a max-heap of k entries kept in
+// global memory.  No distance is stored, so the cost per pair does not grow with n
+// (200,000 points of 5 dimensions, k = 10: 1.9 ps).  Queries are the slots
+// [s0, s0 + nq); heaps are indexed by slot - s0.
+constexpr int kHeapQ = 64;
+constexpr int kHeapR = 32;
+
+__device__ __forceinline__ bool key_less(double da, int ia, double db, int ib) {
+  return da < db || (da == db && ia < ib);
+}
+
+__global__ __launch_bounds__(kKnnThreads) void knn_heap_kernel(const float *__restrict__ X, int n,
+                                                          int dim, int k, double *__restrict__ hd,
+                                                          int *__restrict__ hi, const int *__restrict__ qlist,
+                                                          int s0, int nq) {
+  __shared__ double qs[kKnnDC][kHeapQ + 1];
+  __shared__ double rs[kKnnDC][kHeapR + 1];
+  __shared__ double qd[kHeapQ][kHeapR];
+  __shared__ int qi[kHeapQ][kHeapR];
+  __shared__ int qcnt[kHeapQ];
+  __shared__ double thr_d[kHeapQ];
+  __shared__ int thr_i[kHeapQ];
+  __shared__ int qid[kHeapQ];  // point of each slot (-1: none)
+
+  const int q0 = blockIdx.x * kHeapQ;
+  const int tid = threadIdx.x;
+  const int tq = tid >> 4;   // 0..15 -> queries tq*4 .. tq*4+3
+  const int tr = tid & 15;   // 0..15 -> references tr + 16*c
+  if (tid < kHeapQ) {
+    qcnt[tid] = 0;
+    thr_d[tid] = INFINITY;
+    thr_i[tid] = INT_MAX;
+    const int slot = q0 + tid;
+    qid[tid] = slot < nq ? (qlist ? qlist[s0 + slot] : s0 + slot) : -1;
+    if (slot < nq)
+      for (int e = 0; e < k; ++e) {
+        hd[(size_t)slot * k + e] = INFINITY;
+        hi[(size_t)slot * k + e] = INT_MAX;
+      }
+  }
+  __syncthreads();
+
+  for (int r0 = 0; r0 < n; r0 += kHeapR) {
+    double acc[4][2];
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) acc[a][b] = 0.0;
+    for (int l0 = 0; l0 < dim; l0 += kKnnDC) {
+      for (int idx = tid; idx < kKnnDC * kHeapQ; idx += kKnnThreads) {
+        const int qq = idx / kKnnDC, ll = idx % kKnnDC;
+        const int q = qid[qq], l = l0 + ll;
+        qs[ll][qq] = (q >= 0 && l < dim) ? X[(size_t)q * dim + l] : 0.0;
+        if (qq < kHeapR) {
+          const int r = r0 + qq;
+          rs[ll][qq] = (r < n && l < dim) ? X[(size_t)r * dim + l] : 0.0;
+        }
+      }
+      __syncthreads();
+      const int lc = min(kKnnDC, dim - l0);
+      for (int ll = 0; ll < lc; ++ll) {
+        double qv[4], rv[2];
+#pragma unroll
+        for (int a = 0; a < 4; ++a) qv[a] = qs[ll][tq * 4 + a];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) rv[b] = rs[ll][tr + 16 * b];
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+          for (int b = 0; b < 2; ++b) {
+            const double df = qv[a] - rv[b];
+            acc[a][b] = fma(df, df, acc[a][b]);
+          }
+      }
+      __syncthreads();
+    }
+    // queue candidates
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      const int ql = tq * 4 + a;
+      const int q = qid[ql];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const int r = r0 + tr + 16 * b;
+        if (q >= 0 && r < n && r != q && key_less(acc[a][b], r, thr_d[ql], thr_i[ql])) {
+          const int pos = atomicAdd(&qcnt[ql], 1);
+          qd[ql][pos] = acc[a][b];
+          qi[ql][pos] = r;
+        }
+      }
+    }
+    __syncthreads();
+    // merge queued candidates into the heaps (one thread per query)
+    if (tid < kHeapQ) {
+      const int slot = q0 + tid;
+      const int cnt = qcnt[tid];
+      if (slot < nq && cnt > 0) {
+        double *H = hd + (size_t)slot * k;
+        int *HI = hi + (size_t)slot * k;
+        double rd = H[0];
+        int ri = HI[0];
+        for (int c = 0; c < cnt; ++c) {
+          const double cd = qd[tid][c];
+          const int ci = qi[tid][c];
+          if (!key_less(cd, ci, rd, ri)) continue;
+          int pos = 0;
+          for (;;) {
+            const int l = 2 * pos + 1, rr = l + 1;
+            int m = -1;
+            double md = cd;
+            int mi = ci;
+            if (l < k && key_less(md, mi, H[l], HI[l])) { m = l; md = H[l]; mi = HI[l]; }
+            if (rr < k && key_less(md, mi, H[rr], HI[rr])) { m = rr; md = H[rr]; mi = HI[rr]; }
+            if (m < 0) break;
+            H[pos] = md;
+            HI[pos] = mi;
+            pos = m;
+          }
+          H[pos] = cd;
+          HI[pos] = ci;
+          rd = H[0];
+          ri = HI[0];
+        }
+        thr_d[tid] = rd;
+        thr_i[tid] = ri;
+      }
+      qcnt[tid] = 0;
+    }
+    __syncthreads();
+  }
+}
+
+// Heap -> ascending rows with the point itself first (slots as knn_heap_kernel).
+__global__ void knn_heap_rows_kernel(int s0, int nq, int k, double *__restrict__ hd, int *__restrict__ hi,
+                                     const int *__restrict__ qlist, int32_t *__restrict__ I,
+                                     double *__restrict__ D) {
+  const int slot = blockIdx.x * blockDim.x + threadIdx.x;
+  if (slot >= nq) return;
+  const int q = qlist ? qlist[s0 + slot] : s0 + slot;
+  double *H = hd + (size_t)slot * k;
+  int *HI = hi + (size_t)slot * k;
+  int32_t *Iq = I + (size_t)q * (k + 1);
+  double *Dq = D + (size_t)q * (k + 1);
+  Iq[0] = q;
+  Dq[0] = 0.0;
+  for (int e = k - 1; e >= 0; --e) {
+    Iq[1 + e] = HI[0];
+    Dq[1 + e] = H[0];
+    const double cd = H[e];
+    const int ci = HI[e];
+    int pos = 0;
+    for (;;) {
+      const int l = 2 * pos + 1, rr = l + 1;
+      int m = -1;
+      double md = cd;
+      int mi = ci;
+      if (l < e && key_less(md, mi, H[l], HI[l])) { m = l; md = H[l]; mi = HI[l]; }
+      if (rr < e && key_less(md, mi, H[rr], HI[rr])) { m = rr; md = H[rr]; mi = HI[rr]; }
+      if (m < 0) break;
+      H[pos] = md;
+      HI[pos] = mi;
+      pos = m;
+    }
+    H[pos] = cd;
+    HI[pos] = ci;
+  }
+}
+
 // ---- kNN through an FP32 matrix-core filter --------------------------------
 // The exact distances above cost two FP64 vector operations per (pair,
 // dimension).  Here the squared distances of the mean-centred points, rounded
@@ -2060,6 +2232,54 @@ __global__ void gather_points_kernel(int n, int ds, const int32_t *__restrict__ 
 
 namespace {
 
+constexpr size_t kKnnSlabBytes = (size_t)1 << 29;
+
+// Whether the rows of nq slots come sooner from heaps.  Picoseconds per pair,
+// fitted to 10,000-400,000 points of 2-200 dimensions, k = 10-1000: a slab's rows
+// get fewer as n grows, so the selection leaves the device idle (one work-group
+// per row; 24 ps at 200,000 points); the heaps' tiles are small (0.14 against
+// 0.06 per dimension), their merges serial (k per row), and a list of few slots
+// does not fill the device with work-groups of 64.  All rows, slabs / heaps:
+// 20,000 x 50, k = 90 8.3 / 16.8 ms; 60,000 x 5, k = 90 41.6 / 31.1; 200,000 x
+// 50, k = 90 1091 / 424; 200,000 x 5, k = 10 957 / 78; 100,000 x 200, k = 90
+// 262 / 380; 200,000 x 50, k = 1000 1355 / 1849.  The rule took the slower
+// by more than 15 % only below 30,000 points (k below 30 in few dimensions) and
+// at 60,000 x 20, k = 90.
+bool knn_heaps_better(int n, int dim, int k, int nq) {
+  const double slabs = 2.5 + 1.05e-4 * n + 0.064 * dim;
+  const double heaps = std::max(1.2 + 0.144 * dim + 4500.0 * k / n, (55000.0 + 4800.0 * dim) / nq);
+  return heaps < slabs;
+}
+
+// knn_exact_rows by heaps, in groups of slots whose heaps take 512 MB (of fewer
+// when there is no memory for that).
+int knn_heap_rows(hipStream_t s, ScratchSource &src, const float *X, int n, int dim, int k, const int *qlist, int nq, int32_t *I,
+                  double *D) {
+  const size_t row = (sizeof(double) + sizeof(int)) * (size_t)k;
+  int slab = (int)std::min<int64_t>(nq, (int64_t)(kKnnSlabBytes / row));
+  void *block = nullptr;
+  for (;;) {
+    const int st = src.take(s, row * slab, &block);
+    if (st == SGTSNE_OK) break;
+    if (slab == 1) return st;
+    slab = div_up(slab, 2);
+  }
+  double *hd = static_cast<double *>(block);
+  int *hi = reinterpret_cast<int *>(hd + (size_t)slab * k);
+  auto rows = [&](int s0) -> int {
+    const int m = std::min(slab, nq - s0);
+    knn_heap_kernel<<<div_up(m, kHeapQ), kKnnThreads, 0, s>>>(X, n, dim, k, hd, hi, qlist, s0, m);
+    SGT_LAUNCH_CHECK();
+    knn_heap_rows_kernel<<<div_up(m, 256), 256, 0, s>>>(s0, m, k, hd, hi, qlist, I, D);
+    SGT_LAUNCH_CHECK();
+    return SGTSNE_OK;
+  };
+  int st = SGTSNE_OK;
+  for (int s0 = 0; s0 < nq && !st; s0 += slab) st = rows(s0);
+  src.give(s, block);
+  return st;
+}
+
 // Exact kNN of the query slots [0, nq) (points qlist[slot], or all points),
 // in slabs of slots whose distances to every point take 512 MB, or of 128 slots
 // where those take more (1.3 GB at 1.3M points: whole tiles, and work-groups
@@ -2072,11 +2292,11 @@ namespace {
 // the 39 T operations/s that FP64 issue allows)
 // and 0.17 ms for the selection (one work-group per 64 queries with serial
 // heaps: 37.1 ms); the 82 uncertified rows of a 20,011-point 50-D job 0.08 ms
-// (11.5 ms).  Slabs of up to 64 slots take the small tiles too.
-constexpr size_t kKnnSlabBytes = (size_t)1 << 29;
-
+// (11.5 ms).  Slabs of up to 64 slots take the small tiles too.  Where heaps are
+// the faster way to the same rows (knn_heaps_better) they are taken.
 int knn_exact_rows(hipStream_t s, ScratchSource &src, const float *X, int n, int dim, int k, const int *qlist, int nq, int32_t *I,
                    double *D) {
+  if (knn_heaps_better(n, dim, k, nq)) return knn_heap_rows(s, src, X, n, dim, k, qlist, nq, I, D);
   int slab = (int)std::min<int64_t>(nq, std::max<int64_t>(128, (int64_t)(kKnnSlabBytes / 8 / n) / 128 * 128));
   void *block = nullptr;
   for (;;) {
